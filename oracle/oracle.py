@@ -29,8 +29,8 @@ _REF = None
 def build_ref():
     """Compile the reference's own table-spec sources (src/storage/specs.cc with its headers)
     behind oracle/ref_specs_glue.cc into oracle/_ref/libref_specs.so.  Needs the reference tree;
-    returns False where it is absent (then a library built earlier is used if it is there)."""
-    if not os.path.isdir(REFERENCE_ROOT):
+    returns False where it is absent or empty (then a library built earlier is used if it is there)."""
+    if not os.path.isfile(os.path.join(REFERENCE_ROOT, "src", "storage", "specs.cc")):
         return False
     subprocess.run(["make", "-s", "-B", "-C", _HERE, "ref"], check=True)
     return True

@@ -67,3 +67,10 @@ def test_baseline_tables_equal_the_reference(ref):
     mujoco = [([17], REF_CODE["float32"]), ([6], REF_CODE["float32"]), ([1], REF_CODE["float32"]),
               ([1], REF_CODE["uint8"])]
     assert ref.ref_table_nbytes(64, 4096, mujoco) == 97 * 64 * 4096
+
+
+def test_build_ref_without_the_reference_sources(oracle, tmp_path, monkeypatch):
+    """An absent or empty reference tree is no build error: nothing is compiled."""
+    for root in (tmp_path / "absent", tmp_path):
+        monkeypatch.setattr(oracle, "REFERENCE_ROOT", str(root))
+        assert oracle.build_ref() is False
