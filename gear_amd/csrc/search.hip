@@ -1,11 +1,11 @@
 // Batched upper_bound of draws in an inclusive prefix array (+ importance weights), and the
 // one-call batch sampler (search + ranking sort + split into window arguments), gfx950.
 //
-// One thread per draw, one wave per workgroup.  The first levels of the search touch the same few
-// prefix entries for every draw, so they are served by the caches; the search is latency-bound
-// (a chain of log8(n) + 1 dependent load steps), which is why all draws of a batch run concurrently
-// and spread over many CUs.
+// The search is latency-bound (a chain of dependent loads), so the lanes of a group look for one
+// draw together and a batch spreads over many CUs.
 #include <math.h>
+
+#include <type_traits>
 
 #include "radix_sort.hpp"
 
@@ -13,31 +13,65 @@ namespace gearhip {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kSearchBlock = 64;  // one wave per workgroup: spreads the divergent probes over many CUs
 
-// First index with p[i] > t (n when there is none).  The search is kArity-ary: kArity - 1
-// independent probes per step cut the chain of dependent loads from log2(n) to log_kArity(n)
-// steps, and the chain, not the number of loads, is what a batch of draws waits for.  The last
-// step reads the whole remaining stretch at once.
-constexpr int kArity = 8;  // 16 probes per step measured slower (4.5 against 4.05 us at n = 1e6)
-constexpr int kArityShift = 3;
+// ---- search -------------------------------------------------------------------------------------
+// First index with p[i] > t (n when there is none), worked out by kLanes neighbouring lanes
+// together.  What a batch of draws waits for is the chain of dependent loads, so a step cuts the
+// remaining range [lo, hi) into kLanes parts with one probe per lane: part j ends before
+// lo + (range * (j + 1) >> log2(kLanes)), and the answer lies behind as many parts as have a last
+// entry <= t -- counted, so that a larger t never gives a smaller answer, whatever the array holds.
+// More lanes make the chain shorter (log_kLanes(n) steps) and the loads more: kLanes cache lines a
+// draw and step, and a CU asks for one a clock.  us per batch of draws in a prefix of 1e6 / 1e7
+// entries (back to back; a launch alone takes 3.1), by lanes; 1 = seven probes by one lane:
+//     draws        1              8             16             32
+//       512   4.5 / 5.9     3.7 / 4.5      3.3 / 3.9      3.3 / 3.6
+//      4096   4.9 / 6.2     4.1 / 4.9      3.7 / 4.6      3.9 / 5.3
+//     16384   5.3 / 8.9     4.9 / 7.9      6.2 / 9.9      7.6 / 13
+//     65536  10.1 / 20.6   11.2 / 21.2    16.3 / 28.5    22.7 / 41
+// hence 16 lanes up to 4096 draws, 8 up to 32768, 1 beyond (search_lanes).
+inline int search_lanes(int64_t num) { return num <= 4096 ? 16 : num <= 32768 ? 8 : 1; }
 
+template <int kLanes>
+struct Probe {
+  int64_t lo, range;
+  static constexpr int kShift = kLanes == 16 ? 4 : 3;
+  static_assert(1 << kShift == kLanes, "a power of two");
+  __device__ __forceinline__ int64_t parts_end(int j) const { return (range * (j + 1)) >> kShift; }
+  // the entry that lane `sub` of the group looks at (empty parts at the front look at the first one)
+  template <typename T>
+  __device__ __forceinline__ T load(const T *__restrict__ p, int sub) const {
+    const int64_t e = parts_end(sub);
+    return p[lo + (e > 0 ? e - 1 : 0)];
+  }
+  template <typename T>
+  __device__ __forceinline__ void narrow(T v, T t, int sub) {
+    const uint64_t le = wave_ballot(parts_end(sub) == 0 || v <= t);
+    const int first_lane = (int)(threadIdx.x & (kWave - 1)) & ~(kLanes - 1);
+    const int c = __popc((uint32_t)(le >> first_lane) & ((1u << kLanes) - 1u));
+    const int64_t begin = c > 0 ? parts_end(c - 1) : 0;
+    range = c < kLanes ? parts_end(c) - 1 - begin : 0;
+    lo += begin;
+  }
+};
+
+// One lane alone: seven independent probes per step, and the last step reads the whole remaining
+// stretch at once.
 template <typename T>
-__device__ __forceinline__ int64_t upper_bound_dev(const T *__restrict__ p, int64_t n, T t) {
+__device__ __forceinline__ int64_t lane_search(const T *__restrict__ p, int64_t n, T t) {
+  constexpr int kArity = 8, kArityShift = 3;
   int64_t lo = 0, hi = n;  // the answer lies in [lo, hi]
   while (hi - lo >= kArity) {
     const int64_t step = (hi - lo) >> kArityShift;
     T v[kArity - 1];
 #pragma unroll
     for (int j = 0; j < kArity - 1; ++j) v[j] = p[lo + step * (j + 1) - 1];
-    int c = 0;  // probes are ordered, so the ones <= t form a prefix
+    int c = 0;
 #pragma unroll
     for (int j = 0; j < kArity - 1; ++j) c += (v[j] <= t) ? 1 : 0;
     const int64_t base = lo + step * c;
     if (c < kArity - 1) hi = lo + step * (c + 1) - 1;
     lo = base;
   }
-  // fewer than kArity candidates left: p[lo .. hi) in one go (entries are ordered)
   T v[kArity - 1];
 #pragma unroll
   for (int j = 0; j < kArity - 1; ++j) v[j] = lo + j < hi ? p[lo + j] : t;
@@ -47,29 +81,104 @@ __device__ __forceinline__ int64_t upper_bound_dev(const T *__restrict__ p, int6
   return lo + c;
 }
 
-__global__ __launch_bounds__(kSearchBlock) void search_f64_kernel(
-    const double *__restrict__ prefix, int64_t n, const float *__restrict__ u, int64_t num,
-    int unit, int64_t *__restrict__ idx_out, const float *__restrict__ priorities, double beta,
-    double *__restrict__ wraw, double *__restrict__ block_max) {
-  const int64_t j = (int64_t)blockIdx.x * kSearchBlock + threadIdx.x;
-  const double total = prefix[n - 1];
+// The whole search, by kLanes lanes, for a target that depends on the array's last entry, the
+// total (it is what the group's last lane looks at in the first step).
+template <int kLanes, typename T, typename Target>
+__device__ __forceinline__ int64_t group_search(const T *__restrict__ p, int64_t n, int sub,
+                                                const Target &target) {
+  int64_t at;
+  if constexpr (kLanes == 1) {
+    at = lane_search(p, n, target(p[n - 1]));
+  } else {
+    Probe<kLanes> s{0, n};
+    T v = s.load(p, sub);
+    const T t = target(__shfl(v, kLanes - 1, kLanes));
+    s.narrow(v, t, sub);
+    while (s.range > 0) {
+      v = s.load(p, sub);
+      s.narrow(v, t, sub);
+    }
+    at = s.lo;
+  }
+  return at < n ? at : n - 1;
+}
+
+// The targets of a batch of draws, and keys of the same order to rank the draws by.
+// fp64 prefix: fp32 draws, in [0, 1) (unit) or targets already.  A NaN target compares with nothing
+// and finds entry 0, so a NaN draw has the lowest key (and whatever a NaN or infinite total makes
+// NaN lies next to draws that find entry 0 too).
+struct DrawF64 {
+  typedef double type;
+  typedef uint32_t key_type;
+  const double *prefix;
+  int64_t n;
+  const float *u;
+  int unit;
+  __device__ __forceinline__ double target(int64_t j, double total) const {
+    return unit ? (double)u[j] * total : (double)u[j];
+  }
+  __device__ __forceinline__ uint32_t key(int64_t j, double total) const {
+    const float f = u[j];
+    const uint32_t b = __float_as_uint(f);
+    uint32_t k = b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
+    if (unit && total < 0.0) k = ~k;  // (priorities are not negative; the order holds all the same)
+    return f == f ? k : 0u;
+  }
+};
+// int64 prefix (a sampler over lengths): doubles in [0, 1) (unit) or int64 targets.
+struct DrawI64 {
+  typedef int64_t type;
+  typedef int64_t key_type;
+  const int64_t *prefix;
+  int64_t n;
+  const void *u;
+  int unit;
+  __device__ __forceinline__ int64_t target(int64_t j, int64_t total) const {
+    return unit ? (int64_t)floor(static_cast<const double *>(u)[j] * (double)total)
+                : static_cast<const int64_t *>(u)[j];
+  }
+  __device__ __forceinline__ int64_t key(int64_t j, int64_t total) const { return target(j, total); }
+};
+
+template <int kLanes, typename Draw>
+__global__ __launch_bounds__(kBlock) void search_kernel(Draw draw, int64_t num,
+                                                        int64_t *__restrict__ idx_out) {
+  const int64_t j = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kLanes;
+  const int sub = threadIdx.x & (kLanes - 1);
+  if (j >= num) return;
+  const int64_t i = group_search<kLanes>(
+      draw.prefix, draw.n, sub, [&](typename Draw::type total) { return draw.target(j, total); });
+  if (sub == 0) idx_out[j] = i;
+}
+
+// The same with the raw importance weights (N * p / total) ** -beta of the found entries and their
+// maximum per workgroup.
+template <int kLanes>
+__global__ __launch_bounds__(kBlock) void search_weights_kernel(
+    DrawF64 draw, int64_t num, int64_t *__restrict__ idx_out, const float *__restrict__ priorities,
+    double beta, double *__restrict__ wraw, double *__restrict__ block_max) {
+  __shared__ double wmax[kBlock / kWave];
+  const int64_t j = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kLanes;
+  const int sub = threadIdx.x & (kLanes - 1);
   double w = 0.0;
   if (j < num) {
-    const double t = unit ? (double)u[j] * total : (double)u[j];
-    int64_t i = upper_bound_dev<double>(prefix, n, t);
-    if (i > n - 1) i = n - 1;
-    idx_out[j] = i;
-    if (priorities != nullptr) {
-      w = pow((double)n * (double)priorities[i] / total, -beta);
+    double total = 0.0;
+    const int64_t i = group_search<kLanes>(draw.prefix, draw.n, sub, [&](double last) {
+      total = last;
+      return draw.target(j, last);
+    });
+    w = pow((double)draw.n * (double)priorities[i] / total, -beta);
+    if (sub == 0) {
+      idx_out[j] = i;
       wraw[j] = w;
     }
   }
-  if (priorities != nullptr) {
-    // workgroup (= wave) maximum of the raw weights (weights are positive, padding lanes hold 0)
-    double m = w;
-    for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, kWave));
-    if (threadIdx.x == 0) block_max[blockIdx.x] = m;
-  }
+  // (weights are positive, lanes without a draw hold 0)
+  for (int off = 32; off >= kLanes; off >>= 1) w = fmax(w, __shfl_xor(w, off, kWave));
+  if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x / kWave] = w;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    block_max[blockIdx.x] = fmax(fmax(wmax[0], wmax[1]), fmax(wmax[2], wmax[3]));
 }
 
 __global__ __launch_bounds__(kBlock) void normalise_kernel(const double *__restrict__ wraw,
@@ -85,72 +194,6 @@ __global__ __launch_bounds__(kBlock) void normalise_kernel(const double *__restr
   m = fmax(fmax(wmax[0], wmax[1]), fmax(wmax[2], wmax[3]));
   const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (j < num) out[j] = (float)(wraw[j] / m);
-}
-
-// The draw of an int64 prefix (a sampler over lengths): u holds doubles in [0, 1) (unit) or
-// int64 targets.
-struct DrawI64 {
-  const int64_t *prefix;
-  int64_t n;
-  const void *u;
-  int unit;
-  __device__ __forceinline__ int64_t operator()(int64_t j) const {
-    const int64_t total = prefix[n - 1];
-    int64_t t;
-    if (unit)
-      t = (int64_t)floor(static_cast<const double *>(u)[j] * (double)total);
-    else
-      t = static_cast<const int64_t *>(u)[j];
-    const int64_t i = upper_bound_dev<int64_t>(prefix, n, t);
-    return i > n - 1 ? n - 1 : i;
-  }
-};
-__global__ __launch_bounds__(kSearchBlock) void search_i64_kernel(DrawI64 draw, int64_t num,
-                                                                  int64_t *__restrict__ idx_out) {
-  const int64_t j = (int64_t)blockIdx.x * kSearchBlock + threadIdx.x;
-  if (j < num) idx_out[j] = draw(j);
-}
-
-// The ranking sort of radix_sort.hpp over the found indices, fused with the split into window
-// arguments.  Used for prefixes shorter than 2^32 entries (the compare key is the index as
-// uint32_t); longer ones take the radix sort.
-struct Split {
-  int64_t *sorted_out;
-  int64_t T, modulo;
-  int64_t *idxs, *tss, *lens;
-  // the entry at sorted place `rank` is the flat index `mine` (below 2^32)
-  __device__ __forceinline__ void operator()(int64_t rank, int64_t f) const {
-    const uint32_t mine = (uint32_t)f;
-    if (sorted_out) sorted_out[rank] = f;
-    if (T > 0) {
-      int64_t traj, ts;
-      if (T <= 0xffffffffll && modulo <= 0xffffffffll) {
-        uint32_t f32 = mine;  // 32-bit division is a fraction of the 64-bit one
-        if (modulo > 0) f32 %= (uint32_t)modulo;
-        const uint32_t q = f32 / (uint32_t)T;
-        traj = q;
-        ts = f32 - q * (uint32_t)T;
-      } else {
-        if (modulo > 0) f %= modulo;
-        traj = f / T;
-        ts = f - traj * T;
-      }
-      idxs[rank] = traj;
-      tss[rank] = ts;
-      if (lens) lens[rank] = ts + 1;
-    }
-  }
-};
-
-__global__ __launch_bounds__(radix::kRankBlock) void rank_split_kernel(
-    const int64_t *__restrict__ raw, int num, Split split) {
-  typedef uint32_t K;
-  __shared__ radix::RankSmem<K> sm;
-  K mine;
-  const uint32_t rank = radix::block_rank<K>(sm, num, [&](int j) { return (K)raw[j]; }, &mine);
-  const int e = (int)blockIdx.x * kWave + (threadIdx.x & 63);
-  if (threadIdx.x >= kWave || e >= num) return;
-  split((int64_t)rank, (int64_t)mine);
 }
 
 __global__ __launch_bounds__(kBlock) void split_sorted_kernel(const int64_t *__restrict__ flat,
@@ -170,6 +213,44 @@ __global__ __launch_bounds__(kBlock) void split_sorted_kernel(const int64_t *__r
   if (lens) lens[j] = ts + 1;
 }
 
+// What happens with the entry that takes place r of the sorted batch.  resolve() needs the entry
+// only and runs while the place is still being worked out; store() writes the results.
+
+// Split of a flat step index into window arguments.
+struct Split {
+  int64_t *sorted_out;
+  int64_t T, modulo;
+  int64_t *idxs, *tss, *lens;
+  struct Resolved {
+    int64_t flat, traj, ts;
+  };
+  __device__ __forceinline__ Resolved resolve(int64_t f) const {
+    Resolved r{f, 0, 0};
+    if (T > 0) {
+      if (f <= 0xffffffffll && T <= 0xffffffffll && modulo <= 0xffffffffll) {
+        uint32_t f32 = (uint32_t)f;  // 32-bit division is a fraction of the 64-bit one
+        if (modulo > 0) f32 %= (uint32_t)modulo;
+        const uint32_t q = f32 / (uint32_t)T;
+        r.traj = q;
+        r.ts = f32 - q * (uint32_t)T;
+      } else {
+        if (modulo > 0) f %= modulo;
+        r.traj = f / T;
+        r.ts = f - r.traj * T;
+      }
+    }
+    return r;
+  }
+  __device__ __forceinline__ void store(int64_t rank, const Resolved &r) const {
+    if (sorted_out) sorted_out[rank] = r.flat;
+    if (T > 0) {
+      idxs[rank] = r.traj;
+      tss[rank] = r.ts;
+      if (lens) lens[rank] = r.ts + 1;
+    }
+  }
+};
+
 // What the loader does with a sorted batch of positions before it can gather
 // (gear/loader/offline_loader.py:168-177 and the samplers' concat_indices[draws],
 // gear/sampler/global_sampler.py:131,172,196), for the entry at sorted place r with position p:
@@ -187,39 +268,164 @@ struct Lookup {
   const double *start_u = nullptr;
   int64_t window = 0;
   int64_t *starts = nullptr;
-  __device__ __forceinline__ void operator()(int64_t r, int64_t p) const {
-    int64_t g = p;
-    if (index_table) g = (p >= 0 && p < index_n) ? index_table[p] : 0;
-    const int64_t l = g - index_offset;
-    if (sampled) sampled[r] = g;
-    if (local) local[r] = l;
-    const int64_t len = (lengths_table && l >= 0 && l < lengths_n) ? lengths_table[l] : 0;
-    if (lens) lens[r] = len;
+  struct Resolved {
+    int64_t global, len;
+  };
+  __device__ __forceinline__ Resolved resolve(int64_t p) const {
+    Resolved v;
+    v.global = p;
+    if (index_table) v.global = (p >= 0 && p < index_n) ? index_table[p] : 0;
+    const int64_t l = v.global - index_offset;
+    v.len = (lengths_table && l >= 0 && l < lengths_n) ? lengths_table[l] : 0;
+    return v;
+  }
+  __device__ __forceinline__ void store(int64_t r, const Resolved &v) const {
+    if (sampled) sampled[r] = v.global;
+    if (local) local[r] = v.global - index_offset;
+    if (lens) lens[r] = v.len;
     if (starts) {
-      const int64_t room = len - (window - 1);
+      const int64_t room = v.len - (window - 1);
       starts[r] = room > 0 ? (int64_t)floor(start_u[r] * (double)room) : 0;
     }
   }
 };
 
-// The ranking sort over a batch of positions (at most kRankMax, each below 2^32), with the
-// look-ups of the sorted entry done by the thread that ranked it: one launch instead of a sort
-// and two gathers.
-__global__ __launch_bounds__(radix::kRankBlock) void rank_lookup_kernel(
-    const int64_t *__restrict__ raw, int num, Lookup look) {
-  typedef uint32_t K;
-  __shared__ radix::RankSmem<K> sm;
-  K mine;
-  const uint32_t rank = radix::block_rank<K>(sm, num, [&](int j) { return (K)raw[j]; }, &mine);
-  const int e = (int)blockIdx.x * kWave + (threadIdx.x & 63);
-  if (threadIdx.x >= kWave || e >= num) return;
-  look((int64_t)rank, (int64_t)mine);
+// ---- a sorted batch in one launch ---------------------------------------------------------------
+// Draws are searched and put in order at the same time: a larger target never finds a smaller
+// entry, so the place of a draw in the sorted batch is the place of its TARGET among the targets,
+// and nothing has to be found before the sort can begin.  A workgroup takes kPlaced draws.  Its
+// first waves search them (kLanes lanes each) and do the look-ups; the other waves keep the keys
+// of ALL draws of the batch (at most kRankMax) in LDS and count the smaller ones, and the equal
+// ones at smaller positions (the place after a stable sort); both meet in LDS at the end.
+// 2048 draws in 1e6 / 1e7 entries: 4.3 / 4.9 us (a launch alone 3.1), where a search launch and a
+// ranking launch took 6.8 + 6.3 in the same stream; 8 or 32 lanes a draw: 4.6 / 5.2, 4.4 / 5.0.
+// At 4096 draws (5.1 us) the counting -- kPlaced * num compares a CU -- begins to be what bounds it.
+constexpr int kPlaced = 16;
+constexpr int kPlaceThreads = 1024;
+constexpr int kPlaceWaves = kPlaceThreads / kWave;
+
+template <typename K>
+struct PlaceSmem {
+  __align__(16) K keys[radix::kRankMax];
+  uint32_t part[kPlaceWaves][kPlaced];
+};
+
+// Fills sm.keys, padded to a multiple of kPlaced with the largest key there is: it lies behind
+// every draw and no key exceeds it, so it is never counted.
+template <typename K, typename Key>
+__device__ __forceinline__ void fill_keys(PlaceSmem<K> &sm, int num, const Key &key) {
+  constexpr K kTop = (K)-1 > (K)0 ? ~(K)0 : (K)(((uint64_t)1 << (8 * sizeof(K) - 1)) - 1);
+  const int padded = (num + kPlaced - 1) & ~(kPlaced - 1);
+  for (int j = threadIdx.x; j < padded; j += kPlaceThreads) sm.keys[j] = j < num ? key(j) : kTop;
+}
+
+// The share of rank wave `rw` (of `rws`) in the places of the workgroup's draws: lane = (slice of
+// the keys, draw).  A chunk of kPlaced keys lies before, behind or exactly at the workgroup's own.
+template <typename K>
+__device__ __forceinline__ void count_before(PlaceSmem<K> &sm, int num, int rw, int rws) {
+  typedef K K4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & (kWave - 1);
+  const int d = lane & (kPlaced - 1), slice = lane / kPlaced;
+  const int own = blockIdx.x, chunks = (num + kPlaced - 1) / kPlaced;
+  const K mine = sm.keys[own * kPlaced + d];
+  const K4 *keys4 = reinterpret_cast<const K4 *>(sm.keys) + slice;
+  uint32_t c = 0;
+  int ch = rw;
+#pragma unroll 4
+  for (; ch < own; ch += rws) {
+    const K4 k = keys4[ch * (kPlaced / 4)];
+    c += (k[0] <= mine) + (k[1] <= mine) + (k[2] <= mine) + (k[3] <= mine);
+  }
+  if (ch == own) {
+    const K4 k = keys4[ch * (kPlaced / 4)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c += k[i] < mine || (k[i] == mine && slice * 4 + i < d);
+    ch += rws;
+  }
+#pragma unroll 4
+  for (; ch < chunks; ch += rws) {
+    const K4 k = keys4[ch * (kPlaced / 4)];
+    c += (k[0] < mine) + (k[1] < mine) + (k[2] < mine) + (k[3] < mine);
+  }
+  c += (uint32_t)__shfl_xor((int)c, kPlaced, kWave);
+  c += (uint32_t)__shfl_xor((int)c, 2 * kPlaced, kWave);
+  if (lane < kPlaced) sm.part[rw][d] = c;
+}
+
+template <int kLanes, typename Draw, typename Emit>
+__global__ __launch_bounds__(kPlaceThreads) void place_draws_kernel(Draw draw, int num, Emit emit) {
+  typedef typename Draw::type T;
+  constexpr int kFindWaves = kPlaced * kLanes / kWave;
+  constexpr int kRankWaves = kPlaceWaves - kFindWaves;
+  static_assert(kRankWaves > 0, "somebody ranks");
+  __shared__ PlaceSmem<typename Draw::key_type> sm;
+  __shared__ typename Emit::Resolved found[kPlaced];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int sub = tid & (kLanes - 1), d = tid / kLanes;  // of the search
+  // the first probes go out together with the loads of the draws
+  Probe<kLanes> s{0, draw.n};
+  T v = T(0);
+  if (wave < kFindWaves) v = s.load(draw.prefix, sub);
+  const T total = draw.prefix[draw.n - 1];
+  fill_keys(sm, num, [&](int j) { return draw.key(j, total); });
+  if (wave < kFindWaves) {
+    const int e = (int)blockIdx.x * kPlaced + d;
+    const T t = draw.target(e < num ? e : num - 1, total);
+    __syncthreads();
+    s.narrow(v, t, sub);
+    while (s.range > 0) {
+      v = s.load(draw.prefix, sub);
+      s.narrow(v, t, sub);
+    }
+    if (sub == 0) found[d] = emit.resolve(s.lo < draw.n ? s.lo : draw.n - 1);
+  } else {
+    __syncthreads();
+    count_before(sm, num, wave - kFindWaves, kRankWaves);
+  }
+  __syncthreads();
+  if (tid < kPlaced && (int)blockIdx.x * kPlaced + tid < num) {
+    uint32_t rank = 0;
+#pragma unroll
+    for (int w = 0; w < kRankWaves; ++w) rank += sm.part[w][tid];
+    emit.store((int64_t)rank, found[tid]);
+  }
+}
+
+// The same for positions that are given (no search): sorted and looked up.
+template <typename Emit>
+__global__ __launch_bounds__(kPlaceThreads) void place_positions_kernel(
+    const int64_t *__restrict__ raw, int num, Emit emit) {
+  __shared__ PlaceSmem<int64_t> sm;
+  const int tid = threadIdx.x;
+  const int e = (int)blockIdx.x * kPlaced + tid;
+  const bool mine = tid < kPlaced && e < num;
+  typename Emit::Resolved found = {};
+  if (mine) found = emit.resolve(raw[e]);
+  fill_keys(sm, num, [&](int j) { return raw[j]; });
+  __syncthreads();
+  count_before(sm, num, __builtin_amdgcn_readfirstlane(tid / kWave), kPlaceWaves);
+  __syncthreads();
+  if (mine) {
+    uint32_t rank = 0;
+#pragma unroll
+    for (int w = 0; w < kPlaceWaves; ++w) rank += sm.part[w][tid];
+    emit.store((int64_t)rank, found);
+  }
+}
+
+template <typename Draw, typename Emit>
+int place_draws(const Draw &draw, int64_t num, const Emit &emit, hipStream_t st) {
+  place_draws_kernel<16>
+      <<<dim3((unsigned)ceil_div64(num, kPlaced)), dim3(kPlaceThreads), 0, st>>>(draw, (int)num, emit);
+  GEARHIP_RETURN_IF_LAUNCH_FAILED();
+  return 0;
 }
 
 __global__ __launch_bounds__(kBlock) void lookup_kernel(const int64_t *__restrict__ positions,
                                                         int64_t num, Lookup look) {
   const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (j < num) look(j, positions[j]);
+  if (j < num) look.store(j, look.resolve(positions[j]));
 }
 
 struct SampleWs {
@@ -236,10 +442,34 @@ SampleWs sample_ws(int64_t num) {
   return w;
 }
 
+int64_t search_blocks(int64_t num) { return ceil_div64(num * search_lanes(num), kBlock); }
+
+// calls f(std::integral_constant<int, lanes>) for the batch's number of lanes per draw
+template <typename F>
+void with_search_lanes(int64_t num, const F &f) {
+  const int lanes = search_lanes(num);
+  if (lanes == 16)
+    f(std::integral_constant<int, 16>{});
+  else if (lanes == 8)
+    f(std::integral_constant<int, 8>{});
+  else
+    f(std::integral_constant<int, 1>{});
+}
+template <typename Draw>
+int launch_search(const Draw &draw, int64_t num, int64_t *idx_out, hipStream_t st) {
+  const int64_t blocks = search_blocks(num);
+  if (blocks >= 0x7fffffffll) return GEAR_HIP_ERANGE;
+  with_search_lanes(num, [&](auto lanes) {
+    search_kernel<decltype(lanes)::value><<<dim3((unsigned)blocks), dim3(kBlock), 0, st>>>(draw, num,
+                                                                                        idx_out);
+  });
+  GEARHIP_RETURN_IF_LAUNCH_FAILED();
+  return 0;
+}
+
 size_t search_ws_bytes(int64_t num) {
   if (num <= 0) return 256;
-  const int64_t blocks = ceil_div64(num, kSearchBlock);
-  return align_up((size_t)num * 8, 256) + align_up((size_t)blocks * 8, 256);
+  return align_up((size_t)num * 8, 256) + align_up((size_t)search_blocks(num) * 8, 256);
 }
 
 }  // namespace
@@ -257,7 +487,7 @@ extern "C" int gear_hip_upper_bound_f64(const double *prefix, int64_t n, const f
   if (num == 0) return 0;
   if (n == 0 || !prefix || !u || !idx_out) return GEAR_HIP_EINVAL;
   if ((priorities == nullptr) != (weights_out == nullptr)) return GEAR_HIP_EINVAL;
-  const int64_t blocks = ceil_div64(num, kSearchBlock);
+  const int64_t blocks = search_blocks(num);
   const int64_t nblocks = ceil_div64(num, kBlock);
   if (blocks >= 0x7fffffffll) return GEAR_HIP_ERANGE;
   double *wraw = nullptr, *bmax = nullptr;
@@ -270,14 +500,16 @@ extern "C" int gear_hip_upper_bound_f64(const double *prefix, int64_t n, const f
                                       align_up((size_t)num * 8, 256));
   }
   hipStream_t st = as_stream(stream);
-  search_f64_kernel<<<dim3((unsigned)blocks), dim3(kSearchBlock), 0, st>>>(
-      prefix, n, u, num, unit_uniforms ? 1 : 0, idx_out, priorities, beta, wraw, bmax);
+  const DrawF64 draw{prefix, n, u, unit_uniforms ? 1 : 0};
+  if (!priorities) return launch_search(draw, num, idx_out, st);
+  with_search_lanes(num, [&](auto lanes) {
+    search_weights_kernel<decltype(lanes)::value><<<dim3((unsigned)blocks), dim3(kBlock), 0, st>>>(
+        draw, num, idx_out, priorities, beta, wraw, bmax);
+  });
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
-  if (priorities) {
-    normalise_kernel<<<dim3((unsigned)nblocks), dim3(kBlock), 0, st>>>(wraw, bmax, (int)blocks,
-                                                                      num, weights_out);
-    GEARHIP_RETURN_IF_LAUNCH_FAILED();
-  }
+  normalise_kernel<<<dim3((unsigned)nblocks), dim3(kBlock), 0, st>>>(wraw, bmax, (int)blocks, num,
+                                                                    weights_out);
+  GEARHIP_RETURN_IF_LAUNCH_FAILED();
   return 0;
 }
 
@@ -287,12 +519,7 @@ extern "C" int gear_hip_upper_bound_i64(const int64_t *prefix, int64_t n, const 
   if (n < 0 || num < 0) return GEAR_HIP_EINVAL;
   if (num == 0) return 0;
   if (n == 0 || !prefix || !u || !idx_out) return GEAR_HIP_EINVAL;
-  const int64_t blocks = ceil_div64(num, kSearchBlock);
-  if (blocks >= 0x7fffffffll) return GEAR_HIP_ERANGE;
-  search_i64_kernel<<<dim3((unsigned)blocks), dim3(kSearchBlock), 0, as_stream(stream)>>>(
-      DrawI64{prefix, n, u, unit_uniforms ? 1 : 0}, num, idx_out);
-  GEARHIP_RETURN_IF_LAUNCH_FAILED();
-  return 0;
+  return launch_search(DrawI64{prefix, n, u, unit_uniforms ? 1 : 0}, num, idx_out, as_stream(stream));
 }
 
 extern "C" size_t gear_hip_sample_workspace_bytes(int64_t num) { return sample_ws(num).total; }
@@ -316,20 +543,13 @@ extern "C" int gear_hip_sample_sorted_f64(const double *prefix, int64_t n, const
   char *ws = static_cast<char *>(workspace);
   int64_t *raw = reinterpret_cast<int64_t *>(ws + w.raw);
   const int64_t blocks = ceil_div64(num, kBlock);
-  const int64_t sblocks = ceil_div64(num, kSearchBlock);
-  if (sblocks >= 0x7fffffffll) return GEAR_HIP_ERANGE;
   const Split split{sorted_out, trajectory_length, modulo, idxs, tss, lens};
-  search_f64_kernel<<<dim3((unsigned)sblocks), dim3(kSearchBlock), 0, st>>>(
-      prefix, n, u, num, unit_uniforms ? 1 : 0, raw, nullptr, 0.0, nullptr, nullptr);
-  GEARHIP_RETURN_IF_LAUNCH_FAILED();
-  if (num <= radix::kRankMax && n < (1ll << 32)) {
-    rank_split_kernel<<<dim3((unsigned)ceil_div64(num, kWave)), dim3(radix::kRankBlock), 0, st>>>(
-        raw, (int)num, split);
-    GEARHIP_RETURN_IF_LAUNCH_FAILED();
-    return 0;
-  }
+  const DrawF64 draw{prefix, n, u, unit_uniforms ? 1 : 0};
+  if (num <= radix::kRankMax) return place_draws(draw, num, split, st);
+  int rc = launch_search(draw, num, raw, st);
+  if (rc) return rc;
   int64_t *sorted = sorted_out ? sorted_out : reinterpret_cast<int64_t *>(ws + w.sorted);
-  int rc = radix::sort_pairs<uint64_t, uint64_t>(
+  rc = radix::sort_pairs<uint64_t, uint64_t>(
       reinterpret_cast<const uint64_t *>(raw), reinterpret_cast<uint64_t *>(sorted), nullptr,
       nullptr, reinterpret_cast<uint64_t *>(ws + w.ktmp), nullptr, num, 0, key_bits,
       reinterpret_cast<uint32_t *>(ws + w.hist), st);
@@ -356,8 +576,8 @@ int check_lookup(const Lookup &look) {
 // raw: num positions on the device (each in [0, bound)); sorted ascending, then looked up.
 int sort_and_look_up(const int64_t *raw, int64_t num, int64_t bound, const Lookup &look, char *ws,
                      const SampleWs &w, hipStream_t st) {
-  if (num <= radix::kRankMax && bound <= (1ll << 32)) {
-    rank_lookup_kernel<<<dim3((unsigned)ceil_div64(num, kWave)), dim3(radix::kRankBlock), 0, st>>>(
+  if (num <= radix::kRankMax) {
+    place_positions_kernel<<<dim3((unsigned)ceil_div64(num, kPlaced)), dim3(kPlaceThreads), 0, st>>>(
         raw, (int)num, look);
     GEARHIP_RETURN_IF_LAUNCH_FAILED();
     return 0;
@@ -373,6 +593,17 @@ int sort_and_look_up(const int64_t *raw, int64_t num, int64_t bound, const Looku
   lookup_kernel<<<dim3((unsigned)ceil_div64(num, kBlock)), dim3(kBlock), 0, st>>>(sorted, num, look);
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
   return 0;
+}
+
+// draws: searched, sorted ascending, looked up
+template <typename Draw>
+int draw_and_look_up(const Draw &draw, int64_t num, const Lookup &look, char *ws, const SampleWs &w,
+                     hipStream_t st) {
+  if (num <= radix::kRankMax) return place_draws(draw, num, look, st);
+  int64_t *raw = reinterpret_cast<int64_t *>(ws + w.raw);
+  const int rc = launch_search(draw, num, raw, st);
+  if (rc) return rc;
+  return sort_and_look_up(raw, num, draw.n, look, ws, w, st);
 }
 
 }  // namespace
@@ -395,15 +626,8 @@ extern "C" int gear_hip_sample_lookup_f64(const double *prefix, int64_t n, const
   const SampleWs w = sample_ws(num);
   if (!workspace || workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(workspace) & 7))
     return GEAR_HIP_EWORKSPACE;
-  const int64_t sblocks = ceil_div64(num, kSearchBlock);
-  if (sblocks >= 0x7fffffffll) return GEAR_HIP_ERANGE;
-  char *ws = static_cast<char *>(workspace);
-  int64_t *raw = reinterpret_cast<int64_t *>(ws + w.raw);
-  hipStream_t st = as_stream(stream);
-  search_f64_kernel<<<dim3((unsigned)sblocks), dim3(kSearchBlock), 0, st>>>(
-      prefix, n, u, num, unit_uniforms ? 1 : 0, raw, nullptr, 0.0, nullptr, nullptr);
-  GEARHIP_RETURN_IF_LAUNCH_FAILED();
-  return sort_and_look_up(raw, num, n, look, ws, w, st);
+  return draw_and_look_up(DrawF64{prefix, n, u, unit_uniforms ? 1 : 0}, num, look,
+                          static_cast<char *>(workspace), w, as_stream(stream));
 }
 
 extern "C" int gear_hip_sample_lookup_i64(const int64_t *prefix, int64_t n, const void *u,
@@ -427,15 +651,8 @@ extern "C" int gear_hip_sample_lookup_i64(const int64_t *prefix, int64_t n, cons
   const SampleWs w = sample_ws(num);
   if (!workspace || workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(workspace) & 7))
     return GEAR_HIP_EWORKSPACE;
-  const int64_t sblocks = ceil_div64(num, kSearchBlock);
-  if (sblocks >= 0x7fffffffll) return GEAR_HIP_ERANGE;
-  char *ws = static_cast<char *>(workspace);
-  int64_t *raw = reinterpret_cast<int64_t *>(ws + w.raw);
-  hipStream_t st = as_stream(stream);
-  const DrawI64 draw{prefix, n, u, unit_uniforms ? 1 : 0};
-  search_i64_kernel<<<dim3((unsigned)sblocks), dim3(kSearchBlock), 0, st>>>(draw, num, raw);
-  GEARHIP_RETURN_IF_LAUNCH_FAILED();
-  return sort_and_look_up(raw, num, n, look, ws, w, st);
+  return draw_and_look_up(DrawI64{prefix, n, u, unit_uniforms ? 1 : 0}, num, look,
+                          static_cast<char *>(workspace), w, as_stream(stream));
 }
 
 extern "C" int gear_hip_sort_lookup_i64(const int64_t *positions, int64_t num, int64_t bound,
