@@ -7,12 +7,14 @@
 // the hot loop is an aligned global_store_dwordx4; the matching source bytes are fetched with one
 // global_load_dwordx4 at whatever byte alignment the table layout gives (the table has no
 // padding: a window of fp32[17] steps starts on a 4-byte boundary, a uint8 column on any byte).
-// Vectors that straddle the region edge or the copy/padding edge (at most four per slice) take a
-// byte path.  A group of `tg` threads (power of two, 1..128) owns one chunk of tg*U consecutive
+// Vectors that straddle the region edge or the copy/padding edge (at most four per slice) are
+// moved by words or bytes.  A group of `tg` threads (power of two, 1..128) owns one chunk of tg*U consecutive
 // vectors; lanes of a group take consecutive vectors so a wave reads and writes 1 KiB runs and a
 // 128-thread workgroup covers one contiguous 4 KiB piece of a large window (source cache lines
 // shared by neighbouring pieces are then fetched twice only at 4 KiB boundaries).
 // Each thread issues its U loads before its first store to keep U*16 bytes per lane in flight.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace gearhip {
@@ -24,14 +26,13 @@ constexpr int kMaxGroupShift = 7;  // a group never spans workgroups: at most 12
 enum GatherMode { kSubcopy = 0, kVcopy = 1, kCopy = 2 };
 
 // vector u of a lane: lanes of a group take consecutive vectors (coalesced 1 KiB per wave)
-#define GEARHIP_VEC_INDEX(k0, u, tg, lane, U) ((k0) + (int64_t)(u) * (tg) + (lane))
+#define GEARHIP_VEC_INDEX(k0, u, tg, lane, U) ((k0) + (u) * (tg) + (lane))
 
 struct ColumnArgs {
   uint8_t *dst;
   uint8_t *mask;
   int64_t ofst, span, step_bytes, col_base, dst_stride;
   int64_t cps;          // chunks per slice
-  int64_t block_begin;  // first block of this column in a multi-column grid
   int32_t pad_head, zero_fill;
   int32_t tg_shift;     // log2(threads per group)
   int32_t pad_;
@@ -50,16 +51,19 @@ struct GatherArgs {
 };
 
 struct MultiArgs {
+  uint32_t begin[GEAR_HIP_MAX_COLUMNS];  // first block of the column; beyond the last one: no block
   ColumnArgs col[GEAR_HIP_MAX_COLUMNS];
-  int32_t ncols;
 };
 
+// O: int32_t where every region of the launch is below 2^30 bytes (all but copies of gigabytes).  The
+// kernel is bound by its instructions where windows are short, and 64-bit offsets double them.
+template <typename O>
 struct Slice {
   const uint8_t *sp;  // source of the first copied byte
   uint8_t *rp;        // first byte of the destination region
-  int64_t rl;         // region length
-  int64_t cs;         // copy range start, relative to rp
-  int64_t n;          // copied bytes
+  O rl;               // region length
+  O cs;               // copy range start, relative to rp
+  O n;                // copied bytes
 };
 
 // NT is a bit mask: 1 = non-temporal loads, 2 = non-temporal stores
@@ -77,69 +81,94 @@ __device__ __forceinline__ void store16(uint8_t *p, u32x4 v) {
     *reinterpret_cast<u32x4 *>(p) = v;
 }
 
+struct __attribute__((packed, aligned(1))) u32_any {
+  uint32_t v;
+};
+
+// The vector at offset `lo` of the region when it straddles an edge, in elements of T.  All loads
+// are under way together, without a test around them (an element that is not copied loads the
+// slice's first one and is not looked at): one round trip to memory.  With a load inside a test per byte
+// they followed each other, and windows of a few bytes -- a flag column -- held a whole batch up:
+// 512 windows of 8 steps in four columns took 7.4 us for 0.8 MB, 4.5 now (a launch alone 3.1), 4096
+// whole trajectories of 64 steps 18.1, 13.6 now.
+template <typename T, typename O>
+__device__ __forceinline__ void edge_vector(const Slice<O> &s, O lo) {
+  constexpr int kN = 16 / (int)sizeof(T);
+  typedef typename std::make_unsigned<O>::type UO;
+  T v[kN];
+#pragma unroll
+  for (int j = 0; j < kN; ++j) v[j] = 0;
+  const O at0 = lo - s.cs;
+  if (s.n > 0) {
+#pragma unroll
+    for (int j = 0; j < kN; ++j) {
+      const O at = at0 + j * (int)sizeof(T);
+      const uint8_t *p = s.sp + ((UO)at < (UO)s.n ? at : (O)0);
+      if constexpr (sizeof(T) == 4)
+        v[j] = reinterpret_cast<const u32_any *>(p)->v;
+      else
+        v[j] = *p;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kN; ++j) {
+    const O off = lo + j * (int)sizeof(T), at = at0 + j * (int)sizeof(T);
+    if ((UO)off < (UO)s.rl) *reinterpret_cast<T *>(s.rp + off) = (UO)at < (UO)s.n ? v[j] : (T)0;
+  }
+}
+
 // Copies the part of slice `s` that belongs to group-chunk `c` (and c+cps, ... if the slice is
 // longer than the launch was sized for).
-template <int U, int NT>
-__device__ __forceinline__ void gather_chunks(const Slice &s, int64_t c, int64_t cps, int lane,
-                                              int tg) {
+template <int U, int NT, typename O>
+__device__ __forceinline__ void gather_chunks(const Slice<O> &s, O c, O cps, int lane, int tg) {
   const uintptr_t r0 = reinterpret_cast<uintptr_t>(s.rp);
-  const int64_t head = (int64_t)(r0 & 15);
+  const O head = (O)(r0 & 15);
   uint8_t *ap = s.rp - head;  // 16-byte aligned
-  const int64_t nvec = (head + s.rl + 15) >> 4;
-  const int64_t ce = s.cs + s.n;
-  const int64_t chunk = (int64_t)tg * U;
+  const O nvec = (head + s.rl + 15) >> 4;
+  const O ce = s.cs + s.n;
+  const O chunk = (O)tg * U;
+  // edges that lie between 32-bit words of the destination (all but columns of 1- and 2-byte steps)
+  const bool words = (((O)(r0 & 3) | s.cs | s.n | s.rl) & 3) == 0;
 
-  for (int64_t k0 = c * chunk; k0 < nvec; k0 += cps * chunk) {
+  for (O k0 = c * chunk; k0 < nvec; k0 += cps * chunk) {
     u32x4 v[U];
-    int kind[U];  // 0 nothing, 1 full aligned store, 2 byte path
+    uint32_t whole = 0, edge = 0;  // bit u: vector u is stored as it is / straddles an edge
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t k = GEARHIP_VEC_INDEX(k0, u, tg, lane, U);
-      const int64_t lo = (k << 4) - head;
-      const int64_t hi = lo + 16;
-      kind[u] = 0;
+      const O k = GEARHIP_VEC_INDEX(k0, u, tg, lane, U);
+      const O lo = (k << 4) - head, hi = lo + 16;
       v[u] = u32x4{0u, 0u, 0u, 0u};
       if (k < nvec) {
-        if (lo >= 0 && hi <= s.rl) {
-          if (lo >= s.cs && hi <= ce) {
-            v[u] = load16<NT>(s.sp + (lo - s.cs));
-            kind[u] = 1;
-          } else if (hi <= s.cs || lo >= ce) {
-            kind[u] = 1;  // all padding
-          } else {
-            kind[u] = 2;
-          }
-        } else {
-          kind[u] = 2;
-        }
+        const bool inside = lo >= 0 && hi <= s.rl;
+        const bool copy = lo >= s.cs && hi <= ce, pad = hi <= s.cs || lo >= ce;
+        if (inside && copy) v[u] = load16<NT>(s.sp + (lo - s.cs));
+        if (inside && (copy || pad))
+          whole |= 1u << u;
+        else
+          edge |= 1u << u;
       }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t k = GEARHIP_VEC_INDEX(k0, u, tg, lane, U);
-      if (kind[u] == 1) store16<NT>(ap + (k << 4), v[u]);
+      const O k = GEARHIP_VEC_INDEX(k0, u, tg, lane, U);
+      if ((whole >> u) & 1u) store16<NT>(ap + (k << 4), v[u]);
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (kind[u] == 2) {
-        const int64_t k = GEARHIP_VEC_INDEX(k0, u, tg, lane, U);
-        const int64_t lo = (k << 4) - head;
-        for (int j = 0; j < 16; ++j) {
-          const int64_t off = lo + j;
-          if (off >= 0 && off < s.rl) {
-            uint8_t b = 0;
-            if (off >= s.cs && off < ce) b = s.sp[off - s.cs];
-            s.rp[off] = b;
-          }
-        }
-      }
+    while (edge != 0u) {
+      const int u = __ffs((int)edge) - 1;
+      edge &= edge - 1u;
+      const O lo = (GEARHIP_VEC_INDEX(k0, u, tg, lane, U) << 4) - head;
+      if (words)
+        edge_vector<uint32_t>(s, lo);
+      else
+        edge_vector<uint8_t>(s, lo);
     }
   }
 }
 
 // Window arithmetic of fused_subcopy_collect (src/cuda/copy.cu:110-123) in int64.
-__device__ __forceinline__ Slice resolve_window(const GatherArgs &p, const ColumnArgs &col,
-                                                int64_t g, int64_t *valid_steps) {
+template <typename O>
+__device__ __forceinline__ Slice<O> resolve_window(const GatherArgs &p, const ColumnArgs &col,
+                                                   int64_t g, int64_t *valid_steps) {
   const int64_t idx = p.a[g], ts = p.b[g];
   int64_t len = p.c[g];
   if (p.traj_len > 0 && len > p.traj_len) len = p.traj_len;
@@ -151,14 +180,14 @@ __device__ __forceinline__ Slice resolve_window(const GatherArgs &p, const Colum
   int64_t steps = rsub - lsub;
   if (steps < 0) steps = 0;
   *valid_steps = steps;
-  const int64_t n = steps * col.step_bytes;
-  const int64_t npad = col.pad_head ? col.dst_stride - n : 0;
-  Slice s;
+  const O n = (O)steps * (O)col.step_bytes;
+  const O npad = col.pad_head ? (O)col.dst_stride - n : 0;
+  Slice<O> s;
   s.sp = p.src + idx * p.traj_stride + col.col_base + lsub * col.step_bytes;
   uint8_t *w0 = col.dst + g * col.dst_stride;
   if (col.zero_fill) {
     s.rp = w0;
-    s.rl = col.dst_stride;
+    s.rl = (O)col.dst_stride;
     s.cs = npad;
   } else {
     s.rp = w0 + npad;
@@ -169,13 +198,13 @@ __device__ __forceinline__ Slice resolve_window(const GatherArgs &p, const Colum
   return s;
 }
 
-template <int U, int NT>
+template <int U, int NT, typename O>
 __device__ __forceinline__ void subcopy_body(const GatherArgs &p, const ColumnArgs &col,
                                              int64_t block) {
   const int64_t t = block * kBlock + threadIdx.x;
   const int64_t gid = t >> col.tg_shift;
   const int tg = 1 << col.tg_shift;
-  const int lane = (int)(t & (tg - 1));
+  const int lane = (int)threadIdx.x & (tg - 1);
   int64_t g, c;
   if (col.cps == 1) {
     g = gid;
@@ -189,38 +218,38 @@ __device__ __forceinline__ void subcopy_body(const GatherArgs &p, const ColumnAr
   }
   if (g >= p.num) return;
   int64_t steps;
-  const Slice s = resolve_window(p, col, g, &steps);
+  const Slice<O> s = resolve_window<O>(p, col, g, &steps);
   if (col.mask != nullptr && c == 0) {
     uint8_t *m = col.mask + g * col.span;
     for (int64_t j = lane; j < col.span; j += tg)
       m[j] = col.pad_head ? (uint8_t)(j >= col.span - steps) : (uint8_t)(j < steps);
   }
-  gather_chunks<U, NT>(s, c, col.cps, lane, tg);
+  gather_chunks<U, NT, O>(s, (O)c, (O)col.cps, lane, tg);
 }
 
-template <int U, int NT>
+template <int U, int NT, typename O>
 __global__ __launch_bounds__(kBlock) void subcopy_kernel(GatherArgs p, ColumnArgs col) {
-  subcopy_body<U, NT>(p, col, blockIdx.x);
+  subcopy_body<U, NT, O>(p, col, blockIdx.x);
 }
 
-template <int U, int NT>
+template <int U, int NT, typename O>
 __global__ __launch_bounds__(kBlock) void subcopy_multi_kernel(GatherArgs p, MultiArgs m) {
-  // columns are laid out one after another along the grid; find this block's column
-  int ci = 0;
-  const int64_t b = blockIdx.x;
-#pragma unroll 1
-  for (int i = 1; i < m.ncols; ++i)
-    if (b >= m.col[i].block_begin) ci = i;
-  subcopy_body<U, NT>(p, m.col[ci], b - m.col[ci].block_begin);
+  // columns are laid out one after another along the grid: this block's column is the last one that
+  // begins at or before it (one load brings all the beginnings)
+  int ci = -1;
+  const uint32_t b = blockIdx.x;
+#pragma unroll
+  for (int i = 0; i < GEAR_HIP_MAX_COLUMNS; ++i) ci += b >= m.begin[i] ? 1 : 0;
+  subcopy_body<U, NT, O>(p, m.col[ci], b - m.begin[ci]);
 }
 
-template <int MODE, int U, int NT>
+template <int MODE, int U, int NT, typename O>
 __global__ __launch_bounds__(kBlock) void slices_kernel(GatherArgs p, uint8_t *dst, int64_t cps,
                                                         int tg_shift) {
   const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const int64_t gid = t >> tg_shift;
   const int tg = 1 << tg_shift;
-  const int lane = (int)(t & (tg - 1));
+  const int lane = (int)threadIdx.x & (tg - 1);
   int64_t g, c;
   if (cps == 1) {
     g = gid;
@@ -230,14 +259,14 @@ __global__ __launch_bounds__(kBlock) void slices_kernel(GatherArgs p, uint8_t *d
     c = gid - g * cps;
   }
   if (g >= p.num) return;
-  Slice s;
-  s.n = (MODE == kCopy) ? p.fixed_stride : p.c[g];
+  Slice<O> s;
+  s.n = (O)((MODE == kCopy) ? p.fixed_stride : p.c[g]);
   if (s.n < 0) s.n = 0;
   s.sp = p.src + p.a[g];
   s.rp = dst + p.b[g];
   s.rl = s.n;
   s.cs = 0;
-  gather_chunks<U, NT>(s, c, cps, lane, tg);
+  gather_chunks<U, NT, O>(s, (O)c, (O)cps, lane, tg);
 }
 
 // Device restatement of CpuTrajectoryStorageHandler::sub (src/storage/handler.cc:100-121).
@@ -334,7 +363,6 @@ int fill_column(const gear_hip_column_desc &d, int64_t num, int U, ColumnArgs *o
   out->col_base = d.col_base;
   out->dst_stride = d.dst_stride;
   out->cps = s.cps;
-  out->block_begin = 0;
   out->pad_head = d.pad_head ? 1 : 0;
   out->zero_fill = d.zero_fill ? 1 : 0;
   out->tg_shift = s.tg_shift;
@@ -343,24 +371,42 @@ int fill_column(const gear_hip_column_desc &d, int64_t num, int U, ColumnArgs *o
   return 0;
 }
 
+// regions of a launch below this many bytes: 32-bit offsets inside a slice (a multiple of the
+// chunk of a step may be added to an offset before it is compared)
+constexpr int64_t kNarrowRegion = 1ll << 30;
+
 int launch_subcopy(const GatherArgs &p, const ColumnArgs &col, int64_t blocks, hipStream_t st) {
-  subcopy_kernel<kUnroll, kNt><<<dim3((unsigned)blocks), dim3(kBlock), 0, st>>>(p, col);
+  const dim3 grid((unsigned)blocks), block(kBlock);
+  if (col.dst_stride < kNarrowRegion)
+    subcopy_kernel<kUnroll, kNt, int32_t><<<grid, block, 0, st>>>(p, col);
+  else
+    subcopy_kernel<kUnroll, kNt, int64_t><<<grid, block, 0, st>>>(p, col);
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
   return 0;
 }
 
-int launch_multi(const GatherArgs &p, const MultiArgs &m, int64_t blocks, hipStream_t st) {
-  subcopy_multi_kernel<kUnroll, kNt><<<dim3((unsigned)blocks), dim3(kBlock), 0, st>>>(p, m);
+int launch_multi(const GatherArgs &p, const MultiArgs &m, int ncols, int64_t blocks, hipStream_t st) {
+  bool narrow = true;
+  for (int i = 0; i < ncols; ++i) narrow = narrow && m.col[i].dst_stride < kNarrowRegion;
+  const dim3 grid((unsigned)blocks), block(kBlock);
+  if (narrow)
+    subcopy_multi_kernel<kUnroll, kNt, int32_t><<<grid, block, 0, st>>>(p, m);
+  else
+    subcopy_multi_kernel<kUnroll, kNt, int64_t><<<grid, block, 0, st>>>(p, m);
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
   return 0;
 }
 
+// (a slice of vcopy may be longer than max_len says, up to whatever its stride holds: 64-bit offsets)
 template <int MODE>
 int launch_slices(const GatherArgs &p, uint8_t *dst, int64_t max_len, hipStream_t st) {
   const Shape s = plan(p.num, max_len, kUnroll);
   if (s.blocks >= 0x7fffffffll) return GEAR_HIP_ERANGE;
-  slices_kernel<MODE, kUnroll, kNt><<<dim3((unsigned)s.blocks), dim3(kBlock), 0, st>>>(
-      p, dst, s.cps, s.tg_shift);
+  const dim3 grid((unsigned)s.blocks), block(kBlock);
+  if (MODE == kCopy && max_len < kNarrowRegion)
+    slices_kernel<MODE, kUnroll, kNt, int32_t><<<grid, block, 0, st>>>(p, dst, s.cps, s.tg_shift);
+  else
+    slices_kernel<MODE, kUnroll, kNt, int64_t><<<grid, block, 0, st>>>(p, dst, s.cps, s.tg_shift);
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
   return 0;
 }
@@ -418,20 +464,22 @@ extern "C" int gear_hip_subcopy_multi_checked(const void *src, int64_t num, cons
   if (!src || !idxs || !tss || !lens || !cols || traj_stride < 0) return GEAR_HIP_EINVAL;
   const int U = kUnroll;
   MultiArgs m;
-  m.ncols = ncols;
   int64_t total = 0;
   for (int i = 0; i < ncols; ++i) {
     int64_t blocks = 0;
     int rc = fill_column(cols[i], num, U, &m.col[i], &blocks);
     if (rc) return rc;
-    m.col[i].block_begin = total;
+    m.begin[i] = (uint32_t)total;
     total += blocks;
+    if (total >= 0x7fffffffll) return GEAR_HIP_ERANGE;
   }
-  for (int i = ncols; i < GEAR_HIP_MAX_COLUMNS; ++i) m.col[i] = m.col[0];
-  if (total >= 0x7fffffffll) return GEAR_HIP_ERANGE;
+  for (int i = ncols; i < GEAR_HIP_MAX_COLUMNS; ++i) {
+    m.begin[i] = 0xffffffffu;
+    m.col[i] = m.col[0];
+  }
   GatherArgs p{static_cast<const uint8_t *>(src), num,        idxs, tss, lens, traj_stride, 0,
                capacity,                          trajectory_length};
-  return launch_multi(p, m, total, as_stream(stream));
+  return launch_multi(p, m, ncols, total, as_stream(stream));
 }
 
 extern "C" int gear_hip_vcopy(const void *src, void *dst, int64_t num,
