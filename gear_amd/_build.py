@@ -79,6 +79,31 @@ def build_libgear_ext():
     return out
 
 
+def hostops_path():
+    suffix = sysconfig.get_config_var("EXT_SUFFIX") or ".so"
+    return os.path.join(_PKG, "_hostops" + suffix)
+
+
+def build_hostops():
+    """Compile the host side of gear_amd.ops (gear_amd/_hostops*.so): host C++ over libtorch and the
+    C ABI, no device code."""
+    import torch
+    from torch.utils import cpp_extension
+    inc, lib = [], []
+    for d in cpp_extension.include_paths(device_type="cuda"):
+        inc += ["-isystem", d]
+    for d in cpp_extension.library_paths(device_type="cuda"):
+        lib += ["-L", d, "-Wl,-rpath," + d]
+    out = hostops_path()
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+          "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
+          "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-I", INCLUDE] + inc +
+         ["-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "torchops", "ops.cc"),
+          "-o", out, "-L", _PKG, "-lgearhip", "-Wl,-rpath,$ORIGIN"] + lib +
+         ["-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-lamdhip64"])
+    return out
+
+
 SANITIZE_FLAGS = ["-fsanitize=address,undefined", "-fno-sanitize-recover=undefined",
                   "-fno-omit-frame-pointer", "-O1", "-g"]
 
@@ -108,6 +133,7 @@ def build_all(verbose=False):
     build_libgearhip(verbose)
     if os.path.isdir(os.path.join(CSRC, "host")):
         build_libgear_ext()
+    build_hostops()
 
 
 if __name__ == "__main__":

@@ -17,7 +17,7 @@ from typing import Any, Dict, List, Sequence, Union
 
 import torch
 
-from .. import ops
+from .. import _hostops, ops
 from ..dataset import SharedDataset
 from ..dtypes import CVT_DTYPES_GEAR_TO_TORCH
 from ..libgear import core as glibc
@@ -107,8 +107,23 @@ class OfflineLoader(BasicLoader):
         self._sampler.indices_ascending = True   # arange + offset below
         self._indices = torch.arange(self._iset.local_capacity, dtype=torch.long,
                                      device=self._mpu.device) + self._iset.index_offset
+        self._step = self._native_step()
         self.last_masks = None
         self.last_sampled = None   # global indices of the last batch (device tensor)
+
+    def _native_step(self):
+        """The step after the draws as one native call (LoaderStep of _hostops)."""
+        spec = self._table.get_table_spec()
+        columns = []
+        for col, p in zip(self._sub_cols, self._patterns):
+            cspec = self._table.get_column_spec(col)
+            columns.append((CVT_DTYPES_GEAR_TO_TORCH[cspec.dtype],
+                            [int(p.length)] + [int(v) for v in cspec.shape], int(p.offset),
+                            int(p.length), cspec.size(), self._table.column_base(col),
+                            p.pad_option == glibc.SubscribePattern.PadOption.head))
+        return _hostops.LoaderStep(self._table, self._table.trajectory_stride, spec.capacity,
+                                   spec.trajectory_length, columns, self._with_mask,
+                                   torch.device(self._mpu.device))
 
     def refresh_index(self):
         """Upload priorities and trajectory lengths after the host side changed them."""
@@ -219,31 +234,20 @@ class OfflineLoader(BasicLoader):
         self.last_masks = masks
         return data_batch
 
-    def _select_gather(self, draws, dirty_from):
+    def _select_gather(self, draws, dirty_from, host_timesteps=False):
         """Everything of a step after the draws: the sampler's own preparation (prefix rescan,
         top-k selection), then ONE call that sorts the batch, looks up global index, local index
-        and recorded length of every entry, and gathers all columns
-        (CpuTrajectoryStorageHandler.select_subcopy).  Returns (sampled, lengths, data_batch)."""
+        and recorded length of every entry, and gathers all columns into fresh tensors.  Returns
+        (lengths, data_batch); the lengths on the host, ahead of the gather, when asked for."""
         kind, picks, prefix = self._sampler.prepare(self._indices, self._device_weights, draws,
                                                     dirty_from=dirty_from)
-        n = picks.numel()
-        dev = self._mpu.device
-        looked = torch.empty((3, n), dtype=torch.int64, device=dev)  # sampled, local, lengths
-        data_batch = self._empty_batch(n)
-        masks = None
-        if self._with_mask:
-            masks = [torch.empty((n, p.length), dtype=torch.uint8, device=dev)
-                     for p in self._patterns]
-        self._handler.select_subcopy(kind, picks, prefix, self._indices, self._iset.index_offset,
-                                     self._device_timesteps, self._sub_cols, data_batch, True,
-                                     masks, looked[0], looked[1], looked[2])
-        self.last_masks = masks
-        self.last_sampled = looked[0]
-        return looked[0], looked[2], data_batch
+        self.last_sampled, lengths, data_batch, self.last_masks = self._step.run(
+            kind, picks, prefix, self._indices, self._iset.index_offset, self._device_timesteps,
+            host_timesteps, ops._ws)
+        return lengths, data_batch
 
     def _graph_step(self):
-        _, lengths, data_batch = self._select_gather(self._graph_draws, None)
-        return lengths, data_batch
+        return self._select_gather(self._graph_draws, None)
 
     def _graph_iterate(self):
         n = self._indices.numel()
@@ -273,9 +277,9 @@ class OfflineLoader(BasicLoader):
         if self._use_graph:
             return self._graph_iterate()
         draws = self._sampler.draw(self._indices.numel(), self._batch_size * self._dp_world)
-        _, lengths, data_batch = self._select_gather(draws, self._dirty_from)
+        timesteps, data_batch = self._select_gather(draws, self._dirty_from,
+                                                    not self._timesteps_on_device)
         self._dirty_from = self._device_weights.numel()   # clean until the next update
-        timesteps = lengths if self._timesteps_on_device else lengths.cpu()
         return timesteps, data_batch
 
     def low_level_controlled_iterate(self):

@@ -12,6 +12,13 @@ import torch
 from . import _cabi
 from ._cabi import ColumnDesc, call, load
 
+try:
+    from . import _hostops  # checks, outputs, scratch and calls of the functions below, natively
+except ImportError as _e:  # pragma: no cover - only without a build
+    raise ImportError(
+        "gear_amd.ops: the native module _hostops is not built; run "
+        "`python -c 'import __graft_entry__ as g; g.build()'` in the repository root") from _e
+
 
 # torch's C accessor for the raw current stream (a fraction of the cost of
 # torch.cuda.current_stream(), which builds a Stream object through several Python layers)
@@ -68,23 +75,9 @@ def _ws_bytes(query, *sizes):
     return getattr(load(), query)(*[int(v) for v in sizes])
 
 
-class _Workspace:
-    """Scratch tensors per (purpose, device, stream), grown on demand and reused: no allocation
-    in steady state, and calls enqueued on different streams never share a workspace."""
-
-    def __init__(self):
-        self._bufs = {}
-
-    def get(self, tag, nbytes, device):
-        key = (tag, device, _stream_value(device))
-        buf = self._bufs.get(key)
-        if buf is None or buf.numel() < nbytes:
-            buf = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
-            self._bufs[key] = buf
-        return buf
-
-
-_ws = _Workspace()
+# Scratch tensors per (purpose, device, stream), grown on demand and reused: no allocation in steady
+# state, and calls enqueued on different streams never share a workspace.
+_ws = _hostops.Workspace()
 
 
 def set_device(device_id):
@@ -157,8 +150,8 @@ def subcopy_multi(src, idxs, tss, lens, traj_stride, columns, capacity=0, trajec
 
 class GatherPlan:
     """subcopy_multi for a loop that gathers into the same batch tensors every step: the column
-    descriptors and every argument that does not change are marshalled once, run() is one call
-    into the library with the three index tensors of the step."""
+    descriptors and every argument that does not change are marshalled once, run(idxs, tss, lens)
+    is one call into the library with the three index tensors of the step."""
 
     def __init__(self, src, traj_stride, columns, num, capacity=0, trajectory_length=0):
         n = len(columns)
@@ -185,20 +178,10 @@ class GatherPlan:
             d.zero_fill = int(bool(c.get("zero_fill", True)))
             self._keep.append((dst, m))
         self._keep.append(src)
-        self._fn = load().gear_hip_subcopy_multi_checked
-        self._num = int(num)
-        self._head = (_src_ptr(src), self._num)
-        self._tail = (int(traj_stride), int(capacity), int(trajectory_length), self._descs, n)
-
-    def run(self, idxs, tss, lens):
-        if idxs.numel() != self._num or tss.numel() != self._num or lens.numel() != self._num:
-            raise ValueError("the plan was made for %d windows" % self._num)
-        if idxs.dtype != torch.int64 or tss.dtype != torch.int64 or lens.dtype != torch.int64:
-            raise TypeError("idxs, tss and lens must be int64 tensors")
-        code = self._fn(*self._head, idxs.data_ptr(), tss.data_ptr(), lens.data_ptr(), *self._tail,
-                        _stream_value(idxs.device))
-        if code != 0:
-            _cabi.check("gear_hip_subcopy_multi_checked", code)
+        self.run = _hostops.Gather(
+            _src_ptr(src), int(traj_stride), int(num), int(capacity), int(trajectory_length),
+            [(d.dst, d.mask_out or 0, d.ofst, d.span, d.step_bytes, d.col_base, d.dst_stride,
+              bool(d.pad_head), bool(d.zero_fill)) for d in self._descs[:n]]).run
 
 
 def vcopy(src, dst, src_offsets, dst_offsets, strides, max_stride):
@@ -249,29 +232,12 @@ def split_step_index(flat, trajectory_length, modulo=0, idxs=None, tss=None, len
 
 def take_i64(table, idx, add=0, out=None):
     """out[j] = table[idx[j]] + add (int64, device)."""
-    _need(table, torch.int64, "table")
-    _need(idx, torch.int64, "idx")
-    if out is None:
-        out = torch.empty(idx.numel(), dtype=torch.int64, device=idx.device)
-    call("gear_hip_take_i64", _ptr(table), table.numel(), _ptr(idx), idx.numel(), int(add),
-         _ptr(out), _stream())
-    return out
+    return _hostops.take_i64(table, idx, int(add), out)
 
 
 def prefix_sum(priorities, out=None):
     """fp32[n] -> inclusive fp64 prefix[n] (gear_hip_scan_f32_f64)."""
-    _need(priorities, torch.float32, "priorities")
-    n = priorities.numel()
-    if out is None:
-        out = torch.empty(n, dtype=torch.float64, device=priorities.device)
-    else:
-        _need(out, torch.float64, "out")
-        if out.numel() < n:
-            raise ValueError("out is too small")
-    nbytes = _ws_bytes("gear_hip_scan_workspace_bytes", n)
-    ws = _ws.get("scan", nbytes, priorities.device)
-    call("gear_hip_scan_f32_f64", _ptr(priorities), _ptr(out), n, _ptr(ws), ws.numel(), _stream())
-    return out
+    return _hostops.prefix_sum(priorities, out, _ws)
 
 
 def prefix_sum_static(priorities, out):
@@ -313,28 +279,14 @@ class PrefixState:
             self._valid = False
         if self._src != priorities.data_ptr():
             self._valid = False
-        if not self._valid or first_changed <= 0:
-            call("gear_hip_scan_f32_f64", _ptr(priorities), _ptr(self.out), n, _ptr(self._ws),
-                 self._ws.numel(), _stream())
-        else:
-            call("gear_hip_rescan_f32_f64", _ptr(priorities), _ptr(self.out), n,
-                 int(first_changed), _ptr(self._ws), self._ws.numel(), _stream())
+        _hostops.rescan(priorities, self.out, int(first_changed) if self._valid else 0, self._ws)
         self._src = priorities.data_ptr()
         self._valid = True
         return self.out
 
 
 def prefix_sum_i64(weights, out=None):
-    _need(weights, torch.int64, "weights")
-    n = weights.numel()
-    if out is None:
-        out = torch.empty(n, dtype=torch.int64, device=weights.device)
-    else:
-        _need(out, torch.int64, "out")
-    nbytes = _ws_bytes("gear_hip_scan_workspace_bytes", n)
-    ws = _ws.get("scan", nbytes, weights.device)
-    call("gear_hip_scan_i64", _ptr(weights), _ptr(out), n, _ptr(ws), ws.numel(), _stream())
-    return out
+    return _hostops.prefix_sum_i64(weights, out, _ws)
 
 
 def sum_f32(values, out=None, out_f64=None):
@@ -352,60 +304,15 @@ def sum_f32(values, out=None, out_f64=None):
 def upper_bound(prefix, u, *, unit_uniforms=False, idx_out=None, priorities=None, beta=0.4,
                 weights_out=None):
     """Batched search of draws in an fp64 prefix array; optionally importance weights."""
-    _need(prefix, torch.float64, "prefix")
-    _need(u, torch.float32, "u")
-    num = u.numel()
-    if idx_out is None:
-        idx_out = torch.empty(num, dtype=torch.int64, device=u.device)
-    else:
-        _need(idx_out, torch.int64, "idx_out")
-    ws = None
-    if priorities is not None:
-        _need(priorities, torch.float32, "priorities")
-        if priorities.numel() != prefix.numel():
-            raise ValueError("priorities and prefix differ in length")
-        if weights_out is None:
-            weights_out = torch.empty(num, dtype=torch.float32, device=u.device)
-        nbytes = _ws_bytes("gear_hip_search_workspace_bytes", num)
-        ws = _ws.get("search", nbytes, u.device)
-    call("gear_hip_upper_bound_f64", _ptr(prefix), prefix.numel(), _ptr(u), num,
-         int(bool(unit_uniforms)), _ptr(idx_out), _ptr(priorities), float(beta),
-         _ptr(weights_out) if priorities is not None else None, _ptr(ws),
-         ws.numel() if ws is not None else 0, _stream())
-    if priorities is not None:
-        return idx_out, weights_out
-    return idx_out
+    return _hostops.upper_bound(prefix, u, bool(unit_uniforms), idx_out, priorities, float(beta),
+                                weights_out, _ws)
 
 
 def sample_sorted(prefix, u, *, unit_uniforms=True, sorted_out=None, trajectory_length=0,
                   modulo=0, idxs=None, tss=None, lens=None):
     """Search + ascending sort (+ split into window arguments) of one batch of draws."""
-    _need(prefix, torch.float64, "prefix")
-    _need(u, torch.float32, "u")
-    num = u.numel()
-    dev = u.device
-    if sorted_out is None:
-        sorted_out = torch.empty(num, dtype=torch.int64, device=dev)
-    if trajectory_length > 0:
-        idxs = idxs if idxs is not None else torch.empty(num, dtype=torch.int64, device=dev)
-        tss = tss if tss is not None else torch.empty(num, dtype=torch.int64, device=dev)
-        lens = lens if lens is not None else torch.empty(num, dtype=torch.int64, device=dev)
-    nbytes = _ws_bytes("gear_hip_sample_workspace_bytes", num)
-    ws = _ws.get("sample", nbytes, dev)
-    call("gear_hip_sample_sorted_f64", _ptr(prefix), prefix.numel(), _ptr(u), num,
-         int(bool(unit_uniforms)), _ptr(sorted_out), int(trajectory_length), int(modulo),
-         _ptr(idxs), _ptr(tss), _ptr(lens), _ptr(ws), ws.numel(), _stream())
-    if trajectory_length > 0:
-        return sorted_out, idxs, tss, lens
-    return sorted_out
-
-
-def _lookup_outputs(num, dev, lengths_table, sampled_out, local_out, lens_out):
-    empty = lambda: torch.empty(num, dtype=torch.int64, device=dev)
-    sampled = sampled_out if sampled_out is not None else empty()
-    local = local_out if local_out is not None else empty()
-    lens = lens_out if lens_out is not None else (empty() if lengths_table is not None else None)
-    return sampled, local, lens
+    return _hostops.sample_sorted(prefix, u, bool(unit_uniforms), sorted_out, int(trajectory_length),
+                                  int(modulo), idxs, tss, lens, _ws)
 
 
 def sample_lookup(prefix, u, *, unit_uniforms=True, index_table=None, index_offset=0,
@@ -418,125 +325,41 @@ def sample_lookup(prefix, u, *, unit_uniforms=True, index_table=None, index_offs
     or int64 targets (gear_hip_sample_lookup_i64); there, `start_uniforms` (float64 in [0, 1), one
     per draw) and `window` add a fourth result: starts = floor(start_uniforms * (lens - window + 1)),
     where a window of that many steps begins inside each drawn entry."""
-    if start_uniforms is not None and prefix.dtype != torch.int64:
-        raise ValueError("window starts come with an int64 prefix only")
-    if prefix.dtype == torch.int64:
-        _need(prefix, torch.int64, "prefix")
-        if unit_uniforms:
-            _need(u, torch.float64, "u")
-        else:
-            _need(u, torch.int64, "u")
-        entry = "gear_hip_sample_lookup_i64"
-    else:
-        _need(prefix, torch.float64, "prefix")
-        _need(u, torch.float32, "u")
-        entry = "gear_hip_sample_lookup_f64"
-    num, dev = u.numel(), u.device
-    if index_table is not None:
-        _need(index_table, torch.int64, "index_table")
-        if index_table.numel() != prefix.numel():
-            raise ValueError("index_table and prefix differ in length")
-    if lengths_table is not None:
-        _need(lengths_table, torch.int64, "lengths_table")
-    sampled, local, lens = _lookup_outputs(num, dev, lengths_table, sampled_out, local_out, lens_out)
-    ws = _ws.get("sample", _ws_bytes("gear_hip_sample_workspace_bytes", num), dev)
-    args = [_ptr(prefix), prefix.numel(), _ptr(u), num, int(bool(unit_uniforms)), _ptr(index_table),
-            int(index_offset), _ptr(lengths_table),
-            lengths_table.numel() if lengths_table is not None else 0, _ptr(sampled), _ptr(local),
-            _ptr(lens)]
-    starts = None
-    if prefix.dtype == torch.int64:
-        if start_uniforms is not None:
-            _need(start_uniforms, torch.float64, "start_uniforms")
-            if start_uniforms.numel() != num or lengths_table is None or window < 1:
-                raise ValueError("window starts need a uniform per draw, lengths_table and window >= 1")
-            starts = starts_out if starts_out is not None else torch.empty(
-                num, dtype=torch.int64, device=dev)
-        args += [_ptr(start_uniforms), int(window), _ptr(starts)]
-    call(entry, *args, _ptr(ws), ws.numel(), _stream())
-    if starts is not None:
-        return sampled, local, lens, starts
-    return sampled, local, lens
+    return _hostops.sample_lookup(prefix, u, bool(unit_uniforms), index_table, int(index_offset),
+                                  lengths_table, sampled_out, local_out, lens_out, start_uniforms,
+                                  int(window), starts_out, _ws)
 
 
 def sort_lookup(positions, bound, *, index_table=None, index_offset=0, lengths_table=None,
                 sampled_out=None, local_out=None, lens_out=None):
     """Given positions (each in [0, bound)): ascending sort, then the same look-ups
     (gear_hip_sort_lookup_i64)."""
-    _need(positions, torch.int64, "positions")
-    num, dev = positions.numel(), positions.device
-    if index_table is not None:
-        _need(index_table, torch.int64, "index_table")
-    if lengths_table is not None:
-        _need(lengths_table, torch.int64, "lengths_table")
-    sampled, local, lens = _lookup_outputs(num, dev, lengths_table, sampled_out, local_out, lens_out)
-    ws = _ws.get("sample", _ws_bytes("gear_hip_sample_workspace_bytes", num), dev)
-    call("gear_hip_sort_lookup_i64", _ptr(positions), num, int(bound), _ptr(index_table),
-         index_table.numel() if index_table is not None else 0, int(index_offset),
-         _ptr(lengths_table), lengths_table.numel() if lengths_table is not None else 0,
-         _ptr(sampled), _ptr(local), _ptr(lens), _ptr(ws), ws.numel(), _stream())
-    return sampled, local, lens
+    return _hostops.sort_lookup(positions, int(bound), index_table, int(index_offset), lengths_table,
+                                sampled_out, local_out, lens_out, _ws)
 
 
 def lookup(positions, *, index_table=None, index_offset=0, lengths_table=None, sampled_out=None,
            local_out=None, lens_out=None):
     """The look-ups alone, for positions that are already in the wanted order
     (gear_hip_lookup_i64)."""
-    _need(positions, torch.int64, "positions")
-    num, dev = positions.numel(), positions.device
-    if index_table is not None:
-        _need(index_table, torch.int64, "index_table")
-    if lengths_table is not None:
-        _need(lengths_table, torch.int64, "lengths_table")
-    sampled, local, lens = _lookup_outputs(num, dev, lengths_table, sampled_out, local_out, lens_out)
-    call("gear_hip_lookup_i64", _ptr(positions), num, _ptr(index_table),
-         index_table.numel() if index_table is not None else 0, int(index_offset),
-         _ptr(lengths_table), lengths_table.numel() if lengths_table is not None else 0,
-         _ptr(sampled), _ptr(local), _ptr(lens), _stream())
-    return sampled, local, lens
+    return _hostops.lookup(positions, index_table, int(index_offset), lengths_table, sampled_out,
+                           local_out, lens_out)
 
 
 def upper_bound_i64(prefix, u, *, unit_uniforms=True, idx_out=None):
-    _need(prefix, torch.int64, "prefix")
-    _need(u, torch.float64 if unit_uniforms else torch.int64, "u")
-    num = u.numel()
-    if idx_out is None:
-        idx_out = torch.empty(num, dtype=torch.int64, device=u.device)
-    call("gear_hip_upper_bound_i64", _ptr(prefix), prefix.numel(), _ptr(u), num,
-         int(bool(unit_uniforms)), _ptr(idx_out), _stream())
-    return idx_out
+    return _hostops.upper_bound_i64(prefix, u, bool(unit_uniforms), idx_out)
 
 
 def sort_i64(keys, vals=None, key_bits=63):
-    _need(keys, torch.int64, "keys")
-    num = keys.numel()
-    keys_out = torch.empty_like(keys)
-    vals_out = None
-    if vals is not None:
-        _need(vals, torch.int64, "vals")
-        vals_out = torch.empty_like(vals)
-    nbytes = _ws_bytes("gear_hip_sort_workspace_bytes", num)
-    ws = _ws.get("sort", nbytes, keys.device)
-    call("gear_hip_sort_i64", _ptr(keys), _ptr(keys_out), _ptr(vals), _ptr(vals_out), num,
-         int(key_bits), _ptr(ws), ws.numel(), _stream())
-    return (keys_out, vals_out) if vals is not None else keys_out
+    return _hostops.sort_i64(keys, vals, int(key_bits), _ws)
 
 
 def topk(priorities, k, *, sorted_by_value=True, want_values=True, warm=False, workspace=None):
     """Top-k of fp32 priorities (values, indices), by value descending or by index ascending.
     warm=True: the call may start from the bound that the last call on `workspace` (same n, k and
     order) left there instead of sampling the array; the result is the same either way."""
-    _need(priorities, torch.float32, "priorities")
-    n = priorities.numel()
-    idx = torch.empty(k, dtype=torch.int64, device=priorities.device)
-    vals = torch.empty(k, dtype=torch.float32, device=priorities.device) if want_values else None
-    nbytes = _ws_bytes("gear_hip_topk_workspace_bytes", n, k)
-    ws = workspace if workspace is not None else _ws.get("topk", nbytes, priorities.device)
-    if ws.numel() < nbytes:
-        raise ValueError("top-k workspace holds %d bytes, %d needed" % (ws.numel(), nbytes))
-    call("gear_hip_topk_f32_warm" if warm else "gear_hip_topk_f32", _ptr(priorities), n, int(k),
-         int(bool(sorted_by_value)), _ptr(vals), _ptr(idx), _ptr(ws), ws.numel(), _stream())
-    return vals, idx
+    return _hostops.topk(priorities, int(k), bool(sorted_by_value), bool(want_values), bool(warm),
+                         workspace, _ws)
 
 
 class TopKState:
@@ -564,19 +387,4 @@ class TopKState:
 
 def scatter(weights, idx, values, *, unique_indices=False):
     """weights[idx[j]] = values[j]; duplicates: last one wins.  fp32 or int64 tables."""
-    if weights.dtype not in (torch.float32, torch.int64):
-        raise TypeError("scatter works on float32 or int64 tables")
-    _need(weights, weights.dtype, "weights")
-    _need(idx, torch.int64, "idx")
-    _need(values, weights.dtype, "values")
-    num = idx.numel()
-    if values.numel() != num:
-        raise ValueError("idx and values differ in length")
-    ws = None
-    if not unique_indices:
-        nbytes = _ws_bytes("gear_hip_scatter_workspace_bytes", num)
-        ws = _ws.get("scatter", nbytes, weights.device)
-    fn = "gear_hip_scatter_f32" if weights.dtype == torch.float32 else "gear_hip_scatter_i64"
-    call(fn, _ptr(weights), weights.numel(), _ptr(idx), _ptr(values), num,
-         int(bool(unique_indices)), _ptr(ws), ws.numel() if ws is not None else 0, _stream())
-    return weights
+    return _hostops.scatter(weights, idx, values, bool(unique_indices), _ws)

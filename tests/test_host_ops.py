@@ -1,0 +1,32 @@
+"""Argument checks of gear_amd.ops (made natively): refused before anything reaches the GPU, with
+the name of the argument."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+
+def test_wrong_arguments_are_named():
+    from gear_amd import ops
+    f = torch.zeros(8)
+    with pytest.raises(TypeError, match="priorities must be a torch.Tensor"):
+        ops.prefix_sum([1.0, 2.0])
+    with pytest.raises(TypeError, match="priorities must have dtype torch.float32, got torch.float64"):
+        ops.prefix_sum(f.double())
+    with pytest.raises(ValueError, match="priorities must be contiguous"):
+        ops.prefix_sum(f[::2])
+    with pytest.raises(ValueError, match="priorities must live on the GPU"):
+        ops.prefix_sum(f)
+    with pytest.raises(TypeError, match="weights must have dtype torch.int64"):
+        ops.prefix_sum_i64(f)
+    with pytest.raises(TypeError, match="prefix must have dtype torch.float64"):
+        ops.upper_bound(f, f)
+    with pytest.raises(TypeError, match="prefix must have dtype torch.float64"):
+        ops.sample_sorted(f, f)
+    with pytest.raises(ValueError, match="window starts come with an int64 prefix only"):
+        ops.sample_lookup(f.double(), f, start_uniforms=f.double(), window=2)
+    with pytest.raises(TypeError, match="positions must have dtype torch.int64"):
+        ops.sort_lookup(f, 8)
+    with pytest.raises(TypeError, match="keys must have dtype torch.int64"):
+        ops.sort_i64(f)
+    with pytest.raises(TypeError, match="scatter works on float32 or int64 tables"):
+        ops.scatter(f.double(), f.long(), f.double())
