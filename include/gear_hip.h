@@ -342,7 +342,7 @@ int gear_hip_upper_bound_i64(const int64_t *prefix, int64_t n, const void *u, in
 
 /* ---- sort / top-k / priority update ------------------------------------------------------- */
 
-/* Ascending LSD radix sort of `num` int64 keys (non-negative, < 2^key_bits) with an optional
+/* Ascending sort (by counting, or LSD radix) of `num` int64 keys (non-negative, < 2^key_bits) with an optional
  * int64 payload, stable.  keys_out/vals_out must not alias the inputs.
  * Replaces the torch.sort of sampled indices in every sampler
  * (gear/sampler/global_sampler.py:131,172,195-199) and the unfinished
