@@ -91,12 +91,6 @@ __device__ __forceinline__ bool try_read(const Slot *s, uint64_t tag, uint64_t *
 // row-major order of the memory instructions into the blocked order of the arithmetic and back.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 template <typename T> struct Gran {  // one 16-byte granule of T
   static constexpr int kN = 16 / (int)sizeof(T);
   typedef T type __attribute__((ext_vector_type(kN)));

@@ -97,6 +97,13 @@ __device__ __forceinline__ T wave_sum(T x) {
 
 __device__ __forceinline__ uint64_t wave_ballot(bool p) { return __ballot(p); }
 
+// Orders the LDS accesses of a wave's lanes (a wave-private piece of LDS needs no barrier).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Agent-scope relaxed 64-bit accesses: they reach the device-coherent level, so a word written
 // by a workgroup on one XCD is seen by workgroups on the others without further fences.
 __device__ __forceinline__ uint64_t load_agent(const uint64_t *p) {

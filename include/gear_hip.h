@@ -394,8 +394,8 @@ int gear_hip_topk_f32_warm(const float *priorities, int64_t n, int64_t k, int so
  * semantics of WeightUpdateRequestArray::update (src/index/request.cc:41-51): when an index
  * occurs more than once the LAST occurrence wins.
  *   unique_indices != 0: caller guarantees no duplicates; plain scatter, no workspace needed.
- *   unique_indices == 0: duplicates resolved deterministically with a stable radix sort of the
- *                        indices; workspace of gear_hip_scatter_workspace_bytes(num) bytes.
+ *   unique_indices == 0: duplicates resolved deterministically (a hash table of the indices, or a
+ *                        stable radix sort of them); workspace of gear_hip_scatter_workspace_bytes(num) bytes.
  * Indices outside [0,n) are ignored. */
 size_t gear_hip_scatter_workspace_bytes(int64_t num);
 int gear_hip_scatter_f32(float *weights, int64_t n, const int64_t *idx, const float *values,
