@@ -4,7 +4,7 @@
 // granules of its range, adds them up in order, and one DPP wave scan per range joins the
 // threads (a wave-private LDS row turns the row-major order of the memory instructions, 1 KiB of
 // consecutive addresses per wave and instruction, into that blocked order and back):
-//  * chained single pass, up to 4096 ranges (of up to 16384 fp32 elements: 67 M):
+//  * chained single pass, up to 8192 ranges (of up to 16384 fp32 elements: 134 M):
 //    scan_ranges_kernel<kChained>.  A workgroup
 //    keeps its range in registers, publishes the range's sum and adds the sums of ALL earlier
 //    ranges (fixed order: bit-reproducible), then writes the prefix: the input is read once.
@@ -63,7 +63,9 @@ __device__ __forceinline__ void store_vec(V *p, V v, bool nt) {
 // sum of ALL earlier ranges' sums (each thread adds its share of them, fixed summation order).
 // Nobody waits for an inclusive value, so there is no serial chain across the XCDs, and the result
 // is bit-reproducible from run to run.
-constexpr int kMaxRanges = 4096;      // chained: every thread polls up to 16 range sums
+constexpr int kMaxRanges = 8192;      // chained: every thread polls up to 32 range sums
+constexpr int kMaxRanges8 = 4096;     // ... of ranges of 8 granules per thread
+static_assert(kMaxRanges / 32 <= kBlock, "a thread per word of the missing ranges");
 constexpr int kMaxRangesTwo = 16384;  // two launches: every thread adds up to 64 range sums
 
 // A range sum in flight between workgroups of one launch: three self-validating words.
@@ -643,18 +645,19 @@ int launch_scan(const In *in, Out *out, int64_t n, void *ws, size_t ws_bytes, hi
   // Ranges of 2, 4, 8 or 16 granules per thread (2048 to 16384 fp32 elements): 2 while that
   // leaves at most 256 ranges, 4 up to 512 ranges, then 8 (a workgroup adds up ALL earlier sums, so
   // more ranges cost more than they gain once every CU has work), and 16 -- 190 registers, two
-  // workgroups per CU -- where 8 would need more than 4096 ranges (33.5 to 67 M fp32: one read
-  // instead of two, 187 -> 148 us at 6e7).  The chained kernel and the two launches cut the input
+  // workgroups per CU -- where 8 would need more than 4096 ranges (33.5 to 134 M fp32: one read
+  // instead of two, us at 6e7 / 6.8e7 / 1e8 / 1.3e8: 148 / 167 / 240 / 330 against 187 / 213 / 308 /
+  // 399; int64 at 4e7 / 6e7: 143 / 235 against 183 / 267).  The chained kernel and the two launches cut the input
   // the same way, so a rescan finds the sums of the last full scan.
-  // Beyond 4096 ranges the words to poll outweigh the second read: two launches, up to 16384
-  // ranges of 8 granules.  (8-byte elements: ranges of 2 granules would be smaller than the 2048 elements the
+  // At 8192 ranges the words to poll are 0.8 GB beside 1.6 GB of data; beyond that they outweigh
+  // the second read: two launches, up to 16384 ranges of 8 granules.  (8-byte elements: ranges of 2 granules would be smaller than the 2048 elements the
   // workspace is laid out for, so they start at 4.)
   constexpr int64_t g1 = (int64_t)kBlock * VE;  // elements per range and granule
   if (VE == 4 && ceil_div64(n, 2 * g1) <= 256)
     return launch_ranges<In, Acc, Out, VE, 2>(in, out, n, ws, st, chained, first_changed);
   else if (ceil_div64(n, 4 * g1) <= 512)
     return launch_ranges<In, Acc, Out, VE, 4>(in, out, n, ws, st, chained, first_changed);
-  else if (ceil_div64(n, 8 * g1) <= kMaxRanges)
+  else if (ceil_div64(n, 8 * g1) <= kMaxRanges8)
     return launch_ranges<In, Acc, Out, VE, 8>(in, out, n, ws, st, chained, first_changed);
   else if (ceil_div64(n, 16 * g1) <= kMaxRanges)
     return launch_ranges<In, Acc, Out, VE, 16>(in, out, n, ws, st, chained, first_changed);
