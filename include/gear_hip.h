@@ -296,9 +296,8 @@ int gear_hip_sample_sorted_f64(const double *prefix, int64_t n, const float *u, 
  * for a sampler whose index array ascends (then sort(indices[p]) == indices[sort(p)]), the chain
  * torch.sort(concat_indices[draws]) (gear/sampler/global_sampler.py:131,172,196),
  * indices - index_offset and iset.timesteps[indices.cpu()] on the host
- * (gear/loader/offline_loader.py:161-177): up to 4096 positions take ONE launch after the search
- * (the ranking sort does the look-ups of the entry it places), more take the radix sort and an
- * element-wise launch.
+ * (gear/loader/offline_loader.py:161-177): up to 32768 positions or draws take ONE launch (search,
+ * order and look-ups), more take the radix sort and an element-wise launch.
  *   gear_hip_sample_lookup_f64  positions = upper_bound of the draws u in the fp64 prefix, as
  *                               gear_hip_upper_bound_f64 (index_table, when given, has n entries)
  *   gear_hip_sample_lookup_i64  the same in an int64 prefix (a sampler over lengths), u as for
