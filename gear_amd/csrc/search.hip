@@ -425,7 +425,7 @@ int place_draws(const Draw &draw, int64_t num, const Emit &emit, hipStream_t st)
 // ---- larger batches: the one-launch sort ----------------------------------------------------------
 // The same idea beyond kRankMax draws: the draws are put in order by their keys, and the workgroup
 // that places a draw searches it too -- the search, two launches a digit of the radix sort and the
-// look-ups are one launch: 20 000 draws in 1e6 entries 14.7 us (27.5 with a launch for the search
+// look-ups are one launch: 20 000 draws in 1e6 entries 14.9 us (27.5 with a launch for the search
 // and six for the sort), 20 000 integer draws in 1e5 entries 17.8 (29.5), positions 11.3 (23.9).
 inline __device__ uint32_t sort_key(uint32_t k) { return k; }
 inline __device__ uint64_t sort_key(int64_t k) { return (uint64_t)k ^ (1ull << 63); }
@@ -443,13 +443,15 @@ template <typename Draw, typename Emit>
 struct DrawEmit {
   Draw draw;
   Emit emit;
+  int lanes;  // per draw: the same everywhere, so that a larger target never finds a smaller entry
+              // whatever the prefix holds (an ulp less behind a zero priority)
   template <int kLanes>
   __device__ __forceinline__ int64_t search(int j) const {
     return group_search<kLanes>(draw.prefix, draw.n, (int)threadIdx.x & (kLanes - 1),
                                 [&](typename Draw::type total) { return draw.target(j, total); });
   }
   __device__ __forceinline__ typename Emit::Resolved find(int j) const {
-    return emit.resolve(search<16>(j));
+    return emit.resolve(lanes == 16 ? search<16>(j) : lanes == 8 ? search<8>(j) : search<1>(j));
   }
   __device__ __forceinline__ void put(uint32_t place, int, const typename Emit::Resolved &r) const {
     emit.store((int64_t)place, r);
@@ -457,18 +459,17 @@ struct DrawEmit {
   template <int kLanes, typename L>
   __device__ __forceinline__ void list_by(const L &list, const uint32_t *rank, int n,
                                           uint32_t base) const {
-    const int e = (int)threadIdx.x / kLanes;
-    if (e >= n) return;
-    const auto r = emit.resolve(search<kLanes>(list.pos(e)));
-    if ((threadIdx.x & (kLanes - 1)) == 0) emit.store((int64_t)(base + rank[e]), r);
+    for (int e = (int)threadIdx.x / kLanes; e < n; e += ranges::kThreads / kLanes) {
+      const auto r = emit.resolve(search<kLanes>(list.pos(e)));
+      if ((threadIdx.x & (kLanes - 1)) == 0) emit.store((int64_t)(base + rank[e]), r);
+    }
   }
-  // as many lanes a draw as let the workgroup search its draws at the same time
   template <typename L>
   __device__ __forceinline__ void list(const L &list, const uint32_t *rank, int n,
                                        uint32_t base) const {
-    if (n <= ranges::kThreads / 16)
+    if (lanes == 16)
       list_by<16>(list, rank, n, base);
-    else if (n <= ranges::kThreads / 8)
+    else if (lanes == 8)
       list_by<8>(list, rank, n, base);
     else
       list_by<1>(list, rank, n, base);
@@ -521,8 +522,10 @@ bool one_launch(const Draw &draw, int64_t num, const Emit &emit) {
 template <typename Draw, typename Emit>
 int sort_draws(const Draw &draw, int64_t num, const Emit &emit, hipStream_t st) {
   typedef DrawSrc<Draw> Src;
-  return ranges::sort<typename Src::key_type, false>(Src{draw, {}}, num, DrawEmit<Draw, Emit>{draw, emit},
-                                                     st);
+  // as many lanes a draw as let a workgroup search most shares (num / 256 draws) in one round
+  const int lanes = num <= 12288 ? 16 : num <= 24576 ? 8 : 1;
+  return ranges::sort<typename Src::key_type, false>(
+      Src{draw, {}}, num, DrawEmit<Draw, Emit>{draw, emit, lanes}, st);
 }
 
 __global__ __launch_bounds__(kBlock) void lookup_kernel(const int64_t *__restrict__ positions,
