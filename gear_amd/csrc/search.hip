@@ -421,6 +421,13 @@ int place_draws(const Draw &draw, int64_t num, const Emit &emit, hipStream_t st)
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
   return 0;
 }
+template <typename Emit>
+int place_positions(const int64_t *raw, int64_t num, const Emit &emit, hipStream_t st) {
+  place_positions_kernel<<<dim3((unsigned)ceil_div64(num, kPlaced)), dim3(kPlaceThreads), 0, st>>>(
+      raw, (int)num, emit);
+  GEARHIP_RETURN_IF_LAUNCH_FAILED();
+  return 0;
+}
 
 // ---- larger batches: the one-launch sort ----------------------------------------------------------
 // The same idea beyond kRankMax draws: the draws are put in order by their keys, and the workgroup
@@ -509,14 +516,13 @@ inline bool writes_over(const Lookup &l, const void *p, int64_t bytes, int64_t n
          ranges::overlap(l.lens, num * 8, p, bytes) || ranges::overlap(l.starts, num * 8, p, bytes);
 }
 
-// Whether a batch beyond kRankMax draws goes through the one-launch sort: it fits, and nothing that
-// one workgroup stores is still to be read by another (outputs on top of the draws or the prefix
-// keep the separate launches, where reading ends before writing begins).
+// Whether a batch can be searched and stored by one launch: nothing that one workgroup stores is
+// still to be read by another.  Outputs on top of the draws or the prefix take separate launches,
+// where reading ends before writing begins.
 template <typename Draw, typename Emit>
-bool one_launch(const Draw &draw, int64_t num, const Emit &emit) {
+bool apart(const Draw &draw, int64_t num, const Emit &emit) {
   const int64_t u_bytes = num * (sizeof(typename Draw::type) == 8 && sizeof(typename Draw::key_type) == 8 ? 8 : 4);
-  return ranges::fits(num) &&
-         !writes_over(emit, draw.u, u_bytes, num) && !writes_over(emit, draw.prefix, draw.n * 8, num);
+  return !writes_over(emit, draw.u, u_bytes, num) && !writes_over(emit, draw.prefix, draw.n * 8, num);
 }
 
 template <typename Draw, typename Emit>
@@ -651,10 +657,13 @@ extern "C" int gear_hip_sample_sorted_f64(const double *prefix, int64_t n, const
   const int64_t blocks = ceil_div64(num, kBlock);
   const Split split{sorted_out, trajectory_length, modulo, idxs, tss, lens};
   const DrawF64 draw{prefix, n, u, unit_uniforms ? 1 : 0};
-  if (num <= radix::kRankMax) return place_draws(draw, num, split, st);
-  if (one_launch(draw, num, split)) return sort_draws(draw, num, split, st);
+  if (apart(draw, num, split)) {
+    if (num <= radix::kRankMax) return place_draws(draw, num, split, st);
+    if (ranges::fits(num)) return sort_draws(draw, num, split, st);
+  }
   int rc = launch_search(draw, num, raw, st);
   if (rc) return rc;
+  if (num <= radix::kRankMax) return place_positions(raw, num, split, st);
   int64_t *sorted = sorted_out ? sorted_out : reinterpret_cast<int64_t *>(ws + w.sorted);
   rc = radix::sort_pairs<uint64_t, uint64_t>(
       reinterpret_cast<const uint64_t *>(raw), reinterpret_cast<uint64_t *>(sorted), nullptr,
@@ -683,15 +692,11 @@ int check_lookup(const Lookup &look) {
 // raw: num positions on the device (each in [0, bound)); sorted ascending, then looked up.
 int sort_and_look_up(const int64_t *raw, int64_t num, int64_t bound, const Lookup &look, char *ws,
                      const SampleWs &w, hipStream_t st) {
-  if (num <= radix::kRankMax) {
-    place_positions_kernel<<<dim3((unsigned)ceil_div64(num, kPlaced)), dim3(kPlaceThreads), 0, st>>>(
-        raw, (int)num, look);
-    GEARHIP_RETURN_IF_LAUNCH_FAILED();
-    return 0;
-  }
+  const bool over = writes_over(look, raw, num * 8, num);  // (then reading ends before writing begins)
+  if (num <= radix::kRankMax && !over) return place_positions(raw, num, look, st);
   int key_bits = 1;
   while (key_bits < 63 && ((uint64_t)(bound - 1) >> key_bits) != 0) ++key_bits;
-  if (key_bits <= 32 && ranges::fits(num) && !writes_over(look, raw, num * 8, num))
+  if (key_bits <= 32 && ranges::fits(num) && !over)
     return ranges::sort<uint32_t, false>(PositionSrc{raw, (uint32_t)(((uint64_t)1 << key_bits) - 1)},
                                          num, PositionEmit{raw, look}, st);
   int64_t *sorted = reinterpret_cast<int64_t *>(ws + w.sorted);
@@ -709,8 +714,10 @@ int sort_and_look_up(const int64_t *raw, int64_t num, int64_t bound, const Looku
 template <typename Draw>
 int draw_and_look_up(const Draw &draw, int64_t num, const Lookup &look, char *ws, const SampleWs &w,
                      hipStream_t st) {
-  if (num <= radix::kRankMax) return place_draws(draw, num, look, st);
-  if (one_launch(draw, num, look)) return sort_draws(draw, num, look, st);
+  if (apart(draw, num, look)) {
+    if (num <= radix::kRankMax) return place_draws(draw, num, look, st);
+    if (ranges::fits(num)) return sort_draws(draw, num, look, st);
+  }
   int64_t *raw = reinterpret_cast<int64_t *>(ws + w.raw);
   const int rc = launch_search(draw, num, raw, st);
   if (rc) return rc;
