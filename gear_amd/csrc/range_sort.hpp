@@ -5,15 +5,19 @@
 // which the work is a fraction.  Here every workgroup works alone.  It reads ALL keys (held in
 // registers, so one pass over L2), finds the two keys between which its share of the sorted batch
 // lies -- a histogram of the keys over 4096 equal ranges, refined where one range holds too many
-// -- collects the keys in between in LDS, ranks them there by counting, and writes them out.
+// -- collects the keys in between in LDS, ranks them there by counting, and writes them out.  Keys
+// that are repeated more often than a list holds are not ranked: their order is that of the batch.
 // Nothing passes between workgroups: no scratch, no second launch, and the cuts come out the same
 // everywhere because they depend on the keys alone.  The price is that 256 workgroups each count
 // the whole batch (an LDS atomic a key), which is why larger batches keep the radix sort.
 // us a call, back to back, here / radix sort (63-bit keys need 40 registers a thread more):
-//     keys     20 bits       63 bits     63 bits, in order
-//      4097   7.6 / 20.7    9.7 / 55.1      5.4 / 55.5
-//     20000  12.1 / 21.6   15.9 / 58.0      8.4 / 58.2
-//     32768  16.4 / 22.2   26.9 / 59.2     16.7 / 59.6
+//     keys     20 bits      63 bits      63 bits, in order
+//      4097   7.7 / 20.0    9.1 / 53.6      5.4 / 55.5
+//     20000  12.4 / 21.4   15.3 / 57.5      8.4 / 58.2
+//     32768  16.6 / 22.0   24.2 / 59.1     13.5 / 59.6
+// A batch of a few keys, each many times over, takes longer, for the passes that find its runs: 19.6 /
+// 21.9 for 20000 keys of two values, 26.3 / 22.4 for 32768 of them, 38.5 / 59.8 where they are 63 bits
+// wide, 37.0 / 59.4 for 5000 values and one far away.
 // At 40 000 keys of 20 bits the two meet (64 registers of keys a thread spill: 64 us).
 #pragma once
 #include "radix_sort.hpp"
@@ -29,8 +33,11 @@ constexpr int kBinBits = 12;
 constexpr int kBins = 1 << kBinBits;
 constexpr int kPerThread = kBins / kThreads;
 static_assert(kPerThread == 4, "a thread's bins are one 16-byte word");
+constexpr int kBanks = 64;
+constexpr int kCopies = 8;             // of the counts, where many lanes count in the same bank
+constexpr int kCopy = kBins + 4;       // (in different banks)
 constexpr int kCap = 1024;             // keys ranked at once in LDS
-constexpr int kTol = 512;              // a cut may leave its place by so many keys
+constexpr int kTol = 448;              // a cut may leave its place by so many keys
 constexpr int kMax = 32 * kThreads;    // largest batch: the keys of a thread stay in registers
 static_assert(kMax / kGroups + kTol <= kCap, "a share without repeated keys fits in LDS");
 
@@ -90,11 +97,11 @@ struct Cut {
 
 template <typename C>
 struct Smem {
-  __align__(16) uint32_t hist[kBins + 1];  // counts, then exclusive sums; the last entry is the total
+  __align__(16) uint32_t hist[kCopies * kCopy];
   uint32_t wsum[kWaves];
   C wmin[kWaves], wmax[kWaves], wfirst[kWaves];
   Cut<C> cut[2];
-  int sorted, found, n;
+  int sorted, crowd, n;
   List<C> list;
   uint32_t rank[kCap];
 };
@@ -111,16 +118,13 @@ __device__ __forceinline__ int shift_of(uint64_t last) {
 
 // A thread's elements: wave w holds the elements [w, w + 1) * per * 64, round i of them the elements
 // 64 * i + lane; so elements in order are (wave, round, lane) in order.  The keys (less the smallest
-// one) are in registers for the passes that every batch takes; the passes that only batches with
-// crowded keys take ask the source again (each(), a rolled loop: unrolled ones made the kernel spill).
-template <typename C, int kRounds, typename Src>
+// one) stay in registers for all passes: reading them again is a round trip to L2 a round.
+template <typename C, int kRounds>
 struct Keys {
-  const Src &src;
+  static constexpr int kHeld = kRounds;
   C k[kRounds];
-  C mn;
   int first;   // element of round 0
-  int per;     // rounds in use
-  int rounds;  // of them, this thread's
+  int rounds;  // this thread's
   // the rounds again, unknown to the compiler: comparisons with it are not kept from pass to pass
   __device__ __forceinline__ int own_rounds() const {
     int r = rounds;
@@ -128,35 +132,49 @@ struct Keys {
     return r;
   }
   __device__ __forceinline__ int element(int i) const { return first + i * kWave; }
-  // f(round is this thread's, element, key): as often in every lane of a wave
-  template <typename F>
-  __device__ __forceinline__ void each(const F &f) const {
-#pragma unroll 1
-    for (int i = 0; i < per; ++i) {
-      const bool ok = i < rounds;
-      f(ok, element(i), ok ? (C)(src.key(element(i)) - mn) : (C)0);
-    }
-  }
-  template <typename F>
-  __device__ __forceinline__ void each_held(const F &f) const {
-    const int r = own_rounds();
-#pragma unroll
-    for (int i = 0; i < kRounds; ++i)
-      if (i < r) f(element(i), k[i]);
-  }
 };
 
 template <typename C>
-__device__ __forceinline__ void clear_counts(Smem<C> &sm) {
-  reinterpret_cast<u32x4 *>(sm.hist)[threadIdx.x] = u32x4{0, 0, 0, 0};
+__device__ __forceinline__ void wave_min_max(C &mn, C &mx) {
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) {
+    const C a = __shfl_xor(mn, off, kWave), b = __shfl_xor(mx, off, kWave);
+    mn = a < mn ? a : mn;
+    mx = b > mx ? b : mx;
+  }
 }
 
-// The counts of this thread's bins, and the sum of those before them.
+// A thread's four bins of every copy.
 template <typename C>
-__device__ __forceinline__ uint32_t sum_counts(Smem<C> &sm, u32x4 &c) {
+__device__ __forceinline__ void clear_counts(Smem<C> &sm, int first, int copies) {
+  for (int i = first; i < copies; ++i)
+    reinterpret_cast<u32x4 *>(sm.hist + i * kCopy)[threadIdx.x] = u32x4{0, 0, 0, 0};
+}
+
+// The keys (kAll), or those in [lo, last], counted over ranges of 1 << s keys.  Lanes that count in the
+// same bank are served one after the other; in a crowd neighbours count in different copies.
+template <bool kAll, typename C, typename K>
+__device__ __forceinline__ void count_ranges(Smem<C> &sm, const K &keys, C lo, C last, int s, bool crowd) {
+  const int r = keys.own_rounds();
+  uint32_t *hist = sm.hist + (crowd ? (int)(threadIdx.x & (kCopies - 1)) * kCopy : 0);
+  const C width = (C)(last - lo);
+#pragma unroll
+  for (int i = 0; i < K::kHeld; ++i) {
+    const C at = kAll ? keys.k[i] : (C)(keys.k[i] - lo);
+    if (i < r && (kAll || at <= width)) atomicAdd(&hist[(uint32_t)(at >> s)], 1u);
+  }
+}
+
+// The counts of this thread's bins, and the sum of those before them; the counts are clear again after
+// the next barrier.
+template <typename C>
+__device__ __forceinline__ uint32_t sum_counts(Smem<C> &sm, bool crowd, u32x4 &c) {
   const int tid = threadIdx.x;
   __syncthreads();
   c = reinterpret_cast<const u32x4 *>(sm.hist)[tid];
+  if (__builtin_expect(crowd, 0))
+    for (int i = 1; i < kCopies; ++i) c += reinterpret_cast<const u32x4 *>(sm.hist + i * kCopy)[tid];
+  clear_counts(sm, 0, crowd ? kCopies : 1);
   const int total = (int)(c[0] + c[1] + c[2] + c[3]);
   const int inc = wave_inclusive_sum(total);
   if ((tid & (kWave - 1)) == kWave - 1) sm.wsum[tid / kWave] = (uint32_t)inc;
@@ -167,70 +185,109 @@ __device__ __forceinline__ uint32_t sum_counts(Smem<C> &sm, u32x4 &c) {
   return run;
 }
 
-// The sums for the keys in [lo, last] over ranges of 1 << s keys.
+// The smallest and the largest key in [lo, last].
 template <typename C, typename K>
-__device__ __forceinline__ void count_ranges(Smem<C> &sm, const K &keys, C lo, C last, int s) {
-  clear_counts(sm);
-  __syncthreads();
-  keys.each([&](bool ok, int, C k) {
-    if (ok && k >= lo && k <= last) atomicAdd(&sm.hist[(uint32_t)((k - lo) >> s) & (kBins - 1)], 1u);
-  });
-  u32x4 c;
-  const uint32_t run = sum_counts(sm, c);
-  reinterpret_cast<u32x4 *>(sm.hist)[threadIdx.x] =
-      u32x4{run, run + c[0], run + c[0] + c[1], run + c[0] + c[1] + c[2]};
-  if (threadIdx.x == kThreads - 1) sm.hist[kBins] = run + c[0] + c[1] + c[2] + c[3];
-  __syncthreads();
-}
-
-// The range f with hist[f] <= at < hist[f + 1]; at is below the total, so there is exactly one.
-template <typename C>
-__device__ __forceinline__ int range_at(Smem<C> &sm, uint32_t at) {
-  const int b0 = (int)threadIdx.x * kPerThread;
+__device__ __forceinline__ void tighten(Smem<C> &sm, const K &keys, C &lo, C &last) {
+  const int r = keys.own_rounds();
+  const C width = (C)(last - lo);
+  C mn = width, mx = 0;
 #pragma unroll
-  for (int i = 0; i < kPerThread; ++i)
-    if (sm.hist[b0 + i] <= at && at < sm.hist[b0 + i + 1]) sm.found = b0 + i;
+  for (int i = 0; i < K::kHeld; ++i) {
+    const C at = (C)(keys.k[i] - lo);
+    const bool takes = i < r && at <= width;
+    mn = takes && at < mn ? at : mn;
+    mx = takes && at > mx ? at : mx;
+  }
+  wave_min_max(mn, mx);
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+    sm.wmin[threadIdx.x / kWave] = mn;
+    sm.wmax[threadIdx.x / kWave] = mx;
+  }
   __syncthreads();
-  const int f = sm.found;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    mn = sm.wmin[w] < mn ? sm.wmin[w] : mn;
+    mx = sm.wmax[w] > mx ? sm.wmax[w] : mx;
+  }
+  last = (C)(lo + mx);
+  lo = (C)(lo + mn);
   __syncthreads();
-  return f;
 }
 
-// Moves a cut up towards its place while the range that holds it has too many keys.
+template <typename C>
+__device__ __forceinline__ bool too_many(const Cut<C> &c) { return c.count > (uint32_t)kTol && c.s > 0; }
+
+// The cuts for the places at0 and at1 (num: none) of a batch with keys up to `all`: each moves towards
+// its place until the range that holds it has few keys, or is one key.  A range that holds both is
+// counted once.  When it begins the first copy of the counts is clear; crowd: neighbours' keys share
+// ranges, all copies are clear.
 template <typename C, typename K>
-__device__ __forceinline__ void refine(Smem<C> &sm, const K &keys, Cut<C> &cut, uint32_t at) {
-  while (cut.count > (uint32_t)kTol && cut.s > 0) {
-    const int s = cut.s > kBinBits ? cut.s - kBinBits : 0;
-    count_ranges(sm, keys, cut.lo, (C)(cut.lo + (((C)1 << cut.s) - 1)), s);
-    const int f = range_at(sm, at - cut.below);
-    cut.lo += (C)((C)f << s);
-    cut.count = sm.hist[f + 1] - sm.hist[f];
-    cut.below += sm.hist[f];
-    cut.s = s;
+__device__ __forceinline__ void find_cuts(Smem<C> &sm, const K &keys, C all, uint32_t num, uint32_t at0,
+                                          uint32_t at1, bool crowd, Cut<C> &from, Cut<C> &to) {
+  from = Cut<C>{0, 0u, num, 0};
+  to = at1 < num ? from : Cut<C>{0, num, 0u, 0};
+  if (all == 0) return;
+  const bool split = at1 < num;
+  auto place = [&](C lo, int s, bool crowd, bool mine0, bool mine1) {
+    u32x4 c;
+    uint32_t run = sum_counts(sm, crowd, c);
+#pragma unroll
+    for (int i = 0; i < kPerThread; ++i) {
+      const C low = (C)(lo + ((C)(threadIdx.x * kPerThread + i) << s));
+      const uint32_t p0 = at0 - from.below, p1 = at1 - to.below;
+      if (mine0 && run <= p0 && p0 < run + c[i]) sm.cut[0] = Cut<C>{low, from.below + run, c[i], s};
+      if (mine1 && run <= p1 && p1 < run + c[i]) sm.cut[1] = Cut<C>{low, to.below + run, c[i], s};
+      run += c[i];
+    }
     __syncthreads();
+    if (mine0) from = sm.cut[0];
+    if (mine1) to = sm.cut[1];
+  };
+  count_ranges<true>(sm, keys, (C)0, all, shift_of(all), crowd);
+  place(0, shift_of(all), crowd, true, split);
+  bool clear = crowd;
+  for (;;) {
+    const bool mine0 = too_many(from);
+    const bool mine1 = too_many(to) && (!mine0 || (to.lo == from.lo && to.s == from.s));
+    if (__builtin_expect(!mine0 && !mine1, 1)) return;
+    C lo = mine0 ? from.lo : to.lo;
+    C last = (C)(lo + (((C)1 << (mine0 ? from.s : to.s)) - 1));
+    const bool many = (mine0 ? from.count : to.count) > num / 8;
+    if (many || (mine0 ? from.s : to.s) > 2 * kBinBits) {
+      // a few keys in a corner of the range, or one: a pass instead of one a level
+      tighten(sm, keys, lo, last);
+      if (lo == last) {
+        if (mine0) from.lo = lo, from.s = 0;
+        if (mine1) to.lo = lo, to.s = 0;
+        continue;
+      }
+    }
+    if (many && !clear) {
+      clear_counts(sm, 1, kCopies);
+      __syncthreads();
+      clear = true;
+    }
+    const int s = shift_of((C)(last - lo));
+    count_ranges<false>(sm, keys, lo, last, s, many);
+    place(lo, s, many, mine0, mine1);
   }
 }
 
 // The keys in [lo, last], at most kCap, ranked and handed to emit.list as the places from `base`.
-template <bool kHeld, typename C, typename K, typename Emit>
+template <typename C, typename K, typename Emit>
 __device__ __forceinline__ void emit_window(Smem<C> &sm, const K &keys, C lo, C last, uint32_t base,
                                             uint32_t room, const Emit &emit) {
   const int tid = threadIdx.x;
   if (tid == 0) sm.n = 0;
   sm.rank[tid] = 0;
   __syncthreads();
-  auto collect = [&](int j, C k) {
-    if ((C)(k - lo) <= (C)(last - lo)) {
+  const int r = keys.own_rounds();
+#pragma unroll
+  for (int i = 0; i < K::kHeld; ++i)
+    if (i < r && (C)(keys.k[i] - lo) <= (C)(last - lo)) {
       const int slot = atomicAdd(&sm.n, 1);
-      if (slot < kCap) sm.list.put(slot, k, j);
+      if (slot < kCap) sm.list.put(slot, keys.k[i], keys.element(i));
     }
-  };
-  if constexpr (kHeld)
-    keys.each_held(collect);
-  else
-    keys.each([&](bool ok, int j, C k) {
-      if (ok) collect(j, k);
-    });
   __syncthreads();
   const int limit = room < (uint32_t)kCap ? (int)room : kCap, n = sm.n < limit ? sm.n : limit;
   // thread = (part of the list, key of it)
@@ -250,38 +307,43 @@ __device__ __forceinline__ void emit_window(Smem<C> &sm, const K &keys, C lo, C 
   }
   __syncthreads();
   emit.list(sm.list, sm.rank, n, base);
-  __syncthreads();
 }
 
-// All elements whose key is v, in their order, as the places from `base`.
+// The places [p0, p1) of the sorted batch, at most kCap, which hold elements of the one key v whose
+// elements, in their order, take the places from `start`.
 template <typename C, typename K, typename Emit>
-__device__ __forceinline__ void emit_equal(Smem<C> &sm, const K &keys, C v, uint32_t base,
-                                           uint32_t room, const Emit &emit) {
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+__device__ __forceinline__ void emit_equal(Smem<C> &sm, const K &keys, C v, uint32_t start, uint32_t p0,
+                                           uint32_t p1, const Emit &emit) {
+  if (p0 >= p1) return;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const int r = keys.own_rounds();
   uint32_t mine = 0;
-  keys.each([&](bool ok, int j, C k) {
-    const bool hit = ok && k == v;
-    mine += (uint32_t)__popcll(wave_ballot(hit));
-    if (hit) sm.found = j;  // any of them: equal keys find the same
-  });
+#pragma unroll
+  for (int i = 0; i < K::kHeld; ++i) mine += (uint32_t)__popcll(wave_ballot(i < r && keys.k[i] == v));
   if (lane == 0) sm.wsum[wave] = mine;
+  sm.rank[threadIdx.x] = 0;
   __syncthreads();
-  const auto what = emit.find(sm.found);
-  const uint32_t end = base + room;
-  for (int w = 0; w < wave; ++w) base += sm.wsum[w];
-  keys.each([&](bool ok, int j, C k) {
-    const bool hit = ok && k == v;
-    const uint64_t hits = wave_ballot(hit);
-    const uint32_t place = base + (uint32_t)__popcll(hits & ((1ull << lane) - 1));
-    if (hit && place < end) emit.put(place, j, what);
-    base += (uint32_t)__popcll(hits);
-  });
+  uint32_t place = start;  // of the wave's next element
+  for (int w = 0; w < wave; ++w) place += sm.wsum[w];
+  if (place < p1 && place + mine > p0) {
+#pragma unroll
+    for (int i = 0; i < K::kHeld; ++i) {
+      const bool hit = i < r && keys.k[i] == v;
+      const uint64_t hits = wave_ballot(hit);
+      const uint32_t at = place + (uint32_t)__popcll(hits & ((1ull << lane) - 1));
+      if (hit && at >= p0 && at < p1 && at - p0 < (uint32_t)kCap) sm.rank[at - p0] = (uint32_t)keys.element(i);
+      place += (uint32_t)__popcll(hits);
+    }
+  }
   __syncthreads();
+  emit.equal(sm.rank, (int)(p1 - p0 < (uint32_t)kCap ? p1 - p0 : kCap), p0);
 }
 
-// Src: C key(j), the key of element j.  Emit: list(list, rank, n, base) stores n collected elements
-// at base + rank, by all threads; find(j) + put(place, j, found) store one of many equal keys.
-// kLook: a batch that is in order already is passed on without a histogram.
+// Src: C key(j), the key of element j.  Emit, by all threads: list(list, rank, n, base) stores n
+// collected elements at base + rank; equal(at, n, base) stores the elements at[0..n) of one key at
+// base, base + 1, ...  kLook: a batch that is in order already is passed on without a histogram
+// (Emit::put(place, j) stores element j).
 template <typename C, int kRounds, bool kLook, typename Src, typename Emit>
 __global__ __launch_bounds__(kThreads) void range_sort_kernel(Src src, int num, Emit emit) {
   __shared__ Smem<C> sm;
@@ -290,8 +352,8 @@ __global__ __launch_bounds__(kThreads) void range_sort_kernel(Src src, int num, 
   const int per = (num + kThreads - 1) / kThreads;
   const int first = wave * per * kWave + lane;
   const int left_here = num - first + kWave - 1;
-  Keys<C, kRounds, Src> keys{src, {}, (C)0, first, per,
-                             left_here <= 0 ? 0 : left_here / kWave < per ? left_here / kWave : per};
+  Keys<C, kRounds> keys{
+      {}, first, left_here <= 0 ? 0 : left_here / kWave < per ? left_here / kWave : per};
   const int own0 = (int)((int64_t)blockIdx.x * num / kGroups);
   const int own1 = (int)((int64_t)(blockIdx.x + 1) * num / kGroups);
   src.begin();
@@ -302,7 +364,7 @@ __global__ __launch_bounds__(kThreads) void range_sort_kernel(Src src, int num, 
     keys.k[i] = 0;
     if (i < per) keys.k[i] = src.key(j < num ? j : num - 1);
   }
-  clear_counts(sm);  // (before the first barrier)
+  clear_counts(sm, 0, 1);  // (before the first barrier)
   bool ordered = true;
   C edge = 0;  // the last key of the round before
   {
@@ -322,13 +384,11 @@ __global__ __launch_bounds__(kThreads) void range_sort_kernel(Src src, int num, 
       }
     }
   }
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    const C a = __shfl_xor(mn, off, kWave), b = __shfl_xor(mx, off, kWave);
-    mn = a < mn ? a : mn;
-    mx = b > mx ? b : mx;
+  wave_min_max(mn, mx);
+  if (tid == 0) {
+    sm.sorted = 1;
+    sm.crowd = 0;
   }
-  if (tid == 0) sm.sorted = 1;
   if (lane == 0) {
     sm.wmin[wave] = mn;
     sm.wmax[wave] = mx;
@@ -345,79 +405,55 @@ __global__ __launch_bounds__(kThreads) void range_sort_kernel(Src src, int num, 
     mn = sm.wmin[w] < mn ? sm.wmin[w] : mn;
     mx = sm.wmax[w] > mx ? sm.wmax[w] : mx;
   }
+  // neighbours of a wave's first round that count in one bank of LDS tell whether many keys do
+  const C all = mx - mn;
+  const C before = (C)(lane_before(keys.k[0]) - mn);
+  const bool shared = 0 < keys.own_rounds() && lane > 0 &&
+                      (((before ^ (C)(keys.k[0] - mn)) >> shift_of(all)) & (kBanks - 1)) == 0;
+  if (__popcll(wave_ballot(shared)) >= kWave / 8 && lane == 0) sm.crowd = 1;
   __syncthreads();
-  if (kLook && sm.sorted) {
-    for (int j = own0 + tid; j < own1; j += kThreads) emit.put((uint32_t)j, j, emit.find(j));
-    return;
+  if constexpr (kLook) {
+    if (sm.sorted) {
+      for (int j = own0 + tid; j < own1; j += kThreads) emit.put((uint32_t)j, j);
+      return;
+    }
   }
-  keys.mn = mn;
+  const bool crowd = sm.crowd != 0;
+  if (__builtin_expect(crowd, 0)) {
+    clear_counts(sm, 1, kCopies);
+    __syncthreads();
+  }
 #pragma unroll
   for (int i = 0; i < kRounds; ++i) keys.k[i] -= mn;
-  const C all = mx - mn;
-  const int s = shift_of(all);
-  keys.each_held([&](int, C k) { atomicAdd(&sm.hist[(uint32_t)(k >> s)], 1u); });
-  {
-    u32x4 c;
-    uint32_t run = sum_counts(sm, c);
-#pragma unroll
-    for (int i = 0; i < kPerThread; ++i) {
-      const C lo = (C)((C)(tid * kPerThread + i) << s);
-      if (run <= (uint32_t)own0 && (uint32_t)own0 < run + c[i]) sm.cut[0] = Cut<C>{lo, run, c[i], s};
-      if (run <= (uint32_t)own1 && (uint32_t)own1 < run + c[i]) sm.cut[1] = Cut<C>{lo, run, c[i], s};
-      run += c[i];
-    }
-  }
-  __syncthreads();
-  Cut<C> from = sm.cut[0], to = {0, (uint32_t)num, 0, 0};
-  if (own1 < num) to = sm.cut[1];
-  refine(sm, keys, from, (uint32_t)own0);
-  refine(sm, keys, to, (uint32_t)own1);
-  uint32_t left = to.below - from.below, base = from.below;
-  // (a share is empty where its neighbour's cut is the same; the limits here and below keep every
-  // place inside the batch and every loop finite even if the source changes while it is read)
-  if (to.below <= from.below || to.below > (uint32_t)num) return;
-  const C last = own1 < num ? (C)(to.lo - 1) : all;
-  C cur = from.lo;
-  if (left <= (uint32_t)kCap) {
-    emit_window<true>(sm, keys, cur, last, base, left, emit);
-    return;
-  }
-  // keys that are repeated many times are among the share
-  while (left > 0) {
-    C end = last;
-    int t = shift_of((C)(end - cur));
-    for (;;) {
-      count_ranges(sm, keys, cur, end, t);
-      const uint32_t total = sm.hist[kBins];
-      if (total == 0) return;
-      // the ranges before f together fit in LDS, the one at f no more
-      const int f = total <= (uint32_t)kCap ? kBins : range_at(sm, (uint32_t)kCap);
-      const uint32_t fit = sm.hist[f], next = f < kBins ? sm.hist[f + 1] : 0;
-      __syncthreads();
-      if (fit > 0) {
-        const C stop = (C)(cur + ((C)f << t));
-        emit_window<false>(sm, keys, cur, f < kBins ? (C)(stop - 1) : end, base, left, emit);
-        cur = stop;  // (not used again after the last range)
-        base += fit;
-        left -= fit < left ? fit : left;
-        break;
-      }
-      cur = (C)(cur + ((C)f << t));
-      if (t == 0) {  // one key
-        emit_equal(sm, keys, cur, base, left, emit);
-        base += next;
-        left -= next < left ? next : left;
-        cur = (C)(cur + 1);  // (past the largest key only when nothing is left)
-        break;
-      }
-      const C stop = (C)(cur + (((C)1 << t) - 1));
-      end = stop < end ? stop : end;
-      t = t > kBinBits ? t - kBinBits : 0;
-    }
+  Cut<C> from, to;
+  find_cuts(sm, keys, all, (uint32_t)num, (uint32_t)own0, (uint32_t)own1, crowd, from, to);
+  // A cut lies before the first key of its range, unless the range is one key that is repeated too
+  // often: then it lies at its place among the equal ones.  So a share has at most
+  // num / kGroups + kTol keys that have to be ranked, and the workgroups that a run of equal keys
+  // covers take a part of it each.  (The limits here and above keep every place inside the batch and
+  // every loop finite even if the source changes while it is read.)
+  if (to.below > (uint32_t)num) return;
+  const bool from_run = from.count > (uint32_t)kTol, to_run = to.count > (uint32_t)kTol;
+  const uint32_t base = from.below + (from_run ? from.count : 0u);
+  if (base < to.below)
+    emit_window(sm, keys, from_run ? (C)(from.lo + 1) : from.lo, own1 < num ? (C)(to.lo - 1) : all, base,
+                to.below - base, emit);
+  if (__builtin_expect(!from_run && !to_run, 1)) return;
+#pragma unroll 1
+  for (int end = 0; end < 2; ++end) {
+    if (!(end == 0 ? from_run : to_run && !(from_run && from.lo == to.lo))) continue;
+    __syncthreads();  // (the lists and sums of the part before)
+    const C key = end == 0 ? from.lo : to.lo;
+    const uint32_t p0 = end == 0 ? from.below : to.below, p1 = p0 + (end == 0 ? from.count : to.count);
+    emit_equal(sm, keys, key, p0, p0 > (uint32_t)own0 ? p0 : (uint32_t)own0,
+               p1 < (uint32_t)own1 ? p1 : (uint32_t)own1, emit);
   }
 }
 
 inline bool fits(int64_t num) { return num > 0 && num <= kMax; }
+
+// Up to how many keys this sort is the faster one: a radix sort of one digit takes 9 us, of two 14.4.
+inline int64_t worth(int key_bits) { return key_bits <= 8 ? 0 : key_bits <= 16 ? 20480 : kMax; }
 
 template <typename C, bool kLook, typename Src, typename Emit>
 int sort(const Src &src, int64_t num, const Emit &emit, hipStream_t st) {

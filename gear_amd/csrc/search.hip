@@ -457,11 +457,11 @@ struct DrawEmit {
     return group_search<kLanes>(draw.prefix, draw.n, (int)threadIdx.x & (kLanes - 1),
                                 [&](typename Draw::type total) { return draw.target(j, total); });
   }
-  __device__ __forceinline__ typename Emit::Resolved find(int j) const {
-    return emit.resolve(lanes == 16 ? search<16>(j) : lanes == 8 ? search<8>(j) : search<1>(j));
-  }
-  __device__ __forceinline__ void put(uint32_t place, int, const typename Emit::Resolved &r) const {
-    emit.store((int64_t)place, r);
+  // (equal keys find the same entry: one search)
+  __device__ __forceinline__ void equal(const uint32_t *at, int n, uint32_t base) const {
+    const int j = (int)at[0], e = threadIdx.x;
+    const auto r = emit.resolve(lanes == 16 ? search<16>(j) : lanes == 8 ? search<8>(j) : search<1>(j));
+    if (e < n) emit.store((int64_t)base + e, r);
   }
   template <int kLanes, typename L>
   __device__ __forceinline__ void list_by(const L &list, const uint32_t *rank, int n,
@@ -493,15 +493,15 @@ struct PositionSrc {
 struct PositionEmit {
   const int64_t *raw;
   Lookup look;
-  __device__ __forceinline__ Lookup::Resolved find(int j) const { return look.resolve(raw[j]); }
-  __device__ __forceinline__ void put(uint32_t place, int, const Lookup::Resolved &r) const {
-    look.store((int64_t)place, r);
-  }
   template <typename L>
   __device__ __forceinline__ void list(const L &list, const uint32_t *rank, int n,
                                        uint32_t base) const {
     const int e = threadIdx.x;
-    if (e < n) put(base + rank[e], 0, find(list.pos(e)));
+    if (e < n) look.store((int64_t)(base + rank[e]), look.resolve(raw[list.pos(e)]));
+  }
+  __device__ __forceinline__ void equal(const uint32_t *at, int n, uint32_t base) const {
+    const int e = threadIdx.x;
+    if (e < n) look.store((int64_t)base + e, look.resolve(raw[at[e]]));
   }
 };
 
@@ -689,6 +689,12 @@ int check_lookup(const Lookup &look) {
   return 0;
 }
 
+// Beyond this many positions among at most 256 entries -- one digit of a radix sort, which with the
+// look-ups takes 12.1 us whatever the positions are -- the one-launch sort is the slower one: 10.7 us at
+// 12 288, 12.9 at 20 480, 17.5 at 32 768, a few more where they are the same few entries.  Integer draws
+// take 15.1 us that way, in one launch 15.0 / 17.6 / 25.8.
+constexpr int64_t kFewEntries = 12288;
+
 // raw: num positions on the device (each in [0, bound)); sorted ascending, then looked up.
 int sort_and_look_up(const int64_t *raw, int64_t num, int64_t bound, const Lookup &look, char *ws,
                      const SampleWs &w, hipStream_t st) {
@@ -696,7 +702,7 @@ int sort_and_look_up(const int64_t *raw, int64_t num, int64_t bound, const Looku
   if (num <= radix::kRankMax && !over) return place_positions(raw, num, look, st);
   int key_bits = 1;
   while (key_bits < 63 && ((uint64_t)(bound - 1) >> key_bits) != 0) ++key_bits;
-  if (key_bits <= 32 && ranges::fits(num) && !over)
+  if (key_bits <= 32 && ranges::fits(num) && (key_bits > 8 || num <= kFewEntries) && !over)
     return ranges::sort<uint32_t, false>(PositionSrc{raw, (uint32_t)(((uint64_t)1 << key_bits) - 1)},
                                          num, PositionEmit{raw, look}, st);
   int64_t *sorted = reinterpret_cast<int64_t *>(ws + w.sorted);
@@ -716,7 +722,8 @@ int draw_and_look_up(const Draw &draw, int64_t num, const Lookup &look, char *ws
                      hipStream_t st) {
   if (apart(draw, num, look)) {
     if (num <= radix::kRankMax) return place_draws(draw, num, look, st);
-    if (ranges::fits(num)) return sort_draws(draw, num, look, st);
+    if (ranges::fits(num) && (sizeof(typename Draw::key_type) < 8 || draw.n > 256 || num <= kFewEntries))
+      return sort_draws(draw, num, look, st);
   }
   int64_t *raw = reinterpret_cast<int64_t *>(ws + w.raw);
   const int rc = launch_search(draw, num, raw, st);

@@ -28,9 +28,7 @@ struct Src {
 struct Emit {
   const int64_t *kin, *vin;
   int64_t *kout, *vout;
-  struct Nothing {};
-  __device__ __forceinline__ Nothing find(int) const { return Nothing{}; }
-  __device__ __forceinline__ void put(uint32_t place, int j, Nothing) const {
+  __device__ __forceinline__ void put(uint32_t place, int j) const {
     kout[place] = kin[j];
     if (vin) vout[place] = vin[j];
   }
@@ -38,7 +36,11 @@ struct Emit {
   __device__ __forceinline__ void list(const L &list, const uint32_t *rank, int n,
                                        uint32_t base) const {
     const int e = threadIdx.x;
-    if (e < n) put(base + rank[e], list.pos(e), Nothing{});
+    if (e < n) put(base + rank[e], list.pos(e));
+  }
+  __device__ __forceinline__ void equal(const uint32_t *at, int n, uint32_t base) const {
+    const int e = threadIdx.x;
+    if (e < n) put(base + (uint32_t)e, (int)at[e]);
   }
 };
 
@@ -47,7 +49,7 @@ struct Emit {
 bool one_launch(const int64_t *kin, int64_t *kout, const int64_t *vin, int64_t *vout, int64_t num,
                 int key_bits) {
   const int64_t b = num * 8;
-  return num > radix::kRankMax && key_bits > 0 && ranges::fits(num) &&
+  return num > radix::kRankMax && ranges::fits(num) && num <= ranges::worth(key_bits) &&
          !ranges::overlap(kin, b, kout, b) && !ranges::overlap(kin, b, vout, b) &&
          !ranges::overlap(vin, b, kout, b) && !ranges::overlap(vin, b, vout, b);
 }

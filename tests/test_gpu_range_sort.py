@@ -107,3 +107,75 @@ def test_batches_of_draws(num, crowd):
     assert np.array_equal(got[3].cpu().numpy(), starts)
     pos = np.floor(u * n).astype(np.int64)
     check(pos, ops.sort_lookup(torch.from_numpy(pos).cuda(), n, **look))
+
+
+@pytest.mark.parametrize("num", [4097, 8193, 20_480, 20_481, 32_767, 32_768])
+@pytest.mark.parametrize("bits", [17, 24, 32, 63])
+def test_runs_of_equal_keys(num, bits):
+    """Keys repeated about as often as a list may hold beside a share (448 times), or far more often;
+    spaced evenly (one bank of the counts), far apart, and next to a key that is far from them all."""
+    from gear_amd import ops
+    rng = np.random.default_rng(num + bits)
+    top = (1 << bits) - 1
+    for run in (63, 127, 128, 129, 447, 448, 449, 450, 1000, num // 3, num // 2 + 1):
+        for step in (1, 64, max(top // (num // run + 1), 1)):
+            announce("runs num=%d bits=%d run=%d step=%d" % (num, bits, run, step))
+            k = np.minimum(np.arange(num) // run * step, top)
+            k[:3] = top
+            k = rng.permutation(k)
+            order = np.argsort(k, kind="stable")
+            ko, vo = ops.sort_i64(torch.from_numpy(k).cuda(), torch.arange(num, device="cuda"),
+                                  key_bits=bits)
+            assert np.array_equal(vo.cpu().numpy(), order)
+            assert np.array_equal(ko.cpu().numpy(), k[order])
+
+
+@pytest.mark.parametrize("num", [4097, 12_288, 12_289, 20_481, 32_768])
+@pytest.mark.parametrize("n", [1, 2, 5, 255, 256, 257])
+def test_batches_from_a_few_entries(num, n):
+    """Many positions or draws among few entries: the forms of both sides of the rules."""
+    from gear_amd import ops
+    rng = np.random.default_rng(num + n)
+    announce("few entries num=%d n=%d" % (num, n))
+    pos = rng.integers(0, n, size=num)
+    got = ops.sort_lookup(torch.from_numpy(pos).cuda(), n, index_offset=1)
+    assert np.array_equal(got[0].cpu().numpy(), np.sort(pos))
+    assert np.array_equal(got[1].cpu().numpy(), np.sort(pos) - 1)
+    prefix = np.cumsum(rng.integers(1, 4, size=n))
+    u = rng.random(num)
+    at = np.searchsorted(prefix, np.floor(u * prefix[-1]).astype(np.int64), side="right")
+    got = ops.sample_lookup(torch.from_numpy(prefix).cuda(), torch.from_numpy(u).cuda())
+    assert np.array_equal(got[0].cpu().numpy(), np.sort(at))
+    u[: num // 2] = u[0]
+    u = u.astype(np.float32)
+    at = np.searchsorted(prefix, u.astype(np.float64) * prefix[-1], side="right")
+    got = ops.sample_sorted(torch.from_numpy(prefix.astype(np.float64)).cuda(), torch.from_numpy(u).cuda())
+    assert np.array_equal(got.cpu().numpy(), np.sort(np.minimum(at, n - 1)))
+
+
+@pytest.mark.parametrize("bits", [20, 63])
+def test_a_few_keys_take_no_multiple_of_the_time(bits):
+    """A batch of two keys takes about 1.6 times a batch of distinct ones; it took 6 to 12 times when
+    one workgroup stored a run by itself and the counts of one key followed each other."""
+    from gear_amd import ops
+    num = 32_768
+    announce("time of a few keys, %d bits" % bits)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(bits)
+    distinct = torch.randint(0, 1 << bits if bits < 63 else 1 << 62, (num,), device="cuda", generator=g)
+    two = torch.randint(0, 2, (num,), device="cuda", generator=g) * (1 << (bits - 2))
+
+    def ms(x):
+        best = []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                ops.sort_i64(x, key_bits=bits)
+            b.record()
+            b.synchronize()
+            best.append(a.elapsed_time(b))
+        return min(best)
+
+    ms(distinct)
+    assert ms(two) < 3.0 * ms(distinct)
