@@ -629,11 +629,16 @@ int launch_scan(const In *in, Out *out, int64_t n, void *ws, size_t ws_bytes, hi
   if ((reinterpret_cast<uintptr_t>(in) & (sizeof(In) - 1)) ||
       (reinterpret_cast<uintptr_t>(out) & 15))
     return GEAR_HIP_EALIGN;
+  constexpr int64_t g1 = (int64_t)kBlock * VE;  // elements per range and granule
+  const bool wide = ceil_div64(n, 8 * g1) > kMaxRanges8 && ceil_div64(n, 16 * g1) <= kMaxRanges;
   // GEAR_HIP_SCAN_SINGLE_PASS: 1 = the chained kernel wherever it applies, 0 = never; unset = the
-  // chained kernel for full scans, two launches for the rescan of a suffix.  A launch that is
-  // being captured into a graph would replay its tag, so it takes the two launches.
+  // chained kernel for full scans and, over ranges of 16 granules, for the rescan of a suffix as well:
+  // there it is the faster one for every suffix (us for the last entry / a tenth / the last half of 7e7:
+  // 11.3 / 21.6 / 94 against 13.6 / 29.6 / 96 in two launches, of 1.3e8: 12.9 / 34.7 / 158 against
+  // 13.8 / 44.6 / 212).  A launch that is being captured into a graph would replay its tag, so it takes
+  // the two launches.
   const int forced = env_int("GEAR_HIP_SCAN_SINGLE_PASS", -1);
-  bool chained = forced < 0 ? first_changed <= 0 : forced == 1;
+  bool chained = forced < 0 ? first_changed <= 0 || wide : forced == 1;
   if (chained) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
@@ -647,19 +652,20 @@ int launch_scan(const In *in, Out *out, int64_t n, void *ws, size_t ws_bytes, hi
   // more ranges cost more than they gain once every CU has work), and 16 -- 190 registers, two
   // workgroups per CU -- where 8 would need more than 4096 ranges (33.5 to 134 M fp32: one read
   // instead of two, us at 6e7 / 6.8e7 / 1e8 / 1.3e8: 148 / 167 / 240 / 330 against 187 / 213 / 308 /
-  // 399; int64 at 4e7 / 6e7: 143 / 235 against 183 / 267).  The chained kernel and the two launches cut the input
-  // the same way, so a rescan finds the sums of the last full scan.
+  // 399; int64 at 4e7 / 6e7: 143 / 235 against 183 / 267).  The chained kernel and the two launches cut
+  // the input the same way, so a rescan finds the sums of the last full scan and the bits are the same;
+  // but integers, which have no rescan and the same sums in any order, take 8 granules in two launches
+  // (captured, 4e7 / 6e7: 187 / 276 us, 197 / 281 with 16).
   // At 8192 ranges the words to poll are 0.8 GB beside 1.6 GB of data; beyond that they outweigh
-  // the second read: two launches, up to 16384 ranges of 8 granules.  (8-byte elements: ranges of 2 granules would be smaller than the 2048 elements the
-  // workspace is laid out for, so they start at 4.)
-  constexpr int64_t g1 = (int64_t)kBlock * VE;  // elements per range and granule
+  // the second read: two launches, up to 16384 ranges of 8 granules.  (8-byte elements: ranges of 2
+  // granules would be smaller than the 2048 elements the workspace is laid out for, so they start at 4.)
   if (VE == 4 && ceil_div64(n, 2 * g1) <= 256)
     return launch_ranges<In, Acc, Out, VE, 2>(in, out, n, ws, st, chained, first_changed);
   else if (ceil_div64(n, 4 * g1) <= 512)
     return launch_ranges<In, Acc, Out, VE, 4>(in, out, n, ws, st, chained, first_changed);
   else if (ceil_div64(n, 8 * g1) <= kMaxRanges8)
     return launch_ranges<In, Acc, Out, VE, 8>(in, out, n, ws, st, chained, first_changed);
-  else if (ceil_div64(n, 16 * g1) <= kMaxRanges)
+  else if (wide && (chained || !std::is_integral<Acc>::value))
     return launch_ranges<In, Acc, Out, VE, 16>(in, out, n, ws, st, chained, first_changed);
   return launch_ranges<In, Acc, Out, VE, 8>(in, out, n, ws, st, false, first_changed);
 }
