@@ -539,20 +539,6 @@ class LoaderStep {
     } else {
       throw std::invalid_argument("kind must be 'weighted', 'uniform' or 'positions'");
     }
-    // The lengths go to the host ahead of the gather: the host waits for the selection only.
-    // (The staging buffer leaves the object for the time of the call: another thread that comes
-    // in while this one waits without the GIL makes one of its own.)
-    Staging staged;
-    if (host_timesteps && num > 0) {
-      std::swap(staged, staging_);
-      if (!staged.buf.defined() || staged.buf.numel() < num)
-        staged.buf = at::empty({num}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
-      check("gear_hip_take_i64", gear_hip_take_i64(lengths, timesteps.numel(), l, num, 0,
-                                                   ptr<int64_t>(staged.buf), st));
-      if (staged.arrived == nullptr)
-        hip("event", hipEventCreateWithFlags(&staged.arrived, hipEventDisableTiming));
-      hip("event record", hipEventRecord(staged.arrived, static_cast<hipStream_t>(st)));
-    }
     py::list batch(columns_.size());
     py::object masks = py::none();
     if (with_mask_) masks = py::list(columns_.size());
@@ -586,8 +572,21 @@ class LoaderStep {
                                            traj_stride_, capacity_, trajectory_length_, descs.data(),
                                            (int)descs.size(), st));
     if (!host_timesteps) return py::make_tuple(wrap(sampled), wrap(lens), batch, masks);
+    // The lengths on the host.  The call returns when the gather has ended, as one that copied the
+    // lengths behind it: a table in host memory may be written again, and the batch read on any stream.
+    // (The staging buffer leaves the object for the time of the call: another thread that comes
+    // in while this one waits without the GIL makes one of its own.)
     at::Tensor host = at::empty({num}, at::TensorOptions().dtype(at::kLong));
     if (num > 0) {
+      Staging staged;
+      std::swap(staged, staging_);
+      if (!staged.buf.defined() || staged.buf.numel() < num)
+        staged.buf = at::empty({num}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+      if (staged.arrived == nullptr)
+        hip("event", hipEventCreateWithFlags(&staged.arrived, hipEventDisableTiming));
+      check("gear_hip_take_i64", gear_hip_take_i64(lengths, timesteps.numel(), l, num, 0,
+                                                   ptr<int64_t>(staged.buf), st));
+      hip("event record", hipEventRecord(staged.arrived, static_cast<hipStream_t>(st)));
       {
         py::gil_scoped_release nogil;
         hip("event wait", hipEventSynchronize(staged.arrived));

@@ -9,6 +9,10 @@ What differs from the reference, on purpose (one GPU, one data-parallel rank):
     so the batch tensors are torch.empty, not torch.zeros (offline_loader.py:181-189);
   * lengths are passed as they are (the reference takes them modulo the shard capacity,
     offline_loader.py:196-198).
+
+With the timesteps on the host (the default) next() returns when the batch is complete: a table in
+host memory may be written again, and the batch read on any stream.  With timesteps_on_device=True
+next() only enqueues the step on the current stream.
 """
 import importlib
 import logging
@@ -238,7 +242,7 @@ class OfflineLoader(BasicLoader):
         """Everything of a step after the draws: the sampler's own preparation (prefix rescan,
         top-k selection), then ONE call that sorts the batch, looks up global index, local index
         and recorded length of every entry, and gathers all columns into fresh tensors.  Returns
-        (lengths, data_batch); the lengths on the host, ahead of the gather, when asked for."""
+        (lengths, data_batch); the lengths on the host, after the gather, when asked for."""
         kind, picks, prefix = self._sampler.prepare(self._indices, self._device_weights, draws,
                                                     dirty_from=dirty_from)
         self.last_sampled, lengths, data_batch, self.last_masks = self._step.run(
