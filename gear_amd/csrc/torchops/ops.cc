@@ -458,18 +458,25 @@ void hip(const char *what, hipError_t e) {
   if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// Pinned memory for lengths on their way to the host, and the event of their arrival.
+// Pinned memory for lengths on their way to the host, and the event of their arrival.  Memory that a
+// kernel may still write (an error between its launch and the end of the wait) is waited for, or never
+// given back where not even that works: the next pinned tensor would be written over.
 struct Staging {
   at::Tensor buf;
   hipEvent_t arrived = nullptr;
+  hipStream_t pending = nullptr;  // the stream of a kernel that may write buf
+  bool is_pending = false;
   Staging() = default;
-  Staging(Staging &&o) noexcept : buf(std::move(o.buf)), arrived(o.arrived) { o.arrived = nullptr; }
-  Staging &operator=(Staging &&o) noexcept {
+  Staging(const Staging &) = delete;
+  Staging &operator=(const Staging &) = delete;
+  void swap(Staging &o) {
     std::swap(buf, o.buf);
     std::swap(arrived, o.arrived);
-    return *this;
+    std::swap(pending, o.pending);
+    std::swap(is_pending, o.is_pending);
   }
   ~Staging() {
+    if (is_pending && hipStreamSynchronize(pending) != hipSuccess) (void)buf.unsafeReleaseIntrusivePtr().release();
     if (arrived != nullptr) (void)hipEventDestroy(arrived);
   }
 };
@@ -579,20 +586,23 @@ class LoaderStep {
     at::Tensor host = at::empty({num}, at::TensorOptions().dtype(at::kLong));
     if (num > 0) {
       Staging staged;
-      std::swap(staged, staging_);
+      staged.swap(staging_);
       if (!staged.buf.defined() || staged.buf.numel() < num)
         staged.buf = at::empty({num}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
       if (staged.arrived == nullptr)
         hip("event", hipEventCreateWithFlags(&staged.arrived, hipEventDisableTiming));
+      staged.pending = static_cast<hipStream_t>(st);
+      staged.is_pending = true;
       check("gear_hip_take_i64", gear_hip_take_i64(lengths, timesteps.numel(), l, num, 0,
                                                    ptr<int64_t>(staged.buf), st));
-      hip("event record", hipEventRecord(staged.arrived, static_cast<hipStream_t>(st)));
+      hip("event record", hipEventRecord(staged.arrived, staged.pending));
       {
         py::gil_scoped_release nogil;
         hip("event wait", hipEventSynchronize(staged.arrived));
       }
+      staged.is_pending = false;
       std::memcpy(host.data_ptr(), staged.buf.data_ptr(), (size_t)num * 8);
-      std::swap(staged, staging_);
+      staged.swap(staging_);
     }
     return py::make_tuple(wrap(sampled), wrap(host), batch, masks);
   }

@@ -64,3 +64,65 @@ def test_the_batch_may_be_read_on_another_stream():
         torch.cuda.synchronize()
         assert torch.equal(early, batch[0])
         _check(loader, timesteps, batch)
+
+
+def test_a_step_that_runs_out_of_memory_leaves_nothing_behind():
+    """The batch does not fit: the step raises, nothing on the GPU still writes the pinned memory the
+    lengths would have gone through, and the loader goes on."""
+    loader = _loader("device", 3, batch=16384)      # a batch of 32 GiB
+    small = _loader("device", 4, batch=1024)
+    timesteps, batch = next(small)                  # (what the step keeps is in the caches)
+    del batch
+    torch.cuda.empty_cache()
+    announce("out of memory in a loader's step")
+    torch.cuda.set_per_process_memory_fraction(0.05)
+    try:
+        for _ in range(2):
+            torch.cuda._sleep(50_000_000)           # what the step enqueues runs late
+            with pytest.raises(RuntimeError, match="out of memory"):
+                next(loader)
+            pinned = [torch.full((n,), -7, dtype=torch.int64).pin_memory() for n in (16384, 16384, 16000)]
+            torch.cuda.synchronize()
+            assert all(bool((p == -7).all()) for p in pinned)
+            del pinned
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    timesteps, batch = next(small)
+    at = small.last_sampled.cpu()
+    assert torch.equal(timesteps, 1 + at % T) and torch.equal(batch[0][:, 0, 0].cpu(), at + 1.0)
+
+
+def test_two_threads_in_one_loader():
+    """A thread that comes in while another waits for its lengths has memory of its own for them."""
+    import threading
+    loader = _loader("device", 5, batch=32)
+    step, errors = loader._step, []
+    tables = [torch.randint(1, T + 1, (CAP,), device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    announce("two threads in one loader's step")
+
+    def work(lengths):
+        try:
+            host = lengths.cpu()
+            with torch.cuda.stream(torch.cuda.Stream()):
+                draws = torch.randint(0, CAP, (32,), device="cuda")
+                for _ in range(200):
+                    sampled, ts, _, _ = step.run("uniform", draws, None, loader._indices, 0, lengths, True,
+                                                 _ops()._ws)
+                    if not torch.equal(ts, host[sampled.cpu()]):
+                        errors.append("lengths of another thread's step")
+                        return
+        except Exception as e:  # noqa: BLE001 (reported by the test's own thread)
+            errors.append(repr(e))
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in tables]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+
+
+def _ops():
+    from gear_amd import ops
+    return ops
