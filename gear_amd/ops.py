@@ -150,8 +150,8 @@ def subcopy_multi(src, idxs, tss, lens, traj_stride, columns, capacity=0, trajec
 
 class GatherPlan:
     """subcopy_multi for a loop that gathers into the same batch tensors every step: the column
-    descriptors and every argument that does not change are marshalled once, run(idxs, tss, lens)
-    is one call into the library with the three index tensors of the step."""
+    descriptors and every argument that does not change are marshalled once, run() is one call
+    into the library with the three index tensors of the step."""
 
     def __init__(self, src, traj_stride, columns, num, capacity=0, trajectory_length=0):
         n = len(columns)
@@ -178,10 +178,13 @@ class GatherPlan:
             d.zero_fill = int(bool(c.get("zero_fill", True)))
             self._keep.append((dst, m))
         self._keep.append(src)
-        self.run = _hostops.Gather(
+        self._gather = _hostops.Gather(
             _src_ptr(src), int(traj_stride), int(num), int(capacity), int(trajectory_length),
             [(d.dst, d.mask_out or 0, d.ofst, d.span, d.step_bytes, d.col_base, d.dst_stride,
-              bool(d.pad_head), bool(d.zero_fill)) for d in self._descs[:n]]).run
+              bool(d.pad_head), bool(d.zero_fill)) for d in self._descs[:n]])
+
+    def run(self, idxs, tss, lens):
+        self._gather.run(idxs, tss, lens)
 
 
 def vcopy(src, dst, src_offsets, dst_offsets, strides, max_stride):
