@@ -180,7 +180,7 @@ class GatherPlan:
         self._keep.append(src)
         self._gather = _hostops.Gather(
             _src_ptr(src), int(traj_stride), int(num), int(capacity), int(trajectory_length),
-            [(d.dst, d.mask_out or 0, d.ofst, d.span, d.step_bytes, d.col_base, d.dst_stride,
+            [(d.dst or 0, d.mask_out or 0, d.ofst, d.span, d.step_bytes, d.col_base, d.dst_stride,
               bool(d.pad_head), bool(d.zero_fill)) for d in self._descs[:n]])
 
     def run(self, idxs, tss, lens):

@@ -54,3 +54,12 @@ def test_the_method_keeps_its_tensors():
     assert all(r() is not None for r in alive)
     run(**_args(3))
     torch.cuda.synchronize()
+
+
+def test_a_plan_for_no_windows():
+    from gear_amd import ops
+    announce("gather plan of no windows")
+    plan, dst = _plan(ops.GatherPlan, 0, torch.zeros(64, dtype=torch.uint8, device="cuda"))
+    plan.run(**_args(0))
+    with pytest.raises(ValueError, match="made for 0 windows"):
+        plan.run(**_args(1))
