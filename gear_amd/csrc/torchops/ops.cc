@@ -502,7 +502,8 @@ class LoaderStep {
                                 c[3].cast<int64_t>(), c[4].cast<int64_t>(), c[5].cast<int64_t>(),
                                 c[6].cast<bool>()});
     }
-    if (columns_.size() > GEAR_HIP_MAX_COLUMNS) throw py::value_error("more than 16 columns");
+    if (columns_.size() > GEAR_HIP_MAX_COLUMNS)
+      throw std::runtime_error("more than 16 columns: one launch gathers 16 at most");
   }
 
   // kind, draws, prefix: as WeightedSampler / UniformSampler / TopKSampler.prepare() return them.

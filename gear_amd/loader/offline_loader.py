@@ -111,7 +111,7 @@ class OfflineLoader(BasicLoader):
         self._sampler.indices_ascending = True   # arange + offset below
         self._indices = torch.arange(self._iset.local_capacity, dtype=torch.long,
                                      device=self._mpu.device) + self._iset.index_offset
-        self._step = self._native_step()
+        self._step = None   # made by the first fused step
         self.last_masks = None
         self.last_sampled = None   # global indices of the last batch (device tensor)
 
@@ -245,6 +245,8 @@ class OfflineLoader(BasicLoader):
         (lengths, data_batch); the lengths on the host, after the gather, when asked for."""
         kind, picks, prefix = self._sampler.prepare(self._indices, self._device_weights, draws,
                                                     dirty_from=dirty_from)
+        if self._step is None:
+            self._step = self._native_step()
         self.last_sampled, lengths, data_batch, self.last_masks = self._step.run(
             kind, picks, prefix, self._indices, self._iset.index_offset, self._device_timesteps,
             host_timesteps, ops._ws)

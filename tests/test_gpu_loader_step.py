@@ -96,6 +96,7 @@ def test_two_threads_in_one_loader():
     """A thread that comes in while another waits for its lengths has memory of its own for them."""
     import threading
     loader = _loader("device", 5, batch=32)
+    next(loader)
     step, errors = loader._step, []
     tables = [torch.randint(1, T + 1, (CAP,), device="cuda") for _ in range(2)]
     torch.cuda.synchronize()
@@ -121,6 +122,31 @@ def test_two_threads_in_one_loader():
     for t in threads:
         t.join()
     assert not errors
+
+
+def test_more_columns_than_one_launch_gathers():
+    """A loader of 17 columns can be made; the fused step refuses it, the step column by column does not."""
+    from gear_amd.dataset import SharedDataset
+    from gear_amd.loader import OfflineLoader
+    from gear_amd.mpu import ModelParallelismUnit
+    from gear_amd.specs import TableSpec
+    names = ["c%02d" % c for c in range(17)]
+    spec = TableSpec.create(trajectory_length=4, capacity=6, column_specs=[
+        dict(shape=[c + 1], dtype=torch.float32, name=n) for c, n in enumerate(names)])
+    data = SharedDataset.create(spec, key=(os.getpid() << 8) + 6, placement="pinned")
+    for i in range(6):
+        data[i] = (1.0, 4, [torch.full((4, c + 1), 10.0 * i + c) for c in range(17)])
+    loader = OfflineLoader(data, 3, ModelParallelismUnit(device=torch.device("cuda:0")), "Uniform",
+                           [dict(name=n, offset=-4, length=4, pad="tail") for n in names])
+    announce("a loader of 17 columns")
+    with pytest.raises(RuntimeError, match="more than 16 columns"):
+        next(loader)
+    _, batch = loader.exposed_low_level_controlled_iterate(torch.tensor([4, 0, 5]))
+    for c in range(17):
+        for j, i in enumerate([4, 0, 5]):
+            assert bool((batch[c][j].cpu() == 10.0 * i + c).all())
+    timesteps, batch = loader.low_level_controlled_iterate()
+    assert timesteps.tolist() == [4, 4, 4] and len(batch) == 17
 
 
 def _ops():
