@@ -5,7 +5,9 @@
 // from Python (ctypes marshalling, a torch.empty per output, four to six attribute calls per
 // tensor) took 35 to 60 us, of which the launches themselves are 2.6 us apiece.  Here a tensor
 // costs an unpack and an output an allocation of the caching allocator (0.5 us).  The module links
-// libtorch for that; it computes nothing on tensors.
+// libtorch for that; it computes nothing on tensors.  Allocations and calls into the library run without
+// the GIL: a launch that waits for room in its queue, or an allocation that waits for the driver, stops
+// no other Python thread.
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPGeneratorImpl.h>
 #include <c10/hip/HIPFunctions.h>
@@ -17,8 +19,11 @@
 #include <torch/csrc/utils/pybind.h>
 
 #include <cstring>
-#include <deque>
+#include <memory>
+#include <mutex>
 #include <string>
+#include <tuple>
+#include <unordered_map>
 #include <vector>
 
 #include "gear_hip.h"
@@ -63,7 +68,9 @@ T *ptr_or_null(py::handle h, const char *name) {
   return h.is_none() ? nullptr : static_cast<T *>(any_tensor(h, name).data_ptr());
 }
 
+// (where the GIL is held)
 at::Tensor empty(int64_t n, at::ScalarType dtype, const at::Device &device) {
+  py::gil_scoped_release nogil;
   return at::empty({n}, at::TensorOptions().dtype(dtype).device(device));
 }
 
@@ -71,8 +78,10 @@ py::object wrap(const at::Tensor &t) { return py::reinterpret_steal<py::object>(
 
 void *current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
+// (with or without the GIL)
 void check(const char *fn, int code) {
   if (code == 0) return;
+  py::gil_scoped_acquire gil;
   py::module_::import("gear_amd._cabi").attr("check")(fn, code);  // raises
 }
 
@@ -82,46 +91,76 @@ void check(const char *fn, int code) {
 // get(); an instance whose get() was replaced is asked through it.
 class Workspace {
  public:
-  at::Tensor &get(const char *tag, size_t bytes, const at::Device &device) {
+  struct Entry {
+    at::Tensor buf;
+    std::mutex order;  // held while a call enqueues its launches on the buffer's stream
+  };
+  // (the GIL is held; the entry stays the same while its buffer grows)
+  std::shared_ptr<Entry> get(const char *tag, size_t bytes, const at::Device &device, at::Tensor *buf) {
     const c10::DeviceIndex index = device.has_index() ? device.index() : c10::hip::current_device();
     void *stream = c10::hip::getCurrentHIPStream(index).stream();
-    for (Entry &e : entries_)
-      if (e.device == index && e.stream == stream && e.tag == tag) {
-        if ((size_t)e.buf.numel() < bytes) e.buf = make(bytes, device);
-        return e.buf;
-      }
-    entries_.push_back(Entry{tag, index, stream, make(bytes, device)});
-    return entries_.back().buf;
+    std::shared_ptr<Entry> &slot = entries_[Key{tag, index, stream}];
+    if (!slot) slot = std::make_shared<Entry>();
+    std::shared_ptr<Entry> e = slot;
+    if (!e->buf.defined() || (size_t)e->buf.numel() < bytes) {
+      at::Tensor grown = empty((int64_t)std::max<size_t>(bytes, 256), at::kByte, device);
+      // (another thread may have been here meanwhile)
+      if (!e->buf.defined() || e->buf.numel() < grown.numel()) e->buf = grown;
+    }
+    *buf = e->buf;
+    return e;
   }
 
  private:
-  struct Entry {
+  struct Key {
     std::string tag;
     c10::DeviceIndex device;
     void *stream;
-    at::Tensor buf;
+    bool operator==(const Key &o) const { return stream == o.stream && device == o.device && tag == o.tag; }
   };
-  static at::Tensor make(size_t bytes, const at::Device &device) {
-    return empty((int64_t)std::max<size_t>(bytes, 256), at::kByte, device);
-  }
-  std::deque<Entry> entries_;
+  struct Hash {
+    size_t operator()(const Key &k) const {
+      return std::hash<std::string>()(k.tag) ^ (std::hash<void *>()(k.stream) * 31 + (size_t)k.device);
+    }
+  };
+  std::unordered_map<Key, std::shared_ptr<Entry>, Hash> entries_;
 };
 
 struct Scratch {
-  void *ptr;
-  size_t bytes;
+  void *ptr = nullptr;
+  size_t bytes = 0;
   at::Tensor keep;
+  std::shared_ptr<Workspace::Entry> entry;
+  Scratch() = default;  // none
   Scratch(py::handle ws, const char *tag, size_t want, const at::Device &device) {
     PyObject **dict = _PyObject_GetDictPtr(ws.ptr());
     if (dict != nullptr && *dict != nullptr && PyDict_GET_SIZE(*dict) != 0)
       keep = THPVariable_Unpack(
           ws.attr("get")(tag, want, py::reinterpret_steal<py::object>(THPDevice_New(device))).ptr());
     else
-      keep = ws.cast<Workspace &>().get(tag, want, device);
+      entry = ws.cast<Workspace &>().get(tag, want, device, &keep);
     ptr = keep.data_ptr();
     bytes = (size_t)keep.numel();
   }
 };
+
+// f(args) without the GIL.  Two threads that enqueue on one stream share its scratch: the launches of
+// one call follow each other, so that no other call's lie between them.
+template <typename F>
+int launches(const Scratch &s, const F &f) {
+  if (!s.entry) return f();
+  std::lock_guard<std::mutex> order(s.entry->order);
+  return f();
+}
+template <typename F, typename... A>
+void call(const char *name, const Scratch &s, const F &f, A... args) {
+  int code;
+  {
+    py::gil_scoped_release nogil;
+    code = launches(s, [&] { return f(args...); });
+  }
+  check(name, code);
+}
 
 // ---- prefix sums -----------------------------------------------------------------------------------
 template <typename Launch>
@@ -135,8 +174,8 @@ py::object prefix(py::handle in, py::object out, py::handle ws, at::ScalarType f
     throw py::value_error("out is too small");
   }
   Scratch s(ws, "scan", gear_hip_scan_workspace_bytes(n), p.device());
-  check(fn, launch(p.data_ptr(), THPVariable_Unpack(out.ptr()).data_ptr(), n, s.ptr, s.bytes,
-                   current_stream()));
+  call(fn, s, launch, p.data_ptr(), THPVariable_Unpack(out.ptr()).data_ptr(), n, s.ptr, s.bytes,
+       current_stream());
   return out;
 }
 
@@ -157,13 +196,12 @@ py::object prefix_sum_i64(py::handle in, py::object out, py::handle ws) {
 // first_changed <= 0: full scan
 void rescan(const at::Tensor &in, const at::Tensor &out, int64_t first_changed, const at::Tensor &ws) {
   if (first_changed <= 0)
-    check("gear_hip_scan_f32_f64",
-          gear_hip_scan_f32_f64(ptr<float>(in), ptr<double>(out), in.numel(), ws.data_ptr(),
-                                (size_t)ws.numel(), current_stream()));
+    call("gear_hip_scan_f32_f64", Scratch(), gear_hip_scan_f32_f64, ptr<float>(in), ptr<double>(out),
+         in.numel(), ws.data_ptr(), (size_t)ws.numel(), current_stream());
   else
-    check("gear_hip_rescan_f32_f64",
-          gear_hip_rescan_f32_f64(ptr<float>(in), ptr<double>(out), in.numel(), first_changed,
-                                  ws.data_ptr(), (size_t)ws.numel(), current_stream()));
+    call("gear_hip_rescan_f32_f64", Scratch(), gear_hip_rescan_f32_f64, ptr<float>(in),
+         ptr<double>(out), in.numel(), first_changed, ws.data_ptr(), (size_t)ws.numel(),
+         current_stream());
 }
 
 // ---- draws -----------------------------------------------------------------------------------------
@@ -177,19 +215,17 @@ py::object upper_bound(py::handle prefix_, py::handle u_, bool unit, py::object 
     need(idx_out, at::kLong, "idx_out");
   int64_t *idx = ptr<int64_t>(THPVariable_Unpack(idx_out.ptr()));
   if (pri.is_none()) {
-    check("gear_hip_upper_bound_f64",
-          gear_hip_upper_bound_f64(ptr<double>(prefix), n, ptr<float>(u), num, unit, idx, nullptr, beta,
-                                   nullptr, nullptr, 0, current_stream()));
+    call("gear_hip_upper_bound_f64", Scratch(), gear_hip_upper_bound_f64, ptr<double>(prefix), n,
+         ptr<float>(u), num, unit, idx, nullptr, beta, nullptr, nullptr, 0, current_stream());
     return idx_out;
   }
   const at::Tensor &p = need(pri, at::kFloat, "priorities");
   if (p.numel() != n) throw py::value_error("priorities and prefix differ in length");
   if (weights_out.is_none()) weights_out = wrap(empty(num, at::kFloat, u.device()));
   Scratch s(ws, "search", gear_hip_search_workspace_bytes(num), u.device());
-  check("gear_hip_upper_bound_f64",
-        gear_hip_upper_bound_f64(ptr<double>(prefix), n, ptr<float>(u), num, unit, idx, ptr<float>(p),
-                                 beta, ptr_or_null<float>(weights_out, "weights_out"), s.ptr, s.bytes,
-                                 current_stream()));
+  call("gear_hip_upper_bound_f64", s, gear_hip_upper_bound_f64, ptr<double>(prefix), n, ptr<float>(u),
+       num, unit, idx, ptr<float>(p), beta, ptr_or_null<float>(weights_out, "weights_out"), s.ptr,
+       s.bytes, current_stream());
   return py::make_tuple(std::move(idx_out), std::move(weights_out));
 }
 
@@ -197,9 +233,9 @@ py::object upper_bound_i64(py::handle prefix_, py::handle u_, bool unit, py::obj
   const at::Tensor &prefix = need(prefix_, at::kLong, "prefix");
   const at::Tensor &u = need(u_, unit ? at::kDouble : at::kLong, "u");
   if (idx_out.is_none()) idx_out = wrap(empty(u.numel(), at::kLong, u.device()));
-  check("gear_hip_upper_bound_i64",
-        gear_hip_upper_bound_i64(ptr<int64_t>(prefix), prefix.numel(), u.data_ptr(), u.numel(), unit,
-                                 ptr_or_null<int64_t>(idx_out, "idx_out"), current_stream()));
+  call("gear_hip_upper_bound_i64", Scratch(), gear_hip_upper_bound_i64, ptr<int64_t>(prefix),
+       prefix.numel(), u.data_ptr(), u.numel(), unit, ptr_or_null<int64_t>(idx_out, "idx_out"),
+       current_stream());
   return idx_out;
 }
 
@@ -218,12 +254,10 @@ py::object sample_sorted(py::handle prefix_, py::handle u_, bool unit, py::objec
     output(lens);
   }
   Scratch s(ws, "sample", gear_hip_sample_workspace_bytes(num), u.device());
-  check("gear_hip_sample_sorted_f64",
-        gear_hip_sample_sorted_f64(ptr<double>(prefix), prefix.numel(), ptr<float>(u), num, unit,
-                                   ptr_or_null<int64_t>(sorted_out, "sorted_out"), trajectory_length,
-                                   modulo, ptr_or_null<int64_t>(idxs, "idxs"),
-                                   ptr_or_null<int64_t>(tss, "tss"), ptr_or_null<int64_t>(lens, "lens"),
-                                   s.ptr, s.bytes, current_stream()));
+  call("gear_hip_sample_sorted_f64", s, gear_hip_sample_sorted_f64, ptr<double>(prefix),
+       prefix.numel(), ptr<float>(u), num, unit, ptr_or_null<int64_t>(sorted_out, "sorted_out"),
+       trajectory_length, modulo, ptr_or_null<int64_t>(idxs, "idxs"), ptr_or_null<int64_t>(tss, "tss"),
+       ptr_or_null<int64_t>(lens, "lens"), s.ptr, s.bytes, current_stream());
   if (trajectory_length > 0)
     return py::make_tuple(std::move(sorted_out), std::move(idxs), std::move(tss), std::move(lens));
   return sorted_out;
@@ -272,11 +306,9 @@ py::object sample_lookup(py::handle prefix_, py::handle u_, bool unit, py::handl
     throw py::value_error("index_table and prefix differ in length");
   Scratch s(ws, "sample", gear_hip_sample_workspace_bytes(num), u.device());
   if (!i64) {
-    check("gear_hip_sample_lookup_f64",
-          gear_hip_sample_lookup_f64(ptr<double>(prefix), prefix.numel(), ptr<float>(u), num, unit,
-                                     a.index_table, index_offset, a.lengths_table, a.lengths_n,
-                                     a.sampled_ptr(), a.local_ptr(), a.lens_ptr(), s.ptr, s.bytes,
-                                     current_stream()));
+    call("gear_hip_sample_lookup_f64", s, gear_hip_sample_lookup_f64, ptr<double>(prefix),
+         prefix.numel(), ptr<float>(u), num, unit, a.index_table, index_offset, a.lengths_table,
+         a.lengths_n, a.sampled_ptr(), a.local_ptr(), a.lens_ptr(), s.ptr, s.bytes, current_stream());
     return py::make_tuple(a.sampled, a.local, a.lens);
   }
   const double *v = nullptr;
@@ -289,11 +321,10 @@ py::object sample_lookup(py::handle prefix_, py::handle u_, bool unit, py::handl
     if (starts_out.is_none()) starts_out = wrap(empty(num, at::kLong, u.device()));
     starts = ptr_or_null<int64_t>(starts_out, "starts_out");
   }
-  check("gear_hip_sample_lookup_i64",
-        gear_hip_sample_lookup_i64(ptr<int64_t>(prefix), prefix.numel(), u.data_ptr(), num, unit,
-                                   a.index_table, index_offset, a.lengths_table, a.lengths_n,
-                                   a.sampled_ptr(), a.local_ptr(), a.lens_ptr(), v, window, starts,
-                                   s.ptr, s.bytes, current_stream()));
+  call("gear_hip_sample_lookup_i64", s, gear_hip_sample_lookup_i64, ptr<int64_t>(prefix),
+       prefix.numel(), u.data_ptr(), num, unit, a.index_table, index_offset, a.lengths_table,
+       a.lengths_n, a.sampled_ptr(), a.local_ptr(), a.lens_ptr(), v, window, starts, s.ptr, s.bytes,
+       current_stream());
   if (starts) return py::make_tuple(a.sampled, a.local, a.lens, starts_out);
   return py::make_tuple(a.sampled, a.local, a.lens);
 }
@@ -306,10 +337,9 @@ py::object sort_lookup(py::handle positions_, int64_t bound, py::handle index_ta
   LookupArgs a(num, positions.device(), index_table, lengths_table, std::move(sampled_out),
                std::move(local_out), std::move(lens_out));
   Scratch s(ws, "sample", gear_hip_sample_workspace_bytes(num), positions.device());
-  check("gear_hip_sort_lookup_i64",
-        gear_hip_sort_lookup_i64(ptr<int64_t>(positions), num, bound, a.index_table, a.index_n,
-                                 index_offset, a.lengths_table, a.lengths_n, a.sampled_ptr(),
-                                 a.local_ptr(), a.lens_ptr(), s.ptr, s.bytes, current_stream()));
+  call("gear_hip_sort_lookup_i64", s, gear_hip_sort_lookup_i64, ptr<int64_t>(positions), num, bound,
+       a.index_table, a.index_n, index_offset, a.lengths_table, a.lengths_n, a.sampled_ptr(),
+       a.local_ptr(), a.lens_ptr(), s.ptr, s.bytes, current_stream());
   return py::make_tuple(a.sampled, a.local, a.lens);
 }
 
@@ -320,19 +350,17 @@ py::object lookup(py::handle positions_, py::handle index_table, int64_t index_o
   const int64_t num = positions.numel();
   LookupArgs a(num, positions.device(), index_table, lengths_table, std::move(sampled_out),
                std::move(local_out), std::move(lens_out));
-  check("gear_hip_lookup_i64",
-        gear_hip_lookup_i64(ptr<int64_t>(positions), num, a.index_table, a.index_n, index_offset,
-                            a.lengths_table, a.lengths_n, a.sampled_ptr(), a.local_ptr(), a.lens_ptr(),
-                            current_stream()));
+  call("gear_hip_lookup_i64", Scratch(), gear_hip_lookup_i64, ptr<int64_t>(positions), num,
+       a.index_table, a.index_n, index_offset, a.lengths_table, a.lengths_n, a.sampled_ptr(),
+       a.local_ptr(), a.lens_ptr(), current_stream());
   return py::make_tuple(a.sampled, a.local, a.lens);
 }
 
 py::object take_i64(py::handle table_, py::handle idx_, int64_t add, py::object out) {
   const at::Tensor &table = need(table_, at::kLong, "table"), &idx = need(idx_, at::kLong, "idx");
   if (out.is_none()) out = wrap(empty(idx.numel(), at::kLong, idx.device()));
-  check("gear_hip_take_i64",
-        gear_hip_take_i64(ptr<int64_t>(table), table.numel(), ptr<int64_t>(idx), idx.numel(), add,
-                          ptr_or_null<int64_t>(out, "out"), current_stream()));
+  call("gear_hip_take_i64", Scratch(), gear_hip_take_i64, ptr<int64_t>(table), table.numel(),
+       ptr<int64_t>(idx), idx.numel(), add, ptr_or_null<int64_t>(out, "out"), current_stream());
   return out;
 }
 
@@ -340,18 +368,21 @@ py::object take_i64(py::handle table_, py::handle idx_, int64_t add, py::object 
 py::object sort_i64(py::handle keys_, py::handle vals_, int64_t key_bits, py::handle ws) {
   const at::Tensor &keys = need(keys_, at::kLong, "keys");
   const int64_t num = keys.numel();
-  py::object keys_out = wrap(at::empty_like(keys)), vals_out = py::none();
+  auto like = [](const at::Tensor &t) {
+    py::gil_scoped_release nogil;
+    return at::empty_like(t);
+  };
+  py::object keys_out = wrap(like(keys)), vals_out = py::none();
   const int64_t *vals = nullptr;
   if (!vals_.is_none()) {
     const at::Tensor &v = need(vals_, at::kLong, "vals");
     vals = ptr<int64_t>(v);
-    vals_out = wrap(at::empty_like(v));
+    vals_out = wrap(like(v));
   }
   Scratch s(ws, "sort", gear_hip_sort_workspace_bytes(num), keys.device());
-  check("gear_hip_sort_i64",
-        gear_hip_sort_i64(ptr<int64_t>(keys), ptr_or_null<int64_t>(keys_out, "keys_out"), vals,
-                          ptr_or_null<int64_t>(vals_out, "vals_out"), num, (int)key_bits, s.ptr,
-                          s.bytes, current_stream()));
+  call("gear_hip_sort_i64", s, gear_hip_sort_i64, ptr<int64_t>(keys), ptr_or_null<int64_t>(keys_out,
+       "keys_out"), vals, ptr_or_null<int64_t>(vals_out, "vals_out"), num, (int)key_bits, s.ptr,
+       s.bytes, current_stream());
   if (vals) return py::make_tuple(std::move(keys_out), std::move(vals_out));
   return keys_out;
 }
@@ -364,15 +395,15 @@ py::object topk(py::handle priorities, int64_t k, bool by_value, bool want_value
   if (want_values) vals = wrap(empty(k, at::kFloat, p.device()));
   py::object idx = wrap(empty(k, at::kLong, p.device()));
   const size_t want = gear_hip_topk_workspace_bytes(n, k);
-  at::Tensor buf = workspace.is_none() ? Scratch(ws, "topk", want, p.device()).keep
-                                       : any_tensor(workspace, "workspace");
+  const Scratch s = workspace.is_none() ? Scratch(ws, "topk", want, p.device()) : Scratch();
+  const at::Tensor &buf = workspace.is_none() ? s.keep : any_tensor(workspace, "workspace");
   if ((size_t)buf.numel() < want)
     throw py::value_error("top-k workspace holds " + std::to_string(buf.numel()) + " bytes, " +
                           std::to_string(want) + " needed");
   const auto fn = warm ? gear_hip_topk_f32_warm : gear_hip_topk_f32;
-  check(warm ? "gear_hip_topk_f32_warm" : "gear_hip_topk_f32",
-        fn(ptr<float>(p), n, k, by_value, ptr_or_null<float>(vals, "values"),
-           ptr_or_null<int64_t>(idx, "indices"), buf.data_ptr(), (size_t)buf.numel(), current_stream()));
+  call(warm ? "gear_hip_topk_f32_warm" : "gear_hip_topk_f32", s, fn, ptr<float>(p), n, k, by_value,
+       ptr_or_null<float>(vals, "values"), ptr_or_null<int64_t>(idx, "indices"), buf.data_ptr(),
+       (size_t)buf.numel(), current_stream());
   return py::make_tuple(std::move(vals), std::move(idx));
 }
 
@@ -384,23 +415,14 @@ py::object scatter(py::object weights_, py::handle idx_, py::handle values_, boo
                    &values = need(values_, dtype, "values");
   const int64_t num = idx.numel();
   if (values.numel() != num) throw py::value_error("idx and values differ in length");
-  void *ptr_ws = nullptr;
-  size_t bytes = 0;
-  at::Tensor keep;
-  if (!unique) {
-    Scratch s(ws, "scatter", gear_hip_scatter_workspace_bytes(num), weights.device());
-    ptr_ws = s.ptr;
-    bytes = s.bytes;
-    keep = s.keep;
-  }
+  const Scratch s = unique ? Scratch()
+                           : Scratch(ws, "scatter", gear_hip_scatter_workspace_bytes(num), weights.device());
   if (dtype == at::kFloat)
-    check("gear_hip_scatter_f32",
-          gear_hip_scatter_f32(ptr<float>(weights), weights.numel(), ptr<int64_t>(idx),
-                               ptr<float>(values), num, unique, ptr_ws, bytes, current_stream()));
+    call("gear_hip_scatter_f32", s, gear_hip_scatter_f32, ptr<float>(weights), weights.numel(),
+         ptr<int64_t>(idx), ptr<float>(values), num, unique, s.ptr, s.bytes, current_stream());
   else
-    check("gear_hip_scatter_i64",
-          gear_hip_scatter_i64(ptr<int64_t>(weights), weights.numel(), ptr<int64_t>(idx),
-                               ptr<int64_t>(values), num, unique, ptr_ws, bytes, current_stream()));
+    call("gear_hip_scatter_i64", s, gear_hip_scatter_i64, ptr<int64_t>(weights), weights.numel(),
+         ptr<int64_t>(idx), ptr<int64_t>(values), num, unique, s.ptr, s.bytes, current_stream());
   return weights_;
 }
 
@@ -441,11 +463,10 @@ struct Gather {
         lens.scalar_type() != at::kLong)
       throw py::type_error("idxs, tss and lens must be int64 tensors");
     const c10::DeviceIndex dev = idxs.is_cuda() ? idxs.get_device() : c10::hip::current_device();
-    check("gear_hip_subcopy_multi_checked",
-          gear_hip_subcopy_multi_checked(reinterpret_cast<const void *>(src), num, ptr<int64_t>(idxs),
-                                         ptr<int64_t>(tss), ptr<int64_t>(lens), traj_stride, capacity,
-                                         trajectory_length, descs.data(), (int)descs.size(),
-                                         c10::hip::getCurrentHIPStream(dev).stream()));
+    call("gear_hip_subcopy_multi_checked", Scratch(), gear_hip_subcopy_multi_checked,
+         reinterpret_cast<const void *>(src), num, ptr<int64_t>(idxs), ptr<int64_t>(tss),
+         ptr<int64_t>(lens), traj_stride, capacity, trajectory_length, descs.data(), (int)descs.size(),
+         c10::hip::getCurrentHIPStream(dev).stream());
   }
 };
 
@@ -515,97 +536,104 @@ class LoaderStep {
                      &timesteps = need(timesteps_, at::kLong, "timesteps");
     const bool weighted = kind == "weighted";
     const at::Tensor &draws = need(draws_, weighted ? at::kFloat : at::kLong, "draws");
+    const bool uniform = kind == "uniform";
+    if (!weighted && !uniform && kind != "positions")
+      throw std::invalid_argument("kind must be 'weighted', 'uniform' or 'positions'");
     const int64_t num = draws.numel();
     const uintptr_t base = table_.attr("device_address").cast<uintptr_t>();
     if (base == 0)
       throw std::runtime_error(
           "table memory is not visible to the GPU: connect() it, with placement 'pinned' or 'device'");
-    void *st = current_stream();
-    at::Tensor sampled = empty(num, at::kLong, device_), lens = empty(num, at::kLong, device_),
-               local = empty(num, at::kLong, device_);
-    const int64_t *table = ptr<int64_t>(indices), *lengths = ptr<int64_t>(timesteps);
-    int64_t *s = ptr<int64_t>(sampled), *l = ptr<int64_t>(local), *len = ptr<int64_t>(lens);
+    const double *prefix = nullptr;
     if (weighted) {
-      const at::Tensor &prefix = need(prefix_, at::kDouble, "prefix");
-      if (prefix.numel() != indices.numel())
-        throw std::runtime_error("prefix and indices differ in length");
-      Scratch w(ws, "sample", gear_hip_sample_workspace_bytes(num), device_);
-      check("gear_hip_sample_lookup_f64",
-            gear_hip_sample_lookup_f64(ptr<double>(prefix), prefix.numel(), ptr<float>(draws), num, 1,
-                                       table, index_offset, lengths, timesteps.numel(), s, l, len,
-                                       w.ptr, w.bytes, st));
-    } else if (kind == "uniform") {
-      Scratch w(ws, "sample", gear_hip_sample_workspace_bytes(num), device_);
-      check("gear_hip_sort_lookup_i64",
-            gear_hip_sort_lookup_i64(ptr<int64_t>(draws), num, std::max<int64_t>(indices.numel(), 1),
-                                     table, indices.numel(), index_offset, lengths, timesteps.numel(),
-                                     s, l, len, w.ptr, w.bytes, st));
-    } else if (kind == "positions") {
-      check("gear_hip_lookup_i64",
-            gear_hip_lookup_i64(ptr<int64_t>(draws), num, table, indices.numel(), index_offset, lengths,
-                                timesteps.numel(), s, l, len, st));
-    } else {
-      throw std::invalid_argument("kind must be 'weighted', 'uniform' or 'positions'");
+      const at::Tensor &p = need(prefix_, at::kDouble, "prefix");
+      if (p.numel() != indices.numel()) throw std::runtime_error("prefix and indices differ in length");
+      prefix = ptr<double>(p);
     }
-    py::list batch(columns_.size());
-    py::object masks = py::none();
-    if (with_mask_) masks = py::list(columns_.size());
-    std::vector<gear_hip_column_desc> descs(columns_.size());
-    std::vector<int64_t> shape;
-    for (size_t k = 0; k < columns_.size(); ++k) {
-      const Column &c = columns_[k];
-      shape.assign(1, num);
-      shape.insert(shape.end(), c.shape.begin(), c.shape.end());
-      const at::Tensor t = at::empty(shape, at::TensorOptions().dtype(c.dtype).device(device_));
-      gear_hip_column_desc &d = descs[k];
-      d.dst = t.data_ptr();
-      d.mask_out = nullptr;
-      if (with_mask_) {
-        const at::Tensor m = at::empty({num, c.span}, at::TensorOptions().dtype(at::kByte).device(device_));
-        d.mask_out = ptr<uint8_t>(m);
-        PyList_SET_ITEM(masks.ptr(), (Py_ssize_t)k, THPVariable_Wrap(m));
+    Scratch w;
+    if (weighted || uniform) w = Scratch(ws, "sample", gear_hip_sample_workspace_bytes(num), device_);
+    void *st = current_stream();
+    at::Tensor sampled, lens, host;
+    std::vector<at::Tensor> batch(columns_.size()), masks(with_mask_ ? columns_.size() : 0);
+    Staging staged;
+    if (host_timesteps) staged.swap(staging_);
+    {
+      py::gil_scoped_release nogil;
+      const auto on_gpu = at::TensorOptions().device(device_);
+      sampled = at::empty({num}, on_gpu.dtype(at::kLong));
+      lens = at::empty({num}, on_gpu.dtype(at::kLong));
+      const at::Tensor local = at::empty({num}, on_gpu.dtype(at::kLong));
+      if (host_timesteps) host = at::empty({num}, at::TensorOptions().dtype(at::kLong));
+      std::vector<gear_hip_column_desc> descs(columns_.size());
+      std::vector<int64_t> shape;
+      for (size_t k = 0; k < columns_.size(); ++k) {
+        const Column &c = columns_[k];
+        shape.assign(1, num);
+        shape.insert(shape.end(), c.shape.begin(), c.shape.end());
+        batch[k] = at::empty(shape, on_gpu.dtype(c.dtype));
+        if (with_mask_) masks[k] = at::empty({num, c.span}, on_gpu.dtype(at::kByte));
+        gear_hip_column_desc &d = descs[k];
+        d.dst = batch[k].data_ptr();
+        d.mask_out = with_mask_ ? ptr<uint8_t>(masks[k]) : nullptr;
+        d.ofst = c.ofst;
+        d.span = c.span;
+        d.step_bytes = c.step_bytes;
+        d.col_base = c.col_base;
+        d.dst_stride = c.span * c.step_bytes;
+        d.pad_head = c.pad_head ? 1 : 0;
+        d.zero_fill = 1;
       }
-      d.ofst = c.ofst;
-      d.span = c.span;
-      d.step_bytes = c.step_bytes;
-      d.col_base = c.col_base;
-      d.dst_stride = c.span * c.step_bytes;
-      d.pad_head = c.pad_head ? 1 : 0;
-      d.zero_fill = 1;
-      PyList_SET_ITEM(batch.ptr(), (Py_ssize_t)k, THPVariable_Wrap(t));
-    }
-    if (num > 0)
-      check("gear_hip_subcopy_multi_checked",
-            gear_hip_subcopy_multi_checked(reinterpret_cast<const void *>(base), num, l, len, len,
-                                           traj_stride_, capacity_, trajectory_length_, descs.data(),
-                                           (int)descs.size(), st));
-    if (!host_timesteps) return py::make_tuple(wrap(sampled), wrap(lens), batch, masks);
-    // The lengths on the host.  The call returns when the gather has ended, as one that copied the
-    // lengths behind it: a table in host memory may be written again, and the batch read on any stream.
-    // (The staging buffer leaves the object for the time of the call: another thread that comes
-    // in while this one waits without the GIL makes one of its own.)
-    at::Tensor host = at::empty({num}, at::TensorOptions().dtype(at::kLong));
-    if (num > 0) {
-      Staging staged;
-      staged.swap(staging_);
-      if (!staged.buf.defined() || staged.buf.numel() < num)
-        staged.buf = at::empty({num}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
-      if (staged.arrived == nullptr)
-        hip("event", hipEventCreateWithFlags(&staged.arrived, hipEventDisableTiming));
-      staged.pending = static_cast<hipStream_t>(st);
-      staged.is_pending = true;
-      check("gear_hip_take_i64", gear_hip_take_i64(lengths, timesteps.numel(), l, num, 0,
-                                                   ptr<int64_t>(staged.buf), st));
-      hip("event record", hipEventRecord(staged.arrived, staged.pending));
-      {
-        py::gil_scoped_release nogil;
+      const int64_t *table = ptr<int64_t>(indices), *lengths = ptr<int64_t>(timesteps);
+      int64_t *s = ptr<int64_t>(sampled), *l = ptr<int64_t>(local), *len = ptr<int64_t>(lens);
+      if (weighted)
+        check("gear_hip_sample_lookup_f64", launches(w, [&] {
+                return gear_hip_sample_lookup_f64(prefix, indices.numel(), ptr<float>(draws), num, 1, table,
+                                                  index_offset, lengths, timesteps.numel(), s, l, len, w.ptr,
+                                                  w.bytes, st);
+              }));
+      else if (uniform)
+        check("gear_hip_sort_lookup_i64", launches(w, [&] {
+                return gear_hip_sort_lookup_i64(ptr<int64_t>(draws), num, std::max<int64_t>(indices.numel(), 1),
+                                                table, indices.numel(), index_offset, lengths,
+                                                timesteps.numel(), s, l, len, w.ptr, w.bytes, st);
+              }));
+      else
+        check("gear_hip_lookup_i64",
+              gear_hip_lookup_i64(ptr<int64_t>(draws), num, table, indices.numel(), index_offset, lengths,
+                                  timesteps.numel(), s, l, len, st));
+      if (num > 0)
+        check("gear_hip_subcopy_multi_checked",
+              gear_hip_subcopy_multi_checked(reinterpret_cast<const void *>(base), num, l, len, len,
+                                             traj_stride_, capacity_, trajectory_length_, descs.data(),
+                                             (int)descs.size(), st));
+      // The lengths on the host.  The call returns when the gather has ended, as one that copied the
+      // lengths behind it: a table in host memory may be written again, and the batch read on any stream.
+      // (The staging buffer leaves the object for the time of the call: another thread that comes
+      // in meanwhile makes one of its own.)
+      if (host_timesteps && num > 0) {
+        if (!staged.buf.defined() || staged.buf.numel() < num)
+          staged.buf = at::empty({num}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+        if (staged.arrived == nullptr)
+          hip("event", hipEventCreateWithFlags(&staged.arrived, hipEventDisableTiming));
+        staged.pending = static_cast<hipStream_t>(st);
+        staged.is_pending = true;
+        check("gear_hip_take_i64", gear_hip_take_i64(lengths, timesteps.numel(), l, num, 0,
+                                                     ptr<int64_t>(staged.buf), st));
+        hip("event record", hipEventRecord(staged.arrived, staged.pending));
         hip("event wait", hipEventSynchronize(staged.arrived));
+        staged.is_pending = false;
+        std::memcpy(host.data_ptr(), staged.buf.data_ptr(), (size_t)num * 8);
       }
-      staged.is_pending = false;
-      std::memcpy(host.data_ptr(), staged.buf.data_ptr(), (size_t)num * 8);
-      staged.swap(staging_);
     }
-    return py::make_tuple(wrap(sampled), wrap(host), batch, masks);
+    if (host_timesteps) staged.swap(staging_);
+    py::list batch_list(columns_.size());
+    py::object mask_list = py::none();
+    if (with_mask_) mask_list = py::list(columns_.size());
+    for (size_t k = 0; k < columns_.size(); ++k) {
+      PyList_SET_ITEM(batch_list.ptr(), (Py_ssize_t)k, THPVariable_Wrap(batch[k]));
+      if (with_mask_) PyList_SET_ITEM(mask_list.ptr(), (Py_ssize_t)k, THPVariable_Wrap(masks[k]));
+    }
+    return py::make_tuple(wrap(sampled), wrap(host_timesteps ? host : lens), batch_list, mask_list);
   }
 
  private:
@@ -623,7 +651,9 @@ PYBIND11_MODULE(_hostops, m) {
   py::class_<Workspace>(m, "Workspace", py::dynamic_attr())
       .def(py::init<>())
       .def("get", [](Workspace &w, const std::string &tag, size_t bytes, const at::Device &device) {
-        return wrap(w.get(tag.c_str(), bytes, device));
+        at::Tensor buf;
+        w.get(tag.c_str(), bytes, device, &buf);
+        return wrap(buf);
       });
   m.def("prefix_sum", &prefix_sum);
   m.def("prefix_sum_i64", &prefix_sum_i64);
