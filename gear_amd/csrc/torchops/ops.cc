@@ -95,20 +95,20 @@ class Workspace {
     at::Tensor buf;
     std::mutex order;  // held while a call enqueues its launches on the buffer's stream
   };
-  // (the GIL is held; the entry stays the same while its buffer grows)
-  std::shared_ptr<Entry> get(const char *tag, size_t bytes, const at::Device &device, at::Tensor *buf) {
+  // (the GIL is held)
+  std::shared_ptr<Entry> entry(const char *tag, const at::Device &device) {
     const c10::DeviceIndex index = device.has_index() ? device.index() : c10::hip::current_device();
-    void *stream = c10::hip::getCurrentHIPStream(index).stream();
-    std::shared_ptr<Entry> &slot = entries_[Key{tag, index, stream}];
+    std::shared_ptr<Entry> &slot = entries_[Key{tag, index, c10::hip::getCurrentHIPStream(index).stream()}];
     if (!slot) slot = std::make_shared<Entry>();
-    std::shared_ptr<Entry> e = slot;
-    if (!e->buf.defined() || (size_t)e->buf.numel() < bytes) {
+    return slot;
+  }
+  static at::Tensor buffer(Entry &e, size_t bytes, const at::Device &device) {
+    if (!e.buf.defined() || (size_t)e.buf.numel() < bytes) {
       at::Tensor grown = empty((int64_t)std::max<size_t>(bytes, 256), at::kByte, device);
       // (another thread may have been here meanwhile)
-      if (!e->buf.defined() || e->buf.numel() < grown.numel()) e->buf = grown;
+      if (!e.buf.defined() || e.buf.numel() < grown.numel()) e.buf = grown;
     }
-    *buf = e->buf;
-    return e;
+    return e.buf;
   }
 
  private:
@@ -133,12 +133,13 @@ struct Scratch {
   std::shared_ptr<Workspace::Entry> entry;
   Scratch() = default;  // none
   Scratch(py::handle ws, const char *tag, size_t want, const at::Device &device) {
+    entry = ws.cast<Workspace &>().entry(tag, device);
     PyObject **dict = _PyObject_GetDictPtr(ws.ptr());
     if (dict != nullptr && *dict != nullptr && PyDict_GET_SIZE(*dict) != 0)
       keep = THPVariable_Unpack(
           ws.attr("get")(tag, want, py::reinterpret_steal<py::object>(THPDevice_New(device))).ptr());
     else
-      entry = ws.cast<Workspace &>().get(tag, want, device, &keep);
+      keep = Workspace::buffer(*entry, want, device);
     ptr = keep.data_ptr();
     bytes = (size_t)keep.numel();
   }
@@ -651,9 +652,8 @@ PYBIND11_MODULE(_hostops, m) {
   py::class_<Workspace>(m, "Workspace", py::dynamic_attr())
       .def(py::init<>())
       .def("get", [](Workspace &w, const std::string &tag, size_t bytes, const at::Device &device) {
-        at::Tensor buf;
-        w.get(tag.c_str(), bytes, device, &buf);
-        return wrap(buf);
+        const std::shared_ptr<Workspace::Entry> e = w.entry(tag.c_str(), device);
+        return wrap(Workspace::buffer(*e, bytes, device));
       });
   m.def("prefix_sum", &prefix_sum);
   m.def("prefix_sum_i64", &prefix_sum_i64);
