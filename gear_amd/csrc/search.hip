@@ -29,7 +29,8 @@ constexpr int kBlock = 256;
 //     16384   5.3 / 8.9     4.9 / 7.9      6.2 / 9.9      7.6 / 13
 //     65536  10.1 / 20.6   11.2 / 21.2    16.3 / 28.5    22.7 / 41
 // hence 16 lanes up to 4096 draws, 8 up to 32768, 1 beyond (search_lanes).
-inline int search_lanes(int64_t num) { return num <= 4096 ? 16 : num <= 32768 ? 8 : 1; }
+constexpr int64_t kMost16 = 4096, kMost8 = 32768;
+inline int search_lanes(int64_t num) { return num <= kMost16 ? 16 : num <= kMost8 ? 8 : 1; }
 
 template <int kLanes>
 struct Probe {
@@ -579,9 +580,14 @@ int launch_search(const Draw &draw, int64_t num, int64_t *idx_out, hipStream_t s
   return 0;
 }
 
+// (More draws may take fewer lanes each and so fewer workgroups: what is asked for is enough for every
+// smaller batch as well.)
 size_t search_ws_bytes(int64_t num) {
   if (num <= 0) return 256;
-  return align_up((size_t)num * 8, 256) + align_up((size_t)search_blocks(num) * 8, 256);
+  int64_t blocks = search_blocks(num);
+  for (const int64_t most : {(int64_t)kMost16, (int64_t)kMost8})
+    if (most < num && search_blocks(most) > blocks) blocks = search_blocks(most);
+  return align_up((size_t)num * 8, 256) + align_up((size_t)blocks * 8, 256);
 }
 
 }  // namespace

@@ -88,3 +88,17 @@ def test_header_is_plain_c(tmp_path):
     inc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include")
     subprocess.run([gcc, "-std=c99", "-Wall", "-Wextra", "-pedantic", "-Werror", "-I", inc, "-c",
                     str(src), "-o", str(tmp_path / "use_header.o")], check=True)
+
+
+def test_scratch_sizes_never_shrink_with_the_batch():
+    """Scratch sized for the largest batch serves every smaller one."""
+    from gear_amd import _cabi
+    lib = _cabi.load()
+    sizes = sorted(set(list(range(0, 300)) + list(range(3800, 4400)) + list(range(32_000, 36_000)) +
+                       list(range(131_000, 131_200)) + [1 << k for k in range(30)]))
+    for query in ("gear_hip_search_workspace_bytes", "gear_hip_sample_workspace_bytes",
+                  "gear_hip_sort_workspace_bytes", "gear_hip_scatter_workspace_bytes",
+                  "gear_hip_scan_workspace_bytes"):
+        fn = getattr(lib, query)
+        need = [fn(n) for n in sizes]
+        assert all(a <= b for a, b in zip(need, need[1:])), query
