@@ -1,7 +1,8 @@
 // Priority update weights[idx[j]] = values[j] with "last occurrence wins" for repeated indices.
 //
 // With unique indices this is one scatter.  Otherwise only the last update of an index is written:
-//  * up to kClassMax updates: one launch, a hash table in LDS a workgroup.
+//  * up to kClassMax updates (kClassMaxDigit in a short table): one launch, a hash table in LDS a
+//    workgroup.
 //  * beyond that, and where a buffer overlaps another or a table has more entries than 32 bits
 //    count: the (index, position) pairs go through the stable LSD radix sort on the index, and the
 //    last element of each run is written.
@@ -58,13 +59,18 @@ __global__ __launch_bounds__(kBlock) void scatter_winners_kernel(T *__restrict__
 // overflow (indices that crowd in one class), the class is taken in 2, 4, ... parts by further bits
 // of the hash; part and slot together are at last the whole hash, which no two indices share.
 // us a call, back to back, here / by sorting the pairs (a ranking sort up to 4096):
-//     updates of   1e4 entries    1e7 entries   5 entries
-//         64        4.2 / 11.9     4.1 / 11.9    4.3 / 11.9
-//       4096        4.7 / 13.4     4.6 / 13.4    5.7 / 13.1
-//     16 384        6.3 / 21.3     6.3 / 29.0    8.1 / 20.5
-//     65 536       13.0 / 21.9    13.8 / 31.3   18.8 / 21.6
-//    131 072       21.5 / 26.5    23.1 / 38.1   32.3 / 24.6
-// Beyond that the looks outweigh the launches saved (262 144 updates of 1e6 entries: 40 / 45).
+//     updates of   5 entries    255 entries    1e4 entries    1e7 entries   5 of 1e4 entries
+//         64        4.3 / 11.9                   4.2 / 11.9     4.1 / 11.9
+//       4096        5.7 / 13.1                   4.7 / 13.4     4.6 / 13.4
+//     32 768       11.9 / 12.0    8.8 / 12.9     8.4 / 20.3     8.6 / 29.0    11.0 / 19.7
+//     40 960       13.5 / 12.4   10.0 / 12.9     9.5 / 20.6     9.9 / 30.0    12.5 / 19.8
+//     65 536       18.8 / 12.7   13.6 / 13.4    12.6 / 21.5    13.5 / 31.1    17.9 / 20.6
+//    131 072       32.4 / 14.2   23.3 / 15.6    21.0 / 25.8    22.6 / 38.3    31.7 / 24.0
+//    196 608       46.0 / 15.6   33.1 / 17.3    29.5 / 28.8    32.7 / 43.3    45.7 / 26.2
+// Tables below 256 entries are one digit for the sort, which is the faster one from 40 960 updates on;
+// for others the limit is the last size at which updates spread over the table win at every length of
+// it.  (Indices that repeat thousands of times while the table is long lose a third there, and win
+// below 90 000.)
 constexpr int kClassThreads = 1024;
 constexpr int kClassWaves = kClassThreads / kWave;
 constexpr int kClassBits = 8, kSlotBits = 11, kPartBits = 32 - kSlotBits;
@@ -72,12 +78,13 @@ constexpr int kClasses = 1 << kClassBits, kSlots = 1 << kSlotBits;
 constexpr int kMaxProbes = 128;
 constexpr int kQueue = 2 * kWave;
 constexpr int64_t kClassMax = 131072;  // a quarter of the slots when no index repeats
+constexpr int64_t kClassMaxDigit = 40960;  // tables below 256 entries
 constexpr uint64_t kEmpty = ~0ull;
 
 __device__ __forceinline__ uint32_t class_of(uint32_t x) {
   return (uint32_t)__umul24(x ^ (x >> 15), 0x9E3779u) >> (32 - kClassBits);
 }
-__device__ __forceinline__ uint32_t hash_of(uint32_t x) {  // one to one
+__device__ __forceinline__ uint32_t hash_of(uint32_t x) {  // one to one (multipliers: xxHash32's primes)
   x ^= x >> 16;
   x *= 0x9E3779B1u;
   x ^= x >> 15;
@@ -218,7 +225,7 @@ int scatter_any(T *weights, int64_t n, const int64_t *idx, const T *values, int6
     return GEAR_HIP_EWORKSPACE;
   const int64_t bytes = num * (int64_t)sizeof(T), wbytes = n * (int64_t)sizeof(T);
   if (!ranges::overlap(weights, wbytes, idx, num * 8) && !ranges::overlap(weights, wbytes, values, bytes)) {
-    if (num <= kClassMax && n < (1ll << 32)) {
+    if (num <= (n < 256 ? kClassMaxDigit : kClassMax) && n < (1ll << 32)) {
       scatter_class_kernel<T><<<dim3(kClasses), dim3(kClassThreads), 0, st>>>(weights, (uint32_t)n, idx,
                                                                             values, (int)num);
       GEARHIP_RETURN_IF_LAUNCH_FAILED();
