@@ -75,3 +75,44 @@ def test_look_ups_on_top_of_the_positions(num, bound):
         got = ops.sort_lookup(x, bound, index_offset=5, **{name: x})
         assert np.array_equal(got[0].cpu().numpy(), np.sort(pos)), name
         assert np.array_equal(got[1].cpu().numpy(), np.sort(pos) - 5), name
+
+
+@pytest.mark.parametrize("num", [100, 4096, 4097, 50_000])
+def test_updates_of_a_table_that_holds_their_indices(num):
+    """The indices are read before the table, whose first entries they are, is written over."""
+    from gear_amd import ops
+    rng = np.random.default_rng(num)
+    n = 70_001
+    table = rng.integers(0, n, size=n)
+    val = rng.integers(-5, 0, size=num)
+    want = table.copy()
+    for i, v in zip(table[:num], val):
+        want[i] = v
+    announce("updates num=%d by indices in the table" % num)
+    got = torch.from_numpy(table).cuda()
+    ops.scatter(got, got[:num], torch.from_numpy(val).cuda())
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("num", [4097, 20_000, 32_768])
+def test_sorted_keys_on_top_of_a_part_of_the_payload(num):
+    """Outputs that overlap inputs other than themselves, through the C ABI (the sort refuses outputs that
+    are its inputs)."""
+    import ctypes
+    from gear_amd import _cabi
+    lib = _cabi.load()
+    rng = np.random.default_rng(num)
+    keys = rng.integers(0, 1 << 16, size=num)      # two digits: the payload is read by the first launches
+    order = np.argsort(keys, kind="stable")
+    announce("sort num=%d with the keys stored over half of the payload" % num)
+    block = torch.empty(num + num // 2, dtype=torch.int64, device="cuda")
+    vin, kout = block[:num], block[num // 2:]
+    vin.copy_(torch.arange(num, device="cuda"))
+    kin, vout = torch.from_numpy(keys).cuda(), torch.empty(num, dtype=torch.int64, device="cuda")
+    ws = torch.empty(int(lib.gear_hip_sort_workspace_bytes(num)), dtype=torch.uint8, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    code = lib.gear_hip_sort_i64(p(kin), p(kout), p(vin), p(vout), num, 16, p(ws), ws.numel(),
+                                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert code == 0
+    assert np.array_equal(vout.cpu().numpy(), order)
+    assert np.array_equal(kout.cpu().numpy(), keys[order])
