@@ -105,9 +105,9 @@ __device__ __forceinline__ int64_t group_search(const T *__restrict__ p, int64_t
 }
 
 // The targets of a batch of draws, and keys of the same order to rank the draws by.
-// fp64 prefix: fp32 draws, in [0, 1) (unit) or targets already.  A NaN target compares with nothing
-// and finds entry 0, so a NaN draw has the lowest key (and whatever a NaN or infinite total makes
-// NaN lies next to draws that find entry 0 too).
+// fp64 prefix: fp32 draws, in [0, 1) (unit) or targets already.  A target that is not a number -- the
+// draw or the total is none, or infinite where the other is 0 -- compares with nothing and finds
+// entry 0, so it has the lowest key.
 struct DrawF64 {
   typedef double type;
   typedef uint32_t key_type;
@@ -123,7 +123,8 @@ struct DrawF64 {
     const uint32_t b = __float_as_uint(f);
     uint32_t k = b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
     if (unit && total < 0.0) k = ~k;  // (priorities are not negative; the order holds all the same)
-    return f == f ? k : 0u;
+    const double t = target(j, total);
+    return t == t ? k : 0u;
   }
 };
 // int64 prefix (a sampler over lengths): doubles in [0, 1) (unit) or int64 targets.

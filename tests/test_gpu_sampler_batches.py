@@ -68,3 +68,44 @@ def test_draws_in_an_integer_prefix_and_given_positions(num):
                           lengths_table=torch.from_numpy(lengths).cuda())
     want = np.sort(pos)
     assert np.array_equal(got[0].cpu().numpy(), table.cpu().numpy()[want])
+
+
+@pytest.mark.parametrize("num", [17, 4096, 4097, 20_481, 32_768, 32_769])
+@pytest.mark.parametrize("total", [0.0, np.inf, -np.inf, np.nan])
+def test_batches_ascend_whatever_the_total_is(num, total):
+    """Unit draws times a total of 0, an infinity or no number: some targets are not numbers, which find
+    entry 0, wherever the draw lies among the others."""
+    from gear_amd import ops
+    rng = np.random.default_rng(num)
+    n = 1000
+    prefix = np.zeros(n) if total == 0.0 else np.arange(1.0, n + 1.0)
+    prefix[-3:] = total
+    u = rng.random(num, dtype=np.float32)
+    odd = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1.0, -1.0], np.float32)
+    u[rng.integers(0, num, size=num // 2)] = odd[rng.integers(0, len(odd), size=num // 2)]
+    announce("batch of %d draws, total %r" % (num, total))
+    dev, draws = torch.from_numpy(prefix).cuda(), torch.from_numpy(u).cuda()
+    got = ops.sample_sorted(dev, draws, unit_uniforms=True).cpu().numpy()
+    assert np.all(got[:-1] <= got[1:])
+    found = ops.upper_bound(dev, draws, unit_uniforms=True).cpu().numpy()
+    if total in (0.0, np.inf):       # (the prefix ascends: what is found does not depend on the probes)
+        assert np.array_equal(got, np.sort(found))
+
+
+@pytest.mark.parametrize("num", [4096, 4097, 12_288, 12_289, 24_576, 24_577, 32_768, 32_769])
+def test_batches_ascend_in_a_prefix_with_dips(num):
+    """A prefix of rounded sums can dip by a unit in the last place behind zero priorities."""
+    from gear_amd import ops
+    rng = np.random.default_rng(num)
+    n = 20_011
+    prefix = np.cumsum(rng.random(n) * (rng.random(n) < 0.3))
+    dips = rng.integers(1, n - 1, size=n // 4)
+    prefix[dips] = np.nextafter(prefix[dips], 0.0)
+    u = (prefix[rng.integers(0, n, size=num)] / prefix[-1]).astype(np.float32)   # draws at the entries
+    announce("batch of %d draws, prefix with dips" % num)
+    dev = torch.from_numpy(prefix).cuda()
+    got = ops.sample_sorted(dev, torch.from_numpy(u).cuda(), unit_uniforms=True).cpu().numpy()
+    assert np.all(got[:-1] <= got[1:])
+    t = prefix[rng.integers(0, n, size=num)].astype(np.float32)
+    got = ops.sample_lookup(dev, torch.from_numpy(t).cuda(), unit_uniforms=False)[0].cpu().numpy()
+    assert np.all(got[:-1] <= got[1:])
