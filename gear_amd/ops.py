@@ -361,7 +361,7 @@ def topk(priorities, k, *, sorted_by_value=True, want_values=True, warm=False, w
     """Top-k of fp32 priorities (values, indices), by value descending or by index ascending.
     warm=True: the call may start from the bound that the last call on `workspace` (same n, k and
     order) left there instead of sampling the array; the result is the same either way."""
-    return _hostops.topk(priorities, int(k), bool(sorted_by_value), bool(want_values), bool(warm),
+    return _hostops.topk(priorities, k, bool(sorted_by_value), bool(want_values), bool(warm),
                          workspace, _ws)
 
 

@@ -30,3 +30,16 @@ def test_wrong_arguments_are_named():
         ops.sort_i64(f)
     with pytest.raises(TypeError, match="scatter works on float32 or int64 tables"):
         ops.scatter(f.double(), f.long(), f.double())
+
+
+def test_a_number_of_entries_is_an_integer():
+    """Integers of any type count, a fraction is refused and not cut off."""
+    import numpy as np
+    from gear_amd import ops
+    f = torch.zeros(8)
+    for k in (2, np.int64(2), torch.tensor(2)):
+        with pytest.raises(ValueError, match="priorities must live on the GPU"):
+            ops.topk(f, k)
+    for k in (2.0, 2.7, "2", None):
+        with pytest.raises(TypeError):
+            ops.topk(f, k)
