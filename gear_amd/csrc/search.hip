@@ -28,9 +28,20 @@ constexpr int kBlock = 256;
 //      4096   4.9 / 6.2     4.1 / 4.9      3.7 / 4.6      3.9 / 5.3
 //     16384   5.3 / 8.9     4.9 / 7.9      6.2 / 9.9      7.6 / 13
 //     65536  10.1 / 20.6   11.2 / 21.2    16.3 / 28.5    22.7 / 41
-// hence 16 lanes up to 4096 draws, 8 up to 32768, 1 beyond (search_lanes).
-constexpr int64_t kMost16 = 4096, kMost8 = 32768;
-inline int search_lanes(int64_t num) { return num <= kMost16 ? 16 : num <= kMost8 ? 8 : 1; }
+// hence 16 lanes up to 4096 draws, 8 up to 32768, 1 beyond; with importance weights, which each lane of
+// a group works out, 8 up to 24576 (32768 draws: 12.6 / 18.6 with 8, 11.2 / 17.1 with 1).  With one lane
+// a draw, workgroups of one wave spread fewer draws over more CUs (40000: 7.9 / 14.5, 8.9 / 15.2 in
+// workgroups of four), and are too many for a hundred thousand (15.8 / 32.2, 17.0 / 29.5; with weights
+// 22.1 / 39.0, 22.2 / 35.2; the two meet at 65536).
+struct SearchShape {
+  int lanes, threads;
+};
+constexpr int64_t kMost16 = 4096, kMost8 = 32768, kMost8Weights = 24576, kMostWaves = 49152;
+inline SearchShape search_shape(int64_t num, bool weights) {
+  if (num <= kMost16) return {16, kBlock};
+  if (num <= (weights ? kMost8Weights : kMost8)) return {8, kBlock};
+  return {1, num <= kMostWaves ? kWave : kBlock};
+}
 
 template <int kLanes>
 struct Probe {
@@ -142,10 +153,10 @@ struct DrawI64 {
   __device__ __forceinline__ int64_t key(int64_t j, int64_t total) const { return target(j, total); }
 };
 
-template <int kLanes, typename Draw>
-__global__ __launch_bounds__(kBlock) void search_kernel(Draw draw, int64_t num,
-                                                        int64_t *__restrict__ idx_out) {
-  const int64_t j = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kLanes;
+template <int kLanes, int kThreads, typename Draw>
+__global__ __launch_bounds__(kThreads) void search_kernel(Draw draw, int64_t num,
+                                                          int64_t *__restrict__ idx_out) {
+  const int64_t j = ((int64_t)blockIdx.x * kThreads + threadIdx.x) / kLanes;
   const int sub = threadIdx.x & (kLanes - 1);
   if (j >= num) return;
   const int64_t i = group_search<kLanes>(
@@ -155,12 +166,12 @@ __global__ __launch_bounds__(kBlock) void search_kernel(Draw draw, int64_t num,
 
 // The same with the raw importance weights (N * p / total) ** -beta of the found entries and their
 // maximum per workgroup.
-template <int kLanes>
-__global__ __launch_bounds__(kBlock) void search_weights_kernel(
+template <int kLanes, int kThreads>
+__global__ __launch_bounds__(kThreads) void search_weights_kernel(
     DrawF64 draw, int64_t num, int64_t *__restrict__ idx_out, const float *__restrict__ priorities,
     double beta, double *__restrict__ wraw, double *__restrict__ block_max) {
-  __shared__ double wmax[kBlock / kWave];
-  const int64_t j = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kLanes;
+  __shared__ double wmax[kThreads / kWave];
+  const int64_t j = ((int64_t)blockIdx.x * kThreads + threadIdx.x) / kLanes;
   const int sub = threadIdx.x & (kLanes - 1);
   double w = 0.0;
   if (j < num) {
@@ -177,10 +188,16 @@ __global__ __launch_bounds__(kBlock) void search_weights_kernel(
   }
   // (weights are positive, lanes without a draw hold 0)
   for (int off = 32; off >= kLanes; off >>= 1) w = fmax(w, __shfl_xor(w, off, kWave));
+  if (kThreads == kWave) {
+    if (threadIdx.x == 0) block_max[blockIdx.x] = w;
+    return;
+  }
   if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x / kWave] = w;
   __syncthreads();
-  if (threadIdx.x == 0)
-    block_max[blockIdx.x] = fmax(fmax(wmax[0], wmax[1]), fmax(wmax[2], wmax[3]));
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < kThreads / kWave; ++i) w = fmax(w, wmax[i]);
+    block_max[blockIdx.x] = w;
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void normalise_kernel(const double *__restrict__ wraw,
@@ -556,26 +573,33 @@ SampleWs sample_ws(int64_t num) {
   return w;
 }
 
-int64_t search_blocks(int64_t num) { return ceil_div64(num * search_lanes(num), kBlock); }
+int64_t search_blocks(int64_t num, bool weights) {
+  const SearchShape s = search_shape(num, weights);
+  return ceil_div64(num * s.lanes, s.threads);
+}
 
-// calls f(std::integral_constant<int, lanes>) for the batch's number of lanes per draw
+// calls f(lanes per draw, threads per workgroup), both as std::integral_constant
 template <typename F>
-void with_search_lanes(int64_t num, const F &f) {
-  const int lanes = search_lanes(num);
-  if (lanes == 16)
-    f(std::integral_constant<int, 16>{});
-  else if (lanes == 8)
-    f(std::integral_constant<int, 8>{});
+void with_search_shape(int64_t num, bool weights, const F &f) {
+  const SearchShape s = search_shape(num, weights);
+  const std::integral_constant<int, kBlock> block;
+  if (s.lanes == 16)
+    f(std::integral_constant<int, 16>{}, block);
+  else if (s.lanes == 8)
+    f(std::integral_constant<int, 8>{}, block);
+  else if (s.threads == kWave)
+    f(std::integral_constant<int, 1>{}, std::integral_constant<int, kWave>{});
   else
-    f(std::integral_constant<int, 1>{});
+    f(std::integral_constant<int, 1>{}, block);
 }
 template <typename Draw>
 int launch_search(const Draw &draw, int64_t num, int64_t *idx_out, hipStream_t st) {
-  const int64_t blocks = search_blocks(num);
+  const int64_t blocks = search_blocks(num, false);
   if (blocks >= 0x7fffffffll) return GEAR_HIP_ERANGE;
-  with_search_lanes(num, [&](auto lanes) {
-    search_kernel<decltype(lanes)::value><<<dim3((unsigned)blocks), dim3(kBlock), 0, st>>>(draw, num,
-                                                                                        idx_out);
+  with_search_shape(num, false, [&](auto lanes, auto threads) {
+    constexpr int kThreads = decltype(threads)::value;
+    search_kernel<decltype(lanes)::value, kThreads>
+        <<<dim3((unsigned)blocks), dim3(kThreads), 0, st>>>(draw, num, idx_out);
   });
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
   return 0;
@@ -585,9 +609,9 @@ int launch_search(const Draw &draw, int64_t num, int64_t *idx_out, hipStream_t s
 // smaller batch as well.)
 size_t search_ws_bytes(int64_t num) {
   if (num <= 0) return 256;
-  int64_t blocks = search_blocks(num);
-  for (const int64_t most : {(int64_t)kMost16, (int64_t)kMost8})
-    if (most < num && search_blocks(most) > blocks) blocks = search_blocks(most);
+  int64_t blocks = search_blocks(num, true);
+  for (const int64_t most : {kMost16, kMost8Weights, kMostWaves})
+    if (most < num && search_blocks(most, true) > blocks) blocks = search_blocks(most, true);
   return align_up((size_t)num * 8, 256) + align_up((size_t)blocks * 8, 256);
 }
 
@@ -606,7 +630,7 @@ extern "C" int gear_hip_upper_bound_f64(const double *prefix, int64_t n, const f
   if (num == 0) return 0;
   if (n == 0 || !prefix || !u || !idx_out) return GEAR_HIP_EINVAL;
   if ((priorities == nullptr) != (weights_out == nullptr)) return GEAR_HIP_EINVAL;
-  const int64_t blocks = search_blocks(num);
+  const int64_t blocks = search_blocks(num, priorities != nullptr);
   const int64_t nblocks = ceil_div64(num, kBlock);
   if (blocks >= 0x7fffffffll) return GEAR_HIP_ERANGE;
   double *wraw = nullptr, *bmax = nullptr;
@@ -621,9 +645,10 @@ extern "C" int gear_hip_upper_bound_f64(const double *prefix, int64_t n, const f
   hipStream_t st = as_stream(stream);
   const DrawF64 draw{prefix, n, u, unit_uniforms ? 1 : 0};
   if (!priorities) return launch_search(draw, num, idx_out, st);
-  with_search_lanes(num, [&](auto lanes) {
-    search_weights_kernel<decltype(lanes)::value><<<dim3((unsigned)blocks), dim3(kBlock), 0, st>>>(
-        draw, num, idx_out, priorities, beta, wraw, bmax);
+  with_search_shape(num, true, [&](auto lanes, auto threads) {
+    constexpr int kThreads = decltype(threads)::value;
+    search_weights_kernel<decltype(lanes)::value, kThreads>
+        <<<dim3((unsigned)blocks), dim3(kThreads), 0, st>>>(draw, num, idx_out, priorities, beta, wraw, bmax);
   });
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
   normalise_kernel<<<dim3((unsigned)nblocks), dim3(kBlock), 0, st>>>(wraw, bmax, (int)blocks, num,

@@ -94,7 +94,8 @@ def test_scratch_sizes_never_shrink_with_the_batch():
     """Scratch sized for the largest batch serves every smaller one."""
     from gear_amd import _cabi
     lib = _cabi.load()
-    sizes = sorted(set(list(range(0, 300)) + list(range(3800, 4400)) + list(range(32_000, 36_000)) +
+    sizes = sorted(set(list(range(0, 300)) + list(range(3800, 4400)) + list(range(24_000, 25_200)) +
+                       list(range(32_000, 36_000)) + list(range(49_000, 49_400)) +
                        list(range(131_000, 131_200)) + [1 << k for k in range(30)]))
     for query in ("gear_hip_search_workspace_bytes", "gear_hip_sample_workspace_bytes",
                   "gear_hip_sort_workspace_bytes", "gear_hip_scatter_workspace_bytes",

@@ -109,3 +109,21 @@ def test_batches_ascend_in_a_prefix_with_dips(num):
     t = prefix[rng.integers(0, n, size=num)].astype(np.float32)
     got = ops.sample_lookup(dev, torch.from_numpy(t).cuda(), unit_uniforms=False)[0].cpu().numpy()
     assert np.all(got[:-1] <= got[1:])
+
+
+@pytest.mark.parametrize("num", [1, 17, 4096, 4097, 24_576, 24_577, 32_768, 32_769, 49_152, 49_153])
+def test_importance_weights_at_the_limits_of_the_search(num):
+    """Weights against the same in float64, rounded once: two roundings of float32 apart at most."""
+    from gear_amd import ops
+    rng = np.random.default_rng(num)
+    n = 30_011
+    pri = rng.lognormal(size=n).astype(np.float32)
+    prefix = np.cumsum(pri.astype(np.float64))
+    u = rng.random(num, dtype=np.float32)
+    announce("importance weights num=%d" % num)
+    at, w = ops.upper_bound(torch.from_numpy(prefix).cuda(), torch.from_numpy(u).cuda(),
+                            unit_uniforms=True, priorities=torch.from_numpy(pri).cuda(), beta=0.4)
+    want = np.minimum(np.searchsorted(prefix, u.astype(np.float64) * prefix[-1], side="right"), n - 1)
+    assert np.array_equal(at.cpu().numpy(), want)
+    raw = (n * pri[want].astype(np.float64) / prefix[-1]) ** -0.4
+    assert np.max(np.abs(w.cpu().numpy() / (raw / raw.max()) - 1)) < 2.0 ** -23
