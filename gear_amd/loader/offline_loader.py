@@ -22,6 +22,7 @@ from typing import Any, Dict, List, Sequence, Union
 import torch
 
 from .. import _hostops, ops
+from .._cabi import MAX_COLUMNS
 from ..dataset import SharedDataset
 from ..dtypes import CVT_DTYPES_GEAR_TO_TORCH
 from ..libgear import core as glibc
@@ -111,7 +112,8 @@ class OfflineLoader(BasicLoader):
         self._sampler.indices_ascending = True   # arange + offset below
         self._indices = torch.arange(self._iset.local_capacity, dtype=torch.long,
                                      device=self._mpu.device) + self._iset.index_offset
-        self._step = None   # made by the first fused step
+        # (what the fused step cannot gather is refused by the fused step, not here)
+        self._step = self._native_step() if len(self._sub_cols) <= MAX_COLUMNS else None
         self.last_masks = None
         self.last_sampled = None   # global indices of the last batch (device tensor)
 
