@@ -458,7 +458,9 @@ inline int64_t worth(int key_bits) { return key_bits <= 8 ? 0 : key_bits <= 16 ?
 template <typename C, bool kLook, typename Src, typename Emit>
 int sort(const Src &src, int64_t num, const Emit &emit, hipStream_t st) {
   const dim3 grid(kGroups), block(kThreads);
-  // (rounds beyond the batch's own cost registers and a skipped branch each)
+  // Rounds beyond the batch's own cost registers and a skipped branch each: 8192 keys take 8.5 / 10.1 /
+  // 11.8 us in kernels of 8 / 20 / 32 rounds (20 bits; 10.0 / 12.2 / 17.3 with 63), 20 000 keys 12.3 / 14.1
+  // in 20 / 32 (15.3 / 20.4).  A batch just beyond a step pays for it: 20 480 / 20 481 keys 12.4 / 14.4 us.
   const int n = (int)num, per = (int)ceil_div64(num, kThreads);
   if (per <= 8)
     range_sort_kernel<C, 8, kLook, Src, Emit><<<grid, block, 0, st>>>(src, n, emit);

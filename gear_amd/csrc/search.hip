@@ -134,7 +134,8 @@ struct DrawF64 {
     const uint32_t b = __float_as_uint(f);
     uint32_t k = b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
     if (unit && total < 0.0) k = ~k;  // (priorities are not negative; the order holds all the same)
-    const double t = target(j, total);
+    // (no number where the target is none; as one multiplication in fp32)
+    const float t = f * (unit && (total == 0.0 || __builtin_isinf(total)) ? (float)total : 1.0f);
     return t == t ? k : 0u;
   }
 };
@@ -547,8 +548,16 @@ bool apart(const Draw &draw, int64_t num, const Emit &emit) {
 template <typename Draw, typename Emit>
 int sort_draws(const Draw &draw, int64_t num, const Emit &emit, hipStream_t st) {
   typedef DrawSrc<Draw> Src;
-  // as many lanes a draw as let a workgroup search most shares (num / 256 draws) in one round
-  const int lanes = num <= 12288 ? 16 : num <= 24576 ? 8 : 1;
+  // Lanes a draw: a workgroup searches num / 256 draws, a few more where keys crowd, and 16 lanes each
+  // let it search 64 at once.  us a batch in 1e5 / 1e7 entries by lanes:
+  //     draws         16             8              1
+  //      4097    9.5 /  9.7     9.6 / 10.1    10.0 / 10.6
+  //      8192   10.3 / 11.0    10.5 / 11.1    10.6 / 11.3
+  //     12288   13.5 / 15.7    12.8 / 13.4    12.9 / 13.8
+  //     20000   16.8 / 20.4    15.2 / 17.9    15.1 / 19.2
+  //     24576   19.7 / 25.5    18.4 / 23.9    17.5 / 22.2
+  //     32768   23.1 / 31.4    20.6 / 28.7    19.3 / 27.5
+  const int lanes = num <= 8192 ? 16 : num <= 20480 ? 8 : 1;
   return ranges::sort<typename Src::key_type, false>(
       Src{draw, {}}, num, DrawEmit<Draw, Emit>{draw, emit, lanes}, st);
 }

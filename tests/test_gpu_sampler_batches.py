@@ -92,7 +92,7 @@ def test_batches_ascend_whatever_the_total_is(num, total):
         assert np.array_equal(got, np.sort(found))
 
 
-@pytest.mark.parametrize("num", [4096, 4097, 12_288, 12_289, 24_576, 24_577, 32_768, 32_769])
+@pytest.mark.parametrize("num", [4096, 4097, 8192, 8193, 20_480, 20_481, 32_768, 32_769])
 def test_batches_ascend_in_a_prefix_with_dips(num):
     """A prefix of rounded sums can dip by a unit in the last place behind zero priorities."""
     from gear_amd import ops
