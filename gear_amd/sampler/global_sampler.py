@@ -63,8 +63,8 @@ class UniformSampler:
     def select(self, indices, weights, draws, dirty_from=None):
         return self._take_sorted(indices, draws)
 
-    # For a loader that hands the rest of its step to ONE library call
-    # (CpuTrajectoryStorageHandler.select_subcopy): what is left of select() before the sort and
+    # For a loader that hands the rest of its step to ONE call (its native step, or
+    # CpuTrajectoryStorageHandler.select_subcopy): what is left of select() before the sort and
     # the look-ups, as (kind, positions-or-draws, prefix-or-None).  Only valid where
     # indices_ascending holds.
     def prepare(self, indices, weights, draws, dirty_from=None):

@@ -124,6 +124,31 @@ def test_two_threads_in_one_loader():
     assert not errors
 
 
+@pytest.mark.parametrize("method", ["Uniform", "Weighted", "TopK"])
+@pytest.mark.parametrize("placement", ["pinned", "device"])
+def test_the_handlers_step_is_the_loaders(method, placement):
+    """CpuTrajectoryStorageHandler.select_subcopy into a caller's tensors gives what the loader's step
+    gives in fresh ones."""
+    loader = _loader(placement, {"Uniform": 10, "Weighted": 11, "TopK": 12}[method] + 3 * (placement == "device"),
+                     batch=24, method=method, with_mask=True)
+    loader._device_weights.copy_(torch.rand(CAP, device="cuda") + 0.1)
+    announce("handler.select_subcopy %s %s" % (method, placement))
+    kind, picks, prefix = loader._sampler.prepare(
+        loader._indices, loader._device_weights, loader._sampler.draw(CAP, 24), dirty_from=None)
+    want = loader._step.run(kind, picks, prefix, loader._indices, loader._iset.index_offset,
+                            loader._device_timesteps, False, _ops()._ws)
+    dst = torch.full((24, T, WIDTH), -1.0, device="cuda")
+    mask = torch.full((24, T), 9, dtype=torch.uint8, device="cuda")
+    looked = torch.full((3, 24), -1, dtype=torch.int64, device="cuda")
+    loader._handler.select_subcopy(kind, picks, prefix, loader._indices, loader._iset.index_offset,
+                                   loader._device_timesteps, loader._sub_cols, [dst], True, [mask],
+                                   looked[0], looked[1], looked[2])
+    assert torch.equal(looked[0], want[0]) and torch.equal(looked[2], want[1])
+    assert torch.equal(looked[1], want[0] - loader._iset.index_offset)
+    assert torch.equal(dst, want[2][0]) and torch.equal(mask, want[3][0])
+    _check(type("L", (), {"last_sampled": want[0]}), want[1], want[2])
+
+
 def test_more_columns_than_one_launch_gathers():
     """A loader of 17 columns can be made; the fused step refuses it, the step column by column does not."""
     from gear_amd.dataset import SharedDataset
