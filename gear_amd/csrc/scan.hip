@@ -18,8 +18,8 @@
 //  * two launches, up to 16384 ranges (n <= 134 M fp32): range_sum_kernel writes the sum of every
 //    range; scan_ranges_kernel<kTwoLaunches> re-reads its range (now in L2 / MALL), adds the
 //    sums of all earlier ranges and writes the prefix.  No workgroup waits for another one.  Used
-//    for long inputs, under stream capture (a captured launch would replay its tag) and for the
-//    incremental rescan of a suffix.
+//    under stream capture (a captured launch would replay its tag) and for the incremental rescan of
+//    a suffix of up to 33.5 M elements.
 //  * beyond that: three launches -- range_sum_kernel, range_prefix_kernel (ONE workgroup scans the
 //    range sums in a fixed order) and scan_ranges_kernel<kPrefixed>, which finds the sum of all
 //    earlier ranges in one word.  Same bits on every run, and for the rescan of a suffix.

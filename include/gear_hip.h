@@ -277,8 +277,8 @@ int gear_hip_upper_bound_f64(const double *prefix, int64_t n, const float *u, in
  * reference returns, torch.sort(...).values, gear/sampler/global_sampler.py:131,172,195-199 --
  * and, when trajectory_length > 0, split like gear_hip_split_step_index into idxs/tss/lens
  * (lens may be NULL).  sorted_out may be NULL when trajectory_length > 0.
- * Up to 4096 draws take two launches (search over many workgroups, then the ranking sort,
- * which also splits); larger batches use the multi-pass radix sort.
+ * Up to 32768 draws take one launch (search, order and split); larger batches, and outputs that lie on
+ * top of the draws or the prefix, a search, a sort and a split of their own.
  * workspace: gear_hip_sample_workspace_bytes(num) bytes on the device. */
 size_t gear_hip_sample_workspace_bytes(int64_t num);
 int gear_hip_sample_sorted_f64(const double *prefix, int64_t n, const float *u, int64_t num,
@@ -297,7 +297,8 @@ int gear_hip_sample_sorted_f64(const double *prefix, int64_t n, const float *u, 
  * torch.sort(concat_indices[draws]) (gear/sampler/global_sampler.py:131,172,196),
  * indices - index_offset and iset.timesteps[indices.cpu()] on the host
  * (gear/loader/offline_loader.py:161-177): up to 32768 positions or draws take ONE launch (search,
- * order and look-ups), more take the radix sort and an element-wise launch.
+ * order and look-ups), more take the radix sort and an element-wise launch; so do many among a few
+ * entries, and outputs that lie on top of the draws, the prefix or the positions.
  *   gear_hip_sample_lookup_f64  positions = upper_bound of the draws u in the fp64 prefix, as
  *                               gear_hip_upper_bound_f64 (index_table, when given, has n entries)
  *   gear_hip_sample_lookup_i64  the same in an int64 prefix (a sampler over lengths), u as for
