@@ -18,7 +18,8 @@
 // A batch of a few keys, each many times over, takes longer, for the passes that find its runs: 19.6 /
 // 21.9 for 20000 keys of two values, 26.3 / 22.4 for 32768 of them, 38.5 / 59.8 where they are 63 bits
 // wide, 37.0 / 59.4 for 5000 values and one far away.
-// At 40 000 keys of 20 bits the two meet (64 registers of keys a thread spill: 64 us).
+// At 40 000 keys of 20 bits the two meet (64 registers of keys a thread spill: 64 us); for 63-bit keys the
+// registers are the limit: 32 rounds fill all 128 of them.
 #pragma once
 #include "radix_sort.hpp"
 
@@ -34,10 +35,14 @@ constexpr int kBins = 1 << kBinBits;
 constexpr int kPerThread = kBins / kThreads;
 static_assert(kPerThread == 4, "a thread's bins are one 16-byte word");
 constexpr int kBanks = 64;
-constexpr int kCopies = 8;             // of the counts, where many lanes count in the same bank
+// copies of the counts, where many lanes count in the same bank: 32768 keys of two values take 26.4 us,
+// 29.2 with four, 42.3 with one
+constexpr int kCopies = 8;
 constexpr int kCopy = kBins + 4;       // (in different banks)
 constexpr int kCap = 1024;             // keys ranked at once in LDS
-constexpr int kTol = 448;              // a cut may leave its place by so many keys
+// A cut may leave its place by so many keys: more are slow to rank, fewer take another pass (64 values,
+// 24576 keys / 32768 keys: 23.5 / 27.4 us; with 384 27.3 / 27.4, with 512 23.4 / 33.3).
+constexpr int kTol = 448;
 constexpr int kMax = 32 * kThreads;    // largest batch: the keys of a thread stay in registers
 static_assert(kMax / kGroups + kTol <= kCap, "a share without repeated keys fits in LDS");
 

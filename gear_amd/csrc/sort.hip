@@ -44,7 +44,7 @@ struct Emit {
   }
 };
 
-// Up to kRankMax keys the ranking sort is the faster one; outputs on top of inputs need launches
+// Up to kRankMax keys the ranking sort is the faster one, for a digit or two the radix sort; outputs on top of inputs need launches
 // that end reading before they write.
 bool one_launch(const int64_t *kin, int64_t *kout, const int64_t *vin, int64_t *vout, int64_t num,
                 int key_bits) {
@@ -71,7 +71,8 @@ extern "C" int gear_hip_sort_i64(const int64_t *keys_in, int64_t *keys_out, cons
   if (one_launch(keys_in, keys_out, vals_in, vals_out, num, key_bits)) {
     const uint64_t mask = key_bits >= 64 ? ~0ull : ((uint64_t)1 << key_bits) - 1;
     const Emit emit{keys_in, vals_in, keys_out, vals_out};
-    if (key_bits <= 32) return ranges::sort<uint32_t, true>(Src<uint32_t>{keys_in, mask}, num, emit, as_stream(stream));
+    if (key_bits <= 32)
+      return ranges::sort<uint32_t, true>(Src<uint32_t>{keys_in, mask}, num, emit, as_stream(stream));
     return ranges::sort<uint64_t, true>(Src<uint64_t>{keys_in, mask}, num, emit, as_stream(stream));
   }
   char *ws = static_cast<char *>(workspace);
