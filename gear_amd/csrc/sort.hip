@@ -44,8 +44,8 @@ struct Emit {
   }
 };
 
-// Up to kRankMax keys the ranking sort is the faster one, for a digit or two the radix sort; outputs on top of inputs need launches
-// that end reading before they write.
+// Up to kRankMax keys the ranking sort is the faster one, for a digit or two the radix sort; outputs
+// on top of inputs need launches that end reading before they write.
 bool one_launch(const int64_t *kin, int64_t *kout, const int64_t *vin, int64_t *vout, int64_t num,
                 int key_bits) {
   const int64_t b = num * 8;
