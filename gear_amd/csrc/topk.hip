@@ -1,7 +1,10 @@
 // Top-k of fp32 priorities by radix select + ordered compaction + segmented ordering, gfx950.
 //
+// With a sample, and unless bins are crowded (masses of equal priorities) or a list overflowed, a call is
+// prep, level 0, level 1 -- which writes the result (finish_selection) -- and a launch or two that find
+// nothing left to do.  Otherwise the steps are these:
 // fp32 priorities map to order-preserving uint32 keys, selected top-down in three levels: 16384
-// level-0 bins, then up to 11 and up to 10 bits inside the picked bin.  The launches of one call:
+// level-0 bins, then up to 11 and up to 10 bits inside the picked bin.  The steps of one call:
 //   prep      one workgroup draws 2048 to 32768 samples and lays out the level-0 bins around them (coarse
 //             below the bin that safely lies under the k-th largest priority -- the hint --, fine
 //             from there to the largest sample, the rest above); the others clear the histograms.
@@ -77,6 +80,7 @@ static_assert((1ll << 32 >> kLowShift) + kHintedBins <= kBins0, "every bin has a
 constexpr int kMaxSamplesPerThread = 32;
 constexpr uint32_t kNoLists = 0xffffffffu;   // hint_bin: level 0 writes no candidate lists
 constexpr uint32_t kListFull = 0xffffffffu;  // wave_listed: the wave's list overflowed, the wave reads its range instead
+constexpr int64_t kCoarseMaxK = 65536;       // index order with coarse bins up to this k
 constexpr int64_t kBucketMaxK = 131072;      // value order by buckets up to this k
 constexpr int kSortThreads = 1024;           // segment sort workgroup
 constexpr int kSmallGroup = 256;             // groups up to this size are ranked directly
@@ -186,7 +190,9 @@ struct State {
   uint64_t next_magic;
   uint32_t next_a_end, next_b_last;
   uint32_t low_seg;  // after a failed hint, value order: the segment of the entries below the hint
-  uint32_t pad[39];
+  uint32_t gave_up;  // level 0: a wave gave its list up, so there are no binned lists
+  uint32_t done;     // level 1 has written the result: nothing is left to do
+  uint32_t pad[37];
 };
 static_assert(sizeof(State) == 256, "State is the 256-byte header of the workspace");
 
@@ -244,9 +250,20 @@ Geom geom(int64_t n, int64_t k) {
   return g;
 }
 
+// The binned lists: a workgroup's candidates once more, in the order of their bins, and where every bin
+// starts in them (kStartPitch words of 16 bits a workgroup; see level0_hinted_kernel).
+constexpr int kQueueCap = 512;  // candidates per wave held in LDS by level 0; longer lists overflow
+constexpr int kStartPitch = kHintedBins + 8;
+static_assert(kWavesPerBlock * kQueueCap < 65536, "a place in a workgroup's binned list is a 16-bit word");
+__host__ __device__ __forceinline__ int binned_cap(int64_t list_cap) {
+  return (int)(list_cap < kQueueCap ? list_cap : kQueueCap) * kWavesPerBlock;
+}
+
+constexpr int kHandWords = 3 * kMaxBlocks;  // of struct Hand
+
 struct Layout {
-  size_t hist0, hist1, hist2, wg_bins, histf1, histf2, boff, wave_listed, wave_ge, block_ge, lists, cidx,
-      cand, cand2, cseg, ckey, skey, sidx, tkey, tidx, shist, zero_begin, zero_end, total;
+  size_t hist0, hist1, hist2, wg_bins, histf1, histf2, hand, boff, wave_listed, wave_ge, block_ge, lists, binned,
+      starts, cidx, cand, cand2, cseg, ckey, skey, sidx, tkey, tidx, shist, zero_begin, zero_end, total;
 };
 
 Layout layout(int64_t n, int64_t k) {
@@ -261,12 +278,15 @@ Layout layout(int64_t n, int64_t k) {
   l.wg_bins = o; o += 4 * kMaxBlocks * sizeof(uint32_t);
   l.histf1 = o; o += kBinsF * sizeof(uint32_t);  // after a failed hint: upper / lower 16 key bits
   l.histf2 = o; o += kBinsF * sizeof(uint32_t);
+  l.hand = o;   o += kHandWords * sizeof(uint32_t);
   l.zero_end = o;
   l.boff = o;   o += kBins0 * sizeof(uint32_t);
   l.wave_listed = o; o += (size_t)kMaxBlocks * kWavesPerBlock * sizeof(uint32_t);
   l.wave_ge = o;     o += (size_t)kMaxBlocks * kWavesPerBlock * sizeof(uint64_t);
   l.block_ge = o;    o += (size_t)kMaxBlocks * sizeof(uint64_t);
   l.lists = o;  o += align_up((size_t)(g.blocks * kWavesPerBlock * g.list_cap) * 8, 256);
+  l.binned = o; o += align_up((size_t)g.blocks * (size_t)binned_cap(g.list_cap) * 8, 256);
+  l.starts = o; o += align_up((size_t)g.blocks * kStartPitch * 2, 256);
   l.cidx = o;   o += align_up(kk * 4, 256);
   l.cand = l.cand2 = l.cseg = l.ckey = l.skey = l.sidx = l.tkey = l.tidx = l.shist = 0;
   if (k <= kBucketMaxK) {
@@ -302,7 +322,12 @@ Layout layout(int64_t n, int64_t k) {
 struct Pick {
   uint32_t bin, k_rem, found, total;
 };
-template <int BINS>
+// AGENT: a word that other workgroups of this launch have written
+template <bool AGENT>
+__device__ __forceinline__ uint32_t load_word(const uint32_t *p) {
+  return AGENT ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *p;
+}
+template <int BINS, bool AGENT = false>
 __device__ __forceinline__ Pick pick_bin(uint32_t k_rem, const uint32_t *hist, uint32_t *boff,
                                          uint32_t *wg_bins = nullptr, int seg_shift = 0,
                                          uint32_t rank2 = 0u, uint32_t *bin2 = nullptr) {
@@ -321,7 +346,7 @@ __device__ __forceinline__ Pick pick_bin(uint32_t k_rem, const uint32_t *hist, u
   if (boff && tid < kWave && r_begin + tid < BINS) cb0 = hist[BINS - 1 - (r_begin + tid)];
   uint32_t c[kPerThread];  // c[j] = count of bin BINS-1 - tid*kPerThread - j (top down)
   int tsum = 0;
-  if (kPerThread % 4 == 0) {
+  if (kPerThread % 4 == 0 && !AGENT) {
     // the thread's bins are one contiguous run: 16-byte loads, reversed into top-down order
 #pragma unroll
     for (int v = 0; v < kPerThread / 4; ++v) {
@@ -334,7 +359,7 @@ __device__ __forceinline__ Pick pick_bin(uint32_t k_rem, const uint32_t *hist, u
   } else {
 #pragma unroll
     for (int j = 0; j < kPerThread; ++j) {
-      c[j] = tid < kActive ? hist[BINS - 1 - tid * kPerThread - j] : 0u;
+      c[j] = tid < kActive ? load_word<AGENT>(hist + (BINS - 1 - tid * kPerThread - j)) : 0u;
       tsum += (int)c[j];
     }
   }
@@ -656,6 +681,8 @@ __global__ __launch_bounds__(kThreads) void prep_kernel(const float *__restrict_
   if (tid == 7) state->full = 0u;
   if (tid == 8) state->overflow = (rank == 0u && !list_all) ? 1u : 0u;
   if (tid == 9) state->next_magic = 0ull;  // level 1 of this call leaves the next hint, if any
+  if (tid == 10) state->gave_up = 0u;
+  if (tid == 11) state->done = 0u;
   BinMap map;
   map.uniform = 1u;
   map.a_end = map.b_last = map.nb0 = map.nc0 = map.b_shift = map.c_shift = 0u;
@@ -687,7 +714,6 @@ __global__ __launch_bounds__(kThreads) void prep_kernel(const float *__restrict_
 __device__ __forceinline__ void count_add(uint32_t *cnt, uint32_t d, bool valid);
 
 // ---- level 0: ONE read of the priorities --------------------------------------------------------------
-constexpr int kQueueCap = 512;  // candidates per wave held in LDS; longer lists overflow
 
 // With a hint.  The loop over the priorities is bound by the instructions a CU can issue, not
 // by memory, so an entry below the hint -- forty-nine in fifty -- costs ONE compare and nothing
@@ -715,12 +741,13 @@ __device__ __forceinline__ uint32_t lanes_before(uint64_t mask, uint32_t acc) {
 }
 
 __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
-    const float *__restrict__ p, int64_t n, const State *state, uint32_t *__restrict__ hist0,
+    const float *__restrict__ p, int64_t n, State *state, uint32_t *__restrict__ hist0,
     int64_t wave_len, uint32_t *__restrict__ wave_listed, uint64_t *__restrict__ lists,
-    int list_cap) {
+    int list_cap, uint64_t *__restrict__ binned, uint16_t *__restrict__ starts) {
   __shared__ __align__(16) uint32_t h[kHintedBins];  // the bins from the hint upwards
   __shared__ uint64_t queue[kWavesPerBlock][kQueueCap];
   __shared__ uint32_t s_touched[kHintedBins / kWave];  // runs of 64 bins that hold a count
+  __shared__ uint32_t s_wsum[kWavesPerBlock], s_gave_up;
   const int tid = threadIdx.x, lane = tid & 63;
   // (the same in every lane of a wave: said so, everything that follows from it -- the wave's
   // range, the number of its steps -- stays in scalar registers and branches on it are taken by
@@ -750,6 +777,7 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
   static_assert(kHintedBins == kThreads * 4, "one 16-byte store per thread clears the histogram");
   *reinterpret_cast<u32x4 *>(&h[tid * 4]) = u32x4{0u, 0u, 0u, 0u};
   if (tid < kHintedBins / kWave) s_touched[tid] = 0u;
+  if (tid == 0) s_gave_up = 0u;
   const BinMap map = state->map;
   const float lo_f = lower_bound_float(map.a_end);
   const uint32_t bin_base = map.nb0;  // candidates' bins are counted from here
@@ -836,6 +864,7 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
     // histogram, lanes that share a bin by one atomic (the range is read again: it is in the
     // caches, and the later launches read it again anyway).
     queued = 0;
+    if (lane == 0) s_gave_up = 1u;
     stream_range(p, begin, end, lane, [&](int64_t e0, const float q[4]) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -855,7 +884,7 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
     const uint32_t bin = counted_bin(bin_of(map, key), bin_base);
     atomicAdd(&h[bin], 1u);
     s_touched[bin / kWave] = 1u;
-    list[i] = ((uint64_t)key << 32) | (uint32_t)ent;
+    wq[i] = list[i] = ((uint64_t)key << 32) | (uint32_t)ent;
   }
   // a wave whose list overflowed says so: the later launches read its range of the priorities
   // again, its range only
@@ -874,6 +903,34 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
     const int run = wave + kWavesPerBlock * (__ffsll((unsigned long long)todo) - 1);
     const uint32_t c = h[run * kWave + lane];
     if (c != 0u) atomicAdd(&mine[run * kWave + lane], c);
+  }
+  // The candidates once more, in the order of their bins, with a table of where every bin starts:
+  // whoever needs the entries of a few bins finds them in one short piece of every workgroup's list,
+  // instead of walking all of them.
+  if (s_gave_up != 0u) {
+    if (tid == 0) state->gave_up = 1u;
+    return;
+  }
+  const u32x4 c4 = *reinterpret_cast<const u32x4 *>(&h[tid * 4]);
+  const uint32_t sum4 = (c4[0] + c4[1]) + (c4[2] + c4[3]);
+  const uint32_t inc = (uint32_t)wave_inclusive_sum((int)sum4);
+  if (lane == kWave - 1) s_wsum[wave] = inc;
+  __syncthreads();  // (and every count has been read)
+  u32x4 at4;
+  at4[0] = inc - sum4 + (uint32_t)wave_sum((int)(lane < wave ? s_wsum[lane & (kWavesPerBlock - 1)] : 0u));
+  at4[1] = at4[0] + c4[0];
+  at4[2] = at4[1] + c4[1];
+  at4[3] = at4[2] + c4[2];
+  *reinterpret_cast<u32x4 *>(&h[tid * 4]) = at4;  // cursors
+  uint16_t *my_starts = starts + (int64_t)blockIdx.x * kStartPitch;
+  *reinterpret_cast<u32x2 *>(my_starts + tid * 4) = u32x2{at4[0] | (at4[1] << 16), at4[2] | (at4[3] << 16)};
+  if (tid == kThreads - 1) my_starts[kHintedBins] = (uint16_t)(at4[3] + c4[3]);
+  __syncthreads();
+  uint64_t *mine_binned = binned + (int64_t)blockIdx.x * binned_cap(list_cap);
+  for (uint32_t i = (uint32_t)lane; i < queued; i += kWave) {
+    const uint64_t ent = wq[i];
+    const uint32_t bin = counted_bin(bin_of(map, (uint32_t)(ent >> 32)), bin_base);
+    mine_binned[atomicAdd(&h[bin], 1u)] = ent;
   }
 }
 
@@ -918,58 +975,90 @@ __global__ __launch_bounds__(kThreads) void level0_kernel(const float *__restric
 }
 
 // pick_bin for the level-0 histogram of a map with a hint (see Copies): the bins from the hint
-// upwards, at most kHintedBins, kept in several copies that are added up here into `sums` (LDS,
-// kHintedBins words).  Returns the picked bin under its number in the map; boff, wg_bins and
-// seg_shift as for pick_bin.  Every thread of the workgroup calls.
-__device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const uint32_t *hist, const BinMap &map,
+// upwards, at most kHintedBins, kept in several copies that are added up here.  The words of all copies
+// together are the same 16384 however many copies there are, so a caller asks for them before it knows the
+// map (load_copies) and a round trip to memory is saved.  Returns the picked bin under its number in the
+// map; boff, wg_bins and seg_shift as for pick_bin, not looked at when the launch finishes the selection
+// itself.  sums: LDS, kHintedBins words.  Every thread of the workgroup calls.
+// FINISH (see finish_selection): fin->can says on entry whether there are binned lists, and on return
+// whether the launch can finish: enough candidates, and no bin that it has to order holds too many.
+enum FinishOrder { kNoFinish, kFinishByIndex, kFinishByValue };
+struct Finish {
+  bool can;
+  uint32_t limit;         // most entries of a bin
+  uint32_t lo, hi;        // by value: this workgroup's places in the output
+  uint32_t at_lo, at_hi;  // ... the bins that start there, counted from the hint's
+  uint32_t base, end;     // ... and the places of their entries (base == end: none)
+};
+struct CopyWords {
+  u32x4 q[4];
+};
+__device__ __forceinline__ CopyWords load_copies(const uint32_t *hist) {
+  static_assert(kBins0 == kThreads * 16, "a thread loads sixteen words");
+  CopyWords w;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    w.q[j] = *reinterpret_cast<const u32x4 *>(hist + threadIdx.x * 4 + j * kHintedBins);
+  return w;
+}
+template <int FINISH>
+__device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &words, const BinMap &map,
                                             uint32_t rank2, uint32_t *bin2, uint32_t *sums,
-                                            uint32_t *boff, uint32_t *wg_bins, int seg_shift) {
-  constexpr int kPer = 4;  // bins per thread, top down: thread 0 owns the top four
+                                            uint32_t *boff, uint32_t *wg_bins, int seg_shift,
+                                            Finish *fin) {
+  constexpr int kPer = 4;  // bins per thread
   static_assert(kPer * kThreads == kHintedBins, "every bin of a copy has its thread");
   __shared__ uint32_t wsum[kWavesPerBlock];
   __shared__ Pick s_pick;
   __shared__ uint32_t s_bin2;
   __shared__ uint32_t s_base[kHintedBins / kWave];  // entries above every 64th bin from the top
+  __shared__ uint32_t s_big, s_at_lo, s_at_hi, s_begin, s_end;
   const Copies cp = copies_of(map);
   const int tid = threadIdx.x, lane = tid & 63;
-  // the copies are added up into `sums` (LDS, 4096 words): neighbouring threads take neighbouring
-  // bins, and a thread's loads of the copies of its bin are all under way together
-  for (uint32_t at = (uint32_t)tid; at < cp.used; at += kThreads) {
-    uint32_t v[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) v[r] = (uint32_t)r < cp.copies ? hist[(uint32_t)r * cp.pitch + at] : 0u;
-    sums[at] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  // thread t owns the bins 4t .. 4t + 3; of eight copies its words are those of every other one
+  u32x4 c = (words.q[0] + words.q[1]) + (words.q[2] + words.q[3]);
+  if (cp.copies == 8u) {
+    constexpr int kHalf = kThreads / 2;
+    if (tid >= kHalf) *reinterpret_cast<u32x4 *>(&sums[(tid - kHalf) * kPer]) = c;
+    __syncthreads();
+    if (tid < kHalf)
+      c += *reinterpret_cast<const u32x4 *>(&sums[tid * kPer]);
+    else
+      c = u32x4{0u, 0u, 0u, 0u};
+    __syncthreads();
   }
-  __syncthreads();
-  uint32_t c[kPer];
   uint32_t tsum = 0u;
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
-    const uint32_t from_top = (uint32_t)(tid * kPer + j);
-    c[j] = from_top < cp.used ? sums[cp.used - 1u - from_top] : 0u;
+    if ((uint32_t)(tid * kPer + j) >= cp.used) c[j] = 0u;
     tsum += c[j];
   }
-  const int inc = wave_inclusive_sum((int)tsum);
-  if (lane == 63) wsum[tid >> 6] = (uint32_t)inc;
+  if (boff) *reinterpret_cast<u32x4 *>(&sums[tid * kPer]) = c;
+  const uint32_t inc = (uint32_t)wave_inclusive_sum((int)tsum);
+  if (lane == 63) wsum[tid >> 6] = inc;
   if (tid == 0) {
     s_pick.bin = map.nb0;
     s_pick.k_rem = k_rem;
     s_pick.found = 0u;
     s_bin2 = 0u;
+    s_big = s_at_lo = s_begin = s_end = 0u;
+    s_at_hi = cp.used - 1u;
   }
   __syncthreads();
-  const uint32_t before =
-      (uint32_t)wave_sum((int)(lane < (tid >> 6) && lane < kWavesPerBlock ? wsum[lane] : 0u));
-  const uint32_t running0 = before + (uint32_t)inc - tsum;  // entries above the thread's bins
+  const uint32_t mine = lane < kWavesPerBlock ? wsum[lane] : 0u;
+  const uint32_t total = (uint32_t)wave_sum((int)mine);
+  const uint32_t below = (uint32_t)wave_sum((int)(lane < (tid >> 6) ? mine : 0u)) + inc - tsum;
+  const uint32_t running0 = total - below - tsum;  // entries above the thread's bins
   auto find = [&](uint32_t rank, uint32_t *bin_out, uint32_t *rem_out) {
     if (running0 < rank && running0 + tsum >= rank) {  // one thread
       uint32_t r = running0, pb = 0u, pk = 0u;
       bool found = false;
 #pragma unroll
-      for (int j = 0; j < kPer; ++j) {
+      for (int j = kPer - 1; j >= 0; --j) {
         const bool here = !found && r + c[j] >= rank;
-        pb = here ? map.nb0 + cp.used - 1u - (uint32_t)(tid * kPer + j) : pb;
+        pb = here ? map.nb0 + (uint32_t)(tid * kPer + j) : pb;
         pk = here ? rank - r : pk;
+        if (FINISH == kFinishByIndex && here && c[j] > fin->limit) s_big = 1u;
         found = found || here;
         r += c[j];
       }
@@ -980,11 +1069,42 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const uint32_t *hist
       }
     }
   };
+  if (FINISH == kFinishByValue || boff) {
+    // The bins that start in this workgroup's stretch lie between the one that holds the place before
+    // it (for the first stretch from the highest bin that holds any) and the one that holds its last
+    // place: one writer each.
+    const uint32_t lo = fin->lo, hi = fin->hi < k_rem ? fin->hi : k_rem;
+    uint32_t r = running0;
+#pragma unroll
+    for (int j = kPer - 1; j >= 0; --j) {
+      const uint32_t next = r + c[j], bin = (uint32_t)(tid * kPer + j);
+      if (FINISH == kFinishByValue) {
+        if (lo == 0u ? r == 0u && c[j] != 0u : r < lo && next >= lo) {
+          s_at_hi = lo == 0u ? bin : bin - 1u;
+          s_begin = lo == 0u ? 0u : next;
+        }
+        if (lo < hi && r < hi && next >= hi) {
+          s_at_lo = bin;
+          s_end = next;
+        }
+        if (r < k_rem && c[j] > fin->limit) s_big = 1u;
+      }
+      if (boff && bin < cp.used && (cp.used - 1u - bin) % kWave == 0u) s_base[(cp.used - 1u - bin) / kWave] = r;
+      r = next;
+    }
+  }
   find(k_rem, &s_pick.bin, &s_pick.k_rem);
   if (rank2 != 0u) find(rank2, &s_bin2, nullptr);
-  if (tid == kThreads - 1) s_pick.total = running0 + tsum;
-  if (boff && (tid * kPer) % kWave == 0) s_base[tid * kPer / kWave] = running0;
+  if (tid == 0) s_pick.total = total;
   __syncthreads();
+  if (FINISH != kNoFinish) {
+    fin->can = fin->can && s_pick.found != 0u && s_big == 0u;
+    fin->at_lo = s_at_lo;
+    fin->at_hi = s_at_hi;
+    fin->base = s_begin;
+    fin->end = s_end;
+    if (fin->can) boff = nullptr;
+  }
   // Where the bins at or above the picked one start in value order, and the segment table: as
   // in pick_bin (the workgroups of the launch share the bins in runs of 64, a bin per lane),
   // with the counts taken from the sums in LDS.
@@ -1026,7 +1146,14 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const uint32_t *hist
 
 // ---- when the hint fails: 65536-bin histograms over the entries below it -----------------------------
 // pick_bin for a histogram of 65536 bins in memory: every thread of the workgroup calls.
+// AGENT: other workgroups of this launch have counted in it (64 words a thread: the caches are told, instead
+// of every word being asked for past them).
+template <bool AGENT>
 __device__ __forceinline__ Pick pick_wide(uint32_t rank, const uint32_t *hist) {
+  if (AGENT) {
+    if (threadIdx.x < (unsigned)kWave) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    __syncthreads();
+  }
   constexpr int kPer = kBinsF / kThreads;  // 64 bins per thread, thread 0 the top ones
   __shared__ uint32_t wsum[kWavesPerBlock];
   __shared__ Pick s_pick;
@@ -1118,14 +1245,33 @@ __device__ __forceinline__ void wide_hist(const float *__restrict__ p, int64_t n
 __device__ __forceinline__ int bits_of(uint32_t span) { return span ? 32 - __builtin_clz(span) : 0; }
 __device__ __forceinline__ int level1_shift(int bits0) { return bits0 > 11 ? bits0 - 11 : 0; }
 
-template <int LEVEL>
-__global__ __launch_bounds__(kThreads) void member_hist_kernel(
-    const float *__restrict__ p, int64_t n, int64_t k, int mid_bins, State *state,
-    const uint32_t *hist_prev, uint32_t *__restrict__ hist_out, const uint32_t *histf_prev,
+//
+// FINISH, with a hint: when the binned lists are there and no bin holds too many entries, LEVEL 1 writes the
+// whole result itself (finish_selection) and the launches after it find that nothing is left to do.
+template <int FINISH>
+__device__ __forceinline__ void finish_selection(
+    const float *__restrict__ p, int64_t n, uint32_t k, const Finish &fin, const Pick &pick,
+    const BinMap &map, const uint16_t *__restrict__ starts, const uint64_t *__restrict__ binned,
+    int list_cap, const uint64_t *__restrict__ list, uint32_t listed, uint64_t ent_pre,
+    int64_t wave_len, uint32_t *lds, float *__restrict__ values_out, int64_t *__restrict__ indices_out);
+constexpr uint32_t kFinishCap = 4096;  // entries that a workgroup puts in order
+struct FinishIo {
+  const uint16_t *starts;
+  const uint64_t *binned;
+  float *values_out;
+  int64_t *indices_out;
+};
+
+// (block: the workgroup whose part this is; hp: LDS, kBinsF / 2 words, packed counters after a failed hint;
+// else h, below.  Returns level 2's pick.)
+template <int LEVEL, int FINISH>
+__device__ __forceinline__ Pick member_hist(
+    uint32_t block, uint32_t *hp, const float *__restrict__ p, int64_t n, int64_t k, int mid_bins,
+    State *state, const uint32_t *hist_prev, uint32_t *__restrict__ hist_out, const uint32_t *histf_prev,
     uint32_t *__restrict__ histf_out, uint32_t *boff, uint32_t *wg_bins, int seg_shift,
     int64_t wave_len, const uint32_t *__restrict__ wave_listed,
-    const uint64_t *__restrict__ lists, int list_cap) {
-  __shared__ uint32_t hp[kBinsF / 2];  // packed counters after a failed hint; else h, below
+    const uint64_t *__restrict__ lists, int list_cap, const FinishIo &io) {
+  static_assert(LEVEL == 1 || FINISH == kNoFinish, "level 1 finishes or nobody does");
   uint32_t *h = hp;
   static_assert(kBinsR + kHintedBins <= kBinsF / 2,
                 "the level's histogram and the sums of the level-0 copies fit the same LDS");
@@ -1133,28 +1279,40 @@ __global__ __launch_bounds__(kThreads) void member_hist_kernel(
   for (int i = tid; i < kBinsR; i += kThreads) h[i] = 0u;
   // the wave's list does not depend on the pick: its length and first stretch are asked for
   // before the histogram is walked (used only when the lists are in use)
-  const int64_t gw = (int64_t)blockIdx.x * kWavesPerBlock + wave;
+  const int64_t gw = (int64_t)block * kWavesPerBlock + wave;
   const uint64_t *list = lists + gw * list_cap;
   // (the same word in every lane: said so, the branches on it are taken by whole waves)
   const uint32_t m_raw = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_listed[gw]);
   const int m_pre = (int)m_raw;
   const uint64_t ent_pre = list[lane];
+  CopyWords words{};
+  if (FINISH != kNoFinish) words = load_copies(hist_prev);
   uint32_t lo, hi;  // the keys that are counted
   int shift;        // digit = (key - lo) >> shift
   bool full, fail;
+  Pick picked{};
   uint32_t a_end = 0u, upper16 = 0u;
   // what earlier launches left in the state is asked for before the histogram is walked, not
   // after it (a round trip to memory each time)
   if (LEVEL == 1) {
     const BinMap map = state->map;
     const uint32_t overflow = state->overflow, hint_bin = state->hint_bin;
-    const bool hinted = map.uniform == 0u && hint_bin != kNoLists;
+    const bool hinted = FINISH != kNoFinish || (map.uniform == 0u && hint_bin != kNoLists);
     // (the 2k-th largest key, where the histogram holds that many: the next call's hint)
     uint32_t bin2 = 0u;
+    Finish fin{};
+    if (FINISH != kNoFinish) {
+      const uint32_t share = ((uint32_t)k + gridDim.x - 1u) / gridDim.x;
+      fin.can = state->gave_up == 0u;
+      fin.limit = kFinishCap - (FINISH == kFinishByValue ? share : 0u);
+      fin.lo = block * share;
+      fin.hi = fin.lo + share;
+    }
     // (with a hint the histogram holds the bins from the hint upwards, in copies, which are added
     // up in the part of the LDS that only a failed hint uses, later)
-    const Pick r = hinted ? pick_copies((uint32_t)k, hist_prev, map, 2u * (uint32_t)k, &bin2,
-                                        hp + kBinsR, boff, wg_bins, seg_shift)
+    const Pick r = hinted ? pick_copies<FINISH>((uint32_t)k, FINISH != kNoFinish ? words : load_copies(hist_prev),
+                                                map, 2u * (uint32_t)k, &bin2, hp + kBinsR, boff, wg_bins,
+                                                seg_shift, &fin)
                           : pick_bin<kBins0>((uint32_t)k, hist_prev, boff, wg_bins, seg_shift);
     fail = hinted && r.found == 0u;
     lo = bin_lo_key(map, r.bin);
@@ -1162,7 +1320,7 @@ __global__ __launch_bounds__(kThreads) void member_hist_kernel(
     shift = level1_shift(bits_of(hi - lo));
     full = overflow != 0u || fail;
     a_end = map.a_end;
-    if (blockIdx.x == 0 && tid == 0) {
+    if (block == 0u && tid == 0) {
       state->prefix[0] = r.bin;
       state->k_rem[0] = fail ? (uint32_t)k - r.total : r.k_rem;
       state->full = full ? 1u : 0u;
@@ -1191,6 +1349,12 @@ __global__ __launch_bounds__(kThreads) void member_hist_kernel(
         atomicMax(&wg_bins[4 * w + 2], ~r.total);
         atomicMax(&wg_bins[4 * w + 3], (uint32_t)k);
       }
+      if (FINISH != kNoFinish && fin.can) state->done = 1u;
+    }
+    if (FINISH != kNoFinish && fin.can) {
+      finish_selection<FINISH>(p, n, (uint32_t)k, fin, r, map, io.starts, io.binned, list_cap, list, m_raw,
+                               ent_pre, wave_len, hp + kBinsR, io.values_out, io.indices_out);
+      return picked;
     }
   } else {
     const uint32_t lo0 = state->lo0, hi0 = state->hi0, full0 = state->full;
@@ -1201,7 +1365,7 @@ __global__ __launch_bounds__(kThreads) void member_hist_kernel(
     if (!fail) {
       r = pick_bin<kBinsR>(k_rem0, hist_prev, nullptr);
     } else {
-      r = pick_wide(k_rem0, histf_prev);
+      r = pick_wide<false>(k_rem0, histf_prev);
       upper16 = r.bin;
     }
     const int shift1 = level1_shift(bits_of(hi0 - lo0));
@@ -1210,10 +1374,11 @@ __global__ __launch_bounds__(kThreads) void member_hist_kernel(
     if (hi > hi0 || hi < lo) hi = hi0;
     shift = 0;
     full = full0 != 0u;
-    if (blockIdx.x == 0 && tid == 0) {
+    if (block == 0u && tid == 0) {
       state->prefix[1] = r.bin;
       state->k_rem[1] = r.k_rem;
     }
+    picked = r;
   }
   __syncthreads();
   if (fail) {
@@ -1231,7 +1396,7 @@ __global__ __launch_bounds__(kThreads) void member_hist_kernel(
         return q < lo_f && (key >> 16) == upper16;
       });
     }
-    return;
+    return picked;
   }
   // a wave whose list overflowed reads its own range again, the others walk their lists
   if (!full && m_raw != kListFull) {
@@ -1263,35 +1428,52 @@ __global__ __launch_bounds__(kThreads) void member_hist_kernel(
   __syncthreads();
   for (int i = tid; i < kBinsR; i += kThreads)
     if (h[i]) atomicAdd(&hist_out[i], h[i]);
+  return picked;
+}
+
+template <int LEVEL, int FINISH>
+__global__ __launch_bounds__(kThreads) void member_hist_kernel(
+    const float *__restrict__ p, int64_t n, int64_t k, int mid_bins, State *state,
+    const uint32_t *hist_prev, uint32_t *__restrict__ hist_out, const uint32_t *histf_prev,
+    uint32_t *__restrict__ histf_out, uint32_t *boff, uint32_t *wg_bins, int seg_shift,
+    int64_t wave_len, const uint32_t *__restrict__ wave_listed,
+    const uint64_t *__restrict__ lists, int list_cap, FinishIo io) {
+  __shared__ __align__(16) uint32_t hp[kBinsF / 2];
+  member_hist<LEVEL, FINISH>(blockIdx.x, hp, p, n, k, mid_bins, state, hist_prev, hist_out, histf_prev,
+                             histf_out, boff, wg_bins, seg_shift, wave_len, wave_listed, lists, list_cap, io);
 }
 
 // ---- count: threshold, then (greater, equal) per wave and workgroup ---------------------------------
 // Packed counts: greater << 32 | equal.  When the levels before streamed the priorities, this
 // launch does too and lists every wave's entries at or above the threshold on the way.
-__global__ __launch_bounds__(kThreads) void count_kernel(
-    const float *__restrict__ p, int64_t n, State *state, const uint32_t *hist2,
-    const uint32_t *histf2, int64_t wave_len, uint32_t *__restrict__ wave_listed, uint64_t *__restrict__ lists, int list_cap,
-    uint64_t *__restrict__ wave_ge, uint64_t *__restrict__ block_ge) {
+// AGENT: level 2 ran in this launch, pick1 is its pick and the counts are handed on inside it.  Returns the
+// threshold key as `bin`.
+template <bool AGENT>
+__device__ __forceinline__ Pick count_entries(
+    uint32_t block, const Pick &pick1, const float *__restrict__ p, int64_t n, State *state, const uint32_t *hist2,
+    const uint32_t *histf2, int64_t wave_len, uint32_t *__restrict__ wave_listed,
+    uint64_t *__restrict__ lists, int list_cap, uint64_t *__restrict__ wave_ge,
+    uint64_t *__restrict__ block_ge) {
   __shared__ uint64_t red[kWavesPerBlock];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t gw = (int64_t)blockIdx.x * kWavesPerBlock + wave;
+  const int64_t gw = (int64_t)block * kWavesPerBlock + wave;
   uint64_t *list = lists + gw * list_cap;
   // (the same word in every lane: said so, the branches on it are taken by whole waves)
   const uint32_t m_raw = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_listed[gw]);
   const int m_pre = (int)m_raw;
   const uint64_t ent_pre = list[lane];
-  const uint32_t lo0 = state->lo0, hi0 = state->hi0, digit1 = state->prefix[1];
+  const uint32_t lo0 = state->lo0, hi0 = state->hi0, digit1 = AGENT ? pick1.bin : state->prefix[1];
   const bool full = state->full != 0u || m_raw == kListFull;  // this wave reads its range
   const bool fail = state->fail != 0u;  // digit1: the upper 16 bits, histf2: the lower ones
-  const uint32_t k_rem1 = state->k_rem[1];
+  const uint32_t k_rem1 = AGENT ? pick1.k_rem : state->k_rem[1];
   Pick r;
   if (!fail)
-    r = pick_bin<kBinsR>(k_rem1, hist2, nullptr);
+    r = pick_bin<kBinsR, AGENT>(k_rem1, hist2, nullptr);
   else
-    r = pick_wide(k_rem1, histf2);
+    r = pick_wide<AGENT>(k_rem1, histf2);
   const uint32_t thr = fail ? ((digit1 << 16) | r.bin)
                             : lo0 + (digit1 << level1_shift(bits_of(hi0 - lo0))) + r.bin;
-  if (blockIdx.x == 0 && tid == 0) {
+  if (block == 0u && tid == 0) {
     state->prefix[2] = thr;
     state->k_rem[2] = r.k_rem;
   }
@@ -1338,8 +1520,21 @@ __global__ __launch_bounds__(kThreads) void count_kernel(
     uint64_t t = 0;
 #pragma unroll
     for (int i = 0; i < kWavesPerBlock; ++i) t += red[i];
-    block_ge[blockIdx.x] = t;
+    if (AGENT)
+      store_agent(&block_ge[block], t);
+    else
+      block_ge[block] = t;
   }
+  r.bin = thr;
+  return r;
+}
+__global__ __launch_bounds__(kThreads) void count_kernel(
+    const float *__restrict__ p, int64_t n, State *state, const uint32_t *hist2,
+    const uint32_t *histf2, int64_t wave_len, uint32_t *__restrict__ wave_listed,
+    uint64_t *__restrict__ lists, int list_cap, uint64_t *__restrict__ wave_ge,
+    uint64_t *__restrict__ block_ge) {
+  count_entries<false>(blockIdx.x, Pick{}, p, n, state, hist2, histf2, wave_len, wave_listed, lists, list_cap, wave_ge,
+                block_ge);
 }
 
 // ---- write: ordered compaction -----------------------------------------------------------------------
@@ -1349,9 +1544,10 @@ enum Flavour {
   kBucket   // (key, index) in index order for the bucket sort; ties at T go straight to the output's tail
 };
 
-template <int FLAVOUR>
-__global__ __launch_bounds__(kThreads) void write_kernel(
-    const float *__restrict__ p, int64_t n, int64_t k, const State *state, int64_t wave_len,
+// (AGENT: as for count_entries; pick2 is what that returned)
+template <int FLAVOUR, bool AGENT>
+__device__ __forceinline__ void write_entries(
+    uint32_t block, const Pick &pick2, const float *__restrict__ p, int64_t n, int64_t k, const State *state, int64_t wave_len,
     const uint32_t *__restrict__ wave_listed, const uint64_t *__restrict__ lists, int list_cap,
     const uint64_t *__restrict__ wave_ge, const uint64_t *__restrict__ block_ge,
     uint32_t *__restrict__ ckey, uint32_t *__restrict__ cidx, const uint32_t *__restrict__ boff,
@@ -1359,14 +1555,14 @@ __global__ __launch_bounds__(kThreads) void write_kernel(
     int64_t *__restrict__ indices_out) {
   __shared__ uint64_t red[kWavesPerBlock];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t gw = (int64_t)blockIdx.x * kWavesPerBlock + wave;
+  const int64_t gw = (int64_t)block * kWavesPerBlock + wave;
   const uint64_t *list = lists + gw * list_cap;
   // (the same word in every lane: said so, the branch on it is taken by whole waves)
   const uint32_t m_raw = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_listed[gw]);
   const int m_pre = (int)m_raw;
   const uint64_t ent_pre = list[lane];
-  const uint32_t thr = state->prefix[2];
-  const uint32_t need_eq = state->k_rem[2];
+  const uint32_t thr = AGENT ? pick2.bin : state->prefix[2];
+  const uint32_t need_eq = AGENT ? pick2.k_rem : state->k_rem[2];
   const bool reread = m_raw == kListFull;
   const BinMap map = state->map;
   const uint32_t low_seg = state->low_seg;
@@ -1375,7 +1571,7 @@ __global__ __launch_bounds__(kThreads) void write_kernel(
   // counts of the workgroups before this one (at most kMaxBlocks), then of the waves before
   // this one in its own workgroup
   uint64_t part = 0;
-  if (tid < (int)blockIdx.x) part = block_ge[tid];
+  if (tid < (int)block) part = AGENT ? load_agent(&block_ge[tid]) : block_ge[tid];
   const int64_t pw = wave_sum((int64_t)part);
   if (lane == 0) red[wave] = (uint64_t)pw;
   __syncthreads();
@@ -1383,7 +1579,7 @@ __global__ __launch_bounds__(kThreads) void write_kernel(
 #pragma unroll
   for (int i = 0; i < kWavesPerBlock; ++i) excl += red[i];
   uint64_t own = 0;
-  if (lane < wave) own = wave_ge[(int64_t)blockIdx.x * kWavesPerBlock + lane];
+  if (lane < wave) own = wave_ge[(int64_t)block * kWavesPerBlock + lane];
   excl += (uint64_t)wave_sum((int64_t)own);
   uint32_t gt_run = (uint32_t)(excl >> 32), eq_run = (uint32_t)excl;
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -1468,6 +1664,17 @@ __global__ __launch_bounds__(kThreads) void write_kernel(
     gt_run += (uint32_t)__popcll(bg);
     eq_run += (uint32_t)__popcll(be);
   });
+}
+template <int FLAVOUR>
+__global__ __launch_bounds__(kThreads) void write_kernel(
+    const float *__restrict__ p, int64_t n, int64_t k, const State *state, int64_t wave_len,
+    const uint32_t *__restrict__ wave_listed, const uint64_t *__restrict__ lists, int list_cap,
+    const uint64_t *__restrict__ wave_ge, const uint64_t *__restrict__ block_ge,
+    uint32_t *__restrict__ ckey, uint32_t *__restrict__ cidx, const uint32_t *__restrict__ boff,
+    int seg_shift, uint8_t *__restrict__ cseg, float *__restrict__ values_out,
+    int64_t *__restrict__ indices_out) {
+  write_entries<FLAVOUR, false>(blockIdx.x, Pick{}, p, n, k, state, wave_len, wave_listed, lists, list_cap, wave_ge, block_ge,
+                         ckey, cidx, boff, seg_shift, cseg, values_out, indices_out);
 }
 
 // ---- value order: segments gathered and sorted --------------------------------------------------------
@@ -1626,8 +1833,9 @@ __device__ __forceinline__ int differing_bits(const uint64_t *src, uint32_t off,
 // second buffer and hands them to fin(place, entry); called by every thread of the workgroup.  The two
 // callers pass either the LDS buffers or global ones, so that after inlining every access has a
 // known address space.
+template <typename Out>
 __device__ __forceinline__ void sort_segment(uint64_t *a, uint64_t *b, uint32_t m, int bits,
-                                             const SegmentOut &fin, SortShared &sh) {
+                                             const Out &fin, SortShared &sh) {
   const int tid = threadIdx.x;
   if (tid == 0) {
     sh.stk_off[0] = 0u;
@@ -2063,12 +2271,12 @@ __device__ __forceinline__ bool store_equal_segment(uint32_t seg_id, uint32_t m,
   return true;
 }
 
-__global__ __launch_bounds__(kSortThreads) void segment_sort_kernel(
-    const float *__restrict__ p, int64_t n, int64_t k, const State *state,
-    const uint32_t *__restrict__ seg_table, const uint32_t *__restrict__ ckey,
+// (for kMaxBlocks workgroups, of which this is number `block`; lds_a and lds_b: LDS, kLdsEntries each)
+__device__ __forceinline__ void sort_segments(
+    uint32_t block, uint64_t *lds_a, uint64_t *lds_b, const float *__restrict__ p, int64_t n, int64_t k,
+    const State *state, const uint32_t *__restrict__ seg_table, const uint32_t *__restrict__ ckey,
     const uint32_t *__restrict__ cidx, const uint8_t *__restrict__ cseg, uint64_t *buf0,
     uint64_t *buf1, float *__restrict__ values_out, int64_t *__restrict__ indices_out) {
-  __shared__ uint64_t lds_a[kLdsEntries], lds_b[kLdsEntries];
   __shared__ uint32_t s_cur;
   __shared__ SortShared sh;
   __shared__ BigShared bg;
@@ -2076,7 +2284,7 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_kernel(
   // The segment ids of the selected entries (a byte each; every workgroup reads them all) do
   // not depend on what this workgroup owns: their loads go out first, sixteen ids per load.
   const uint32_t kk = (uint32_t)k;
-  const uint32_t pattern = blockIdx.x * 0x01010101u;
+  const uint32_t pattern = block * 0x01010101u;
   constexpr int kLoads = 8;  // covers kBucketMaxK ids
   static_assert((int64_t)kLoads * kSortThreads * 16 >= kBucketMaxK, "one batch of loads reads every id");
   u32x4 q[kLoads];
@@ -2088,7 +2296,7 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_kernel(
   }
   // this workgroup's segment: its bins (highest + 1, kBins0 - lowest; 0 = none) and its stretch
   // of the output, one load; the entries equal to the threshold are not part of any segment
-  u32x4 mine4 = *reinterpret_cast<const u32x4 *>(seg_table + 4 * blockIdx.x);
+  u32x4 mine4 = *reinterpret_cast<const u32x4 *>(seg_table + 4 * block);
   const uint32_t need_eq = state->k_rem[2];
   const BinMap map = state->map;
   if (tid == 0) s_cur = 0u;
@@ -2100,7 +2308,7 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_kernel(
   };
   uint32_t out_lo;
   uint32_t m = stretch(mine4, &out_lo);
-  uint32_t seg_id = blockIdx.x, slot = 0u, parts = 1u;
+  uint32_t seg_id = block, slot = 0u, parts = 1u;
   // The workgroups that own no segment, and the owners of segments that exceed LDS, look at the
   // whole table: which segments are long, which workgroups idle.  The idle ones are dealt out to
   // the long segments (see store_equal_segment).  (The others have no use for it: a barrier and a
@@ -2111,7 +2319,7 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_kernel(
     if (tid < kMaxBlocks) {
       const u32x4 e = *reinterpret_cast<const u32x4 *>(seg_table + 4 * tid);
       uint32_t lo;
-      const uint32_t mt = tid < (int)gridDim.x ? stretch(e, &lo) : 0u;
+      const uint32_t mt = tid < kMaxBlocks ? stretch(e, &lo) : 0u;
       const uint64_t lm = wave_ballot(mt > (uint32_t)kLdsEntries), im = wave_ballot(mt == 0u);
       if (lane == 0) {
         s_long[tid >> 6] = lm;
@@ -2125,8 +2333,8 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_kernel(
       const uint64_t lm = s_long[w], im = s_idle[w];
       nlong += (uint32_t)__popcll(lm);
       nidle += (uint32_t)__popcll(im);
-      if (w * kWave < (int)blockIdx.x) {
-        const int below = (int)blockIdx.x - w * kWave;
+      if (w * kWave < (int)block) {
+        const int below = (int)block - w * kWave;
         const uint64_t mask = below >= kWave ? ~0ull : ((1ull << below) - 1ull);
         long_before += (uint32_t)__popcll(lm & mask);
         idle_before += (uint32_t)__popcll(im & mask);
@@ -2258,7 +2466,7 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_kernel(
     constexpr int kWaves = kSortThreads / kWave;
     __shared__ uint32_t s_wcnt[kWaves];
     const int wave = tid >> 6;
-    const uint8_t seg = (uint8_t)blockIdx.x;
+    const uint8_t seg = (uint8_t)block;
     const uint32_t per_wave = (kk + kWaves * kWave - 1) / (kWaves * kWave) * kWave;
     const uint32_t w_begin = (uint32_t)wave * per_wave < kk ? (uint32_t)wave * per_wave : kk;
     const uint32_t w_end = w_begin + per_wave < kk ? w_begin + per_wave : kk;
@@ -2327,7 +2535,306 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_kernel(
     sort_big_segment(buf0 + out_lo, buf1 + out_lo, m, big_bits < bits ? big_bits : bits, out, sh, bg,
                      lds_a, lds_b);
 }
+__global__ __launch_bounds__(kSortThreads) void segment_sort_kernel(
+    const float *__restrict__ p, int64_t n, int64_t k, const State *state,
+    const uint32_t *__restrict__ seg_table, const uint32_t *__restrict__ ckey,
+    const uint32_t *__restrict__ cidx, const uint8_t *__restrict__ cseg, uint64_t *buf0,
+    uint64_t *buf1, float *__restrict__ values_out, int64_t *__restrict__ indices_out) {
+  __shared__ uint64_t lds_a[kLdsEntries], lds_b[kLdsEntries];
+  if (state->done != 0u) return;
+  sort_segments(blockIdx.x, lds_a, lds_b, p, n, k, state, seg_table, ckey, cidx, cseg, buf0, buf1, values_out,
+                indices_out);
+}
 static_assert(kSortThreads >= kSortBins, "a thread per digit in the segment sort's scan");
+
+// ---- the selection finished by level 1 -----------------------------------------------------------------
+// The entries of a few bins are one short piece of every workgroup's binned list (the table of starts says
+// where), so a workgroup fetches them itself -- four lanes a list, two dependent loads -- and puts them in
+// order in LDS: no list is walked, and nothing passes between the workgroups.
+// us a call, back to back, as five to seven launches / finished by level 1 (lognormal priorities, cold):
+// 20000 of 3e6 by value 39.0 / 25.4, 65536 of 1e7 by value 49.5 / 33.2 and by index 32.8 / 31.4, 1000 of 3e5 by
+// index (with the look-up and the gather of a loader's step) 37.2 / 29.2.  What level 1 cannot finish takes 4
+// to 7 us longer than before, for the binned lists and the hand-overs: 60000 ties above the threshold 56 /
+// 63 by value, 36 / 43 by index; all priorities equal 104 / 111.
+// By value a workgroup takes the bins that start in its stretch of the output; the bin that holds the k-th
+// key is ordered whole and what lies beyond place k is not stored, so no threshold is needed.  By index
+// every workgroup takes the bin of the k-th key, finds the last entry of it that is selected, and from that
+// and the tables of starts how many selected entries lie before its own list, which it then writes in order.
+constexpr uint32_t kFinishSlots = 2 * kThreads;
+constexpr uint32_t kFinishSlot = 64;   // up to so many entries of a slot are ranked by counting, by a lane each
+
+struct FinishOut {
+  const float *p;
+  int64_t n;
+  float *values;
+  int64_t *indices;
+  uint32_t base, key_base, k;
+  __device__ __forceinline__ void operator()(uint32_t i, uint64_t ent) const {
+    const uint32_t index = ~(uint32_t)ent, key = (uint32_t)(ent >> 32) + key_base;
+    if (base + i >= k) return;
+    indices[base + i] = (int64_t)index;
+    if (values)
+      values[base + i] =
+          key != 0x80000000u ? key_to_float(key) : ((int64_t)index < n ? p[index] : 0.0f);
+  }
+};
+
+// fin(place, entry) for the m entries, larger ones first, which were counted in cnt (kFinishSlots words) by
+// slot_of(entry): a counting sort by slots, of which most hold an entry or none, and a rank inside the slot.
+// Both buffers hold kFinishCap.
+template <typename Slot, typename Out>
+__device__ __forceinline__ void order_entries(uint64_t *ents, uint64_t *other, uint32_t *cnt, uint32_t m,
+                                              int bits, const Slot &slot_of, const Out &fin, SortShared &sh) {
+  __shared__ uint32_t s_wsum[kWavesPerBlock];
+  const uint32_t tid = threadIdx.x;
+  const int lane = (int)tid & 63, wave = __builtin_amdgcn_readfirstlane((int)tid >> 6);
+  static_assert(kFinishSlots == 2 * kThreads, "two slots a thread");
+  const u32x2 c2 = reinterpret_cast<const u32x2 *>(cnt)[tid];
+  const uint32_t inc = (uint32_t)wave_inclusive_sum((int)(c2[0] + c2[1]));
+  if (lane == kWave - 1) s_wsum[wave] = inc;
+  const bool crowded = __syncthreads_or(c2[0] > kFinishSlot || c2[1] > kFinishSlot);
+  if (crowded) {
+    sort_segment(ents, other, m, bits, fin, sh);
+    return;
+  }
+  const uint32_t start = inc - c2[0] - c2[1] +
+                         (uint32_t)wave_sum((int)(lane < wave ? s_wsum[lane & (kWavesPerBlock - 1)] : 0u));
+  reinterpret_cast<u32x2 *>(cnt)[tid] = u32x2{start, start + c2[0]};
+  __syncthreads();
+  for (uint32_t i = tid; i < m; i += kThreads) other[atomicAdd(&cnt[slot_of(ents[i])], 1u)] = ents[i];
+  __syncthreads();
+  for (uint32_t i = tid; i < m; i += kThreads) {
+    const uint64_t own = other[i];
+    const uint32_t slot = slot_of(own), b = slot > 0u ? cnt[slot - 1u] : 0u;
+    fin(b + larger_in(other, b, cnt[slot], own), own);
+  }
+}
+
+template <int FINISH>
+__device__ __forceinline__ void finish_selection(
+    const float *__restrict__ p, int64_t n, uint32_t k, const Finish &fin, const Pick &pick,
+    const BinMap &map, const uint16_t *__restrict__ starts, const uint64_t *__restrict__ binned,
+    int list_cap, const uint64_t *__restrict__ list, uint32_t listed, uint64_t ent_pre,
+    int64_t wave_len, uint32_t *lds, float *__restrict__ values_out, int64_t *__restrict__ indices_out) {
+  __shared__ SortShared sh;
+  __shared__ uint32_t s_n, s_red[kWavesPerBlock], s_own[kWavesPerBlock];
+  __shared__ uint64_t s_last;  // by index: the last entry of the picked bin that is selected
+  static_assert(kBinsR + 4 * kFinishCap + kFinishSlots <= kBinsF / 2 && kBinsR % 2 == 0,
+                "the entries fit the LDS that only a failed hint uses");
+  uint64_t *ents = reinterpret_cast<uint64_t *>(lds), *other = ents + kFinishCap;
+  uint32_t *cnt = lds + 4 * kFinishCap;  // entries of a slot
+  constexpr bool kByValue = FINISH == kFinishByValue;
+  if (kByValue && fin.base >= fin.end) return;  // no bin starts in this workgroup's stretch
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  const uint32_t at_hi = kByValue ? fin.at_hi : pick.bin - map.nb0;
+  const uint32_t at_lo = kByValue ? fin.at_lo : at_hi;
+  const uint32_t lo_key = bin_lo_key(map, map.nb0 + at_lo), hi_key = bin_hi_key(map, map.nb0 + at_hi);
+  // the key range in kFinishSlots slots, the largest keys first (the last slot also takes what
+  // NaN samples put outside of it)
+  const int key_bits = bits_of(hi_key - lo_key);
+  const int slot_shift = key_bits > 11 ? key_bits - 11 : 0;
+  static_assert(kFinishSlots == 1u << 11, "eleven bits of slots");
+  auto slot_of = [&](uint64_t own) {
+    const uint32_t s = (hi_key - lo_key - (uint32_t)(own >> 32)) >> slot_shift;
+    return s < kFinishSlots ? s : kFinishSlots - 1u;
+  };
+  // four lanes per list
+  static_assert(kThreads == 4 * kMaxBlocks, "every list has its lanes");
+  const uint32_t src = (uint32_t)tid >> 2;
+  const bool real = src < gridDim.x;
+  const uint16_t *row = starts + (real ? src : 0u) * kStartPitch;
+  const uint64_t *from = binned + (int64_t)(real ? src : 0u) * binned_cap(list_cap);
+  uint32_t c = row[at_lo], end = row[at_hi + 1u];
+  const uint32_t all = kByValue ? 0u : row[kHintedBins];
+  if (tid == 0) {
+    s_n = 0u;
+    s_last = 0ull;
+  }
+  reinterpret_cast<u32x2 *>(cnt)[tid] = u32x2{0u, 0u};
+  __syncthreads();
+  if (!real) end = 0u;
+  uint32_t before = 0u;  // by index: this lane's share of the selected entries of earlier lists
+  if (!kByValue && (tid & 3) == 0 && src < blockIdx.x) before = all - end;
+  constexpr int kAtOnce = 2;
+  for (c += (uint32_t)tid & 3u; wave_ballot(c < end) != 0ull; c += 4u * kAtOnce) {
+    uint64_t e[kAtOnce];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) e[u] = from[c + 4u * u < end ? c + 4u * u : 0u];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) {
+      const bool hit = c + 4u * u < end;
+      const uint64_t hits = wave_ballot(hit);
+      if (hits == 0ull) break;
+      uint32_t slot = 0u;
+      if (lane == 0) slot = atomicAdd(&s_n, (uint32_t)__popcll(hits));
+      slot = (uint32_t)__builtin_amdgcn_readlane((int)slot, 0) + (uint32_t)__popcll(hits & lt_mask);
+      if (hit && slot < kFinishCap) {
+        const uint64_t own = ((e[u] >> 32) - lo_key) << 32 | (uint32_t)~(uint32_t)e[u];
+        ents[slot] = own;
+        atomicAdd(&cnt[slot_of(own)], 1u);
+      }
+    }
+  }
+  __syncthreads();
+  const uint32_t m = s_n < kFinishCap ? s_n : kFinishCap;
+  const int bits = 32 + key_bits;
+  if (kByValue) {
+    order_entries(ents, other, cnt, m, bits, slot_of,
+                  FinishOut{p, n, values_out, indices_out, fin.base, lo_key, k}, sh);
+    return;
+  }
+  const int64_t first_index = (int64_t)blockIdx.x * kWavesPerBlock * wave_len;
+  order_entries(
+      ents, other, cnt, m, bits, slot_of,
+      [&](uint32_t i, uint64_t ent) {
+        if (i + 1u == pick.k_rem) s_last = ent;
+        if (i < pick.k_rem && (int64_t)(uint32_t)~(uint32_t)ent < first_index) ++before;
+      },
+      sh);
+  const uint32_t wave_before = (uint32_t)wave_sum((int)before);
+  if (lane == 0) s_red[wave] = wave_before;
+  __syncthreads();
+  const uint64_t last = s_last;
+  auto selected = [&](uint64_t ent, bool valid) {
+    const uint32_t key = (uint32_t)(ent >> 32), at = counted_bin(bin_of(map, key), map.nb0);
+    const uint64_t own = ((uint64_t)(key - lo_key) << 32) | (uint32_t)~(uint32_t)ent;
+    return valid && (at > at_hi || (at == at_hi && own >= last));
+  };
+  uint32_t mine = 0u;
+  for (uint32_t c0 = 0; c0 < listed; c0 += kWave) {
+    const bool valid = c0 + lane < listed;
+    const uint64_t ent = valid ? (c0 == 0 ? ent_pre : list[c0 + lane]) : 0ull;
+    mine += (uint32_t)__popcll(wave_ballot(selected(ent, valid)));
+  }
+  if (lane == 0) s_own[wave] = mine;
+  __syncthreads();
+  uint32_t pos = (uint32_t)wave_sum(
+      (int)((lane < kWavesPerBlock ? s_red[lane & (kWavesPerBlock - 1)] : 0u) +
+            (lane < wave ? s_own[lane & (kWavesPerBlock - 1)] : 0u)));
+  for (uint32_t c0 = 0; c0 < listed; c0 += kWave) {
+    const bool valid = c0 + lane < listed;
+    const uint64_t ent = valid ? (c0 == 0 ? ent_pre : list[c0 + lane]) : 0ull;
+    const bool sel = selected(ent, valid);
+    const uint64_t b = wave_ballot(sel);
+    const uint32_t at = pos + (uint32_t)__popcll(b & lt_mask);
+    if (sel && at < k) {
+      const uint32_t index = (uint32_t)ent, key = (uint32_t)(ent >> 32);
+      indices_out[at] = (int64_t)index;
+      if (values_out)
+        values_out[at] = key != 0x80000000u ? key_to_float(key) : ((int64_t)index < n ? p[index] : 0.0f);
+    }
+    pos += (uint32_t)__popcll(b);
+  }
+}
+
+// ---- what is left when level 1 could not finish --------------------------------------------------------
+// Level 2, the count and the writing, each of which needs what all workgroups did before it, in ONE launch: a
+// launch that finds nothing to do costs 1.6 us on the GPU and 2.5 on the host, and four of them took a
+// third of an ordinary selection.  Each of the three is cut into one task for every workgroup of the
+// launches that it replaces.  A workgroup claims its own task, does it, waits until all tasks of the phase are
+// done -- it claims and does what nobody has claimed by then --, and goes on to the next phase of the tasks
+// that it claimed.  So it waits for claimed tasks only, which running workgroups are at, and a task waits for
+// nothing: every wait ends, however many of the workgroups the GPU holds at a time and whatever else it runs.
+// What passes between workgroups are counts in agent-scope words; lists and counts of a task stay with the
+// workgroup that claimed it.  (A release and an acquire of everything a workgroup wrote and may read take 4.5
+// us each with 31 workgroups at one L2, the hand-over without them 2.2: no more than another launch.)
+constexpr int kHandOvers = 2;  // level 2 -> count -> write
+struct Hand {
+  uint32_t claimed[kMaxBlocks], done[kHandOvers][kMaxBlocks];  // zeroed by prep
+};
+static_assert(sizeof(Hand) == kHandWords * sizeof(uint32_t), "as the workspace is laid out");
+
+// Says that this workgroup's tasks of a phase are done and waits for everybody's; with `steal` it looks for a
+// task that nobody has claimed when the wait gets long, and returns its number (kNone otherwise).  What the
+// tasks hand on are agent-scope accesses, complete once they are waited for.
+constexpr uint32_t kNone = 0xffffffffu;
+__device__ __forceinline__ uint32_t hand_over(const uint32_t *claimed, uint32_t *done, uint32_t tasks,
+                                              const uint8_t *mine, uint32_t from, uint32_t count, bool steal) {
+  __shared__ uint32_t s_free;
+  constexpr int kPolls = 64;
+  const uint32_t tid = threadIdx.x;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  for (uint32_t i = from + tid; i < count; i += kThreads)
+    __hip_atomic_store(&done[mine[i]], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (;;) {
+    if (tid == 0) s_free = kNone;
+    bool missing = tid < tasks;
+    for (int poll = 0; missing && poll < kPolls; ++poll) {
+      missing = load_word<true>(&done[tid]) == 0u;
+      if (missing) __builtin_amdgcn_s_sleep(1);
+    }
+    if (!__syncthreads_or(missing)) return kNone;
+    if (!steal) continue;
+    if (missing && load_word<true>(&claimed[tid]) == 0u) atomicMin(&s_free, tid);
+    __syncthreads();
+    const uint32_t free = s_free;
+    __syncthreads();
+    if (free != kNone) return free;
+  }
+}
+
+struct Rest {
+  const float *p;
+  int64_t n, k;
+  State *state;
+  Hand *hand;
+  uint32_t *hist1, *hist2, *histf1, *histf2;
+  int64_t wave_len;
+  uint32_t *wave_listed;
+  uint64_t *lists;
+  int list_cap;
+  uint64_t *wave_ge, *block_ge;
+  uint32_t *ckey, *cidx, *boff;
+  int seg_shift;
+  uint8_t *cseg;
+  float *values_out;
+  int64_t *indices_out;
+};
+template <bool BY_VALUE>
+__global__ __launch_bounds__(kThreads) void rest_kernel(Rest r) {
+  __shared__ __align__(16) uint32_t hp[kBinsF / 2];
+  __shared__ uint8_t mine[kMaxBlocks];
+  __shared__ uint32_t s_claimed;
+  static_assert(kMaxBlocks <= 256, "a task's number is a byte");
+  uint32_t taken = 1u;
+  if (threadIdx.x == 0) taken = atomicExch(&r.hand->claimed[blockIdx.x], 1u);  // (on its way meanwhile)
+  if (r.state->done != 0u) return;
+  Pick pick{};  // (the same whatever the task)
+  uint32_t count = 0u, told = 0u;
+  for (uint32_t next = blockIdx.x; next != kNone;) {
+    if (threadIdx.x == 0) {
+      s_claimed = taken == 0u ? 1u : 0u;
+      mine[count] = (uint8_t)next;
+    }
+    __syncthreads();
+    if (s_claimed != 0u) {
+      pick = member_hist<2, kNoFinish>(next, hp, r.p, r.n, r.k, 0, r.state, r.hist1, r.hist2, r.histf1, r.histf2,
+                                       nullptr, nullptr, 0, r.wave_len, r.wave_listed, r.lists, r.list_cap,
+                                       FinishIo{});
+      ++count;
+    }
+    next = hand_over(r.hand->claimed, r.hand->done[0], gridDim.x, mine, told, count, true);
+    told = count;
+    if (next != kNone && threadIdx.x == 0) taken = atomicExch(&r.hand->claimed[next], 1u);
+  }
+  if (count == 0u) return;  // others have this workgroup's task
+  Pick pick2{};
+  for (uint32_t i = 0; i < count; ++i) {
+    pick2 = count_entries<true>(mine[i], pick, r.p, r.n, r.state, r.hist2, r.histf2, r.wave_len, r.wave_listed,
+                                r.lists, r.list_cap, r.wave_ge, r.block_ge);
+    __syncthreads();
+  }
+  hand_over(r.hand->claimed, r.hand->done[1], gridDim.x, mine, 0u, count, false);
+  for (uint32_t i = 0; i < count; ++i) {
+    write_entries<BY_VALUE ? kBucket : kDirect, true>(
+        mine[i], pick2, r.p, r.n, r.k, r.state, r.wave_len, r.wave_listed, r.lists, r.list_cap, r.wave_ge, r.block_ge,
+        r.ckey, r.cidx, r.boff, r.seg_shift, r.cseg, r.values_out, r.indices_out);
+    __syncthreads();
+  }
+}
 
 // Final store of the value-ordered form for k > kBucketMaxK, fused into the last digit of the
 // candidate sort.
@@ -2377,6 +2884,8 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   uint64_t *wave_ge = reinterpret_cast<uint64_t *>(ws + l.wave_ge);
   uint64_t *block_ge = reinterpret_cast<uint64_t *>(ws + l.block_ge);
   uint64_t *lists = reinterpret_cast<uint64_t *>(ws + l.lists);
+  uint64_t *binned = reinterpret_cast<uint64_t *>(ws + l.binned);
+  uint16_t *starts = reinterpret_cast<uint16_t *>(ws + l.starts);
   uint32_t *cidx = reinterpret_cast<uint32_t *>(ws + l.cidx);
   hipStream_t st = as_stream(stream);
   const Geom g = geom(n, k);
@@ -2417,7 +2926,8 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   const dim3 block(kThreads), grid((unsigned)g.blocks);
   // Finer bins pay off in the value-order sort (small, even segments) but cost level 0 more
   // cache lines to add its counts to; the index-ordered selection takes coarse ones.
-  const int mid_bins = (sorted_by_value && k <= kBucketMaxK) ? kMidBins : kMidBinsCoarse;
+  // (Of a large selection a coarse bin would hold too many entries for level 1 to finish.)
+  const int mid_bins = (sorted_by_value ? k <= kBucketMaxK : k > kCoarseMaxK) ? kMidBins : kMidBinsCoarse;
   {
     uint32_t *zero = reinterpret_cast<uint32_t *>(ws + l.zero_begin);
     const dim3 pgrid(1 + zero_blocks);
@@ -2433,7 +2943,7 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   }
   if (rank != 0u)
     level0_hinted_kernel<<<grid, block, 0, st>>>(priorities, n, state, hist0, g.wave_len,
-                                                 wave_listed, lists, (int)g.list_cap);
+                                                 wave_listed, lists, (int)g.list_cap, binned, starts);
   else
     level0_kernel<<<grid, block, 0, st>>>(priorities, n, state, hist0, g.wave_len, wave_listed,
                                           lists, (int)g.list_cap);
@@ -2443,17 +2953,39 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   int seg_shift = 0;
   while ((k >> seg_shift) >= kNoSegment) ++seg_shift;  // segment ids stay below kNoSegment
   uint32_t *wg_bins = reinterpret_cast<uint32_t *>(ws + l.wg_bins);
-  member_hist_kernel<1><<<grid, block, 0, st>>>(priorities, n, k, mid_bins, state, hist0, hist1,
-                                                nullptr, histf1, by_segments ? boff : nullptr,
-                                                wg_bins, seg_shift, g.wave_len, wave_listed, lists,
-                                                (int)g.list_cap);
-  member_hist_kernel<2><<<grid, block, 0, st>>>(priorities, n, k, mid_bins, state, hist1, hist2,
-                                                histf1, histf2, nullptr, nullptr, 0, g.wave_len,
-                                                wave_listed, lists, (int)g.list_cap);
+  const FinishIo io{starts, binned, values_out, indices_out};
+  const auto level1 = [&](auto finish) {
+    member_hist_kernel<1, decltype(finish)::value><<<grid, block, 0, st>>>(
+        priorities, n, k, mid_bins, state, hist0, hist1, nullptr, histf1, by_segments ? boff : nullptr, wg_bins,
+        seg_shift, g.wave_len, wave_listed, lists, (int)g.list_cap, io);
+  };
+  uint8_t *cseg = reinterpret_cast<uint8_t *>(ws + l.cseg);
+  uint64_t *cand = reinterpret_cast<uint64_t *>(ws + l.cand);
+  uint64_t *cand2 = reinterpret_cast<uint64_t *>(ws + l.cand2);
+  uint32_t *ckey = reinterpret_cast<uint32_t *>(ws + l.ckey);
+  if (rank != 0u && (!sorted_by_value || (by_segments && ceil_div64(k, g.blocks) <= kFinishCap / 2))) {
+    const Rest rest{priorities, n, k, state, reinterpret_cast<Hand *>(ws + l.hand), hist1, hist2, histf1, histf2,
+                    g.wave_len, wave_listed, lists, (int)g.list_cap, wave_ge, block_ge, ckey, cidx, boff,
+                    seg_shift, cseg, values_out, indices_out};
+    if (sorted_by_value) {
+      level1(std::integral_constant<int, kFinishByValue>{});
+      rest_kernel<true><<<grid, block, 0, st>>>(rest);
+      segment_sort_kernel<<<dim3(kMaxBlocks), dim3(kSortThreads), 0, st>>>(
+          priorities, n, k, state, wg_bins, ckey, cidx, cseg, cand, cand2, values_out, indices_out);
+    } else {
+      level1(std::integral_constant<int, kFinishByIndex>{});
+      rest_kernel<false><<<grid, block, 0, st>>>(rest);
+    }
+    GEARHIP_RETURN_IF_LAUNCH_FAILED();
+    return 0;
+  }
+  level1(std::integral_constant<int, kNoFinish>{});
+  member_hist_kernel<2, kNoFinish><<<grid, block, 0, st>>>(
+      priorities, n, k, mid_bins, state, hist1, hist2, histf1, histf2, nullptr, nullptr, 0, g.wave_len,
+      wave_listed, lists, (int)g.list_cap, io);
   count_kernel<<<grid, block, 0, st>>>(priorities, n, state, hist2, histf2, g.wave_len,
                                        wave_listed, lists, (int)g.list_cap, wave_ge, block_ge);
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
-  uint8_t *cseg = reinterpret_cast<uint8_t *>(ws + l.cseg);
 #define GEARHIP_WRITE(F, CKEY)                                                                     \
   write_kernel<F><<<grid, block, 0, st>>>(priorities, n, k, state, g.wave_len, wave_listed, lists,  \
                                           (int)g.list_cap, wave_ge, block_ge, CKEY, cidx, boff,     \
@@ -2464,16 +2996,12 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
     return 0;
   }
   if (k <= kBucketMaxK) {
-    uint64_t *cand = reinterpret_cast<uint64_t *>(ws + l.cand);
-    uint64_t *cand2 = reinterpret_cast<uint64_t *>(ws + l.cand2);
-    uint32_t *bkey = reinterpret_cast<uint32_t *>(ws + l.ckey);
-    GEARHIP_WRITE(kBucket, bkey);
+    GEARHIP_WRITE(kBucket, ckey);
     segment_sort_kernel<<<dim3(kMaxBlocks), dim3(kSortThreads), 0, st>>>(
-        priorities, n, k, state, wg_bins, bkey, cidx, cseg, cand, cand2, values_out, indices_out);
+        priorities, n, k, state, wg_bins, ckey, cidx, cseg, cand, cand2, values_out, indices_out);
     GEARHIP_RETURN_IF_LAUNCH_FAILED();
     return 0;
   }
-  uint32_t *ckey = reinterpret_cast<uint32_t *>(ws + l.ckey);
   GEARHIP_WRITE(kPairs, ckey);
 #undef GEARHIP_WRITE
   GEARHIP_RETURN_IF_LAUNCH_FAILED();

@@ -1,0 +1,82 @@
+"""Top-k finished by its first level: a workgroup orders the few bins that concern it, fetched from every
+workgroup's binned list.  Edges: bins that hold nearly, exactly and more than a workgroup orders (4096, less its
+share of the output), a slot of equal keys, the zeros, the first and the last place; and what is left to the
+launch behind it, whose phases hand over inside it, with several of them on the GPU at once."""
+import numpy as np
+import pytest
+
+from conftest import announce
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def _values(n, seed):
+    return (np.random.default_rng(seed).lognormal(0, 1, size=n) ** 0.6).astype(np.float32)
+
+
+def _check(oracle, w, k, label):
+    from gear_amd import ops
+    dw = torch.from_numpy(w).cuda()
+    for by_value in (True, False):
+        announce("topk %s n=%d k=%d by_value=%d" % (label, len(w), k, by_value))
+        _, expected = oracle.topk_f32(w, k, by_value)
+        state = ops.TopKState()
+        for _ in range(2):  # from a sample, from the bound of the call before
+            values, index = state.select(dw, k, sorted_by_value=by_value)
+            torch.cuda.synchronize()
+            assert np.array_equal(index.cpu().numpy(), expected), (label, by_value)
+            assert np.array_equal(values.cpu().numpy().view(np.uint32), w[expected].view(np.uint32))
+        none, index = ops.topk(dw, k, sorted_by_value=by_value, want_values=False)
+        assert none is None and np.array_equal(index.cpu().numpy(), expected)
+
+
+@pytest.mark.parametrize("n,k", [(262_144, 1), (262_145, 64), (262_207, 32_768), (1_048_577, 131_072),
+                                 (1_500_001, 255), (1_500_001, 65_537), (5_000_011, 100_000)])
+def test_sizes(oracle, n, k):
+    _check(oracle, _values(n, n + k), k, "lognormal")
+
+
+@pytest.mark.parametrize("ties", [64, 65, 2_000, 3_800, 4_094, 4_097, 30_000])
+def test_equal_priorities_inside_the_selection(oracle, ties):
+    n, k = 600_001, 20_000
+    w = _values(n, ties)
+    at = np.random.default_rng(ties).permutation(n)[:ties]
+    order = np.sort(w)
+    for where, value in (("at the top", order[-1]), ("at the threshold", order[-k]),
+                         ("in the middle", order[-k // 2])):
+        v = w.copy()
+        v[at] = value
+        _check(oracle, v, k, "%d ties %s" % (ties, where))
+
+
+def test_zeros_and_infinities(oracle):
+    n, k = 400_003, 30_000
+    w = np.full(n, -1.0, np.float32) - _values(n, 5)
+    rng = np.random.default_rng(6)
+    at = rng.permutation(n)[:k + 500]
+    w[at] = rng.random(k + 500, dtype=np.float32)
+    w[at[:900]] = np.where(rng.random(900) < 0.5, np.float32(0.0), np.float32(-0.0))
+    w[at[900:1000]] = np.inf
+    _check(oracle, w, k, "both zeros around the threshold")
+
+
+def test_what_level_1_leaves_on_two_streams(oracle):
+    """Selections that level 1 cannot finish, of two streams at once: neither launch has the GPU to itself."""
+    from gear_amd import ops
+    n, k = 1_000_003, 50_000
+    w = np.random.default_rng(8).integers(0, 50, size=n).astype(np.float32)
+    dw = torch.from_numpy(w).cuda()
+    expected = [torch.from_numpy(oracle.topk_f32(w, k, bool(v))[1]).cuda() for v in (0, 1)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    announce("topk of ties on two streams")
+    torch.cuda.synchronize()
+    got = []
+    for turn in range(20):
+        for s, stream in enumerate(streams):
+            with torch.cuda.stream(stream):
+                by_value = (turn + s) % 2
+                got.append((by_value, ops.topk(dw, k, sorted_by_value=bool(by_value))[1]))
+    torch.cuda.synchronize()
+    for by_value, index in got:
+        assert torch.equal(index, expected[by_value])
