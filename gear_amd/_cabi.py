@@ -87,6 +87,9 @@ SIGNATURES = {
     "gear_hip_upper_bound_i64": (c_int, [c_void_p, c_i64, c_void_p, c_i64, c_int, c_void_p,
                                          c_void_p]),
     "gear_hip_sort_workspace_bytes": (c_size_t, [c_i64]),
+    "gear_hip_take_sorted_workspace_bytes": (c_size_t, [c_i64]),
+    "gear_hip_take_sorted_i64": (c_int, [c_void_p, c_i64, c_void_p, c_i64, c_void_p, c_void_p, c_size_t,
+                                         c_void_p]),
     "gear_hip_sort_i64": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_i64, c_int, c_void_p,
                                   c_size_t, c_void_p]),
     "gear_hip_topk_workspace_bytes": (c_size_t, [c_i64, c_i64]),

@@ -342,13 +342,28 @@ __device__ __forceinline__ uint32_t block_rank(RankSmem<C> &sm, int num, Load lo
 // Stable sort of bits [begin_bit, end_bit) of num <= kRankMax keys (and payloads): grid = num / 64
 // workgroups.  C is the compare type: uint32_t where end_bit - begin_bit <= 32.  A padding key
 // equal to the largest real key is harmless because it sits behind every real position.
+
+// Words of an earlier launch that say whether the keys are in order already, and where they have to go:
+// nothing is left to sort then.  No words: they are not known to be.
+struct InOrder {
+  const uint32_t *words = nullptr;
+  int count = 0;
+  __device__ __forceinline__ bool holds() const {
+    if (words == nullptr) return false;
+    bool out = false;
+    for (int i = threadIdx.x; i < count; i += blockDim.x) out = out || words[i] == 0u;
+    return !__syncthreads_or(out);
+  }
+};
+
 template <typename K, typename V, typename C, bool HAS_V>
 __global__ __launch_bounds__(kRankBlock) void rank_sort_kernel(const K *__restrict__ kin,
                                                                K *__restrict__ kout,
                                                                const V *__restrict__ vin,
                                                                V *__restrict__ vout, int num,
-                                                               int begin_bit, int end_bit) {
+                                                               int begin_bit, int end_bit, InOrder done) {
   __shared__ RankSmem<C> sm;
+  if (done.holds()) return;
   const int width = end_bit - begin_bit;
   const K mask = width >= (int)(8 * sizeof(K)) ? (K) ~(K)0 : (K)(((K)1 << width) - 1);
   C mine;
@@ -370,10 +385,11 @@ __global__ void copy_kernel(const T *__restrict__ in, T *__restrict__ out, int64
 // result lands in kout/vout; ktmp/vtmp are scratch of the same size; hist has hist_bytes(num).
 // vin == nullptr sorts keys only.  num < 2^32.
 // `fin` (see StoreSorted) replaces the stores of the last digit on the radix path; batches of at
-// most kRankMax keys take the ranking sort, which ignores it (the caller checks num).
+// most kRankMax keys take the ranking sort, which ignores it (the caller checks num) and alone looks at `done`.
 template <typename K, typename V, typename Final = StoreSorted>
 int sort_pairs(const K *kin, K *kout, const V *vin, V *vout, K *ktmp, V *vtmp, int64_t num,
-               int begin_bit, int end_bit, uint32_t *hist, hipStream_t st, Final fin = Final()) {
+               int begin_bit, int end_bit, uint32_t *hist, hipStream_t st, Final fin = Final(),
+               InOrder done = InOrder()) {
   if (num <= 0) return 0;
   if (num >= (1ll << 32)) return GEAR_HIP_ERANGE;
   const Plan p = plan(num);
@@ -383,7 +399,7 @@ int sort_pairs(const K *kin, K *kout, const V *vin, V *vout, K *ktmp, V *vtmp, i
     const dim3 grid((unsigned)ceil_div64(num, kWave)), block(kRankBlock);
     const bool narrow = end_bit - begin_bit <= 32;
 #define GEARHIP_RANK_SORT(C, HV) \
-  rank_sort_kernel<K, V, C, HV><<<grid, block, 0, st>>>(kin, kout, vin, vout, (int)num, begin_bit, end_bit)
+  rank_sort_kernel<K, V, C, HV><<<grid, block, 0, st>>>(kin, kout, vin, vout, (int)num, begin_bit, end_bit, done)
     if (narrow) {
       if (has_v) GEARHIP_RANK_SORT(uint32_t, true); else GEARHIP_RANK_SORT(uint32_t, false);
     } else {

@@ -21,6 +21,8 @@
 // At 40 000 keys of 20 bits the two meet (64 registers of keys a thread spill: 64 us); for 63-bit keys the
 // registers are the limit: 32 rounds fill all 128 of them.
 #pragma once
+#include <type_traits>
+
 #include "radix_sort.hpp"
 
 namespace gearhip {
@@ -349,9 +351,18 @@ __device__ __forceinline__ void emit_equal(Smem<C> &sm, const K &keys, C v, uint
 // collected elements at base + rank; equal(at, n, base) stores the elements at[0..n) of one key at
 // base, base + 1, ...  kLook: a batch that is in order already is passed on without a histogram
 // (Emit::put(place, j) stores element j).
+// Src::kGuarded: src.done() says, to all threads alike, that there is nothing to sort.
+template <typename Src, typename = void>
+struct Guarded : std::false_type {};
+template <typename Src>
+struct Guarded<Src, std::enable_if_t<Src::kGuarded>> : std::true_type {};
+
 template <typename C, int kRounds, bool kLook, typename Src, typename Emit>
 __global__ __launch_bounds__(kThreads) void range_sort_kernel(Src src, int num, Emit emit) {
   __shared__ Smem<C> sm;
+  if constexpr (Guarded<Src>::value) {
+    if (src.done()) return;
+  }
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int per = (num + kThreads - 1) / kThreads;

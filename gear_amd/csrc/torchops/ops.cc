@@ -365,6 +365,16 @@ py::object take_i64(py::handle table_, py::handle idx_, int64_t add, py::object 
   return out;
 }
 
+py::object take_sorted(py::handle table_, py::handle idx_, py::handle ws) {
+  const at::Tensor &table = need(table_, at::kLong, "table"), &idx = need(idx_, at::kLong, "idx");
+  const int64_t num = idx.numel();
+  py::object out = wrap(empty(num, at::kLong, idx.device()));
+  Scratch s(ws, "take_sorted", gear_hip_take_sorted_workspace_bytes(num), idx.device());
+  call("gear_hip_take_sorted_i64", s, gear_hip_take_sorted_i64, ptr<int64_t>(table), table.numel(),
+       ptr<int64_t>(idx), num, ptr<int64_t>(THPVariable_Unpack(out.ptr())), s.ptr, s.bytes, current_stream());
+  return out;
+}
+
 // ---- sort, top-k, updates --------------------------------------------------------------------------
 py::object sort_i64(py::handle keys_, py::handle vals_, int64_t key_bits, py::handle ws) {
   const at::Tensor &keys = need(keys_, at::kLong, "keys");
@@ -668,6 +678,7 @@ PYBIND11_MODULE(_hostops, m) {
   m.def("sort_lookup", &sort_lookup);
   m.def("lookup", &lookup);
   m.def("take_i64", &take_i64);
+  m.def("take_sorted", &take_sorted);
   m.def("sort_i64", &sort_i64);
   m.def("topk", &topk);
   m.def("scatter", &scatter);

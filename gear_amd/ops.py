@@ -238,6 +238,11 @@ def take_i64(table, idx, add=0, out=None):
     return _hostops.take_i64(table, idx, int(add), out)
 
 
+def take_sorted_i64(table, idx):
+    """sort(table[idx]) (int64, device), for entries that are mostly in order already."""
+    return _hostops.take_sorted(table, idx, _ws)
+
+
 def prefix_sum(priorities, out=None):
     """fp32[n] -> inclusive fp64 prefix[n] (gear_hip_scan_f32_f64)."""
     return _hostops.prefix_sum(priorities, out, _ws)

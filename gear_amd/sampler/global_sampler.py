@@ -46,11 +46,12 @@ class UniformSampler:
 
     def _take_sorted(self, indices, positions, positions_sorted=False):
         """sort(indices[positions]) on the device."""
+        if positions_sorted and not self.indices_ascending:
+            return ops.take_sorted_i64(indices, positions)  # in order if the indices are
         picked = ops.take_i64(indices, positions)
-        if positions_sorted and self.indices_ascending:
+        if positions_sorted:
             return picked
-        bits = 63
-        return ops.sort_i64(picked, key_bits=bits)
+        return ops.sort_i64(picked, key_bits=63)
 
     # Every sampler is split into draw() -- the random numbers, produced by torch -- and
     # select() -- everything after them, deterministic and free of host synchronisation, so a

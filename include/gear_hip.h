@@ -353,6 +353,15 @@ int gear_hip_sort_i64(const int64_t *keys_in, int64_t *keys_out, const int64_t *
                       int64_t *vals_out, int64_t num, int key_bits, void *workspace,
                       size_t workspace_bytes, void *stream);
 
+/* The entries table[idx[j]] (0 for an index outside [0, n)) in ascending order of their low 63 bits, stable: what
+ * gear_hip_take_i64 and gear_hip_sort_i64 give.  For entries that are in order already more often than not
+ * (ascending positions in a table that is usually ascending too): up to 32768 of them, the sort is a launch
+ * that finds nothing to do.  out must not alias the inputs.
+ * workspace: gear_hip_take_sorted_workspace_bytes(num) bytes on the device. */
+size_t gear_hip_take_sorted_workspace_bytes(int64_t num);
+int gear_hip_take_sorted_i64(const int64_t *table, int64_t n, const int64_t *idx, int64_t num, int64_t *out,
+                             void *workspace, size_t workspace_bytes, void *stream);
+
 /* Top-k of fp32 priorities, largest first; among equal priorities the smaller index wins
  * (i.e. the first k entries of a stable descending sort).  NaN is not a valid priority.
  * Replaces torch.topk(weights, k, largest=True) of TopKSampler
