@@ -4,10 +4,11 @@
 // granules of its range, adds them up in order, and one DPP wave scan per range joins the
 // threads (a wave-private LDS row turns the row-major order of the memory instructions, 1 KiB of
 // consecutive addresses per wave and instruction, into that blocked order and back):
-//  * chained single pass, up to 8192 ranges (of up to 16384 fp32 elements: 134 M):
+//  * chained single pass, up to 16384 ranges (of up to 16384 fp32 elements: 268 M):
 //    scan_ranges_kernel<kChained>.  A workgroup
 //    keeps its range in registers, publishes the range's sum and adds the sums of ALL earlier
-//    ranges (fixed order: bit-reproducible), then writes the prefix: the input is read once.
+//    ranges -- beyond 6656 ranges, of the earlier ones of its group of 64 and of all earlier groups --
+//    (fixed order: bit-reproducible), then writes the prefix: the input is read once.
 //    Range r belongs to workgroup r (no ticket).  A published sum travels as three 64-bit words
 //    that each carry 42 bits of the call's tag next to 21 or 22 bits of payload, so a word is valid
 //    on its own: no fence, no flag, nothing to clear before a call (a host counter hands every
@@ -15,11 +16,11 @@
 //    The wait for a predecessor is bounded: when it runs out, the workgroup sums that
 //    predecessor's range itself, with the same reduction tree, and publishes it on the
 //    predecessor's behalf, so no kernel can spin forever and the result does not change.
-//  * two launches, up to 16384 ranges (n <= 134 M fp32): range_sum_kernel writes the sum of every
-//    range; scan_ranges_kernel<kTwoLaunches> re-reads its range (now in L2 / MALL), adds the
-//    sums of all earlier ranges and writes the prefix.  No workgroup waits for another one.  Used
-//    under stream capture (a captured launch would replay its tag) and for the incremental rescan of
-//    a suffix of up to 33.5 M elements.
+//  * two launches, up to 16384 ranges: range_sum_kernel writes the sum of every range;
+//    scan_ranges_kernel<kTwoLaunches> re-reads its range (now in L2 / MALL), adds the same sums in the same
+//    order (those of whole groups come from a small launch in between) and writes the prefix.  No
+//    workgroup waits for another one.  Used under stream capture (a captured launch would replay its
+//    tag) and for the incremental rescan of a suffix of up to 33.5 M elements.
 //  * beyond that: three launches -- range_sum_kernel, range_prefix_kernel (ONE workgroup scans the
 //    range sums in a fixed order) and scan_ranges_kernel<kPrefixed>, which finds the sum of all
 //    earlier ranges in one word.  Same bits on every run, and for the rescan of a suffix.
@@ -63,10 +64,18 @@ __device__ __forceinline__ void store_vec(V *p, V v, bool nt) {
 // sum of ALL earlier ranges' sums (each thread adds its share of them, fixed summation order).
 // Nobody waits for an inclusive value, so there is no serial chain across the XCDs, and the result
 // is bit-reproducible from run to run.
-constexpr int kMaxRanges = 8192;      // chained: every thread polls up to 32 range sums
-constexpr int kMaxRanges8 = 4096;     // ... of ranges of 8 granules per thread
-static_assert(kMaxRanges / 32 <= kBlock, "a thread per word of the missing ranges");
-constexpr int kMaxRangesTwo = 16384;  // two launches: every thread adds up to 64 range sums
+constexpr int kMaxRanges8 = 4096;     // of ranges of 8 granules per thread
+// Up to kFlatRanges ranges a workgroup adds up the sums of all earlier ranges; of more, those of the
+// earlier ranges of its own group of 64 and those of the groups before it, which the last workgroup of a
+// group publishes.  At 8192 ranges the words of all earlier ranges were 0.8 GB beside 1.6 GB of data, and
+// more of them were not worth it.  A group's sum comes a hand-over later: us all earlier / by groups, fp32
+// 2e7 43 / 55, 3.3e7 83 / 100 (ranges of 8 granules, at most 4096), 6e7 147 / 146, 1e8 240 / 243, 1.3e8 324 / 309
+// (of 16: 3663, 6104 and 7935 ranges); int64 6e7 (7325) 241 / 210; where three launches took 649 (fp32, 2e8)
+// and 480 (int64, 1e8): 475 and 348.
+constexpr int kFlatRanges = 6656;
+constexpr int kGroup = 64;
+constexpr int kMaxRanges = kGroup * kBlock;  // a thread per group
+static_assert(kGroup == kWave, "a group's sum is a wave's");
 
 // A range sum in flight between workgroups of one launch: three self-validating words.
 constexpr int kTagBits = 42;
@@ -243,6 +252,28 @@ __global__ __launch_bounds__(kBlock) void range_sum_kernel(const In *__restrict_
   if (threadIdx.x == 0) sums[range] = Bits<Acc>::to(total);
 }
 
+// The words of more than kFlatRanges ranges behind the slots of the ranges: a slot a group and the plain sums
+// of the groups (kept between calls as those of the ranges are).
+struct Groups {
+  Slot *slots;
+  uint64_t *sums;
+};
+__host__ __device__ __forceinline__ Groups groups_of(Slot *range_slots, int64_t ranges) {
+  Slot *slots = range_slots + ranges;
+  return Groups{slots, reinterpret_cast<uint64_t *>(slots + ceil_div64(ranges, kGroup))};
+}
+
+// Sums of whole groups, a wave each: between the two launches of the variant that waits for nobody.
+template <typename Acc>
+__global__ __launch_bounds__(kBlock) void group_sum_kernel(const uint64_t *__restrict__ sums,
+                                                           uint64_t *__restrict__ group_sums, int64_t first_group,
+                                                           int64_t whole_groups) {
+  const int64_t g = first_group + (int64_t)blockIdx.x * (kBlock / kWave) + (threadIdx.x >> 6);
+  if (g >= whole_groups) return;
+  const Acc total = wave_sum(Bits<Acc>::from(sums[g * kGroup + (threadIdx.x & (kWave - 1))]));
+  if ((threadIdx.x & (kWave - 1)) == 0) group_sums[g] = Bits<Acc>::to(total);
+}
+
 // Exclusive prefix of the range sums by ONE workgroup, in an order that depends on nothing but
 // the number of ranges (thread t adds its stretch of the sums one after the other, the stretches'
 // totals are scanned, the stretch is walked again): the third launch between the two above for
@@ -280,24 +311,29 @@ enum RangeMode {
   kChained = 1,      // ... and the sums of this launch's ranges arrive while it runs
   kPrefixed = 2      // the sum of all earlier ranges is ready: slots holds one word per range
 };
-template <typename In, typename Acc, typename Out, int G, int MODE>
+//
+// GROUPED: more than kFlatRanges ranges (then `ranges` says how many).
+template <typename In, typename Acc, typename Out, int G, int MODE, bool GROUPED>
 __global__ __launch_bounds__(kBlock) void scan_ranges_kernel(const In *__restrict__ in,
                                                              Out *__restrict__ out, int64_t n,
                                                              uint64_t *__restrict__ sums,
                                                              Slot *__restrict__ slots,
                                                              int64_t first_range, uint64_t tag,
                                                              int spin_limit, int stagger,
-                                                             int first_wave) {
+                                                             int first_wave, int64_t ranges) {
   typedef Geo<In, Out, G> geo;
   typedef typename Gran<Out>::type out_gran;
   constexpr bool CHAINED = MODE == kChained;
   constexpr int kWaves = kBlock / kWave;
-  constexpr int kPolls = MODE == kPrefixed ? 0 : (CHAINED ? kMaxRanges : kMaxRangesTwo) / kBlock;
+  constexpr int kPolls = MODE == kPrefixed || GROUPED ? 0 : kFlatRanges / kBlock;
   constexpr int kBatch = 4;
+  constexpr int kMissing = GROUPED ? kGroup + kBlock : kFlatRanges;  // words that may be waited for
   __shared__ u32x4 stage_all[kWaves][geo::kStage];
   __shared__ Acc wtot[kWaves];
   __shared__ Acc red[kWaves];
-  __shared__ uint32_t s_missing[CHAINED ? kMaxRanges / 32 : 1];  // one bit per unpublished range
+  __shared__ uint32_t s_missing[CHAINED ? kMissing / 32 : 1];  // one bit per unpublished range or group
+  __shared__ Acc s_in_group;
+  static_assert(kMissing / 32 <= kBlock, "a thread per word of the missing ranges");
 
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
   const int64_t tile = first_range + (int64_t)blockIdx.x;
@@ -305,7 +341,7 @@ __global__ __launch_bounds__(kBlock) void scan_ranges_kernel(const In *__restric
   u32x4 *stage = stage_all[wave];
 
   if (CHAINED) {
-    if (tid < kMaxRanges / 32) s_missing[tid] = 0u;
+    if (tid < kMissing / 32) s_missing[tid] = 0u;
     // All workgroups that fit the GPU at once start within a microsecond.  Left alone, their loads
     // queue up together and come back in no particular order, every workgroup then waits for the
     // slowest load of ALL its predecessors, and the whole GPU first reads and then writes.  Starting
@@ -385,28 +421,91 @@ __global__ __launch_bounds__(kBlock) void scan_ranges_kernel(const In *__restric
         }
       }
     }
+    if constexpr (GROUPED) {
+      const int64_t group = tile / kGroup, group_begin = group * kGroup;
+      const int pos = (int)(tile - group_begin);
+      const Groups gs = groups_of(slots, ranges);
+      // a word that is plain or arrives while this launch runs
+      const auto fetch = [&](const uint64_t *plain, const Slot *slot, int64_t first_new, int64_t j, int bit) {
+        uint64_t v = 0ull;
+        if (!CHAINED || j < first_new) return Bits<Acc>::from(plain[j]);
+        bool have = try_read(&slot[j], tag, &v);
+        for (int spin = 0; !have && spin < spin_limit; ++spin) {
+          __builtin_amdgcn_s_sleep(1);
+          have = try_read(&slot[j], tag, &v);
+        }
+        if (!have) {
+          atomicOr(&s_missing[bit >> 5], 1u << (bit & 31));
+          miss = true;
+          return (Acc)0;
+        }
+        return Bits<Acc>::from(v);
+      };
+      if (wave == 0) {
+        Acc v = (Acc)0;
+        if (lane < pos) v = fetch(sums, slots, first_range, group_begin + lane, lane);
+        const Acc before = wave_sum(v);
+        if (lane == 0) s_in_group = before;
+        if (CHAINED && pos == kGroup - 1 && wave_ballot(miss) == 0ull) {
+          const Acc whole = wave_sum(lane == pos ? (w0 + w1) + (w2 + w3) : v);
+          if (lane == 0) {
+            publish(&gs.slots[group], tag, Bits<Acc>::to(whole));
+            gs.sums[group] = Bits<Acc>::to(whole);
+          }
+        }
+      }
+      if (tid < group) part = fetch(gs.sums, gs.slots, first_range / kGroup, tid, kGroup + tid);
+    }
     if (!CHAINED) break;
     if (!__syncthreads_or(miss)) {
       failed = false;
       break;
     }
-    for (int word = 0; word < kMaxRanges / 32; ++word) {
+    for (int word = 0; word < kMissing / 32; ++word) {
       uint32_t bits = s_missing[word];
       while (bits) {
-        const int j = word * 32 + (__ffs((int)bits) - 1);
+        int64_t j = word * 32 + (__ffs((int)bits) - 1);
         bits &= bits - 1u;
+        if (GROUPED && j >= kGroup) {
+          // a group: its ranges' sums, those that have not been published from the input
+          const int64_t g = j - kGroup;
+          Acc mine = (Acc)0;
+          for (int i = 0; i < kGroup; ++i) {
+            const int64_t range = g * kGroup + i;
+            uint64_t v = 0ull;
+            bool have = range < first_range;
+            if (have)
+              v = sums[range];
+            else
+              have = try_read(&slots[range], tag, &v);
+            Acc total = Bits<Acc>::from(v);
+            if (__syncthreads_or(!have)) {
+              total = range_total_direct<In, Acc, Out, G>(in, n, range, red);
+              if (tid == 0) publish(&slots[range], tag, Bits<Acc>::to(total));
+            }
+            if (lane == i) mine = total;
+          }
+          const Acc whole = wave_sum(mine);
+          if (tid == 0) {
+            publish(&groups_of(slots, ranges).slots[g], tag, Bits<Acc>::to(whole));
+            groups_of(slots, ranges).sums[g] = Bits<Acc>::to(whole);
+          }
+          continue;
+        }
+        if (GROUPED) j += tile / kGroup * kGroup;
         const Acc total = range_total_direct<In, Acc, Out, G>(in, n, j, red);
         if (tid == 0) publish(&slots[j], tag, Bits<Acc>::to(total));
       }
     }
     __syncthreads();
-    if (tid < kMaxRanges / 32) s_missing[tid] = 0u;
+    if (tid < kMissing / 32) s_missing[tid] = 0u;
     __syncthreads();
   }
   const Acc pw = wave_sum(part);
   if (lane == 0) red[wave] = pw;
   __syncthreads();
   Acc excl = (red[0] + red[1]) + (red[2] + red[3]);
+  if (GROUPED) excl += s_in_group;
   if (MODE == kPrefixed) excl = Bits<Acc>::from(reinterpret_cast<const uint64_t *>(slots)[tile]);
   // Three passes cannot fail (the second one reads what this workgroup published itself); should
   // they -- two launches that share one workspace at the same time --, the range is marked rather
@@ -585,18 +684,26 @@ int launch_ranges(const In *in, Out *out, int64_t n, void *ws, hipStream_t st, b
   Slot *slots = reinterpret_cast<Slot *>(sums + max_ranges);
   const int64_t first = first_changed > 0 ? first_changed / range_elems : 0;
   const dim3 grid((unsigned)(ranges - first)), block(kBlock);
+  const bool grouped = ranges > kFlatRanges && ranges <= kMaxRanges;
   if (!chained) {
     range_sum_kernel<In, Acc, Out, G><<<grid, block, 0, st>>>(in, n, sums, first);
-    if (ranges <= kMaxRangesTwo) {
-      scan_ranges_kernel<In, Acc, Out, G, kTwoLaunches><<<grid, block, 0, st>>>(
-          in, out, n, sums, slots, first, 0ull, 0, 0, 0);
+    if (G >= 8 && grouped) {
+      const int64_t first_group = first / kGroup, whole = ranges / kGroup;
+      if (whole > first_group)
+        group_sum_kernel<Acc><<<dim3((unsigned)ceil_div64(whole - first_group, kBlock / kWave)), block, 0, st>>>(
+            sums, groups_of(slots, ranges).sums, first_group, whole);
+      scan_ranges_kernel<In, Acc, Out, G >= 8 ? G : 8, kTwoLaunches, true><<<grid, block, 0, st>>>(
+          in, out, n, sums, slots, first, 0ull, 0, 0, 0, ranges);
+    } else if (ranges <= kFlatRanges) {
+      scan_ranges_kernel<In, Acc, Out, G, kTwoLaunches, false><<<grid, block, 0, st>>>(
+          in, out, n, sums, slots, first, 0ull, 0, 0, 0, ranges);
     } else {
-      // more ranges than a workgroup adds up by itself: their prefix comes from a launch in
-      // between (into the words that the chained variant uses for its slots)
+      // more groups than a workgroup has threads: the ranges' prefix comes from a launch in between (into
+      // the words that the chained variant uses for its slots)
       range_prefix_kernel<Acc><<<dim3(1), dim3(kPrefixThreads), 0, st>>>(
           sums, reinterpret_cast<uint64_t *>(slots), ranges);
-      scan_ranges_kernel<In, Acc, Out, G, kPrefixed><<<grid, block, 0, st>>>(
-          in, out, n, sums, slots, first, 0ull, 0, 0, 0);
+      scan_ranges_kernel<In, Acc, Out, G, kPrefixed, false><<<grid, block, 0, st>>>(
+          in, out, n, sums, slots, first, 0ull, 0, 0, 0, ranges);
     }
     GEARHIP_RETURN_IF_LAUNCH_FAILED();
     return 0;
@@ -607,13 +714,18 @@ int launch_ranges(const In *in, Out *out, int64_t n, void *ws, hipStream_t st, b
   // on; below that they only delay the launch): 5 ns per range of 8192 fp32 elements.
   int stagger = 0, first_wave = 0;
   if (ranges - first > 512) {
-    static const Residency res = residency((const void *)scan_ranges_kernel<In, Acc, Out, G, kChained>);
+    static const Residency res =
+        residency((const void *)scan_ranges_kernel<In, Acc, Out, G, kChained, false>);
     const int64_t ps = env_int("GEAR_HIP_SCAN_STAGGER_PS", 5000) * (int64_t)(G * 16) / 128;
     stagger = (int)(ps * res.clock_khz * 1024 / 1000000000ll);
     first_wave = res.workgroups;
   }
-  scan_ranges_kernel<In, Acc, Out, G, kChained><<<grid, block, 0, st>>>(
-      in, out, n, sums, slots, first, tag, spin_limit, stagger, first_wave);
+  if (G >= 8 && grouped)
+    scan_ranges_kernel<In, Acc, Out, G >= 8 ? G : 8, kChained, true><<<grid, block, 0, st>>>(
+        in, out, n, sums, slots, first, tag, spin_limit, stagger, first_wave, ranges);
+  else
+    scan_ranges_kernel<In, Acc, Out, G, kChained, false><<<grid, block, 0, st>>>(
+        in, out, n, sums, slots, first, tag, spin_limit, stagger, first_wave, ranges);
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
   return 0;
 }
@@ -650,15 +762,15 @@ int launch_scan(const In *in, Out *out, int64_t n, void *ws, size_t ws_bytes, hi
   // Ranges of 2, 4, 8 or 16 granules per thread (2048 to 16384 fp32 elements): 2 while that
   // leaves at most 256 ranges, 4 up to 512 ranges, then 8 (a workgroup adds up ALL earlier sums, so
   // more ranges cost more than they gain once every CU has work), and 16 -- 190 registers, two
-  // workgroups per CU -- where 8 would need more than 4096 ranges (33.5 to 134 M fp32: one read
-  // instead of two, us at 6e7 / 6.8e7 / 1e8 / 1.3e8: 148 / 167 / 240 / 330 against 187 / 213 / 308 /
-  // 399; int64 at 4e7 / 6e7: 143 / 235 against 183 / 267).  The chained kernel and the two launches cut
+  // workgroups per CU -- where 8 would need more than 4096 ranges (33.5 to 268 M fp32: one read
+  // instead of two, us at 6e7 / 6.8e7 / 1e8 / 1.3e8: 147 / 167 / 240 / 309 against 187 / 213 / 308 /
+  // 399; int64 at 4e7 / 6e7: 143 / 210 against 183 / 267).  The chained kernel and the two launches cut
   // the input the same way, so a rescan finds the sums of the last full scan and the bits are the same;
   // but integers, which have no rescan and the same sums in any order, take 8 granules in two launches
   // (captured, 4e7 / 6e7: 187 / 276 us, 197 / 281 with 16).
-  // At 8192 ranges the words to poll are 0.8 GB beside 1.6 GB of data; beyond that they outweigh
-  // the second read: two launches, up to 16384 ranges of 8 granules.  (8-byte elements: ranges of 2
-  // granules would be smaller than the 2048 elements the workspace is laid out for, so they start at 4.)
+  // Beyond 16384 ranges a workgroup has fewer threads than there are groups: three launches of 8 granules.
+  // (8-byte elements: ranges of 2 granules would be smaller than the 2048 elements the workspace is laid
+  // out for, so they start at 4.)
   if (VE == 4 && ceil_div64(n, 2 * g1) <= 256)
     return launch_ranges<In, Acc, Out, VE, 2>(in, out, n, ws, st, chained, first_changed);
   else if (ceil_div64(n, 4 * g1) <= 512)

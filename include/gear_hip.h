@@ -178,12 +178,11 @@ int gear_hip_take_i64(const int64_t *table, int64_t n, const int64_t *idx, int64
 
 /* Inclusive prefix sum of fp32 priorities accumulated and written in fp64:
  *     out[i] = sum_{j<=i} (double) in[j]
- * One pass over the input for up to 4096 ranges (n <= 67.1 M): every workgroup publishes the sum
+ * One pass over the input for up to 16384 ranges (n <= 268 M): every workgroup publishes the sum
  * of its range and adds the sums of all earlier ranges, with a bounded wait (a workgroup that
  * waited too long sums the missing range itself and publishes it: same bits, no kernel can
- * hang).  Two launches (range sums, then the scan) beyond that, for a stream under graph capture,
- * and with GEAR_HIP_SCAN_SINGLE_PASS=0; three (a launch in between scans the range sums) beyond
- * 16384 ranges (n > 134 M).  The result is bit-identical in all cases and on every run.  Replaces
+ * hang).  Two launches (range sums, then the scan) for a stream under graph capture and with
+ * GEAR_HIP_SCAN_SINGLE_PASS=0; three (a launch in between scans the range sums) beyond that.  The result is bit-identical in all cases and on every run.  Replaces
  * gear::cuda::launch_prefix_sum /
  * one_dimension_prefix_sum (src/cuda/one_dim_prefix_sum.cu:125-273; libgear.core.prefix_sum,
  * :276-278), which is fp32 and only correct for one block.
