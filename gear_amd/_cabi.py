@@ -10,6 +10,7 @@ _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, "libgearhip.so")
 
 c_i64 = ctypes.c_int64
+c_u64 = ctypes.c_uint64
 c_int = ctypes.c_int
 c_void_p = ctypes.c_void_p
 c_size_t = ctypes.c_size_t
@@ -87,6 +88,12 @@ SIGNATURES = {
     "gear_hip_upper_bound_i64": (c_int, [c_void_p, c_i64, c_void_p, c_i64, c_int, c_void_p,
                                          c_void_p]),
     "gear_hip_sort_workspace_bytes": (c_size_t, [c_i64]),
+    "gear_hip_draw_max": (c_i64, []),
+    "gear_hip_draw_lookup_f64": (c_int, [c_void_p, c_i64, c_u64, c_u64, c_i64, c_void_p, c_i64, c_void_p,
+                                         c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "gear_hip_draw_sort_lookup_i64": (c_int, [c_u64, c_u64, c_i64, c_i64, c_void_p, c_i64, c_i64, c_void_p,
+                                              c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t,
+                                              c_void_p]),
     "gear_hip_take_sorted_workspace_bytes": (c_size_t, [c_i64]),
     "gear_hip_take_sorted_i64": (c_int, [c_void_p, c_i64, c_void_p, c_i64, c_void_p, c_void_p, c_size_t,
                                          c_void_p]),

@@ -7,6 +7,7 @@
 
 #include <type_traits>
 
+#include "philox.hpp"
 #include "range_sort.hpp"
 
 namespace gearhip {
@@ -119,15 +120,21 @@ __device__ __forceinline__ int64_t group_search(const T *__restrict__ p, int64_t
 // fp64 prefix: fp32 draws, in [0, 1) (unit) or targets already.  A target that is not a number -- the
 // draw or the total is none, or infinite where the other is 0 -- compares with nothing and finds
 // entry 0, so it has the lowest key.
-struct DrawF64 {
+struct PhiloxU {  // draws that are worked out where they are asked for
+  Philox rng;
+  __device__ __forceinline__ float operator[](int64_t j) const { return rng.uniform((uint64_t)j); }
+};
+template <typename U>
+struct DrawF64From {
   typedef double type;
   typedef uint32_t key_type;
   const double *prefix;
   int64_t n;
-  const float *u;
+  U u;
   int unit;
   __device__ __forceinline__ double target(int64_t j, double total) const {
-    return unit ? (double)u[j] * total : (double)u[j];
+    const float f = u[j];
+    return unit ? (double)f * total : (double)f;
   }
   __device__ __forceinline__ uint32_t key(int64_t j, double total) const {
     const float f = u[j];
@@ -139,6 +146,7 @@ struct DrawF64 {
     return t == t ? k : 0u;
   }
 };
+typedef DrawF64From<const float *> DrawF64;
 // int64 prefix (a sampler over lengths): doubles in [0, 1) (unit) or int64 targets.
 struct DrawI64 {
   typedef int64_t type;
@@ -412,10 +420,14 @@ __global__ __launch_bounds__(kPlaceThreads) void place_draws_kernel(Draw draw, i
   }
 }
 
-// The same for positions that are given (no search): sorted and looked up.
-template <typename Emit>
-__global__ __launch_bounds__(kPlaceThreads) void place_positions_kernel(
-    const int64_t *__restrict__ raw, int num, Emit emit) {
+// The same for positions that are given (no search): sorted and looked up.  raw[j]: from memory, or drawn.
+struct PhiloxPositions {
+  Philox rng;
+  uint32_t range;
+  __device__ __forceinline__ int64_t operator[](int j) const { return rng.below(range, (uint64_t)j); }
+};
+template <typename Raw, typename Emit>
+__global__ __launch_bounds__(kPlaceThreads) void place_positions_kernel(Raw raw, int num, Emit emit) {
   __shared__ PlaceSmem<int64_t> sm;
   const int tid = threadIdx.x;
   const int e = (int)blockIdx.x * kPlaced + tid;
@@ -441,8 +453,8 @@ int place_draws(const Draw &draw, int64_t num, const Emit &emit, hipStream_t st)
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
   return 0;
 }
-template <typename Emit>
-int place_positions(const int64_t *raw, int64_t num, const Emit &emit, hipStream_t st) {
+template <typename Raw, typename Emit>
+int place_positions(const Raw &raw, int64_t num, const Emit &emit, hipStream_t st) {
   place_positions_kernel<<<dim3((unsigned)ceil_div64(num, kPlaced)), dim3(kPlaceThreads), 0, st>>>(
       raw, (int)num, emit);
   GEARHIP_RETURN_IF_LAUNCH_FAILED();
@@ -561,6 +573,21 @@ int sort_draws(const Draw &draw, int64_t num, const Emit &emit, hipStream_t st) 
   return ranges::sort<typename Src::key_type, false>(
       Src{draw, {}}, num, DrawEmit<Draw, Emit>{draw, emit, lanes}, st);
 }
+
+// Draws of a batch that other launches read.
+__global__ __launch_bounds__(kBlock) void draw_uniform_kernel(Philox rng, int64_t num, float *__restrict__ out) {
+  const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (j < num) out[j] = rng.uniform((uint64_t)j);
+}
+__global__ __launch_bounds__(kBlock) void draw_positions_kernel(PhiloxPositions raw, int64_t num,
+                                                                int64_t *__restrict__ out) {
+  const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (j < num) out[j] = raw[(int)j];
+}
+// Up to so many draws -- all that are placed by one launch -- every workgroup works out the draws of the whole
+// batch itself, four a thread at most.  us a batch of uniforms in 1e6 entries / of positions, so and with a
+// launch for the draws: 256 3.8 / 2.9 and 5.3 / 4.6, 1024 4.2 / 3.5 and 5.5 / 5.1, 4096 6.4 / 6.3 and 7.0 / 7.1.
+constexpr int64_t kDrawnInPlace = radix::kRankMax;
 
 __global__ __launch_bounds__(kBlock) void lookup_kernel(const int64_t *__restrict__ positions,
                                                         int64_t num, Lookup look) {
@@ -794,6 +821,61 @@ extern "C" int gear_hip_sample_lookup_f64(const double *prefix, int64_t n, const
     return GEAR_HIP_EWORKSPACE;
   return draw_and_look_up(DrawF64{prefix, n, u, unit_uniforms ? 1 : 0}, num, look,
                           static_cast<char *>(workspace), w, as_stream(stream));
+}
+
+extern "C" int64_t gear_hip_draw_max(void) { return kMaxDraws; }
+
+extern "C" int gear_hip_draw_lookup_f64(const double *prefix, int64_t n, uint64_t seed, uint64_t offset,
+                                        int64_t num, const int64_t *index_table, int64_t index_offset,
+                                        const int64_t *lengths_table, int64_t lengths_n,
+                                        int64_t *sampled_out, int64_t *local_out, int64_t *lens_out,
+                                        void *workspace, size_t workspace_bytes, void *stream) {
+  if (n < 0 || num < 0) return GEAR_HIP_EINVAL;
+  if (num == 0) return 0;
+  if (n == 0 || !prefix) return GEAR_HIP_EINVAL;
+  if (num > kMaxDraws) return GEAR_HIP_ERANGE;
+  const Lookup look{index_table, n, index_offset, lengths_table, lengths_n, sampled_out, local_out,
+                    lens_out};
+  int rc = check_lookup(look);
+  if (rc) return rc;
+  const SampleWs w = sample_ws(num);
+  if (!workspace || workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(workspace) & 7))
+    return GEAR_HIP_EWORKSPACE;
+  hipStream_t st = as_stream(stream);
+  const Philox rng{seed, offset};
+  if (num <= kDrawnInPlace && !writes_over(look, prefix, n * 8, num))
+    return place_draws(DrawF64From<PhiloxU>{prefix, n, {rng}, 1}, num, look, st);
+  char *ws = static_cast<char *>(workspace);
+  float *u = reinterpret_cast<float *>(ws + w.ktmp);  // (free until the draws have been searched)
+  draw_uniform_kernel<<<dim3((unsigned)ceil_div64(num, kBlock)), dim3(kBlock), 0, st>>>(rng, num, u);
+  GEARHIP_RETURN_IF_LAUNCH_FAILED();
+  return draw_and_look_up(DrawF64{prefix, n, u, 1}, num, look, ws, w, st);
+}
+
+extern "C" int gear_hip_draw_sort_lookup_i64(uint64_t seed, uint64_t offset, int64_t num, int64_t bound,
+                                             const int64_t *index_table, int64_t index_n,
+                                             int64_t index_offset, const int64_t *lengths_table,
+                                             int64_t lengths_n, int64_t *sampled_out, int64_t *local_out,
+                                             int64_t *lens_out, void *workspace, size_t workspace_bytes,
+                                             void *stream) {
+  if (num < 0 || bound <= 0) return GEAR_HIP_EINVAL;
+  if (num == 0) return 0;
+  if (num > kMaxDraws || bound > 0xffffffffll) return GEAR_HIP_ERANGE;
+  const Lookup look{index_table, index_n, index_offset, lengths_table, lengths_n, sampled_out,
+                    local_out, lens_out};
+  int rc = check_lookup(look);
+  if (rc) return rc;
+  const SampleWs w = sample_ws(num);
+  if (!workspace || workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(workspace) & 7))
+    return GEAR_HIP_EWORKSPACE;
+  hipStream_t st = as_stream(stream);
+  const PhiloxPositions drawn{{seed, offset}, (uint32_t)bound};
+  if (num <= kDrawnInPlace) return place_positions(drawn, num, look, st);
+  char *ws = static_cast<char *>(workspace);
+  int64_t *raw = reinterpret_cast<int64_t *>(ws + w.raw);
+  draw_positions_kernel<<<dim3((unsigned)ceil_div64(num, kBlock)), dim3(kBlock), 0, st>>>(drawn, num, raw);
+  GEARHIP_RETURN_IF_LAUNCH_FAILED();
+  return sort_and_look_up(raw, num, bound, look, ws, w, st);
 }
 
 extern "C" int gear_hip_sample_lookup_i64(const int64_t *prefix, int64_t n, const void *u,

@@ -23,6 +23,7 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <tuple>
 #include <unordered_map>
@@ -536,6 +537,37 @@ struct Staging {
   }
 };
 
+// ---- draws -----------------------------------------------------------------------------------------
+// A batch of random numbers from a torch generator costs a call of torch's, 6 us of the host and a launch of
+// 2.2 us, for numbers that a few instructions give where they are used (philox.hpp).  Only where a call
+// of torch's would take one block of the generator's stream a draw, and not while the stream is captured,
+// when the generator's state is not the host's to read.
+bool draws_here(const at::Generator &gen, bool weighted, int64_t range, int64_t num, const at::Device &device) {
+  if (!gen.defined() || gen.device().type() != at::kCUDA || num < 1 || num > gear_hip_draw_max()) return false;
+  if (gen.device().index() != (device.has_index() ? device.index() : c10::hip::current_device())) return false;
+  if (!weighted && (range < 1 || range > 0xffffffffll)) return false;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(static_cast<hipStream_t>(current_stream()), &capture) == hipSuccess &&
+         capture == hipStreamCaptureStatusNone;
+}
+py::object torch_draws(const at::Generator &gen, bool weighted, int64_t range, int64_t num,
+                       const at::Device &device) {
+  at::Tensor t;
+  {
+    py::gil_scoped_release nogil;
+    const auto options = at::TensorOptions().device(device);
+    t = weighted ? at::rand({num}, gen, options.dtype(at::kFloat))
+                 : at::randint(range, {num}, gen, options.dtype(at::kLong));
+  }
+  return wrap(t);
+}
+// the seed and the offset of the next call's numbers, which are taken from the generator
+std::pair<uint64_t, uint64_t> next_block(at::Generator &gen) {
+  std::lock_guard<std::mutex> lock(gen.mutex());
+  const auto state = at::check_generator<at::CUDAGeneratorImpl>(gen)->philox_cuda_state(4);
+  return {state.seed_.val, state.offset_.val};
+}
+
 class LoaderStep {
  public:
   struct Column {
@@ -561,19 +593,29 @@ class LoaderStep {
       throw std::runtime_error("more than 16 columns: one launch gathers 16 at most");
   }
 
-  // kind, draws, prefix: as WeightedSampler / UniformSampler / TopKSampler.prepare() return them.
+  // kind, draws, prefix: as WeightedSampler / UniformSampler / TopKSampler.prepare() return them; or the
+  // generator to draw from and how many draws there are: the same draws, worked out where they are used.
   // Returns (sampled, timesteps, [batch tensors], [masks] or None); the timesteps on the host when
   // host_timesteps is set.
-  py::tuple run(const std::string &kind, py::handle draws_, py::handle prefix_, py::handle indices_,
-                int64_t index_offset, py::handle timesteps_, bool host_timesteps, py::handle ws) {
+  py::tuple run(const std::string &kind, py::object draws_, py::handle prefix_, py::handle indices_,
+                int64_t index_offset, py::handle timesteps_, bool host_timesteps, py::handle ws, int64_t to_draw) {
     const at::Tensor &indices = need(indices_, at::kLong, "indices"),
                      &timesteps = need(timesteps_, at::kLong, "timesteps");
     const bool weighted = kind == "weighted";
-    const at::Tensor &draws = need(draws_, weighted ? at::kFloat : at::kLong, "draws");
     const bool uniform = kind == "uniform";
     if (!weighted && !uniform && kind != "positions")
       throw std::invalid_argument("kind must be 'weighted', 'uniform' or 'positions'");
-    const int64_t num = draws.numel();
+    std::optional<at::Generator> generator;
+    if (to_draw >= 0) {
+      generator = draws_.cast<at::Generator>();
+      if (!draws_here(*generator, weighted, indices.numel(), to_draw, device_)) {
+        draws_ = torch_draws(*generator, weighted, indices.numel(), to_draw, device_);
+        generator.reset();
+      }
+    }
+    const at::Tensor none;
+    const at::Tensor &draws = generator ? none : need(draws_, weighted ? at::kFloat : at::kLong, "draws");
+    const int64_t num = generator ? to_draw : draws.numel();
     const uintptr_t base = table_.attr("device_address").cast<uintptr_t>();
     if (base == 0)
       throw std::runtime_error(
@@ -619,7 +661,20 @@ class LoaderStep {
       }
       const int64_t *table = ptr<int64_t>(indices), *lengths = ptr<int64_t>(timesteps);
       int64_t *s = ptr<int64_t>(sampled), *l = ptr<int64_t>(local), *len = ptr<int64_t>(lens);
-      if (weighted)
+      const int64_t count = indices.numel();
+      uint64_t seed = 0, offset = 0;
+      if (generator) std::tie(seed, offset) = next_block(*generator);
+      if (generator && weighted)
+        check("gear_hip_draw_lookup_f64", launches(w, [&] {
+                return gear_hip_draw_lookup_f64(prefix, count, seed, offset, num, table, index_offset, lengths,
+                                                timesteps.numel(), s, l, len, w.ptr, w.bytes, st);
+              }));
+      else if (generator)
+        check("gear_hip_draw_sort_lookup_i64", launches(w, [&] {
+                return gear_hip_draw_sort_lookup_i64(seed, offset, num, count, table, count, index_offset,
+                                                     lengths, timesteps.numel(), s, l, len, w.ptr, w.bytes, st);
+              }));
+      else if (weighted)
         check("gear_hip_sample_lookup_f64", launches(w, [&] {
                 return gear_hip_sample_lookup_f64(prefix, indices.numel(), ptr<float>(draws), num, 1, table,
                                                   index_offset, lengths, timesteps.numel(), s, l, len, w.ptr,
@@ -709,5 +764,7 @@ PYBIND11_MODULE(_hostops, m) {
       .def("run", &Gather::run);
   py::class_<LoaderStep>(m, "LoaderStep")
       .def(py::init<py::object, int64_t, int64_t, int64_t, const py::list &, bool, const at::Device &>())
-      .def("run", &LoaderStep::run);
+      .def("run", &LoaderStep::run, py::arg("kind"), py::arg("draws"), py::arg("prefix"), py::arg("indices"),
+           py::arg("index_offset"), py::arg("timesteps"), py::arg("host_timesteps"), py::arg("ws"),
+           py::arg("to_draw") = -1);
 }

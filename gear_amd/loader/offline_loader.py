@@ -240,18 +240,19 @@ class OfflineLoader(BasicLoader):
         self.last_masks = masks
         return data_batch
 
-    def _select_gather(self, draws, dirty_from, host_timesteps=False):
+    def _select_gather(self, draws, dirty_from, host_timesteps=False, draws_num=-1):
         """Everything of a step after the draws: the sampler's own preparation (prefix rescan,
         top-k selection), then ONE call that sorts the batch, looks up global index, local index
         and recorded length of every entry, and gathers all columns into fresh tensors.  Returns
-        (lengths, data_batch); the lengths on the host, after the gather, when asked for."""
+        (lengths, data_batch); the lengths on the host, after the gather, when asked for.  draws: the
+        batch's random numbers, or the generator that gives them in the call, draws_num of them."""
         kind, picks, prefix = self._sampler.prepare(self._indices, self._device_weights, draws,
                                                     dirty_from=dirty_from)
         if self._step is None:
             self._step = self._native_step()
         self.last_sampled, lengths, data_batch, self.last_masks = self._step.run(
             kind, picks, prefix, self._indices, self._iset.index_offset, self._device_timesteps,
-            host_timesteps, ops._ws)
+            host_timesteps, ops._ws, -1 if isinstance(draws, torch.Tensor) else draws_num)
         return lengths, data_batch
 
     def _graph_step(self):
@@ -284,9 +285,10 @@ class OfflineLoader(BasicLoader):
     def fused_iterate(self):
         if self._use_graph:
             return self._graph_iterate()
-        draws = self._sampler.draw(self._indices.numel(), self._batch_size * self._dp_world)
+        bsz = self._batch_size * self._dp_world
+        draws = self._sampler.draws_of_a_step(self._indices.numel(), bsz)
         timesteps, data_batch = self._select_gather(draws, self._dirty_from,
-                                                    not self._timesteps_on_device)
+                                                    not self._timesteps_on_device, bsz)
         self._dirty_from = self._device_weights.numel()   # clean until the next update
         return timesteps, data_batch
 

@@ -61,6 +61,14 @@ class UniformSampler:
                              generator=self._generator, dtype=torch.long,
                              device=self._mpu.device)
 
+    # What a loader's step draws from: the generator, from which the native step takes the numbers that draw()
+    # would have got out of it, or those numbers where draw() or prepare() are not the ones of this module.
+    def draws_of_a_step(self, num_indices, batch_size):
+        cls = type(self)
+        if cls in (UniformSampler, WeightedSampler) and not {"draw", "prepare"} & self.__dict__.keys():
+            return self._generator
+        return self.draw(num_indices, batch_size)
+
     def select(self, indices, weights, draws, dirty_from=None):
         return self._take_sorted(indices, draws)
 

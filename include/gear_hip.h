@@ -341,6 +341,23 @@ int gear_hip_upper_bound_i64(const int64_t *prefix, int64_t n, const void *u, in
 
 /* ---- sort / top-k / priority update ------------------------------------------------------- */
 
+/* gear_hip_sample_lookup_f64 for uniforms, and gear_hip_sort_lookup_i64 for integers in [0, bound), that the
+ * call draws itself: the numbers that torch's GPU generator of this seed and offset gives to one rand
+ * (float32) or randint (int64) call of `num` elements (Philox4x32-10; the caller advances the offset by 4).
+ * num <= gear_hip_draw_max(), bound < 2^32, else GEAR_HIP_ERANGE.  They take the place of the torch.randint
+ * and torch.multinomial of gear/sampler/global_sampler.py:121-199. */
+int64_t gear_hip_draw_max(void);
+int gear_hip_draw_lookup_f64(const double *prefix, int64_t n, uint64_t seed, uint64_t offset, int64_t num,
+                             const int64_t *index_table, int64_t index_offset,
+                             const int64_t *lengths_table, int64_t lengths_n, int64_t *sampled_out,
+                             int64_t *local_out, int64_t *lens_out, void *workspace,
+                             size_t workspace_bytes, void *stream);
+int gear_hip_draw_sort_lookup_i64(uint64_t seed, uint64_t offset, int64_t num, int64_t bound,
+                                  const int64_t *index_table, int64_t index_n, int64_t index_offset,
+                                  const int64_t *lengths_table, int64_t lengths_n, int64_t *sampled_out,
+                                  int64_t *local_out, int64_t *lens_out, void *workspace,
+                                  size_t workspace_bytes, void *stream);
+
 /* Ascending sort (by counting, or LSD radix) of `num` int64 keys (non-negative, < 2^key_bits) with an optional
  * int64 payload, stable.  keys_out/vals_out must not alias the inputs.
  * Replaces the torch.sort of sampled indices in every sampler
