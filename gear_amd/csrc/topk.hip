@@ -911,6 +911,7 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
     if (tid == 0) state->gave_up = 1u;
     return;
   }
+  if (binned == nullptr) return;  // (nobody will ask)
   const u32x4 c4 = *reinterpret_cast<const u32x4 *>(&h[tid * 4]);
   const uint32_t sum4 = (c4[0] + c4[1]) + (c4[2] + c4[3]);
   const uint32_t inc = (uint32_t)wave_inclusive_sum((int)sum4);
@@ -2640,9 +2641,11 @@ __device__ __forceinline__ void finish_selection(
     const uint32_t s = (hi_key - lo_key - (uint32_t)(own >> 32)) >> slot_shift;
     return s < kFinishSlots ? s : kFinishSlots - 1u;
   };
-  // four lanes per list
+  // four lanes per list, more where there are fewer lists
   static_assert(kThreads == 4 * kMaxBlocks, "every list has its lanes");
-  const uint32_t src = (uint32_t)tid >> 2;
+  uint32_t lanes = 4u;
+  while (lanes < (uint32_t)kWave && gridDim.x * lanes * 2u <= (uint32_t)kThreads) lanes *= 2u;
+  const uint32_t src = (uint32_t)tid / lanes, sub = (uint32_t)tid & (lanes - 1u);
   const bool real = src < gridDim.x;
   const uint16_t *row = starts + (real ? src : 0u) * kStartPitch;
   const uint64_t *from = binned + (int64_t)(real ? src : 0u) * binned_cap(list_cap);
@@ -2653,28 +2656,62 @@ __device__ __forceinline__ void finish_selection(
     s_last = 0ull;
   }
   reinterpret_cast<u32x2 *>(cnt)[tid] = u32x2{0u, 0u};
-  __syncthreads();
-  if (!real) end = 0u;
+  if (!real) end = c;
   uint32_t before = 0u;  // by index: this lane's share of the selected entries of earlier lists
-  if (!kByValue && (tid & 3) == 0 && src < blockIdx.x) before = all - end;
+  if (!kByValue && sub == 0u && src < blockIdx.x) before = all - end;
+  auto take = [&](uint32_t slot, uint64_t ent) {
+    const uint64_t own = ((ent >> 32) - lo_key) << 32 | (uint32_t)~(uint32_t)ent;
+    ents[slot] = own;
+    atomicAdd(&cnt[slot_of(own)], 1u);
+  };
   constexpr int kAtOnce = 2;
-  for (c += (uint32_t)tid & 3u; wave_ballot(c < end) != 0ull; c += 4u * kAtOnce) {
-    uint64_t e[kAtOnce];
+  // Most pieces are a few entries.  Where one is long -- neighbours in the input that are neighbours in value --
+  // its lanes would fetch it one round trip after the other: then the entries of all pieces are dealt
+  // out to the threads.
+  if (!__syncthreads_or(end - c > lanes * kAtOnce * 8u)) {
+    for (c += sub; wave_ballot(c < end) != 0ull; c += lanes * kAtOnce) {
+      uint64_t e[kAtOnce];
 #pragma unroll
-    for (int u = 0; u < kAtOnce; ++u) e[u] = from[c + 4u * u < end ? c + 4u * u : 0u];
+      for (int u = 0; u < kAtOnce; ++u) e[u] = from[c + lanes * u < end ? c + lanes * u : 0u];
 #pragma unroll
-    for (int u = 0; u < kAtOnce; ++u) {
-      const bool hit = c + 4u * u < end;
-      const uint64_t hits = wave_ballot(hit);
-      if (hits == 0ull) break;
-      uint32_t slot = 0u;
-      if (lane == 0) slot = atomicAdd(&s_n, (uint32_t)__popcll(hits));
-      slot = (uint32_t)__builtin_amdgcn_readlane((int)slot, 0) + (uint32_t)__popcll(hits & lt_mask);
-      if (hit && slot < kFinishCap) {
-        const uint64_t own = ((e[u] >> 32) - lo_key) << 32 | (uint32_t)~(uint32_t)e[u];
-        ents[slot] = own;
-        atomicAdd(&cnt[slot_of(own)], 1u);
+      for (int u = 0; u < kAtOnce; ++u) {
+        const bool hit = c + lanes * u < end;
+        const uint64_t hits = wave_ballot(hit);
+        if (hits == 0ull) break;
+        uint32_t slot = 0u;
+        if (lane == 0) slot = atomicAdd(&s_n, (uint32_t)__popcll(hits));
+        slot = (uint32_t)__builtin_amdgcn_readlane((int)slot, 0) + (uint32_t)__popcll(hits & lt_mask);
+        if (hit && slot < kFinishCap) take(slot, e[u]);
       }
+    }
+  } else {
+    __shared__ uint32_t s_begin[kMaxBlocks], s_at[kMaxBlocks];  // a piece's begin, the entries up to its end
+    if (tid < kMaxBlocks) s_at[tid] = 0u;
+    __syncthreads();
+    if (sub == 0u && real) {
+      s_begin[src] = c;
+      s_at[src] = end - c;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      uint32_t run = 0u;
+#pragma unroll
+      for (int w = 0; w < kMaxBlocks / kWave; ++w) {
+        const uint32_t inc = run + (uint32_t)wave_inclusive_sum((int)s_at[w * kWave + lane]);
+        s_at[w * kWave + lane] = inc;
+        run = (uint32_t)wave_read_lane((int)inc, kWave - 1);
+      }
+      if (lane == 0) s_n = run;
+    }
+    __syncthreads();
+    const uint32_t entries = s_n < kFinishCap ? s_n : kFinishCap;
+    for (uint32_t i = (uint32_t)tid; i < entries; i += kThreads) {
+      uint32_t lo = 0u;  // the first piece that ends behind entry i
+#pragma unroll
+      for (uint32_t step = kMaxBlocks / 2; step != 0u; step /= 2)
+        if (s_at[lo + step - 1u] <= i) lo += step;
+      const uint32_t before_it = lo > 0u ? s_at[lo - 1u] : 0u;
+      take(i, binned[(int64_t)lo * binned_cap(list_cap) + s_begin[lo] + (i - before_it)]);
     }
   }
   __syncthreads();
@@ -2915,11 +2952,17 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   };
   int per = 2;
   while (per < kMaxSamplesPerThread && !lists_hold(per)) per *= 4;
-  while (per > 2 && n < 128 * (int64_t)per * kThreads) per /= 4;  // strides of 128 elements or more
-  if ((list_all || lists_hold(per)) && n >= 128 * (int64_t)per * kThreads && k <= n / 8 &&
+  const auto strides = [&](int p) { return n / ((int64_t)p * kThreads); };
+  while (per > 2 && strides(per) < 128) per /= 4;
+  // Strides of 128 elements and more, and k up to n / 8, where the steps below follow; any stride, and k up to
+  // n / 4, where level 1 finishes: us without and with a sample, by index / by value, 2048 of 16384 23.4 /
+  // 34.3 and 18.6 / 20.2, 25000 of 200000 24.5 / 37.4 and 20.0 / 20.8, 60000 of 300000 25.2 / 41.4 and 22.2 /
+  // 21.9, 750000 of 3e6 by index 51.4 and 43.3.  (With more of the input selected the lists hold most of it.)
+  const bool ends_early = !sorted_by_value || k <= kBucketMaxK;
+  if ((list_all || lists_hold(per)) && strides(per) >= (ends_early ? 1 : 128) && k <= n / (ends_early ? 4 : 8) &&
       env_int("GEAR_HIP_TOPK_HINT", 1) != 0) {
     const double r = hint_rank(per);
-    if (r < (double)per * kThreads / 4) rank = (uint32_t)r + 1u;
+    if (r < (double)per * kThreads / 2) rank = (uint32_t)r + 1u;
   }
   const int64_t zero_words = (int64_t)((l.zero_end - l.zero_begin) / 4);
   const unsigned zero_blocks = (unsigned)ceil_div64(zero_words, (int64_t)kThreads * 4);
@@ -2941,15 +2984,18 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
       prep_kernel<32><<<pgrid, block, 0, st>>>(priorities, n, k, rank, list_all, mid_bins, warm, state,
                                                zero, zero_words);
   }
+  // Whether level 1 may finish: not the values of a selection that is sorted by radix.
+  const bool by_segments = sorted_by_value && k <= kBucketMaxK;
+  const bool finishes = rank != 0u && (!sorted_by_value || (by_segments && ceil_div64(k, g.blocks) <= kFinishCap / 2));
   if (rank != 0u)
     level0_hinted_kernel<<<grid, block, 0, st>>>(priorities, n, state, hist0, g.wave_len,
-                                                 wave_listed, lists, (int)g.list_cap, binned, starts);
+                                                 wave_listed, lists, (int)g.list_cap, finishes ? binned : nullptr,
+                                                 starts);
   else
     level0_kernel<<<grid, block, 0, st>>>(priorities, n, state, hist0, g.wave_len, wave_listed,
                                           lists, (int)g.list_cap);
   // value order by segments: workgroup w of the sort owns the bins that start in the output
   // places [w << seg_shift, (w + 1) << seg_shift)
-  const bool by_segments = sorted_by_value && k <= kBucketMaxK;
   int seg_shift = 0;
   while ((k >> seg_shift) >= kNoSegment) ++seg_shift;  // segment ids stay below kNoSegment
   uint32_t *wg_bins = reinterpret_cast<uint32_t *>(ws + l.wg_bins);
@@ -2963,7 +3009,7 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   uint64_t *cand = reinterpret_cast<uint64_t *>(ws + l.cand);
   uint64_t *cand2 = reinterpret_cast<uint64_t *>(ws + l.cand2);
   uint32_t *ckey = reinterpret_cast<uint32_t *>(ws + l.ckey);
-  if (rank != 0u && (!sorted_by_value || (by_segments && ceil_div64(k, g.blocks) <= kFinishCap / 2))) {
+  if (finishes) {
     const Rest rest{priorities, n, k, state, reinterpret_cast<Hand *>(ws + l.hand), hist1, hist2, histf1, histf2,
                     g.wave_len, wave_listed, lists, (int)g.list_cap, wave_ge, block_ge, ckey, cidx, boff,
                     seg_shift, cseg, values_out, indices_out};

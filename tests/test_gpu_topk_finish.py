@@ -80,3 +80,20 @@ def test_what_level_1_leaves_on_two_streams(oracle):
     torch.cuda.synchronize()
     for by_value, index in got:
         assert torch.equal(index, expected[by_value])
+
+
+@pytest.mark.parametrize("n,k", [(2_048, 1), (2_049, 512), (4_097, 1_024), (10_007, 2_501), (32_768, 8_192),
+                                 (131_073, 32_768), (1_048_576, 131_072), (1_048_576, 250_000)])
+def test_small_inputs_and_large_shares(oracle, n, k):
+    w = _values(n, n + k)
+    _check(oracle, w, k, "lognormal")
+    _check(oracle, np.full(n, 1.0, np.float32), k, "all equal")
+
+
+@pytest.mark.parametrize("n,k", [(5_000, 600), (60_000, 3_000), (1_000_000, 50_000)])
+def test_neighbours_in_the_input_that_are_neighbours_in_value(oracle, n, k):
+    """A workgroup's entries lie in one other's list: dealt out to its threads."""
+    w = np.sort(_values(n, k))
+    _check(oracle, w, k, "ascending")
+    _check(oracle, w[::-1].copy(), k, "descending")
+    _check(oracle, np.arange(n, dtype=np.float32), k, "0 to n - 1")
