@@ -667,7 +667,7 @@ __global__ __launch_bounds__(kThreads) void prep_kernel(const float *__restrict_
   }
   float v[kPer];
   if (rank != 0u && !reuse) {
-    const int64_t stride = n / (kPer * kThreads);  // >= 128 (the caller's condition), < 2^20
+    const int64_t stride = n / (kPer * kThreads);  // >= 1 (the caller's condition), < 2^20
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
       const uint32_t s = (uint32_t)(tid + j * kThreads);
@@ -2554,9 +2554,9 @@ static_assert(kSortThreads >= kSortBins, "a thread per digit in the segment sort
 // order in LDS: no list is walked, and nothing passes between the workgroups.
 // us a call, back to back, as five to seven launches / finished by level 1 (lognormal priorities, cold):
 // 20000 of 3e6 by value 39.0 / 25.4, 65536 of 1e7 by value 49.5 / 33.2 and by index 32.8 / 31.4, 1000 of 3e5 by
-// index (with the look-up and the gather of a loader's step) 37.2 / 29.2.  What level 1 cannot finish takes 4
-// to 7 us longer than before, for the binned lists and the hand-overs: 60000 ties above the threshold 56 /
-// 63 by value, 36 / 43 by index; all priorities equal 104 / 111.
+// index (with the look-up and the gather of a loader's step) 37.2 / 29.2.  What level 1 cannot finish takes
+// longer than before, for the binned lists and the hand-overs: 60000 ties above the threshold 56 / 63 by
+// value, 36 / 43 by index; all priorities equal 104 / 111, of 1e6 41 / 53, 20000 of them 30 / 40.
 // By value a workgroup takes the bins that start in its stretch of the output; the bin that holds the k-th
 // key is ordered whole and what lies beyond place k is not stored, so no threshold is needed.  By index
 // every workgroup takes the bin of the k-th key, finds the last entry of it that is selected, and from that
@@ -2582,7 +2582,11 @@ struct FinishOut {
 
 // fin(place, entry) for the m entries, larger ones first, which were counted in cnt (kFinishSlots words) by
 // slot_of(entry): a counting sort by slots, of which most hold an entry or none, and a rank inside the slot.
-// Both buffers hold kFinishCap.
+// Both buffers hold kFinishCap, cnt two tables of slots.
+// A slot that is crowded -- priorities that are equal: new entries at the largest one -- is cut again, by what its
+// entries differ in (equal priorities: the index), instead of a radix sort of everything, which stays for
+// more than one such slot and for crowds within the crowd: us a call on 300000 priorities with 1808 equal ones
+// above the rest, 1000 by index 40.9 / 27.6 without and with it, 2000 by value 47.6 / 29.2 by segments and here.
 template <typename Slot, typename Out>
 __device__ __forceinline__ void order_entries(uint64_t *ents, uint64_t *other, uint32_t *cnt, uint32_t m,
                                               int bits, const Slot &slot_of, const Out &fin, SortShared &sh) {
@@ -2593,8 +2597,13 @@ __device__ __forceinline__ void order_entries(uint64_t *ents, uint64_t *other, u
   const u32x2 c2 = reinterpret_cast<const u32x2 *>(cnt)[tid];
   const uint32_t inc = (uint32_t)wave_inclusive_sum((int)(c2[0] + c2[1]));
   if (lane == kWave - 1) s_wsum[wave] = inc;
-  const bool crowded = __syncthreads_or(c2[0] > kFinishSlot || c2[1] > kFinishSlot);
-  if (crowded) {
+  __shared__ uint32_t s_crowd;
+  __shared__ uint64_t s_max[kWavesPerBlock], s_min[kWavesPerBlock];
+  const bool crowded0 = c2[0] > kFinishSlot, crowded1 = c2[1] > kFinishSlot;
+  if (crowded0 || crowded1) s_crowd = 2u * tid + (crowded1 ? 1u : 0u) + (crowded0 && crowded1 ? kFinishSlots : 0u);
+  const int crowds = __syncthreads_count(crowded0 || crowded1);
+  const uint32_t crowd = crowds != 0 ? s_crowd : 0u;
+  if (crowds > 1 || crowd >= kFinishSlots) {
     sort_segment(ents, other, m, bits, fin, sh);
     return;
   }
@@ -2604,7 +2613,62 @@ __device__ __forceinline__ void order_entries(uint64_t *ents, uint64_t *other, u
   __syncthreads();
   for (uint32_t i = tid; i < m; i += kThreads) other[atomicAdd(&cnt[slot_of(ents[i])], 1u)] = ents[i];
   __syncthreads();
+  uint32_t crowd_at = 0u, crowd_end = 0u;
+  if (crowds != 0) {
+    crowd_at = crowd > 0u ? cnt[crowd - 1u] : 0u;
+    crowd_end = cnt[crowd];
+    uint32_t *part = cnt + kFinishSlots;
+    uint64_t largest = 0ull, smallest = ~0ull;
+    for (uint32_t i = crowd_at + tid; i < crowd_end; i += kThreads) {
+      const uint64_t own = other[i];
+      largest = own > largest ? own : largest;
+      smallest = own < smallest ? own : smallest;
+    }
+#pragma unroll
+    for (int step = 1; step < kWave; step *= 2) {
+      const uint64_t a = __shfl_xor((unsigned long long)largest, step);
+      const uint64_t b = __shfl_xor((unsigned long long)smallest, step);
+      largest = a > largest ? a : largest;
+      smallest = b < smallest ? b : smallest;
+    }
+    if (lane == 0) {
+      s_max[wave] = largest;
+      s_min[wave] = smallest;
+    }
+    reinterpret_cast<u32x2 *>(part)[tid] = u32x2{0u, 0u};
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kWavesPerBlock; ++w) {
+      largest = s_max[w] > largest ? s_max[w] : largest;
+      smallest = s_min[w] < smallest ? s_min[w] : smallest;
+    }
+    const int differ = largest > smallest ? 64 - __builtin_clzll(largest - smallest) : 0;
+    const int shift = differ > 11 ? differ - 11 : 0;
+    const auto part_of = [&](uint64_t own) { return (uint32_t)((largest - own) >> shift); };
+    for (uint32_t i = crowd_at + tid; i < crowd_end; i += kThreads) atomicAdd(&part[part_of(other[i])], 1u);
+    __syncthreads();
+    const u32x2 p2 = reinterpret_cast<const u32x2 *>(part)[tid];
+    const uint32_t sum = (uint32_t)wave_inclusive_sum((int)(p2[0] + p2[1]));
+    if (lane == kWave - 1) s_wsum[wave] = sum;
+    if (__syncthreads_or(p2[0] > kFinishSlot || p2[1] > kFinishSlot)) {
+      sort_segment(other, ents, m, bits, fin, sh);
+      return;
+    }
+    const uint32_t at = crowd_at + sum - p2[0] - p2[1] +
+                        (uint32_t)wave_sum((int)(lane < wave ? s_wsum[lane & (kWavesPerBlock - 1)] : 0u));
+    reinterpret_cast<u32x2 *>(part)[tid] = u32x2{at, at + p2[0]};
+    __syncthreads();
+    for (uint32_t i = crowd_at + tid; i < crowd_end; i += kThreads)
+      ents[atomicAdd(&part[part_of(other[i])], 1u)] = other[i];
+    __syncthreads();
+    for (uint32_t i = crowd_at + tid; i < crowd_end; i += kThreads) {
+      const uint64_t own = ents[i];
+      const uint32_t to = part_of(own), b = to > 0u ? part[to - 1u] : crowd_at;
+      fin(b + larger_in(ents, b, part[to], own), own);
+    }
+  }
   for (uint32_t i = tid; i < m; i += kThreads) {
+    if (i >= crowd_at && i < crowd_end) continue;
     const uint64_t own = other[i];
     const uint32_t slot = slot_of(own), b = slot > 0u ? cnt[slot - 1u] : 0u;
     fin(b + larger_in(other, b, cnt[slot], own), own);
@@ -2620,7 +2684,7 @@ __device__ __forceinline__ void finish_selection(
   __shared__ SortShared sh;
   __shared__ uint32_t s_n, s_red[kWavesPerBlock], s_own[kWavesPerBlock];
   __shared__ uint64_t s_last;  // by index: the last entry of the picked bin that is selected
-  static_assert(kBinsR + 4 * kFinishCap + kFinishSlots <= kBinsF / 2 && kBinsR % 2 == 0,
+  static_assert(kBinsR + 4 * kFinishCap + 2 * kFinishSlots <= kBinsF / 2 && kBinsR % 2 == 0,
                 "the entries fit the LDS that only a failed hint uses");
   uint64_t *ents = reinterpret_cast<uint64_t *>(lds), *other = ents + kFinishCap;
   uint32_t *cnt = lds + 4 * kFinishCap;  // entries of a slot
@@ -2928,9 +2992,9 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   const Geom g = geom(n, k);
 
   // The hint: rank of the sample that safely lies below the k-th largest priority -- the sample's
-  // expected share of k plus six standard deviations and a little.  No sample when the input is
-  // small or when k is a large part of it (the lists would hold most of the input: the levels
-  // stream instead).  (Lists that hold whole ranges cannot overflow; with a sample they hold the
+  // expected share of k plus six standard deviations and a little.  No sample when the input has
+  // fewer elements than the sample or when k is a large part of it (the lists would hold most of the
+  // input: the levels stream instead).  (Lists that hold whole ranges cannot overflow; with a sample they hold the
   // candidates only, and the launches after level 0 walk a tenth of the input instead of all.)
   const int list_all = g.list_cap >= g.wave_len ? 1 : 0;
   uint32_t rank = 0;

@@ -97,3 +97,23 @@ def test_neighbours_in_the_input_that_are_neighbours_in_value(oracle, n, k):
     _check(oracle, w, k, "ascending")
     _check(oracle, w[::-1].copy(), k, "descending")
     _check(oracle, np.arange(n, dtype=np.float32), k, "0 to n - 1")
+
+
+@pytest.mark.parametrize("crowd", ["stretch", "two values", "neighbours", "two stretches"])
+@pytest.mark.parametrize("ties", [65, 1_025, 3_000])
+def test_a_crowded_slot(oracle, crowd, ties):
+    n, k = 300_007, 2_500
+    w = _values(n, ties)
+    rng = np.random.default_rng(ties)
+    top = np.float32(2) * w.max()
+    at = rng.permutation(n)[:ties]
+    if crowd == "stretch":
+        w[100_000:100_000 + ties] = top
+    elif crowd == "two values":
+        w[at] = np.where(rng.random(ties) < 0.5, top, np.float32(1.5) * top)
+    elif crowd == "neighbours":  # a few ulps apart
+        w[at] = (np.full(ties, top).view(np.uint32) + rng.integers(0, 5, ties).astype(np.uint32)).view(np.float32)
+    else:
+        w[5:5 + ties // 2] = top
+        w[n - ties // 2:] = top
+    _check(oracle, w, k, "%d %s" % (ties, crowd))
