@@ -3021,8 +3021,11 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   // Strides of 128 elements and more, and k up to n / 8, where the steps below follow; any stride, and k up to
   // n / 4, where level 1 finishes: us without and with a sample, by index / by value, 2048 of 16384 23.4 /
   // 34.3 and 18.6 / 20.2, 25000 of 200000 24.5 / 37.4 and 20.0 / 20.8, 60000 of 300000 25.2 / 41.4 and 22.2 /
-  // 21.9, 750000 of 3e6 by index 51.4 and 43.3.  (With more of the input selected the lists hold most of it.)
-  const bool ends_early = !sorted_by_value || k <= kBucketMaxK;
+  // 21.9.  (With more of the input selected the lists hold most of it.)  Level 1 finishes k up to kBucketMaxK:
+  // values beyond are sorted by radix; by index it gains nothing there, and the binned lists cost: as steps /
+  // finished, 250000 of 1e7 35.5 / 35.2, with every 166th priority at one value above the rest 35.8 / 42.2,
+  // 700000 of 7e6 45.7 / 47.8 (from the bound of the call before 37.3 / 44.8).
+  const bool ends_early = k <= kBucketMaxK;
   if ((list_all || lists_hold(per)) && strides(per) >= (ends_early ? 1 : 128) && k <= n / (ends_early ? 4 : 8) &&
       env_int("GEAR_HIP_TOPK_HINT", 1) != 0) {
     const double r = hint_rank(per);
@@ -3034,7 +3037,7 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   // Finer bins pay off in the value-order sort (small, even segments) but cost level 0 more
   // cache lines to add its counts to; the index-ordered selection takes coarse ones.
   // (Of a large selection a coarse bin would hold too many entries for level 1 to finish.)
-  const int mid_bins = (sorted_by_value ? k <= kBucketMaxK : k > kCoarseMaxK) ? kMidBins : kMidBinsCoarse;
+  const int mid_bins = k <= kBucketMaxK && (sorted_by_value || k > kCoarseMaxK) ? kMidBins : kMidBinsCoarse;
   {
     uint32_t *zero = reinterpret_cast<uint32_t *>(ws + l.zero_begin);
     const dim3 pgrid(1 + zero_blocks);
@@ -3048,9 +3051,10 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
       prep_kernel<32><<<pgrid, block, 0, st>>>(priorities, n, k, rank, list_all, mid_bins, warm, state,
                                                zero, zero_words);
   }
-  // Whether level 1 may finish: not the values of a selection that is sorted by radix.
+  // Whether level 1 may finish: no selection beyond kBucketMaxK (see above).
   const bool by_segments = sorted_by_value && k <= kBucketMaxK;
-  const bool finishes = rank != 0u && (!sorted_by_value || (by_segments && ceil_div64(k, g.blocks) <= kFinishCap / 2));
+  const bool finishes =
+      rank != 0u && ends_early && (!by_segments || ceil_div64(k, g.blocks) <= kFinishCap / 2);
   if (rank != 0u)
     level0_hinted_kernel<<<grid, block, 0, st>>>(priorities, n, state, hist0, g.wave_len,
                                                  wave_listed, lists, (int)g.list_cap, finishes ? binned : nullptr,
