@@ -1096,8 +1096,8 @@ def run_topk(args):
     return _line(n / (ms * 1e-3), "priorities/s", args, ms,
                  "topk: top %d of %d fp32 priorities (%s), ordered by %s%s" %
                  (k, n, args.topk_input, args.topk_order, ", warm calls" if args.topk_warm else ""),
-                 {"bound": "hbm", "kernel": "top-k chain (prep, level0, member_hist x2, count, "
-                                            "write" + (", segment_sort)" if by_value else ")"),
+                 {"bound": "hbm", "kernel": "top-k chain (prep, level0, member_hist, then what "
+                                            "level 1 leaves" + (", segment_sort)" if by_value else ")"),
                   "achieved": alg / (avg * 1e-3) / 1e9, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                   "frac": alg / (avg * 1e-3) / 1e9 / HBM_PEAK_GBPS, "avg_launch_ms": avg,
                   "median_launch_ms": sms[len(sms) // 2], "algorithmic_bytes": alg,

@@ -1,6 +1,7 @@
 // Top-k of fp32 priorities by radix select + ordered compaction + segmented ordering, gfx950.
 //
-// With a sample, and unless bins are crowded (masses of equal priorities) or a list overflowed, a call is
+// With a sample, for at most 131072 entries, and unless bins hold too many (masses of equal priorities) or a
+// list overflowed, a call is
 // prep, level 0, level 1 -- which writes the result (finish_selection) -- and a launch or two that find
 // nothing left to do.  Otherwise the steps are these:
 // fp32 priorities map to order-preserving uint32 keys, selected top-down in three levels: 16384
@@ -80,7 +81,7 @@ static_assert((1ll << 32 >> kLowShift) + kHintedBins <= kBins0, "every bin has a
 constexpr int kMaxSamplesPerThread = 32;
 constexpr uint32_t kNoLists = 0xffffffffu;   // hint_bin: level 0 writes no candidate lists
 constexpr uint32_t kListFull = 0xffffffffu;  // wave_listed: the wave's list overflowed, the wave reads its range instead
-constexpr int64_t kCoarseMaxK = 65536;       // index order with coarse bins up to this k
+constexpr int64_t kCoarseMaxK = 65536;       // index order with coarse bins up to this k (and beyond kBucketMaxK)
 constexpr int64_t kBucketMaxK = 131072;      // value order by buckets up to this k
 constexpr int kSortThreads = 1024;           // segment sort workgroup
 constexpr int kSmallGroup = 256;             // groups up to this size are ranked directly
