@@ -11,6 +11,9 @@
 namespace gearhip {
 
 constexpr int64_t kMaxDraws = 524288;
+// Ranges from 2^28 on take two words a draw in torch's randint (of one word, taken modulo such a range, some
+// entries would come up visibly more often): those are left to torch.
+constexpr int64_t kMaxBound = (1ll << 28) - 1;
 
 struct Philox {
   uint64_t seed, offset;
@@ -36,7 +39,7 @@ struct Philox {
     const float scale = 1.0f / 4294967296.0f, u = scale + (float)word(j) * scale;
     return u == 1.0f ? 0.0f : u;
   }
-  // in [0, range)
+  // in [0, range), range <= kMaxBound
   __device__ __forceinline__ int64_t below(uint32_t range, uint64_t j) const { return (int64_t)(word(j) % range); }
 };
 

@@ -824,6 +824,7 @@ extern "C" int gear_hip_sample_lookup_f64(const double *prefix, int64_t n, const
 }
 
 extern "C" int64_t gear_hip_draw_max(void) { return kMaxDraws; }
+extern "C" int64_t gear_hip_draw_max_bound(void) { return kMaxBound; }
 
 extern "C" int gear_hip_draw_lookup_f64(const double *prefix, int64_t n, uint64_t seed, uint64_t offset,
                                         int64_t num, const int64_t *index_table, int64_t index_offset,
@@ -860,7 +861,7 @@ extern "C" int gear_hip_draw_sort_lookup_i64(uint64_t seed, uint64_t offset, int
                                              void *stream) {
   if (num < 0 || bound <= 0) return GEAR_HIP_EINVAL;
   if (num == 0) return 0;
-  if (num > kMaxDraws || bound > 0xffffffffll) return GEAR_HIP_ERANGE;
+  if (num > kMaxDraws || bound > kMaxBound) return GEAR_HIP_ERANGE;
   const Lookup look{index_table, index_n, index_offset, lengths_table, lengths_n, sampled_out,
                     local_out, lens_out};
   int rc = check_lookup(look);

@@ -545,7 +545,7 @@ struct Staging {
 bool draws_here(const at::Generator &gen, bool weighted, int64_t range, int64_t num, const at::Device &device) {
   if (!gen.defined() || gen.device().type() != at::kCUDA || num < 1 || num > gear_hip_draw_max()) return false;
   if (gen.device().index() != (device.has_index() ? device.index() : c10::hip::current_device())) return false;
-  if (!weighted && (range < 1 || range > 0xffffffffll)) return false;
+  if (!weighted && (range < 1 || range > gear_hip_draw_max_bound())) return false;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(static_cast<hipStream_t>(current_stream()), &capture) == hipSuccess &&
          capture == hipStreamCaptureStatusNone;

@@ -50,6 +50,12 @@ def test_error_paths_without_gpu():
     assert lib.gear_hip_scan_f32_f64(None, None, -1, None, 0, None) == -1
     assert lib.gear_hip_topk_f32(None, 10, 11, 1, None, None, None, 0, None) == -1
     assert lib.gear_hip_sort_i64(None, None, None, None, 5, 70, None, 0, None) == -1
+    # batches that torch would draw in another way are not drawn here
+    draw = [0, 0, 4, 0, None, 0, 0, None, 0, None, None, None, None, 0, None]
+    for bound, code in ((0, -1), ((1 << 28) - 1, -1), (1 << 28, -3), (1 << 32, -3)):
+        draw[3] = bound  # (what is in range is refused for the missing outputs)
+        assert lib.gear_hip_draw_sort_lookup_i64(*draw) == code, bound
+    assert lib.gear_hip_draw_max_bound() == (1 << 28) - 1
     # zero-sized work succeeds without touching the device
     assert lib.gear_hip_subcopy(None, None, 0, None, None, None, 0, 0, 1, 1, 1, 0, 1, 1, None,
                                 None) == 0

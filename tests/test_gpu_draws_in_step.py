@@ -63,6 +63,23 @@ def test_draws(weighted, num):
             assert torch.equal(got[0], draws.sort().values + 5)
 
 
+@pytest.mark.parametrize("n", [(1 << 28) - 1, 1 << 28, (1 << 28) + 1])
+def test_ranges_beyond_one_word_a_draw(n):
+    """From 2^28 on torch's randint takes two words a draw."""
+    step = _loader(46, batch=8)._step
+    g = torch.Generator("cuda")
+    table, lengths = torch.arange(n, device="cuda") + 5, torch.zeros(1, dtype=torch.int64, device="cuda")
+    for num in (48, 5000):
+        g.manual_seed(num)
+        announce("draws num=%d n=%d" % (num, n))
+        got = step.run("uniform", g, None, table, 5, lengths, False, _ops()._ws, num)
+        offset = g.get_offset()
+        g.manual_seed(num)
+        want = torch.randint(0, n, (num,), generator=g, device="cuda")
+        assert torch.equal(got[0], want.sort().values + 5)
+        assert g.get_offset() == offset
+
+
 def test_uniforms_bit_for_bit():
     """The draws themselves: searched in a prefix whose entries are the draws of a call."""
     step = _loader(41, batch=8)._step
