@@ -89,6 +89,7 @@ SIGNATURES = {
                                          c_void_p]),
     "gear_hip_sort_workspace_bytes": (c_size_t, [c_i64]),
     "gear_hip_draw_max": (c_i64, []),
+    "gear_hip_draw_max_of": (c_i64, [c_int, c_int]),
     "gear_hip_draw_max_bound": (c_i64, []),
     "gear_hip_draw_lookup_f64": (c_int, [c_void_p, c_i64, c_u64, c_u64, c_i64, c_void_p, c_i64, c_void_p,
                                          c_i64, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),

@@ -3,14 +3,18 @@
 //
 // A draw of a batch is the first word of the block with counter (offset / 4, number of the draw) under the
 // seed as the key, which is how torch's GPU generator numbers the elements of one rand or randint call of up
-// to kMaxDraws elements; a call takes 4 of the generator's offset.  So a batch drawn here is the
+// to most_draws() elements; a call takes 4 of the generator's offset.  So a batch drawn here is the
 // batch that torch would have drawn from the same generator, bit for bit.
 #pragma once
 #include "common.hpp"
 
 namespace gearhip {
 
-constexpr int64_t kMaxDraws = 524288;
+// torch gives a thread to every element up to the threads that the GPU holds at once, in workgroups of 256;
+// beyond, a thread takes further words of its block.  (256 compute units of 2048 threads: 524 288.)
+inline int64_t most_draws(int64_t compute_units, int64_t threads_per_unit) {
+  return compute_units > 0 && threads_per_unit > 0 ? compute_units * (threads_per_unit / 256 * 256) : 0;
+}
 // Ranges from 2^28 on take two words a draw in torch's randint (of one word, taken modulo such a range, some
 // entries would come up visibly more often): those are left to torch.
 constexpr int64_t kMaxBound = (1ll << 28) - 1;

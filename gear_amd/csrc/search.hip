@@ -5,6 +5,7 @@
 // draw together and a batch spreads over many CUs.
 #include <math.h>
 
+#include <atomic>
 #include <type_traits>
 
 #include "philox.hpp"
@@ -823,7 +824,27 @@ extern "C" int gear_hip_sample_lookup_f64(const double *prefix, int64_t n, const
                           static_cast<char *>(workspace), w, as_stream(stream));
 }
 
-extern "C" int64_t gear_hip_draw_max(void) { return kMaxDraws; }
+extern "C" int64_t gear_hip_draw_max_of(int compute_units, int threads_per_unit) {
+  return most_draws(compute_units, threads_per_unit);
+}
+extern "C" int64_t gear_hip_draw_max(void) {
+  static std::atomic<int64_t> known[64];  // per device; 0: not asked yet
+  int dev = 0, units = 0, threads = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  const bool keep = dev < 64;
+  if (keep && known[dev].load(std::memory_order_relaxed) != 0) return known[dev].load(std::memory_order_relaxed);
+  if (hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipDeviceGetAttribute(&threads, hipDeviceAttributeMaxThreadsPerMultiProcessor, dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  const int64_t most = most_draws(units, threads);
+  if (keep) known[dev].store(most, std::memory_order_relaxed);
+  return most;
+}
 extern "C" int64_t gear_hip_draw_max_bound(void) { return kMaxBound; }
 
 extern "C" int gear_hip_draw_lookup_f64(const double *prefix, int64_t n, uint64_t seed, uint64_t offset,
@@ -834,11 +855,11 @@ extern "C" int gear_hip_draw_lookup_f64(const double *prefix, int64_t n, uint64_
   if (n < 0 || num < 0) return GEAR_HIP_EINVAL;
   if (num == 0) return 0;
   if (n == 0 || !prefix) return GEAR_HIP_EINVAL;
-  if (num > kMaxDraws) return GEAR_HIP_ERANGE;
   const Lookup look{index_table, n, index_offset, lengths_table, lengths_n, sampled_out, local_out,
                     lens_out};
   int rc = check_lookup(look);
   if (rc) return rc;
+  if (num > gear_hip_draw_max()) return GEAR_HIP_ERANGE;
   const SampleWs w = sample_ws(num);
   if (!workspace || workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(workspace) & 7))
     return GEAR_HIP_EWORKSPACE;
@@ -861,11 +882,12 @@ extern "C" int gear_hip_draw_sort_lookup_i64(uint64_t seed, uint64_t offset, int
                                              void *stream) {
   if (num < 0 || bound <= 0) return GEAR_HIP_EINVAL;
   if (num == 0) return 0;
-  if (num > kMaxDraws || bound > kMaxBound) return GEAR_HIP_ERANGE;
+  if (bound > kMaxBound) return GEAR_HIP_ERANGE;
   const Lookup look{index_table, index_n, index_offset, lengths_table, lengths_n, sampled_out,
                     local_out, lens_out};
   int rc = check_lookup(look);
   if (rc) return rc;
+  if (num > gear_hip_draw_max()) return GEAR_HIP_ERANGE;
   const SampleWs w = sample_ws(num);
   if (!workspace || workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(workspace) & 7))
     return GEAR_HIP_EWORKSPACE;

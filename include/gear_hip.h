@@ -344,10 +344,12 @@ int gear_hip_upper_bound_i64(const int64_t *prefix, int64_t n, const void *u, in
 /* gear_hip_sample_lookup_f64 for uniforms, and gear_hip_sort_lookup_i64 for integers in [0, bound), that the
  * call draws itself: the numbers that torch's GPU generator of this seed and offset gives to one rand
  * (float32) or randint (int64) call of `num` elements (Philox4x32-10; the caller advances the offset by 4).
- * num <= gear_hip_draw_max(), bound <= gear_hip_draw_max_bound() (2^28 - 1: from 2^28 on torch's randint takes
+ * num <= gear_hip_draw_max() -- as many as the current GPU holds threads at once, gear_hip_draw_max_of(its compute
+ * units, threads apiece): torch numbers the elements of larger calls in another way --, bound <= gear_hip_draw_max_bound() (2^28 - 1: from 2^28 on torch's randint takes
  * two words a draw), else GEAR_HIP_ERANGE.  They take the place of the torch.randint
  * and torch.multinomial of gear/sampler/global_sampler.py:121-199. */
 int64_t gear_hip_draw_max(void);
+int64_t gear_hip_draw_max_of(int compute_units, int threads_per_unit);
 int64_t gear_hip_draw_max_bound(void);
 int gear_hip_draw_lookup_f64(const double *prefix, int64_t n, uint64_t seed, uint64_t offset, int64_t num,
                              const int64_t *index_table, int64_t index_offset,

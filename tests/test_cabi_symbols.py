@@ -56,6 +56,9 @@ def test_error_paths_without_gpu():
         draw[3] = bound  # (what is in range is refused for the missing outputs)
         assert lib.gear_hip_draw_sort_lookup_i64(*draw) == code, bound
     assert lib.gear_hip_draw_max_bound() == (1 << 28) - 1
+    # torch's grid of 256-thread workgroups: all of a GPU, a partition of it, none
+    for units, threads, most in ((256, 2048, 524_288), (32, 2048, 65_536), (3, 2047, 5376), (0, 2048, 0)):
+        assert lib.gear_hip_draw_max_of(units, threads) == most
     # zero-sized work succeeds without touching the device
     assert lib.gear_hip_subcopy(None, None, 0, None, None, None, 0, 0, 1, 1, 1, 0, 1, 1, None,
                                 None) == 0

@@ -80,6 +80,30 @@ def test_ranges_beyond_one_word_a_draw(n):
         assert g.get_offset() == offset
 
 
+@pytest.mark.parametrize("weighted", [False, True])
+def test_more_draws_than_the_gpu_holds_threads(weighted):
+    from gear_amd import _cabi
+    props = torch.cuda.get_device_properties(0)
+    most = _cabi.load().gear_hip_draw_max()
+    assert most == props.multi_processor_count * (props.max_threads_per_multi_processor // 256) * 256
+    step = _loader(48 + weighted, batch=8)._step
+    g = torch.Generator("cuda")
+    table, lengths = _tables(1000)
+    prefix = _ops().prefix_sum(torch.rand(1000, device="cuda") + 0.01) if weighted else None
+    kind = "weighted" if weighted else "uniform"
+    for num in (most, most + 1):
+        g.manual_seed(num)
+        announce("%s draws num=%d" % (kind, num))
+        got = step.run(kind, g, prefix, table, 5, lengths, False, _ops()._ws, num)
+        offset = g.get_offset()
+        g.manual_seed(num)
+        draws = torch.rand(num, generator=g, device="cuda") if weighted else \
+            torch.randint(0, 1000, (num,), generator=g, device="cuda")
+        assert g.get_offset() == offset
+        want = step.run(kind, draws, prefix, table, 5, lengths, False, _ops()._ws)
+        assert torch.equal(got[0], want[0])
+
+
 def test_uniforms_bit_for_bit():
     """The draws themselves: searched in a prefix whose entries are the draws of a call."""
     step = _loader(41, batch=8)._step
