@@ -62,10 +62,12 @@ class UniformSampler:
                              device=self._mpu.device)
 
     # What a loader's step draws from: the generator, from which the native step takes the numbers that draw()
-    # would have got out of it, or those numbers where draw() or prepare() are not the ones of this module.
+    # would have got out of it, or those numbers where draw() or prepare() are not the ones of this module (of
+    # another class, or replaced in the class or in the sampler).
     def draws_of_a_step(self, num_indices, batch_size):
         cls = type(self)
-        if cls in (UniformSampler, WeightedSampler) and not {"draw", "prepare"} & self.__dict__.keys():
+        if _DRAWN_IN_A_STEP.get(cls) == (cls.draw, cls.prepare) and \
+                not {"draw", "prepare"} & self.__dict__.keys():
             return self._generator
         return self.draw(num_indices, batch_size)
 
@@ -150,3 +152,6 @@ class TopKSampler(UniformSampler):
         _, positions = self._topk_state.select(weights, draws.numel(), sorted_by_value=False,
                                                want_values=False)
         return "positions", positions, None
+
+
+_DRAWN_IN_A_STEP = {cls: (cls.draw, cls.prepare) for cls in (UniformSampler, WeightedSampler)}

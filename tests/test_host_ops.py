@@ -43,3 +43,30 @@ def test_a_number_of_entries_is_an_integer():
     for k in (2.0, 2.7, "2", None):
         with pytest.raises(TypeError):
             ops.topk(f, k)
+
+
+@pytest.mark.parametrize("name", ["draw", "prepare"])
+@pytest.mark.parametrize("where", ["class", "sampler", "subclass"])
+def test_replaced_draws_are_asked_for(monkeypatch, name, where):
+    """A loader's step draws by itself only where draw() and prepare() are the sampler's own."""
+    from gear_amd.mpu import ModelParallelismUnit
+    from gear_amd.sampler import UniformSampler, WeightedSampler
+    mpu = ModelParallelismUnit(device=torch.device("cpu"))
+    for cls in (UniformSampler, WeightedSampler):
+        sampler = cls(mpu)
+        assert sampler.draws_of_a_step(10, 4) is sampler._generator
+        called = []
+
+        def draw(*a, **kw):
+            called.append(a)
+            return torch.zeros(4)
+
+        with monkeypatch.context() as m:
+            if where == "sampler":
+                m.setattr(sampler, name, draw, raising=False)
+            elif where == "class":
+                m.setattr(cls, name, draw)
+            else:
+                sampler = type("Own", (cls,), {name: draw})(mpu)
+            assert isinstance(sampler.draws_of_a_step(10, 4), torch.Tensor)
+            assert len(called) == (name == "draw")
