@@ -59,6 +59,7 @@ bool one_launch(const int64_t *kin, int64_t *kout, const int64_t *vin, int64_t *
 // of them in every workgroup (20 000 in order: 12.4 us behind 4.7 for the look-up).  The look-up sees a
 // neighbour for the price of another load, so it says so, workgroup by workgroup, and stores its
 // entries where they belong if all of them say so; the sort looks at those words and ends (4.0 + 2.8 us).
+// Beyond what one launch sorts nobody looks at such words: an ordinary look-up then, and the sort.
 constexpr int kTakeBlock = 256;
 struct Taken : Src<uint64_t> {
   static constexpr bool kGuarded = true;
@@ -79,6 +80,8 @@ __global__ __launch_bounds__(kTakeBlock) void take_in_order_kernel(
   if (threadIdx.x == 0) in_order[blockIdx.x] = ordered ? 1u : 0u;
 }
 
+bool guarded(int64_t num) { return num <= radix::kRankMax || ranges::fits(num); }
+
 struct TakeWs {
   size_t sort, taken, words, total;
 };
@@ -88,7 +91,7 @@ TakeWs take_ws(int64_t num) {
   w.sort = 0;
   w.taken = align_up(sort_ws(num).total, 256);
   w.words = w.taken + align_up(n * 8, 256);
-  w.total = w.words + align_up((size_t)ceil_div64((int64_t)n, kTakeBlock) * 4, 256);
+  w.total = w.words + (guarded(num) ? align_up((size_t)ceil_div64((int64_t)n, kTakeBlock) * 4, 256) : 0);
   return w;
 }
 }  // namespace
@@ -105,15 +108,21 @@ extern "C" int gear_hip_take_sorted_i64(const int64_t *table, int64_t n, const i
   const TakeWs w = take_ws(num);
   if (!workspace || workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(workspace) & 7))
     return GEAR_HIP_EWORKSPACE;
-  const int64_t blocks = ceil_div64(num, kTakeBlock);
-  if (blocks >= 0x7fffffffll) return GEAR_HIP_ERANGE;
   char *ws = static_cast<char *>(workspace);
   hipStream_t st = as_stream(stream);
   int64_t *taken = reinterpret_cast<int64_t *>(ws + w.taken);
-  uint32_t *words = reinterpret_cast<uint32_t *>(ws + w.words);
-  take_in_order_kernel<<<dim3((unsigned)blocks), dim3(kTakeBlock), 0, st>>>(table, n, idx, num, taken, out, words);
-  GEARHIP_RETURN_IF_LAUNCH_FAILED();
-  const radix::InOrder in_order{words, (int)blocks};
+  radix::InOrder in_order;
+  if (guarded(num)) {
+    const int64_t blocks = ceil_div64(num, kTakeBlock);
+    uint32_t *words = reinterpret_cast<uint32_t *>(ws + w.words);
+    take_in_order_kernel<<<dim3((unsigned)blocks), dim3(kTakeBlock), 0, st>>>(table, n, idx, num, taken, out, words);
+    GEARHIP_RETURN_IF_LAUNCH_FAILED();
+    in_order = radix::InOrder{words, (int)blocks};
+  } else {
+    // (no entries: every index is outside, nothing is read)
+    const int rc = gear_hip_take_i64(n > 0 ? table : idx, n, idx, num, 0, taken, stream);
+    if (rc) return rc;
+  }
   if (num > radix::kRankMax && ranges::fits(num)) {
     Taken src{};
     src.keys = taken;

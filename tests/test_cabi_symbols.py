@@ -59,6 +59,12 @@ def test_error_paths_without_gpu():
     # torch's grid of 256-thread workgroups: all of a GPU, a partition of it, none
     for units, threads, most in ((256, 2048, 524_288), (32, 2048, 65_536), (3, 2047, 5376), (0, 2048, 0)):
         assert lib.gear_hip_draw_max_of(units, threads) == most
+    # beyond what one launch sorts, entries are taken and sorted without a look at their order
+    for num, words in ((4096, 16), (32_768, 128), (32_769, 0), (100_000, 0)):
+        taken = -(-num * 8 // 256) * 256
+        assert lib.gear_hip_take_sorted_workspace_bytes(num) == \
+            lib.gear_hip_sort_workspace_bytes(num) // 256 * 256 + \
+            (256 if lib.gear_hip_sort_workspace_bytes(num) % 256 else 0) + taken + -(-words * 4 // 256) * 256
     # zero-sized work succeeds without touching the device
     assert lib.gear_hip_subcopy(None, None, 0, None, None, None, 0, 0, 1, 1, 1, 0, 1, 1, None,
                                 None) == 0
