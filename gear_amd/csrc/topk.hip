@@ -1060,7 +1060,7 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
         const bool here = !found && r + c[j] >= rank;
         pb = here ? map.nb0 + (uint32_t)(tid * kPer + j) : pb;
         pk = here ? rank - r : pk;
-        if (FINISH == kFinishByIndex && here && c[j] > fin->limit) s_big = 1u;
+        if (FINISH == kFinishByIndex && rem_out && here && c[j] > fin->limit) s_big = 1u;
         found = found || here;
         r += c[j];
       }

@@ -31,6 +31,29 @@ def _check(oracle, w, k, label):
         assert none is None and np.array_equal(index.cpu().numpy(), expected)
 
 
+def _finished(state):
+    """Whether level 1 of the state's last selection wrote the result (`done` of the workspace's header)."""
+    return bool(state._ws[:256].view(torch.int32)[26].item())
+
+
+@pytest.mark.parametrize("ties,at,finished", [(100, 5_000, True), (6_000, 10_000, True)])
+def test_what_level_1_finishes_by_index(oracle, ties, at, finished):
+    """A bin that holds too many entries is in the way only where the selection ends: not at the 2k-th key, the
+    next call's bound."""
+    from gear_amd import ops
+    n, k = 600_001, 5_000
+    w = _values(n, 3)
+    order = np.argsort(-w, kind="stable")
+    w[order[at:at + ties]] = w[order[at]]
+    state = ops.TopKState()
+    dw = torch.from_numpy(w).cuda()
+    for _ in range(2):
+        announce("topk by index, %d ties at the %d-th" % (ties, at))
+        _, index = state.select(dw, k, sorted_by_value=False)
+        assert np.array_equal(index.cpu().numpy(), oracle.topk_f32(w, k, False)[1])
+        assert _finished(state) == finished
+
+
 @pytest.mark.parametrize("n,k", [(262_144, 1), (262_145, 64), (262_207, 32_768), (1_048_577, 131_072),
                                  (1_500_001, 255), (1_500_001, 65_537), (5_000_011, 100_000)])
 def test_sizes(oracle, n, k):
