@@ -286,8 +286,11 @@ Layout layout(int64_t n, int64_t k) {
   l.wave_ge = o;     o += (size_t)kMaxBlocks * kWavesPerBlock * sizeof(uint64_t);
   l.block_ge = o;    o += (size_t)kMaxBlocks * sizeof(uint64_t);
   l.lists = o;  o += align_up((size_t)(g.blocks * kWavesPerBlock * g.list_cap) * 8, 256);
-  l.binned = o; o += align_up((size_t)g.blocks * (size_t)binned_cap(g.list_cap) * 8, 256);
-  l.starts = o; o += align_up((size_t)g.blocks * kStartPitch * 2, 256);
+  l.binned = l.starts = o;  // (level 1 finishes no larger selections)
+  if (k <= kBucketMaxK) {
+    o += align_up((size_t)g.blocks * (size_t)binned_cap(g.list_cap) * 8, 256);
+    l.starts = o; o += align_up((size_t)g.blocks * kStartPitch * 2, 256);
+  }
   l.cidx = o;   o += align_up(kk * 4, 256);
   l.cand = l.cand2 = l.cseg = l.ckey = l.skey = l.sidx = l.tkey = l.tidx = l.shist = 0;
   if (k <= kBucketMaxK) {

@@ -59,6 +59,9 @@ def test_error_paths_without_gpu():
     # torch's grid of 256-thread workgroups: all of a GPU, a partition of it, none
     for units, threads, most in ((256, 2048, 524_288), (32, 2048, 65_536), (3, 2047, 5376), (0, 2048, 0)):
         assert lib.gear_hip_draw_max_of(units, threads) == most
+    # selections that the first level does not finish need no room for its lists
+    bytes_of = lib.gear_hip_topk_workspace_bytes
+    assert bytes_of(10_000_000, 131_073) < bytes_of(10_000_000, 131_072) - 10_000_000
     # beyond what one launch sorts, entries are taken and sorted without a look at their order
     for num, words in ((4096, 16), (32_768, 128), (32_769, 0), (100_000, 0)):
         taken = -(-num * 8 // 256) * 256
