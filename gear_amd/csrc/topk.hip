@@ -3057,8 +3057,11 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   }
   // Whether level 1 may finish: no selection beyond kBucketMaxK (see above).
   const bool by_segments = sorted_by_value && k <= kBucketMaxK;
-  const bool finishes =
-      rank != 0u && ends_early && (!by_segments || ceil_div64(k, g.blocks) <= kFinishCap / 2);
+  // (A workgroup's share of the output is small beside kFinishCap: k <= n / 4 with a sample, so four times a
+  // wave's 256 elements while that is a wave's range, and of more elements there are at least 129 workgroups.)
+  const bool finishes = rank != 0u && ends_early;
+  static_assert(kBucketMaxK / (kMaxBlocks / 2) <= (int64_t)kFinishCap / 4 && 4 * kStep <= (int)kFinishCap / 4,
+                "a workgroup's share of the output is at most a quarter of what it orders");
   if (rank != 0u)
     level0_hinted_kernel<<<grid, block, 0, st>>>(priorities, n, state, hist0, g.wave_len,
                                                  wave_listed, lists, (int)g.list_cap, finishes ? binned : nullptr,
