@@ -252,10 +252,19 @@ Geom geom(int64_t n, int64_t k) {
 }
 
 // The binned lists: a workgroup's candidates once more, in the order of their bins, and where every bin
-// starts in them (kStartPitch words of 16 bits a workgroup; see level0_hinted_kernel).
+// starts in them (kStartPitch words of 16 bits a workgroup; see level0_hinted_kernel).  A bin's word also says
+// whether the workgroup has met two keys in it.  Where a wave of the workgroup gave its list up the word behind
+// the bins' says so, and in place of the binned list stand a key of every bin and where the bins would start,
+// in words of 32 bits (struct Unlisted).
 constexpr int kQueueCap = 512;  // candidates per wave held in LDS by level 0; longer lists overflow
 constexpr int kStartPitch = kHintedBins + 8;
-static_assert(kWavesPerBlock * kQueueCap < 65536, "a place in a workgroup's binned list is a 16-bit word");
+constexpr uint32_t kStartMask = 0x7fffu, kTwoKeys = 0x8000u, kGaveUp = 0xffffu;
+static_assert(kWavesPerBlock * kQueueCap < (int)kStartMask, "a place in a workgroup's binned list is a word of 15 bits");
+struct Unlisted {
+  uint32_t key[kHintedBins], start[kHintedBins];  // (kTwoKeysHere in a start)
+};
+constexpr uint32_t kTwoKeysHere = 0x80000000u;
+static_assert(sizeof(Unlisted) <= 256 * kWavesPerBlock * sizeof(uint64_t), "fits the shortest binned list");
 __host__ __device__ __forceinline__ int binned_cap(int64_t list_cap) {
   return (int)(list_cap < kQueueCap ? list_cap : kQueueCap) * kWavesPerBlock;
 }
@@ -749,9 +758,11 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
     int64_t wave_len, uint32_t *__restrict__ wave_listed, uint64_t *__restrict__ lists,
     int list_cap, uint64_t *__restrict__ binned, uint16_t *__restrict__ starts) {
   __shared__ __align__(16) uint32_t h[kHintedBins];  // the bins from the hint upwards
+  __shared__ __align__(16) uint32_t a_key[kHintedBins];    // a key of every bin that has any
+  __shared__ __align__(4) uint8_t two_keys[kHintedBins];  // 1: another one was met, or may have been
   __shared__ uint64_t queue[kWavesPerBlock][kQueueCap];
   __shared__ uint32_t s_touched[kHintedBins / kWave];  // runs of 64 bins that hold a count
-  __shared__ uint32_t s_wsum[kWavesPerBlock], s_gave_up;
+  __shared__ uint32_t s_wsum[kWavesPerBlock], s_gave_up, s_mixed;
   const int tid = threadIdx.x, lane = tid & 63;
   // (the same in every lane of a wave: said so, everything that follows from it -- the wave's
   // range, the number of its steps -- stays in scalar registers and branches on it are taken by
@@ -780,8 +791,9 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
   for (int a = 0; a < kAhead; ++a) load_step(a, qa[a]);
   static_assert(kHintedBins == kThreads * 4, "one 16-byte store per thread clears the histogram");
   *reinterpret_cast<u32x4 *>(&h[tid * 4]) = u32x4{0u, 0u, 0u, 0u};
+  *reinterpret_cast<uint32_t *>(&two_keys[tid * 4]) = 0u;
   if (tid < kHintedBins / kWave) s_touched[tid] = 0u;
-  if (tid == 0) s_gave_up = 0u;
+  if (tid == 0) s_gave_up = s_mixed = 0u;
   const BinMap map = state->map;
   const float lo_f = lower_bound_float(map.a_end);
   const uint32_t bin_base = map.nb0;  // candidates' bins are counted from here
@@ -790,6 +802,7 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
   uint64_t *wq = queue[wave];
   uint32_t queued = 0;    // candidates of the wave so far, all in the queue (the same in every lane)
   bool given_up = false;  // ... until they outgrow it
+  uint32_t mass = 0u;     // ... with one key above all
   __syncthreads();
   // v: the lane's four entries of the step at offset s of the range
   auto take = [&](int s, const f4 &v) {
@@ -867,29 +880,64 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
     // wave gives its list up and counts the candidates of its whole range straight into the
     // histogram, lanes that share a bin by one atomic (the range is read again: it is in the
     // caches, and the later launches read it again anyway).
+    // Of masses of one key the queue holds many: only that key's bin may be one key, and only if the range
+    // holds no other key in it.  In a wave without such a key no bin is looked at.
+    const uint32_t some = queued != 0u ? order_key(__uint_as_float((uint32_t)(wq[lane < (int)queued ? lane : 0] >> 32))) : 0u;
+    int most = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t key = (uint32_t)__builtin_amdgcn_readlane((int)some, i * 21);
+      const int same = __popcll(wave_ballot(some == key));
+      if (same > most) {
+        most = same;
+        mass = key;
+      }
+    }
+    if (most < kWave / 4) mass = 0u;
     queued = 0;
-    if (lane == 0) s_gave_up = 1u;
+    if (lane == 0) {
+      s_gave_up = 1u;
+      if (mass == 0u) s_mixed = 1u;
+    }
+    const bool one_mass = mass != 0u;
     stream_range(p, begin, end, lane, [&](int64_t e0, const float q[4]) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const bool cand = e0 + j < end && q[j] >= lo_f;
         if (wave_ballot(cand) == 0ull) continue;
-        const uint32_t bin = counted_bin(bin_of(map, order_key(q[j])), bin_base);
+        const uint32_t key = order_key(q[j]), bin = counted_bin(bin_of(map, key), bin_base);
         count_add(h, bin, cand);
-        if (cand) s_touched[bin / kWave] = 1u;
+        if (cand) {
+          s_touched[bin / kWave] = 1u;
+          if (one_mass && key != mass) two_keys[bin] = 1u;
+        }
       }
     });
+    if (one_mass && lane == 0) a_key[counted_bin(bin_of(map, mass), bin_base)] = mass;
   }
   // the queue, in index order, becomes the wave's list and is counted
   uint64_t *list = lists + gw * list_cap;
+  uint64_t ent0 = 0ull;  // (the lane's first one and its bin, which most often are all, stay at hand)
+  uint32_t bin0 = 0u;
   for (uint32_t i = (uint32_t)lane; i < queued; i += kWave) {
     const uint64_t ent = wq[i];
     const uint32_t key = order_key(__uint_as_float((uint32_t)(ent >> 32)));
     const uint32_t bin = counted_bin(bin_of(map, key), bin_base);
+    const uint64_t own = ((uint64_t)key << 32) | (uint32_t)ent;
     atomicAdd(&h[bin], 1u);
     s_touched[bin / kWave] = 1u;
-    wq[i] = list[i] = ((uint64_t)key << 32) | (uint32_t)ent;
+    a_key[bin] = key;
+    wq[i] = list[i] = own;
+    if (i < kWave) {
+      ent0 = own;
+      bin0 = bin;
+    }
   }
+  const auto each_queued = [&](const auto &f) {
+    if ((uint32_t)lane < queued) f(ent0, bin0);
+    for (uint32_t i = (uint32_t)lane + kWave; i < queued; i += kWave)
+      f(wq[i], counted_bin(bin_of(map, (uint32_t)(wq[i] >> 32)), bin_base));
+  };
   // a wave whose list overflowed says so: the later launches read its range of the priorities
   // again, its range only
   if (lane == 0) wave_listed[gw] = given_up ? kListFull : queued;
@@ -911,32 +959,50 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
   // The candidates once more, in the order of their bins, with a table of where every bin starts:
   // whoever needs the entries of a few bins finds them in one short piece of every workgroup's list,
   // instead of walking all of them.
-  if (s_gave_up != 0u) {
-    if (tid == 0) state->gave_up = 1u;
-    return;
-  }
+  const bool gave_up = s_gave_up != 0u;
+  if (gave_up && tid == 0) state->gave_up = 1u;
   if (binned == nullptr) return;  // (nobody will ask)
   const u32x4 c4 = *reinterpret_cast<const u32x4 *>(&h[tid * 4]);
   const uint32_t sum4 = (c4[0] + c4[1]) + (c4[2] + c4[3]);
   const uint32_t inc = (uint32_t)wave_inclusive_sum((int)sum4);
   if (lane == kWave - 1) s_wsum[wave] = inc;
+  each_queued([&](uint64_t ent, uint32_t bin) {
+    if (a_key[bin] != (uint32_t)(ent >> 32)) two_keys[bin] = 1u;
+  });
+  if (mass != 0u && lane == 0) {
+    const uint32_t bin = counted_bin(bin_of(map, mass), bin_base);
+    if (a_key[bin] != mass) two_keys[bin] = 1u;
+  }
   __syncthreads();  // (and every count has been read)
   u32x4 at4;
   at4[0] = inc - sum4 + (uint32_t)wave_sum((int)(lane < wave ? s_wsum[lane & (kWavesPerBlock - 1)] : 0u));
   at4[1] = at4[0] + c4[0];
   at4[2] = at4[1] + c4[1];
   at4[3] = at4[2] + c4[2];
-  *reinterpret_cast<u32x4 *>(&h[tid * 4]) = at4;  // cursors
   uint16_t *my_starts = starts + (int64_t)blockIdx.x * kStartPitch;
-  *reinterpret_cast<u32x2 *>(my_starts + tid * 4) = u32x2{at4[0] | (at4[1] << 16), at4[2] | (at4[3] << 16)};
-  if (tid == kThreads - 1) my_starts[kHintedBins] = (uint16_t)(at4[3] + c4[3]);
-  __syncthreads();
   uint64_t *mine_binned = binned + (int64_t)blockIdx.x * binned_cap(list_cap);
-  for (uint32_t i = (uint32_t)lane; i < queued; i += kWave) {
-    const uint64_t ent = wq[i];
-    const uint32_t bin = counted_bin(bin_of(map, (uint32_t)(ent >> 32)), bin_base);
-    mine_binned[atomicAdd(&h[bin], 1u)] = ent;
+  uint32_t two4 = *reinterpret_cast<const uint32_t *>(&two_keys[tid * 4]);  // a byte a bin, 0 or 1
+  if (gave_up) {
+    if (s_mixed != 0u) two4 = 0x01010101u;
+    Unlisted *mine_unlisted = reinterpret_cast<Unlisted *>(mine_binned);
+    *reinterpret_cast<u32x4 *>(&mine_unlisted->key[tid * 4]) = *reinterpret_cast<const u32x4 *>(&a_key[tid * 4]);
+    static_assert(kTwoKeysHere == 1u << 31, "the byte's lowest bit");
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mine_unlisted->start[tid * 4 + e] = at4[e] | ((two4 >> (8 * e)) << 31);
+    if (tid == kThreads - 1) {
+      my_starts[kHintedBins] = (uint16_t)kGaveUp;
+      *reinterpret_cast<uint32_t *>(my_starts + kHintedBins + 2) = at4[3] + c4[3];
+    }
+    return;
   }
+  static_assert(kTwoKeys == 1u << 15, "the byte's lowest bit");
+  *reinterpret_cast<u32x2 *>(my_starts + tid * 4) =
+      u32x2{at4[0] | (at4[1] << 16) | ((two4 & 1u) << 15) | ((two4 & 0x100u) << 23),
+            at4[2] | (at4[3] << 16) | ((two4 & 0x10000u) >> 1) | ((two4 & 0x1000000u) << 7)};
+  if (tid == kThreads - 1) my_starts[kHintedBins] = (uint16_t)(at4[3] + c4[3]);
+  *reinterpret_cast<u32x4 *>(&h[tid * 4]) = at4;  // cursors
+  __syncthreads();
+  each_queued([&](uint64_t ent, uint32_t bin) { mine_binned[atomicAdd(&h[bin], 1u)] = ent; });
 }
 
 // Without a hint: every entry is counted in its level-0 bin (uniform bins of the top 14 key
@@ -985,12 +1051,30 @@ __global__ __launch_bounds__(kThreads) void level0_kernel(const float *__restric
 // map (load_copies) and a round trip to memory is saved.  Returns the picked bin under its number in the
 // map; boff, wg_bins and seg_shift as for pick_bin, not looked at when the launch finishes the selection
 // itself.  sums: LDS, kHintedBins words.  Every thread of the workgroup calls.
-// FINISH (see finish_selection): fin->can says on entry whether there are binned lists, and on return
-// whether the launch can finish: enough candidates, and no bin that it has to order holds too many.
+// FINISH (see finish_selection): fin->can says on return whether the launch can finish: enough candidates,
+// and no bin that it has to order holds too many, unless they all have the same key (the crowds), or is missing in
+// the binned lists because a wave gave its list up.
 enum FinishOrder { kNoFinish, kFinishByIndex, kFinishByValue };
+constexpr uint32_t kFinishCap = 4096;  // entries that a workgroup puts in order
+constexpr uint32_t kMaxCrowds = 64;
+static_assert(kBucketMaxK / (kFinishCap - kFinishCap / 4) + 2 <= kMaxCrowds && kMaxCrowds <= kWave,
+              "a lane for every bin that is crowded and selected");
+// Bins with more entries than that, counted from the hint's (by value all that are selected, by index the one of
+// the k-th key), and the entries of the workgroups before this one.
+struct Crowds {
+  uint32_t n, bin[kMaxCrowds];
+  uint32_t base[kMaxCrowds];    // by value: entries above the bin
+  uint32_t before[kMaxCrowds];  // entries of the bin in the workgroups before this one
+  uint32_t own[kMaxCrowds];     // ... in this one
+  uint32_t above, own_above;    // by index: the same for the bins above
+};
 struct Finish {
-  bool can;
+  bool can, gave_up;
+  uint32_t crowds;        // how many
   uint32_t limit;         // most entries of a bin
+  const uint16_t *starts;
+  const uint64_t *binned;
+  int list_cap;
   uint32_t lo, hi;        // by value: this workgroup's places in the output
   uint32_t at_lo, at_hi;  // ... the bins that start there, counted from the hint's
   uint32_t base, end;     // ... and the places of their entries (base == end: none)
@@ -1006,18 +1090,86 @@ __device__ __forceinline__ CopyWords load_copies(const uint32_t *hist) {
     w.q[j] = *reinterpret_cast<const u32x4 *>(hist + threadIdx.x * 4 + j * kHintedBins);
   return w;
 }
+
+// Whether every crowd is one key, by the keys that the workgroups left of it; and its entries of the workgroups
+// before this one.  All threads of the workgroup call, in all workgroups with the same answer.
+template <int FINISH>
+__device__ __forceinline__ bool one_key_each(Crowds &cr, const Finish &fin) {
+  constexpr uint32_t kParts = kMaxBlocks / kWave;  // waves that look at a bin, a lane a workgroup
+  __shared__ uint32_t s_key[kMaxCrowds][kParts], s_sum[kMaxCrowds][kParts], s_above[kParts];
+  const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1);
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / kWave));
+  const uint32_t n = cr.n, part = wave % kParts, src = part * kWave + lane;
+  const bool real = src < gridDim.x;
+  const uint16_t *row = fin.starts + (int64_t)(real ? src : 0u) * kStartPitch;
+  const uint64_t *list = fin.binned + (int64_t)(real ? src : 0u) * binned_cap(fin.list_cap);
+  const Unlisted *unlisted = reinterpret_cast<const Unlisted *>(list);
+  const bool listed = row[kHintedBins] != kGaveUp;
+  uint32_t all = row[kHintedBins];  // candidates
+  if (!listed) all = *reinterpret_cast<const uint32_t *>(row + kHintedBins + 2);
+  bool other = false;
+  for (uint32_t q = wave / kParts; q < n; q += kWavesPerBlock / kParts) {
+    const uint32_t bin = cr.bin[q];
+    uint32_t at, end, key = 0u;
+    bool two;
+    if (listed) {
+      at = row[bin] & kStartMask;
+      end = bin + 1u < (uint32_t)kHintedBins ? row[bin + 1u] & kStartMask : all;
+      two = (row[bin] & kTwoKeys) != 0u;
+      if (at < end) key = (uint32_t)(list[at] >> 32);
+    } else {
+      at = unlisted->start[bin] & ~kTwoKeysHere;
+      end = bin + 1u < (uint32_t)kHintedBins ? unlisted->start[bin + 1u] & ~kTwoKeysHere : all;
+      two = (unlisted->start[bin] & kTwoKeysHere) != 0u;
+      key = unlisted->key[bin];
+    }
+    const uint32_t cnt = real ? end - at : 0u;
+    const uint64_t has = wave_ballot(cnt != 0u);
+    const uint32_t some =
+        has != 0ull ? (uint32_t)__builtin_amdgcn_readlane((int)key, __builtin_ctzll(has)) : 0u;
+    other = other || (cnt != 0u && (two || key != some));
+    const uint32_t sum = (uint32_t)wave_sum((int)(src < blockIdx.x ? cnt : 0u));
+    if (src == blockIdx.x) cr.own[q] = cnt;
+    if (lane == 0) {
+      s_key[q][part] = some;
+      s_sum[q][part] = sum;
+    }
+    if (FINISH == kFinishByIndex) {
+      const uint32_t over = all - end;
+      const uint32_t above = (uint32_t)wave_sum((int)(src < blockIdx.x ? over : 0u));
+      if (src == blockIdx.x) cr.own_above = over;
+      if (lane == 0) s_above[part] = above;
+    }
+  }
+  __syncthreads();
+  if (tid < n) {
+    uint32_t key = 0u, sum = 0u;
+#pragma unroll
+    for (uint32_t w = 0; w < kParts; ++w) {
+      const uint32_t some = s_key[tid][w];
+      other = other || (some != 0u && key != 0u && some != key);
+      key = some != 0u ? some : key;
+      sum += s_sum[tid][w];
+    }
+    cr.before[tid] = sum;
+  }
+  if (FINISH == kFinishByIndex && tid == 0) cr.above = (s_above[0] + s_above[1]) + (s_above[2] + s_above[3]);
+  static_assert(kParts == 4, "four parts are added up");
+  return !__syncthreads_or(other);
+}
+
 template <int FINISH>
 __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &words, const BinMap &map,
                                             uint32_t rank2, uint32_t *bin2, uint32_t *sums,
                                             uint32_t *boff, uint32_t *wg_bins, int seg_shift,
-                                            Finish *fin) {
+                                            Finish *fin, Crowds &cr) {
   constexpr int kPer = 4;  // bins per thread
   static_assert(kPer * kThreads == kHintedBins, "every bin of a copy has its thread");
   __shared__ uint32_t wsum[kWavesPerBlock];
   __shared__ Pick s_pick;
   __shared__ uint32_t s_bin2;
   __shared__ uint32_t s_base[kHintedBins / kWave];  // entries above every 64th bin from the top
-  __shared__ uint32_t s_big, s_at_lo, s_at_hi, s_begin, s_end;
+  __shared__ uint32_t s_big, s_plain, s_at_lo, s_at_hi, s_begin, s_end;
   const Copies cp = copies_of(map);
   const int tid = threadIdx.x, lane = tid & 63;
   // thread t owns the bins 4t .. 4t + 3; of eight copies its words are those of every other one
@@ -1046,7 +1198,8 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
     s_pick.k_rem = k_rem;
     s_pick.found = 0u;
     s_bin2 = 0u;
-    s_big = s_at_lo = s_begin = s_end = 0u;
+    s_big = s_plain = s_at_lo = s_begin = s_end = 0u;
+    if (FINISH != kNoFinish) cr.n = 0u;
     s_at_hi = cp.used - 1u;
   }
   __syncthreads();
@@ -1103,7 +1256,42 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
   if (tid == 0) s_pick.total = total;
   __syncthreads();
   if (FINISH != kNoFinish) {
-    fin->can = fin->can && s_pick.found != 0u && s_big == 0u;
+    fin->can = s_pick.found != 0u;
+    fin->crowds = 0u;
+    if (__builtin_expect(fin->can && (s_big != 0u || fin->gave_up), 0)) {
+      if (FINISH == kFinishByIndex) {
+        if (tid == 0) {
+          cr.n = s_big;
+          cr.bin[0] = s_pick.bin - map.nb0;
+          s_plain = 1u - s_big;
+        }
+      } else {
+        const uint32_t hi = fin->hi < k_rem ? fin->hi : k_rem;
+        uint32_t r = running0;
+#pragma unroll
+        for (int j = kPer - 1; j >= 0; --j) {
+          const uint32_t next = r + c[j], bin = (uint32_t)(tid * kPer + j);
+          if (r < k_rem && c[j] > fin->limit) {
+            const uint32_t q = atomicAdd(&cr.n, 1u);
+            if (q < kMaxCrowds) {
+              cr.bin[q] = bin;
+              cr.base[q] = r;
+            }
+            if (fin->lo < hi && r < hi && next >= hi) {  // (the last bin of the stretch, or one before it)
+              s_at_lo = bin + 1u;
+              s_end = r;
+            }
+          } else if (r < k_rem && c[j] != 0u) {
+            s_plain = 1u;
+          }
+          r = next;
+        }
+      }
+      __syncthreads();
+      fin->crowds = cr.n;
+      fin->can = cr.n <= kMaxCrowds && !(fin->gave_up && s_plain != 0u);
+      if (fin->can && cr.n != 0u) fin->can = one_key_each<FINISH>(cr, *fin);
+    }
     fin->at_lo = s_at_lo;
     fin->at_hi = s_at_hi;
     fin->base = s_begin;
@@ -1255,11 +1443,11 @@ __device__ __forceinline__ int level1_shift(int bits0) { return bits0 > 11 ? bit
 // whole result itself (finish_selection) and the launches after it find that nothing is left to do.
 template <int FINISH>
 __device__ __forceinline__ void finish_selection(
-    const float *__restrict__ p, int64_t n, uint32_t k, const Finish &fin, const Pick &pick,
-    const BinMap &map, const uint16_t *__restrict__ starts, const uint64_t *__restrict__ binned,
-    int list_cap, const uint64_t *__restrict__ list, uint32_t listed, uint64_t ent_pre,
-    int64_t wave_len, uint32_t *lds, float *__restrict__ values_out, int64_t *__restrict__ indices_out);
-constexpr uint32_t kFinishCap = 4096;  // entries that a workgroup puts in order
+    const float *__restrict__ p, int64_t n, uint32_t k, const Finish &fin, const Crowds &crowds,
+    const Pick &pick, const BinMap &map, const uint16_t *__restrict__ starts,
+    const uint64_t *__restrict__ binned, int list_cap, const uint64_t *__restrict__ list, uint32_t listed,
+    uint64_t ent_pre, int64_t wave_len, uint32_t *lds, float *__restrict__ values_out,
+    int64_t *__restrict__ indices_out);
 struct FinishIo {
   const uint16_t *starts;
   const uint64_t *binned;
@@ -1306,9 +1494,13 @@ __device__ __forceinline__ Pick member_hist(
     // (the 2k-th largest key, where the histogram holds that many: the next call's hint)
     uint32_t bin2 = 0u;
     Finish fin{};
+    __shared__ Crowds crowds;
     if (FINISH != kNoFinish) {
       const uint32_t share = ((uint32_t)k + gridDim.x - 1u) / gridDim.x;
-      fin.can = state->gave_up == 0u;
+      fin.gave_up = state->gave_up != 0u;
+      fin.starts = io.starts;
+      fin.binned = io.binned;
+      fin.list_cap = list_cap;
       fin.limit = kFinishCap - (FINISH == kFinishByValue ? share : 0u);
       fin.lo = block * share;
       fin.hi = fin.lo + share;
@@ -1317,7 +1509,7 @@ __device__ __forceinline__ Pick member_hist(
     // up in the part of the LDS that only a failed hint uses, later)
     const Pick r = hinted ? pick_copies<FINISH>((uint32_t)k, FINISH != kNoFinish ? words : load_copies(hist_prev),
                                                 map, 2u * (uint32_t)k, &bin2, hp + kBinsR, boff, wg_bins,
-                                                seg_shift, &fin)
+                                                seg_shift, &fin, crowds)
                           : pick_bin<kBins0>((uint32_t)k, hist_prev, boff, wg_bins, seg_shift);
     fail = hinted && r.found == 0u;
     lo = bin_lo_key(map, r.bin);
@@ -1357,8 +1549,8 @@ __device__ __forceinline__ Pick member_hist(
       if (FINISH != kNoFinish && fin.can) state->done = 1u;
     }
     if (FINISH != kNoFinish && fin.can) {
-      finish_selection<FINISH>(p, n, (uint32_t)k, fin, r, map, io.starts, io.binned, list_cap, list, m_raw,
-                               ent_pre, wave_len, hp + kBinsR, io.values_out, io.indices_out);
+      finish_selection<FINISH>(p, n, (uint32_t)k, fin, crowds, r, map, io.starts, io.binned, list_cap, list,
+                               m_raw, ent_pre, wave_len, hp + kBinsR, io.values_out, io.indices_out);
       return picked;
     }
   } else {
@@ -2679,20 +2871,121 @@ __device__ __forceinline__ void order_entries(uint64_t *ents, uint64_t *other, u
   }
 }
 
+// The crowds: an entry's place follows from how many of its bin come before it, so every workgroup stores those
+// of its own entries, in index order -- out of the waves' lists, or out of the input where those overflowed.
+template <int FINISH>
+__device__ __forceinline__ void store_crowds(const float *__restrict__ p, int64_t n, uint32_t k,
+                                             const Crowds &cr, const Pick &pick, const BinMap &map,
+                                             const uint64_t *__restrict__ list, uint32_t listed,
+                                             uint64_t ent_pre, int64_t wave_len, uint32_t *counts,
+                                             float *__restrict__ values_out,
+                                             int64_t *__restrict__ indices_out) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  // f(bin, index, key, valid) for 64 entries at a time
+  const auto own_entries = [&](const auto &f) {
+    if (listed != kListFull) {
+      for (uint32_t c0 = 0; c0 < listed; c0 += kWave) {
+        const bool valid = c0 + lane < listed;
+        const uint64_t ent = valid ? (c0 == 0 ? ent_pre : list[c0 + lane]) : 0ull;
+        const uint32_t key = (uint32_t)(ent >> 32);
+        f(counted_bin(bin_of(map, key), map.nb0), (uint32_t)ent, key, valid);
+      }
+      return;
+    }
+    const int64_t begin = ((int64_t)blockIdx.x * kWavesPerBlock + wave) * wave_len;
+    const int64_t end = begin + wave_len < n ? begin + wave_len : n;
+    const float lo_f = lower_bound_float(map.a_end);
+    stream_rows(p, begin, end, lane, [&](int64_t i, float v, bool in) {
+      const bool valid = in && v >= lo_f;
+      if (wave_ballot(valid) == 0ull) return;
+      const uint32_t key = order_key(v);
+      f(counted_bin(bin_of(map, key), map.nb0), (uint32_t)i, key, valid);
+    });
+  };
+  const auto store = [&](uint32_t at, uint32_t index, uint32_t key) {
+    indices_out[at] = (int64_t)index;
+    if (values_out)
+      values_out[at] = key != 0x80000000u ? key_to_float(key) : ((int64_t)index < n ? p[index] : 0.0f);
+  };
+  if (FINISH == kFinishByIndex) {
+    const uint32_t at_hi = cr.bin[0], need = pick.k_rem;
+    uint32_t gt_run = cr.above, eq_run = cr.before[0];
+    if (cr.own_above == 0u && (cr.own[0] == 0u || eq_run >= need)) return;
+    uint32_t gt = 0u, eq = 0u;
+    own_entries([&](uint32_t bin, uint32_t, uint32_t, bool valid) {
+      gt += (uint32_t)__popcll(wave_ballot(valid && bin > at_hi));
+      eq += (uint32_t)__popcll(wave_ballot(valid && bin == at_hi));
+    });
+    if (lane == 0) {
+      counts[wave] = gt;
+      counts[kWavesPerBlock + wave] = eq;
+    }
+    __syncthreads();
+    gt_run += (uint32_t)wave_sum((int)(lane < wave ? counts[lane & (kWavesPerBlock - 1)] : 0u));
+    eq_run += (uint32_t)wave_sum((int)(lane < wave ? counts[kWavesPerBlock + (lane & (kWavesPerBlock - 1))] : 0u));
+    own_entries([&](uint32_t bin, uint32_t index, uint32_t key, bool valid) {
+      const bool is_gt = valid && bin > at_hi, is_eq = valid && bin == at_hi;
+      const uint64_t bg = wave_ballot(is_gt), be = wave_ballot(is_eq);
+      const uint32_t g = gt_run + (uint32_t)__popcll(bg & lt_mask);
+      const uint32_t e = eq_run + (uint32_t)__popcll(be & lt_mask);
+      const uint32_t at = g + (e < need ? e : need);
+      if ((is_gt || (is_eq && e < need)) && at < k) store(at, index, key);
+      gt_run += (uint32_t)__popcll(bg);
+      eq_run += (uint32_t)__popcll(be);
+    });
+    return;
+  }
+  // by value: lane q counts for crowd q
+  const bool mine = (uint32_t)lane < cr.n;
+  uint32_t run = mine ? cr.base[lane] + cr.before[lane] : 0u;
+  const uint64_t wanted = wave_ballot(mine && run < k && cr.own[lane] != 0u);  // (the same in every wave)
+  if (wanted == 0ull) return;
+  const auto own_crowds = [&](const auto &f) {  // f(crowd, its lanes, index, key)
+    own_entries([&](uint32_t bin, uint32_t index, uint32_t key, bool valid) {
+      for (uint64_t todo = wanted; todo != 0ull; todo &= todo - 1ull) {
+        const int q = __builtin_ctzll(todo);
+        const uint64_t lanes = wave_ballot(valid && bin == cr.bin[q]);
+        if (lanes != 0ull) f(q, lanes, index, key);
+      }
+    });
+  };
+  uint32_t count = 0u;
+  own_crowds([&](int q, uint64_t lanes, uint32_t, uint32_t) {
+    count += lane == q ? (uint32_t)__popcll(lanes) : 0u;
+  });
+  counts[wave * kWave + lane] = count;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) run += counts[w * kWave + lane];
+  own_crowds([&](int q, uint64_t lanes, uint32_t index, uint32_t key) {
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)run, q) + (uint32_t)__popcll(lanes & lt_mask);
+    if (((lanes >> lane) & 1ull) != 0ull && at < k) store(at, index, key);
+    run += lane == q ? (uint32_t)__popcll(lanes) : 0u;
+  });
+}
+
 template <int FINISH>
 __device__ __forceinline__ void finish_selection(
-    const float *__restrict__ p, int64_t n, uint32_t k, const Finish &fin, const Pick &pick,
-    const BinMap &map, const uint16_t *__restrict__ starts, const uint64_t *__restrict__ binned,
-    int list_cap, const uint64_t *__restrict__ list, uint32_t listed, uint64_t ent_pre,
-    int64_t wave_len, uint32_t *lds, float *__restrict__ values_out, int64_t *__restrict__ indices_out) {
+    const float *__restrict__ p, int64_t n, uint32_t k, const Finish &fin, const Crowds &crowds,
+    const Pick &pick, const BinMap &map, const uint16_t *__restrict__ starts,
+    const uint64_t *__restrict__ binned, int list_cap, const uint64_t *__restrict__ list, uint32_t listed,
+    uint64_t ent_pre, int64_t wave_len, uint32_t *lds, float *__restrict__ values_out,
+    int64_t *__restrict__ indices_out) {
   __shared__ SortShared sh;
   __shared__ uint32_t s_n, s_red[kWavesPerBlock], s_own[kWavesPerBlock];
   __shared__ uint64_t s_last;  // by index: the last entry of the picked bin that is selected
-  static_assert(kBinsR + 4 * kFinishCap + 2 * kFinishSlots <= kBinsF / 2 && kBinsR % 2 == 0,
+  constexpr int kCrowdCounts = 4 * kFinishCap + 2 * kFinishSlots;
+  static_assert(kBinsR + kCrowdCounts + kWavesPerBlock * kWave <= kBinsF / 2 && kBinsR % 2 == 0,
                 "the entries fit the LDS that only a failed hint uses");
   uint64_t *ents = reinterpret_cast<uint64_t *>(lds), *other = ents + kFinishCap;
   uint32_t *cnt = lds + 4 * kFinishCap;  // entries of a slot
   constexpr bool kByValue = FINISH == kFinishByValue;
+  if (__builtin_expect(fin.crowds != 0u, 0)) {
+    store_crowds<FINISH>(p, n, k, crowds, pick, map, list, listed, ent_pre, wave_len, lds + kCrowdCounts,
+                         values_out, indices_out);
+    if (!kByValue) return;
+  }
   if (kByValue && fin.base >= fin.end) return;  // no bin starts in this workgroup's stretch
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2717,8 +3010,8 @@ __device__ __forceinline__ void finish_selection(
   const bool real = src < gridDim.x;
   const uint16_t *row = starts + (real ? src : 0u) * kStartPitch;
   const uint64_t *from = binned + (int64_t)(real ? src : 0u) * binned_cap(list_cap);
-  uint32_t c = row[at_lo], end = row[at_hi + 1u];
-  const uint32_t all = kByValue ? 0u : row[kHintedBins];
+  uint32_t c = row[at_lo] & kStartMask, end = row[at_hi + 1u] & kStartMask;
+  const uint32_t all = kByValue ? 0u : row[kHintedBins];  // (no wave gave its list up)
   if (tid == 0) {
     s_n = 0u;
     s_last = 0ull;

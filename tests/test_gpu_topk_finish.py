@@ -84,11 +84,89 @@ def test_zeros_and_infinities(oracle):
     _check(oracle, w, k, "both zeros around the threshold")
 
 
+def _crowds(n, kind, rng):
+    w = _values(n, n)
+    top = np.float32(2) * w.max()
+    if kind == "equal":
+        w[:] = 1.0
+    elif kind == "equal and negative":
+        w[:] = -3.5
+    elif kind == "both zeros":
+        w = np.where(rng.random(n) < 0.5, np.float32(0.0), np.float32(-0.0))
+    elif kind == "infinite":
+        w[rng.random(n) < 0.4] = np.inf
+    elif kind == "most at the top":
+        w[rng.random(n) < 0.9] = top
+    elif kind == "the last tenth at the top":
+        w[-(n // 10):] = top
+    elif kind == "ten values":
+        w = rng.integers(0, 10, size=n).astype(np.float32)
+    elif kind == "many values":  # bins of some 4500 entries each
+        w = rng.integers(0, n // 4500 + 1, size=n).astype(np.float32)
+    elif kind == "a mass below the best":
+        w[rng.random(n) < 0.05] = top
+        w[rng.permutation(n)[:300]] = top + np.arange(300, dtype=np.float32)
+    return w
+
+
+# n: one wave's ranges as long as its list (up to 1048576) and longer ones, whose lists a mass overflows
+@pytest.mark.parametrize("kind", ["equal", "equal and negative", "both zeros", "infinite", "most at the top",
+                                  "the last tenth at the top", "ten values", "many values",
+                                  "a mass below the best"])
+@pytest.mark.parametrize("n", [20_000, 262_145, 1_048_576, 1_048_577, 3_000_017])
+def test_masses_of_equal_priorities_are_finished(oracle, n, kind):
+    """A bin that holds more entries than a workgroup orders, all of the same priority."""
+    from gear_amd import ops
+    rng = np.random.default_rng(n)
+    w = _crowds(n, kind, rng)
+    ks = {1, 255, 5_000, min(n // 4, 131_072), min(n // 8 + 1, 100_001)}
+    first = int((w == w.max()).sum())  # the largest priority's last place, and its neighbours
+    ks |= {v for v in (first - 1, first, first + 1) if 0 < v <= min(n // 4, 131_072)}
+    dw = torch.from_numpy(w).cuda()
+    for k in sorted(ks):
+        for by_value in (False, True):
+            announce("topk %s n=%d k=%d by_value=%d" % (kind, n, k, by_value))
+            _, expected = oracle.topk_f32(w, k, by_value)
+            state = ops.TopKState()
+            for _ in range(2):
+                values, index = state.select(dw, k, sorted_by_value=by_value)
+                assert np.array_equal(index.cpu().numpy(), expected), (kind, k, by_value)
+                assert np.array_equal(values.cpu().numpy().view(np.uint32), w[expected].view(np.uint32))
+            # (where lists overflow only crowds are left to place)
+            if n <= 1_048_576 or kind in ("equal", "equal and negative", "both zeros") or \
+                    kind == "most at the top" and k <= first:
+                assert _finished(state), (kind, k, by_value)
+
+
+def test_a_mass_with_neighbours_in_its_bin(oracle):
+    n, k = 1_000_003, 40_000
+    w = _values(n, 11)
+    rng = np.random.default_rng(12)
+    at = rng.permutation(n)[:k + 7_000]
+    w[at] = np.float32(100.0)
+    w[at[:50]] = np.nextafter(np.float32(100.0), np.float32(200.0))
+    _check(oracle, w, k, "47000 ties, 50 an ulp above")
+    w[at[50:90]] = np.nextafter(np.float32(100.0), np.float32(0.0))
+    _check(oracle, w, k, "and 40 an ulp below")
+
+
 def test_what_level_1_leaves_on_two_streams(oracle):
     """Selections that level 1 cannot finish, of two streams at once: neither launch has the GPU to itself."""
-    from gear_amd import ops
     n, k = 1_000_003, 50_000
     w = np.random.default_rng(8).integers(0, 50, size=n).astype(np.float32)
+    _on_two_streams(oracle, w, k)
+
+
+def test_bins_of_two_keys_on_two_streams(oracle):
+    n, k = 1_000_003, 50_000
+    rng = np.random.default_rng(9)
+    w = rng.integers(0, 50, size=n).astype(np.float32)
+    w[rng.permutation(n)[:2000]] += np.float32(1e-5)
+    _on_two_streams(oracle, w, k)
+
+
+def _on_two_streams(oracle, w, k):
+    from gear_amd import ops
     dw = torch.from_numpy(w).cuda()
     expected = [torch.from_numpy(oracle.topk_f32(w, k, bool(v))[1]).cuda() for v in (0, 1)]
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
