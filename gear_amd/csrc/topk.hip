@@ -1,9 +1,9 @@
 // Top-k of fp32 priorities by radix select + ordered compaction + segmented ordering, gfx950.
 //
-// With a sample, for at most 131072 entries, and unless bins hold too many (masses of equal priorities) or a
-// list overflowed, a call is
-// prep, level 0, level 1 -- which writes the result (finish_selection) -- and a launch or two that find
-// nothing left to do.  Otherwise the steps are these:
+// With a sample, for at most 131072 entries, and unless bins hold too many entries of different keys or a
+// list overflowed of more than masses of one key, a call is
+// prep, level 0, level 1 -- which writes the result (finish_selection, store_crowds) -- and a launch or two that
+// find nothing left to do.  Otherwise the steps are these:
 // fp32 priorities map to order-preserving uint32 keys, selected top-down in three levels: 16384
 // level-0 bins, then up to 11 and up to 10 bits inside the picked bin.  The steps of one call:
 //   prep      one workgroup draws 2048 to 32768 samples and lays out the level-0 bins around them (coarse
@@ -740,6 +740,9 @@ __device__ __forceinline__ void count_add(uint32_t *cnt, uint32_t d, bool valid)
 // histogram in memory (a sweep over all 16384 bins by every workgroup cost 4 us of a 16 us
 // launch).  A wave whose candidates outgrow the queue gives its list up (the later launches read
 // its range again) and counts the candidates of its range straight into the histogram.
+// For every bin the workgroup says whether its candidates have two keys or one, and which: for the price of a
+// store and a look at LDS per candidate (0.1 us of a launch).  A wave that gave its list up keeps to one key, that
+// of the mass which overflowed it (a look at every candidate's bin took 6 to 10 us of an ascending input).
 // Where a candidate's bin is counted: from the hint's bin upwards.  (A map laid out around NaN
 // samples -- NaN is not a valid priority -- can take an infinity for a candidate whose bin lies
 // below the hint's: whatever the result then is, the count stays inside the histogram.)
@@ -2750,9 +2753,12 @@ static_assert(kSortThreads >= kSortBins, "a thread per digit in the segment sort
 // order in LDS: no list is walked, and nothing passes between the workgroups.
 // us a call, back to back, as five to seven launches / finished by level 1 (lognormal priorities, cold):
 // 20000 of 3e6 by value 39.0 / 25.4, 65536 of 1e7 by value 49.5 / 33.2 and by index 32.8 / 31.4, 1000 of 3e5 by
-// index (with the look-up and the gather of a loader's step) 37.2 / 29.2.  What level 1 cannot finish takes
-// longer than before, for the binned lists and the hand-overs: 60000 ties above the threshold 56 / 63 by
-// value, 36 / 43 by index; all priorities equal 104 / 111, of 1e6 41 / 53, 20000 of them 30 / 40.
+// index (with the look-up and the gather of a loader's step) 37.2 / 29.2.
+// A bin that holds more than a workgroup orders is most often a mass of equal priorities -- new entries at the
+// largest one, integers --, which needs no order but the index (store_crowds): as launches / left to the launch
+// behind / finished, by index and by value: all equal 20000 30 / 40 / 29 and 34 / 44 / 32, 1e6 41 / 53 / 33 and
+// 46 / 57 / 37, 1e7 104 / 111 / 72 and 115 / 122 / 82; nine in ten of 1e6 40 / 52 / 33 and 45 / 56 / 36;
+// 65536 of 1e7 integers below 1000 37 / 45 / 31 and 60 / 68 / 44, of 1e7 with 60000 ties by value 53 / 59 / 37.
 // By value a workgroup takes the bins that start in its stretch of the output; the bin that holds the k-th
 // key is ordered whole and what lies beyond place k is not stored, so no threshold is needed.  By index
 // every workgroup takes the bin of the k-th key, finds the last entry of it that is selected, and from that
