@@ -269,7 +269,8 @@ __host__ __device__ __forceinline__ int binned_cap(int64_t list_cap) {
   return (int)(list_cap < kQueueCap ? list_cap : kQueueCap) * kWavesPerBlock;
 }
 
-constexpr int kHandWords = 3 * kMaxBlocks;  // of struct Hand
+constexpr int kBinsC = kBinsF / 128;         // sums of 128 bins
+constexpr int kHandWords = 2 * kMaxBlocks + kBinsC;  // of struct Hand
 
 struct Layout {
   size_t hist0, hist1, hist2, wg_bins, histf1, histf2, hand, boff, wave_listed, wave_ge, block_ge, lists, binned,
@@ -289,11 +290,11 @@ Layout layout(int64_t n, int64_t k) {
   l.histf1 = o; o += kBinsF * sizeof(uint32_t);  // after a failed hint: upper / lower 16 key bits
   l.histf2 = o; o += kBinsF * sizeof(uint32_t);
   l.hand = o;   o += kHandWords * sizeof(uint32_t);
+  l.block_ge = o;    o += (size_t)kMaxBlocks * sizeof(uint64_t);
   l.zero_end = o;
   l.boff = o;   o += kBins0 * sizeof(uint32_t);
   l.wave_listed = o; o += (size_t)kMaxBlocks * kWavesPerBlock * sizeof(uint32_t);
   l.wave_ge = o;     o += (size_t)kMaxBlocks * kWavesPerBlock * sizeof(uint64_t);
-  l.block_ge = o;    o += (size_t)kMaxBlocks * sizeof(uint64_t);
   l.lists = o;  o += align_up((size_t)(g.blocks * kWavesPerBlock * g.list_cap) * 8, 256);
   l.binned = l.starts = o;  // (level 1 finishes no larger selections)
   if (k <= kBucketMaxK) {
@@ -334,16 +335,19 @@ Layout layout(int64_t n, int64_t k) {
 // taken off k_rem and `found` is 0; `total` is the number of entries in the histogram.
 struct Pick {
   uint32_t bin, k_rem, found, total;
+  uint32_t in;  // entries of the bin (pick_bin and pick_wide)
 };
 // AGENT: a word that other workgroups of this launch have written
 template <bool AGENT>
 __device__ __forceinline__ uint32_t load_word(const uint32_t *p) {
   return AGENT ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *p;
 }
+// (used: bins from this one on hold nothing)
 template <int BINS, bool AGENT = false>
 __device__ __forceinline__ Pick pick_bin(uint32_t k_rem, const uint32_t *hist, uint32_t *boff,
                                          uint32_t *wg_bins = nullptr, int seg_shift = 0,
-                                         uint32_t rank2 = 0u, uint32_t *bin2 = nullptr) {
+                                         uint32_t rank2 = 0u, uint32_t *bin2 = nullptr,
+                                         int used = BINS) {
   constexpr int kPerThread = BINS / kThreads > 0 ? BINS / kThreads : 1;
   constexpr int kActive = BINS / kPerThread;  // threads that own bins
   __shared__ uint32_t wsum[kWavesPerBlock];
@@ -372,7 +376,8 @@ __device__ __forceinline__ Pick pick_bin(uint32_t k_rem, const uint32_t *hist, u
   } else {
 #pragma unroll
     for (int j = 0; j < kPerThread; ++j) {
-      c[j] = tid < kActive ? load_word<AGENT>(hist + (BINS - 1 - tid * kPerThread - j)) : 0u;
+      const int bin = BINS - 1 - tid * kPerThread - j;
+      c[j] = tid < kActive && bin < used ? load_word<AGENT>(hist + bin) : 0u;
       tsum += (int)c[j];
     }
   }
@@ -382,6 +387,7 @@ __device__ __forceinline__ Pick pick_bin(uint32_t k_rem, const uint32_t *hist, u
     s_pick.bin = 0u;
     s_pick.k_rem = k_rem;
     s_pick.found = 0u;
+    s_pick.in = 0u;
     s_bin2 = 0u;
   }
   __syncthreads();
@@ -397,13 +403,14 @@ __device__ __forceinline__ Pick pick_bin(uint32_t k_rem, const uint32_t *hist, u
   // are bound by instruction issue: 1.5 us).
   auto find = [&](uint32_t rank, uint32_t *bin_out, uint32_t *rem_out) {
     if (active && running0 < rank && running0 + (uint32_t)tsum >= rank) {
-      uint32_t r = running0, pb = 0u, pk = 0u;
+      uint32_t r = running0, pb = 0u, pk = 0u, in = 0u;
       bool found = false;
 #pragma unroll
       for (int j = 0; j < kPerThread; ++j) {
         const bool here = !found && r + c[j] >= rank;
         pb = here ? (uint32_t)(BINS - 1 - tid * kPerThread - j) : pb;
         pk = here ? rank - r : pk;
+        in = here ? c[j] : in;
         found = found || here;
         r += c[j];
       }
@@ -411,6 +418,7 @@ __device__ __forceinline__ Pick pick_bin(uint32_t k_rem, const uint32_t *hist, u
       if (rem_out) {
         *rem_out = pk;
         s_pick.found = 1u;
+        s_pick.in = in;
       }
     }
   };
@@ -1342,14 +1350,7 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
 
 // ---- when the hint fails: 65536-bin histograms over the entries below it -----------------------------
 // pick_bin for a histogram of 65536 bins in memory: every thread of the workgroup calls.
-// AGENT: other workgroups of this launch have counted in it (64 words a thread: the caches are told, instead
-// of every word being asked for past them).
-template <bool AGENT>
 __device__ __forceinline__ Pick pick_wide(uint32_t rank, const uint32_t *hist) {
-  if (AGENT) {
-    if (threadIdx.x < (unsigned)kWave) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    __syncthreads();
-  }
   constexpr int kPer = kBinsF / kThreads;  // 64 bins per thread, thread 0 the top ones
   __shared__ uint32_t wsum[kWavesPerBlock];
   __shared__ Pick s_pick;
@@ -1367,6 +1368,7 @@ __device__ __forceinline__ Pick pick_wide(uint32_t rank, const uint32_t *hist) {
     s_pick.bin = 0u;
     s_pick.k_rem = rank;
     s_pick.found = 0u;
+    s_pick.in = 0u;
   }
   __syncthreads();
   const uint32_t before =
@@ -1380,6 +1382,7 @@ __device__ __forceinline__ Pick pick_wide(uint32_t rank, const uint32_t *hist) {
         s_pick.bin = (uint32_t)(kBinsF - (tid + 1) * kPer + j);
         s_pick.k_rem = rank - r;
         s_pick.found = 1u;
+        s_pick.in = c;
         break;
       }
       r += c;
@@ -1388,6 +1391,55 @@ __device__ __forceinline__ Pick pick_wide(uint32_t rank, const uint32_t *hist) {
   if (tid == kThreads - 1) s_pick.total = running0 + tsum;
   __syncthreads();
   return s_pick;
+}
+
+// The same where other workgroups of this launch count in it: by way of the sums of 128 bins, since words that
+// are asked for past the caches are few, and acquiring all 65536 cost 10 us in the workgroups of an L2 together.
+// `total` is what the sums say, or nothing that can be while the bins of the picked sum lag behind it.
+__device__ __forceinline__ Pick pick_wide_shared(uint32_t rank, const uint32_t *hist, const uint32_t *sums) {
+  static_assert(kBinsC == kWave * 8 && kBinsF / kBinsC == 2 * kWave, "eight waves a sum each, two for its bins");
+  __shared__ uint32_t wsum[8], wsum2[2];
+  __shared__ uint32_t s_group, s_group_rank, s_group_sum;
+  __shared__ Pick s_pick;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (tid == 0) {
+    s_group = 0u;
+    s_group_rank = rank;
+    s_group_sum = 0u;
+    s_pick = Pick{0u, rank, 0u, 0u, 0u};
+  }
+  const uint32_t c = tid < kBinsC ? load_word<true>(&sums[kBinsC - 1 - tid]) : 0u;
+  uint32_t inc = (uint32_t)wave_inclusive_sum((int)c);
+  if (lane == kWave - 1 && wave < 8) wsum[wave] = inc;
+  __syncthreads();
+  const uint32_t part = lane < 8 ? wsum[lane] : 0u;
+  const uint32_t total = (uint32_t)wave_sum((int)part);
+  inc += (uint32_t)wave_sum((int)(lane < wave ? part : 0u));
+  if (tid < kBinsC && inc >= rank && inc - c < rank) {  // one thread
+    s_group = (uint32_t)(kBinsC - 1 - tid);
+    s_group_rank = rank - (inc - c);
+    s_group_sum = c;
+  }
+  __syncthreads();
+  constexpr int kPer = kBinsF / kBinsC;
+  const uint32_t group = s_group, group_rank = s_group_rank, group_sum = s_group_sum;
+  const int bin = (int)group * kPer + kPer - 1 - tid;
+  const uint32_t b = tid < kPer ? load_word<true>(&hist[bin]) : 0u;
+  uint32_t up_to = (uint32_t)wave_inclusive_sum((int)b);
+  if (lane == kWave - 1 && wave < 2) wsum2[wave] = up_to;
+  __syncthreads();
+  const uint32_t in_group = wsum2[0] + wsum2[1];
+  if (wave == 1) up_to += wsum2[0];
+  if (tid < kPer && group_sum != 0u && up_to >= group_rank && up_to - b < group_rank) {
+    s_pick.bin = (uint32_t)bin;
+    s_pick.k_rem = group_rank - (up_to - b);
+    s_pick.found = 1u;
+    s_pick.in = b;
+  }
+  __syncthreads();
+  Pick r = s_pick;
+  r.total = in_group == group_sum ? total : 0xffffffffu;
+  return r;
 }
 
 // Every wave streams its range and counts digit(q) for the entries that member(q) takes, in a
@@ -1399,7 +1451,7 @@ static_assert(kFlushSteps * kStep * kWavesPerBlock < 65536, "a 16-bit counter ho
 template <typename F>
 __device__ __forceinline__ void wide_hist(const float *__restrict__ p, int64_t n, int64_t wave_len,
                                           int64_t gw, uint32_t *hp, uint32_t *__restrict__ hist_out,
-                                          F digit_of) {
+                                          uint32_t *__restrict__ sums_out, F digit_of) {
   const int tid = threadIdx.x, lane = tid & 63;
   for (int i = tid; i < kBinsF / 2; i += kThreads) hp[i] = 0u;
   __syncthreads();
@@ -1417,12 +1469,17 @@ __device__ __forceinline__ void wide_hist(const float *__restrict__ p, int64_t n
       }
     });
     __syncthreads();
+#pragma unroll 1
     for (int i = tid; i < kBinsF / 2; i += kThreads) {
       const uint32_t w = hp[i];
       if (w != 0u) {
         if (w & 0xffffu) atomicAdd(&hist_out[2 * i], w & 0xffffu);
         if (w >> 16) atomicAdd(&hist_out[2 * i + 1], w >> 16);
         hp[i] = 0u;
+      }
+      if (sums_out != nullptr) {  // (a wave's words are 128 bins)
+        const uint32_t sum = (uint32_t)wave_sum((int)((w & 0xffffu) + (w >> 16)));
+        if (lane == 0 && sum != 0u) atomicAdd(&sums_out[i / kWave], sum);
       }
     }
     __syncthreads();
@@ -1459,10 +1516,11 @@ struct FinishIo {
 };
 
 // (block: the workgroup whose part this is; hp: LDS, kBinsF / 2 words, packed counters after a failed hint;
-// else h, below.  Returns level 2's pick.)
-template <int LEVEL, int FINISH>
+// else h, below.  ours(), called by all threads: a barrier, and whether anything is to be added to the
+// histograms in memory.  Returns level 2's pick.)
+template <int LEVEL, int FINISH, typename Ours>
 __device__ __forceinline__ Pick member_hist(
-    uint32_t block, uint32_t *hp, const float *__restrict__ p, int64_t n, int64_t k, int mid_bins,
+    uint32_t block, const Ours &ours, uint32_t *histf_sums, uint32_t *hp, const float *__restrict__ p, int64_t n, int64_t k, int mid_bins,
     State *state, const uint32_t *hist_prev, uint32_t *__restrict__ hist_out, const uint32_t *histf_prev,
     uint32_t *__restrict__ histf_out, uint32_t *boff, uint32_t *wg_bins, int seg_shift,
     int64_t wave_len, const uint32_t *__restrict__ wave_listed,
@@ -1471,7 +1529,7 @@ __device__ __forceinline__ Pick member_hist(
   uint32_t *h = hp;
   static_assert(kBinsR + kHintedBins <= kBinsF / 2,
                 "the level's histogram and the sums of the level-0 copies fit the same LDS");
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   for (int i = tid; i < kBinsR; i += kThreads) h[i] = 0u;
   // the wave's list does not depend on the pick: its length and first stretch are asked for
   // before the histogram is walked (used only when the lists are in use)
@@ -1565,7 +1623,7 @@ __device__ __forceinline__ Pick member_hist(
     if (!fail) {
       r = pick_bin<kBinsR>(k_rem0, hist_prev, nullptr);
     } else {
-      r = pick_wide<false>(k_rem0, histf_prev);
+      r = pick_wide(k_rem0, histf_prev);
       upper16 = r.bin;
     }
     const int shift1 = level1_shift(bits_of(hi0 - lo0));
@@ -1584,13 +1642,14 @@ __device__ __forceinline__ Pick member_hist(
   if (fail) {
     // the entries below the hint: exactly the ones level 0 did not take for candidates
     const float lo_f = lower_bound_float(a_end);
+    if (!ours()) return picked;
     if (LEVEL == 1) {
-      wide_hist(p, n, wave_len, gw, hp, histf_out, [&](float q, uint32_t *d) {
+      wide_hist(p, n, wave_len, gw, hp, histf_out, nullptr, [&](float q, uint32_t *d) {
         *d = order_key(q) >> 16;
         return q < lo_f;
       });
     } else {
-      wide_hist(p, n, wave_len, gw, hp, histf_out, [&](float q, uint32_t *d) {
+      wide_hist(p, n, wave_len, gw, hp, histf_out, histf_sums, [&](float q, uint32_t *d) {
         const uint32_t key = order_key(q);
         *d = key & 0xffffu;
         return q < lo_f && (key >> 16) == upper16;
@@ -1625,11 +1684,17 @@ __device__ __forceinline__ Pick member_hist(
       }
     });
   }
-  __syncthreads();
+  if (!ours()) return picked;
   for (int i = tid; i < kBinsR; i += kThreads)
     if (h[i]) atomicAdd(&hist_out[i], h[i]);
   return picked;
 }
+struct AlwaysOurs {
+  __device__ __forceinline__ bool operator()() const {
+    __syncthreads();
+    return true;
+  }
+};
 
 template <int LEVEL, int FINISH>
 __global__ __launch_bounds__(kThreads) void member_hist_kernel(
@@ -1639,23 +1704,24 @@ __global__ __launch_bounds__(kThreads) void member_hist_kernel(
     int64_t wave_len, const uint32_t *__restrict__ wave_listed,
     const uint64_t *__restrict__ lists, int list_cap, FinishIo io) {
   __shared__ __align__(16) uint32_t hp[kBinsF / 2];
-  member_hist<LEVEL, FINISH>(blockIdx.x, hp, p, n, k, mid_bins, state, hist_prev, hist_out, histf_prev,
+  member_hist<LEVEL, FINISH>(blockIdx.x, AlwaysOurs{}, nullptr, hp, p, n, k, mid_bins, state, hist_prev, hist_out, histf_prev,
                              histf_out, boff, wg_bins, seg_shift, wave_len, wave_listed, lists, list_cap, io);
 }
 
 // ---- count: threshold, then (greater, equal) per wave and workgroup ---------------------------------
 // Packed counts: greater << 32 | equal.  When the levels before streamed the priorities, this
 // launch does too and lists every wave's entries at or above the threshold on the way.
-// AGENT: level 2 ran in this launch, pick1 is its pick and the counts are handed on inside it.  Returns the
-// threshold key as `bin`.
+// AGENT: level 2 ran in this launch, pick1 and pick2 are its pick and the last digit's, and the counts are handed
+// on inside it, as words that say of themselves that they are there.  Returns the threshold key as `bin`.
+constexpr uint64_t kCounted = 1ull << 63;
 template <bool AGENT>
 __device__ __forceinline__ Pick count_entries(
-    uint32_t block, const Pick &pick1, const float *__restrict__ p, int64_t n, State *state, const uint32_t *hist2,
+    uint32_t block, const Pick &pick1, const Pick &pick2, const float *__restrict__ p, int64_t n, State *state, const uint32_t *hist2,
     const uint32_t *histf2, int64_t wave_len, uint32_t *__restrict__ wave_listed,
     uint64_t *__restrict__ lists, int list_cap, uint64_t *__restrict__ wave_ge,
     uint64_t *__restrict__ block_ge) {
   __shared__ uint64_t red[kWavesPerBlock];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t gw = (int64_t)block * kWavesPerBlock + wave;
   uint64_t *list = lists + gw * list_cap;
   // (the same word in every lane: said so, the branches on it are taken by whole waves)
@@ -1667,10 +1733,12 @@ __device__ __forceinline__ Pick count_entries(
   const bool fail = state->fail != 0u;  // digit1: the upper 16 bits, histf2: the lower ones
   const uint32_t k_rem1 = AGENT ? pick1.k_rem : state->k_rem[1];
   Pick r;
-  if (!fail)
-    r = pick_bin<kBinsR, AGENT>(k_rem1, hist2, nullptr);
+  if (AGENT)
+    r = pick2;
+  else if (!fail)
+    r = pick_bin<kBinsR>(k_rem1, hist2, nullptr);
   else
-    r = pick_wide<AGENT>(k_rem1, histf2);
+    r = pick_wide(k_rem1, histf2);
   const uint32_t thr = fail ? ((digit1 << 16) | r.bin)
                             : lo0 + (digit1 << level1_shift(bits_of(hi0 - lo0))) + r.bin;
   if (block == 0u && tid == 0) {
@@ -1721,7 +1789,7 @@ __device__ __forceinline__ Pick count_entries(
 #pragma unroll
     for (int i = 0; i < kWavesPerBlock; ++i) t += red[i];
     if (AGENT)
-      store_agent(&block_ge[block], t);
+      store_agent(&block_ge[block], t | kCounted);
     else
       block_ge[block] = t;
   }
@@ -1733,7 +1801,7 @@ __global__ __launch_bounds__(kThreads) void count_kernel(
     const uint32_t *histf2, int64_t wave_len, uint32_t *__restrict__ wave_listed,
     uint64_t *__restrict__ lists, int list_cap, uint64_t *__restrict__ wave_ge,
     uint64_t *__restrict__ block_ge) {
-  count_entries<false>(blockIdx.x, Pick{}, p, n, state, hist2, histf2, wave_len, wave_listed, lists, list_cap, wave_ge,
+  count_entries<false>(blockIdx.x, Pick{}, Pick{}, p, n, state, hist2, histf2, wave_len, wave_listed, lists, list_cap, wave_ge,
                 block_ge);
 }
 
@@ -1754,7 +1822,7 @@ __device__ __forceinline__ void write_entries(
     int seg_shift, uint8_t *__restrict__ cseg, float *__restrict__ values_out,
     int64_t *__restrict__ indices_out) {
   __shared__ uint64_t red[kWavesPerBlock];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t gw = (int64_t)block * kWavesPerBlock + wave;
   const uint64_t *list = lists + gw * list_cap;
   // (the same word in every lane: said so, the branch on it is taken by whole waves)
@@ -1771,7 +1839,14 @@ __device__ __forceinline__ void write_entries(
   // counts of the workgroups before this one (at most kMaxBlocks), then of the waves before
   // this one in its own workgroup
   uint64_t part = 0;
-  if (tid < (int)block) part = AGENT ? load_agent(&block_ge[tid]) : block_ge[tid];
+  if (tid < (int)block) {
+    part = AGENT ? load_agent(&block_ge[tid]) : block_ge[tid];
+    while (AGENT && (part & kCounted) == 0ull) {  // (every task is claimed: a running workgroup is at it)
+      __builtin_amdgcn_s_sleep(1);
+      part = load_agent(&block_ge[tid]);
+    }
+    part &= ~kCounted;
+  }
   const int64_t pw = wave_sum((int64_t)part);
   if (lane == 0) red[wave] = (uint64_t)pw;
   __syncthreads();
@@ -3144,25 +3219,33 @@ __device__ __forceinline__ void finish_selection(
 // What passes between workgroups are counts in agent-scope words; lists and counts of a task stay with the
 // workgroup that claimed it.  (A release and an acquire of everything a workgroup wrote and may read take 4.5
 // us each with 31 workgroups at one L2, the hand-over without them 2.2: no more than another launch.)
-constexpr int kHandOvers = 2;  // level 2 -> count -> write
+// us a call, 65536 of 1e7 by index and by value, as separate launches / so, without and with the words below:
+// a sample that misleads 86 / 97 / 85 and 434 / 437 / 426, ascending 75 / 80 / 77 and 93 / 98 / 95, half of it a
+// stretch of neighbours 63 / 68 / 65 and 99 / 104 / 101, 60000 ties and others in their bin by value 153 / 160 / 158.
+// Words that say of themselves that they are complete save the flag beside them and a round trip: the counts of
+// a workgroup carry a bit, and the histogram of level 2 is complete when it adds up to what level 1 counted in
+// the picked digit.  That alone is not waited for -- an input that changes while it is read counts otherwise --:
+// after a few looks the flags decide.
 struct Hand {
-  uint32_t claimed[kMaxBlocks], done[kHandOvers][kMaxBlocks];  // zeroed by prep
+  uint32_t claimed[kMaxBlocks], done[kMaxBlocks], histf_sums[kBinsC];  // zeroed by prep
 };
 static_assert(sizeof(Hand) == kHandWords * sizeof(uint32_t), "as the workspace is laid out");
 
-// Says that this workgroup's tasks of a phase are done and waits for everybody's; with `steal` it looks for a
-// task that nobody has claimed when the wait gets long, and returns its number (kNone otherwise).  What the
-// tasks hand on are agent-scope accesses, complete once they are waited for.
+// Says that level 2 is done for this workgroup's tasks: what they hand on are agent-scope accesses, complete once
+// they are waited for.
+__device__ __forceinline__ void tell_done(uint32_t *done, const uint8_t *mine, uint32_t from, uint32_t count) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  for (uint32_t i = from + threadIdx.x; i < count; i += kThreads)
+    __hip_atomic_store(&done[mine[i]], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Waits until all tasks are done; looks for a task that nobody has claimed when the wait gets long, and returns
+// its number (kNone otherwise).
 constexpr uint32_t kNone = 0xffffffffu;
-__device__ __forceinline__ uint32_t hand_over(const uint32_t *claimed, uint32_t *done, uint32_t tasks,
-                                              const uint8_t *mine, uint32_t from, uint32_t count, bool steal) {
+__device__ __forceinline__ uint32_t wait_done(const uint32_t *claimed, const uint32_t *done, uint32_t tasks) {
   __shared__ uint32_t s_free;
   constexpr int kPolls = 64;
   const uint32_t tid = threadIdx.x;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  for (uint32_t i = from + tid; i < count; i += kThreads)
-    __hip_atomic_store(&done[mine[i]], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (;;) {
     if (tid == 0) s_free = kNone;
     bool missing = tid < tasks;
@@ -3171,7 +3254,6 @@ __device__ __forceinline__ uint32_t hand_over(const uint32_t *claimed, uint32_t 
       if (missing) __builtin_amdgcn_s_sleep(1);
     }
     if (!__syncthreads_or(missing)) return kNone;
-    if (!steal) continue;
     if (missing && load_word<true>(&claimed[tid]) == 0u) atomicMin(&s_free, tid);
     __syncthreads();
     const uint32_t free = s_free;
@@ -3196,6 +3278,7 @@ struct Rest {
   uint8_t *cseg;
   float *values_out;
   int64_t *indices_out;
+  int looks;  // at the histogram of level 2 before the flags decide
 };
 template <bool BY_VALUE>
 __global__ __launch_bounds__(kThreads) void rest_kernel(Rest r) {
@@ -3203,40 +3286,60 @@ __global__ __launch_bounds__(kThreads) void rest_kernel(Rest r) {
   __shared__ uint8_t mine[kMaxBlocks];
   __shared__ uint32_t s_claimed;
   static_assert(kMaxBlocks <= 256, "a task's number is a byte");
+  const uint32_t tid = threadIdx.x;
+  const uint32_t done = r.state->done, fail = r.state->fail, span = r.state->hi0 - r.state->lo0;
+  if (done != 0u) return;
   uint32_t taken = 1u;
-  if (threadIdx.x == 0) taken = atomicExch(&r.hand->claimed[blockIdx.x], 1u);  // (on its way meanwhile)
-  if (r.state->done != 0u) return;
-  Pick pick{};  // (the same whatever the task)
-  uint32_t count = 0u, told = 0u;
+  if (tid == 0) taken = atomicExch(&r.hand->claimed[blockIdx.x], 1u);  // (looked at when the counting is done)
+  Pick pick1{}, pick2{};  // (the same whatever the task)
+  uint32_t count = 0u;
+  // the last digit; what its bins hold comes from everybody
+  const auto last_digit = [&]() {
+    return fail == 0u ? pick_bin<kBinsR, true>(pick1.k_rem, r.hist2, nullptr, nullptr, 0, 0u, nullptr,
+                                               1 << level1_shift(bits_of(span)))
+                      : pick_wide_shared(pick1.k_rem, r.histf2, r.hand->histf_sums);
+  };
   for (uint32_t next = blockIdx.x; next != kNone;) {
-    if (threadIdx.x == 0) {
-      s_claimed = taken == 0u ? 1u : 0u;
-      mine[count] = (uint8_t)next;
+    const auto ours = [&]() {
+      if (tid == 0) {
+        s_claimed = taken == 0u ? 1u : 0u;
+        mine[count] = (uint8_t)next;
+      }
+      __syncthreads();
+      return s_claimed != 0u;
+    };
+    pick1 = member_hist<2, kNoFinish>(next, ours, r.hand->histf_sums, hp, r.p, r.n, r.k, 0, r.state, r.hist1, r.hist2,
+                                      r.histf1, r.histf2, nullptr, nullptr, 0, r.wave_len, r.wave_listed,
+                                      r.lists, r.list_cap, FinishIo{});
+    const uint32_t told = count;
+    count += s_claimed;
+    if (count == 0u) return;  // others have this workgroup's task
+    bool complete = false;
+#pragma unroll 1
+    for (int look = 0; look < r.looks && !complete; ++look) {
+      const bool unclaimed = tid < gridDim.x && load_word<true>(&r.hand->claimed[tid]) == 0u;
+      pick2 = last_digit();
+      complete = !__syncthreads_or(unclaimed) && pick2.total == pick1.in;
     }
-    __syncthreads();
-    if (s_claimed != 0u) {
-      pick = member_hist<2, kNoFinish>(next, hp, r.p, r.n, r.k, 0, r.state, r.hist1, r.hist2, r.histf1, r.histf2,
-                                       nullptr, nullptr, 0, r.wave_len, r.wave_listed, r.lists, r.list_cap,
-                                       FinishIo{});
-      ++count;
-    }
-    next = hand_over(r.hand->claimed, r.hand->done[0], gridDim.x, mine, told, count, true);
-    told = count;
-    if (next != kNone && threadIdx.x == 0) taken = atomicExch(&r.hand->claimed[next], 1u);
+    tell_done(r.hand->done, mine, told, count);
+    if (complete) break;
+    next = wait_done(r.hand->claimed, r.hand->done, gridDim.x);
+    if (next == kNone)
+      pick2 = last_digit();
+    else if (tid == 0)
+      taken = atomicExch(&r.hand->claimed[next], 1u);
   }
-  if (count == 0u) return;  // others have this workgroup's task
-  Pick pick2{};
+  const uint32_t last = pick2.bin;
   for (uint32_t i = 0; i < count; ++i) {
-    pick2 = count_entries<true>(mine[i], pick, r.p, r.n, r.state, r.hist2, r.histf2, r.wave_len, r.wave_listed,
-                                r.lists, r.list_cap, r.wave_ge, r.block_ge);
     __syncthreads();
+    pick2 = count_entries<true>(mine[i], pick1, Pick{last, pick2.k_rem, 0u, 0u, 0u}, r.p, r.n, r.state, r.hist2,
+                                r.histf2, r.wave_len, r.wave_listed, r.lists, r.list_cap, r.wave_ge, r.block_ge);
   }
-  hand_over(r.hand->claimed, r.hand->done[1], gridDim.x, mine, 0u, count, false);
   for (uint32_t i = 0; i < count; ++i) {
+    __syncthreads();
     write_entries<BY_VALUE ? kBucket : kDirect, true>(
         mine[i], pick2, r.p, r.n, r.k, r.state, r.wave_len, r.wave_listed, r.lists, r.list_cap, r.wave_ge, r.block_ge,
         r.ckey, r.cidx, r.boff, r.seg_shift, r.cseg, r.values_out, r.indices_out);
-    __syncthreads();
   }
 }
 
@@ -3386,7 +3489,7 @@ int topk_launch(const float *priorities, int64_t n, int64_t k, int sorted_by_val
   if (finishes) {
     const Rest rest{priorities, n, k, state, reinterpret_cast<Hand *>(ws + l.hand), hist1, hist2, histf1, histf2,
                     g.wave_len, wave_listed, lists, (int)g.list_cap, wave_ge, block_ge, ckey, cidx, boff,
-                    seg_shift, cseg, values_out, indices_out};
+                    seg_shift, cseg, values_out, indices_out, env_int("GEAR_HIP_TOPK_LOOKS", 8)};
     if (sorted_by_value) {
       level1(std::integral_constant<int, kFinishByValue>{});
       rest_kernel<true><<<grid, block, 0, st>>>(rest);

@@ -165,6 +165,24 @@ def test_bins_of_two_keys_on_two_streams(oracle):
     _on_two_streams(oracle, w, k)
 
 
+@pytest.mark.parametrize("looks", ["0", "1", "8"])
+def test_what_level_1_leaves_whatever_says_that_it_is_complete(oracle, monkeypatch, looks):
+    """Level 2's histogram that adds up, or the flags of the workgroups; after a sample that misleads too."""
+    monkeypatch.setenv("GEAR_HIP_TOPK_LOOKS", looks)
+    rng = np.random.default_rng(10)
+    n, k = 1_500_007, 20_000
+    w = _values(n, 13)
+    w[rng.random(n) < 0.04] = np.float32(7.0)
+    w[rng.permutation(n)[:500]] = np.nextafter(np.float32(7.0), np.float32(8.0))
+    _check(oracle, w, k, "two keys a bin, %s looks" % looks)
+    s = np.arange(2048, dtype=np.uint64)
+    stride = np.uint64(n // 2048)
+    at = s * stride + (((s * np.uint64(2654435761)) & np.uint64(0xffffffff)) * stride >> np.uint64(32))
+    w = _values(n, 14)
+    w[at.astype(np.int64)] = 1000.0 + np.arange(2048, dtype=np.float32)
+    _check(oracle, w, k, "a sample of the largest, %s looks" % looks)
+
+
 def _on_two_streams(oracle, w, k):
     from gear_amd import ops
     dw = torch.from_numpy(w).cuda()
