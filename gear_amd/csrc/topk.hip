@@ -191,7 +191,7 @@ struct State {
   uint64_t next_magic;
   uint32_t next_a_end, next_b_last;
   uint32_t low_seg;  // after a failed hint, value order: the segment of the entries below the hint
-  uint32_t gave_up;  // level 0: a wave gave its list up, so there are no binned lists
+  uint32_t gave_up;  // level 0: a wave gave its list up, so there are no binned lists (2: for more than one mass)
   uint32_t done;     // level 1 has written the result: nothing is left to do
   uint32_t pad[37];
 };
@@ -769,8 +769,10 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
     int64_t wave_len, uint32_t *__restrict__ wave_listed, uint64_t *__restrict__ lists,
     int list_cap, uint64_t *__restrict__ binned, uint16_t *__restrict__ starts) {
   __shared__ __align__(16) uint32_t h[kHintedBins];  // the bins from the hint upwards
-  __shared__ __align__(16) uint32_t a_key[kHintedBins];    // a key of every bin that has any
-  __shared__ __align__(4) uint8_t two_keys[kHintedBins];  // 1: another one was met, or may have been
+  // a key of every bin that has any, kNoKey where another one was met; and where a mass met one
+  __shared__ __align__(16) uint32_t a_key[kHintedBins];
+  __shared__ __align__(4) uint8_t two_keys[kHintedBins];
+  constexpr uint32_t kNoKey = 0xffffffffu;  // (that of a NaN)
   __shared__ uint64_t queue[kWavesPerBlock][kQueueCap];
   __shared__ uint32_t s_touched[kHintedBins / kWave];  // runs of 64 bins that hold a count
   __shared__ uint32_t s_wsum[kWavesPerBlock], s_gave_up, s_mixed;
@@ -891,40 +893,54 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
     // wave gives its list up and counts the candidates of its whole range straight into the
     // histogram, lanes that share a bin by one atomic (the range is read again: it is in the
     // caches, and the later launches read it again anyway).
-    // Of masses of one key the queue holds many: only that key's bin may be one key, and only if the range
-    // holds no other key in it.  In a wave without such a key no bin is looked at.
-    const uint32_t some = queued != 0u ? order_key(__uint_as_float((uint32_t)(wq[lane < (int)queued ? lane : 0] >> 32))) : 0u;
-    int most = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t key = (uint32_t)__builtin_amdgcn_readlane((int)some, i * 21);
-      const int same = __popcll(wave_ballot(some == key));
-      if (same > most) {
-        most = same;
-        mass = key;
-      }
+    // Of a mass of one key the queue holds many: only that key's bin may be one key, and only if the range
+    // holds no other key in it.  A wave without such a key leaves the selection to the launch behind level 1.
+    if (queued != 0u) {
+      const uint32_t some = order_key(__uint_as_float((uint32_t)(wq[lane < (int)queued ? lane : 0] >> 32)));
+      const uint32_t key0 = (uint32_t)__builtin_amdgcn_readlane((int)some, 0);
+      const uint32_t key1 = (uint32_t)__builtin_amdgcn_readlane((int)some, kWave / 2);
+      const int same0 = __popcll(wave_ballot(some == key0)), same1 = __popcll(wave_ballot(some == key1));
+      if (same0 >= kWave / 4 || same1 >= kWave / 4) mass = same0 >= same1 ? key0 : key1;
     }
-    if (most < kWave / 4) mass = 0u;
     queued = 0;
     if (lane == 0) {
       s_gave_up = 1u;
       if (mass == 0u) s_mixed = 1u;
     }
-    const bool one_mass = mass != 0u;
-    stream_range(p, begin, end, lane, [&](int64_t e0, const float q[4]) {
+    if (mass != 0u) {
+      uint32_t many = 0u;
+      stream_range(p, begin, end, lane, [&](int64_t e0, const float q[4]) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const bool cand = e0 + j < end && q[j] >= lo_f;
-        if (wave_ballot(cand) == 0ull) continue;
-        const uint32_t key = order_key(q[j]), bin = counted_bin(bin_of(map, key), bin_base);
-        count_add(h, bin, cand);
-        if (cand) {
-          s_touched[bin / kWave] = 1u;
-          if (one_mass && key != mass) two_keys[bin] = 1u;
+        for (int j = 0; j < 4; ++j) {
+          const bool cand = e0 + j < end && q[j] >= lo_f;
+          const uint32_t key = order_key(q[j]);
+          many += (uint32_t)__popcll(wave_ballot(cand && key == mass));
+          if (cand && key != mass) {
+            const uint32_t bin = counted_bin(bin_of(map, key), bin_base);
+            atomicAdd(&h[bin], 1u);
+            s_touched[bin / kWave] = 1u;
+            two_keys[bin] = 1u;
+          }
         }
+      });
+      if (lane == 0) {
+        const uint32_t bin = counted_bin(bin_of(map, mass), bin_base);
+        atomicAdd(&h[bin], many);
+        s_touched[bin / kWave] = 1u;
+        a_key[bin] = mass;
       }
-    });
-    if (one_mass && lane == 0) a_key[counted_bin(bin_of(map, mass), bin_base)] = mass;
+    } else {
+      stream_range(p, begin, end, lane, [&](int64_t e0, const float q[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const bool cand = e0 + j < end && q[j] >= lo_f;
+          if (wave_ballot(cand) == 0ull) continue;
+          const uint32_t bin = counted_bin(bin_of(map, order_key(q[j])), bin_base);
+          count_add(h, bin, cand);
+          if (cand) s_touched[bin / kWave] = 1u;
+        }
+      });
+    }
   }
   // the queue, in index order, becomes the wave's list and is counted
   uint64_t *list = lists + gw * list_cap;
@@ -971,18 +987,18 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
   // whoever needs the entries of a few bins finds them in one short piece of every workgroup's list,
   // instead of walking all of them.
   const bool gave_up = s_gave_up != 0u;
-  if (gave_up && tid == 0) state->gave_up = 1u;
-  if (binned == nullptr) return;  // (nobody will ask)
+  if (gave_up && tid == 0) atomicMax(&state->gave_up, 1u + s_mixed);
+  if (binned == nullptr || s_mixed != 0u) return;  // (nobody will ask)
   const u32x4 c4 = *reinterpret_cast<const u32x4 *>(&h[tid * 4]);
   const uint32_t sum4 = (c4[0] + c4[1]) + (c4[2] + c4[3]);
   const uint32_t inc = (uint32_t)wave_inclusive_sum((int)sum4);
   if (lane == kWave - 1) s_wsum[wave] = inc;
   each_queued([&](uint64_t ent, uint32_t bin) {
-    if (a_key[bin] != (uint32_t)(ent >> 32)) two_keys[bin] = 1u;
+    if (a_key[bin] != (uint32_t)(ent >> 32)) a_key[bin] = kNoKey;
   });
   if (mass != 0u && lane == 0) {
     const uint32_t bin = counted_bin(bin_of(map, mass), bin_base);
-    if (a_key[bin] != mass) two_keys[bin] = 1u;
+    if (a_key[bin] != mass) a_key[bin] = kNoKey;
   }
   __syncthreads();  // (and every count has been read)
   u32x4 at4;
@@ -992,24 +1008,24 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
   at4[3] = at4[2] + c4[2];
   uint16_t *my_starts = starts + (int64_t)blockIdx.x * kStartPitch;
   uint64_t *mine_binned = binned + (int64_t)blockIdx.x * binned_cap(list_cap);
-  uint32_t two4 = *reinterpret_cast<const uint32_t *>(&two_keys[tid * 4]);  // a byte a bin, 0 or 1
+  const u32x4 key4 = *reinterpret_cast<const u32x4 *>(&a_key[tid * 4]);
   if (gave_up) {
-    if (s_mixed != 0u) two4 = 0x01010101u;
     Unlisted *mine_unlisted = reinterpret_cast<Unlisted *>(mine_binned);
-    *reinterpret_cast<u32x4 *>(&mine_unlisted->key[tid * 4]) = *reinterpret_cast<const u32x4 *>(&a_key[tid * 4]);
-    static_assert(kTwoKeysHere == 1u << 31, "the byte's lowest bit");
+    *reinterpret_cast<u32x4 *>(&mine_unlisted->key[tid * 4]) = key4;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) mine_unlisted->start[tid * 4 + e] = at4[e] | ((two4 >> (8 * e)) << 31);
+    for (int e = 0; e < 4; ++e)
+      mine_unlisted->start[tid * 4 + e] =
+          at4[e] | (key4[e] == kNoKey || two_keys[tid * 4 + e] != 0u ? kTwoKeysHere : 0u);
     if (tid == kThreads - 1) {
       my_starts[kHintedBins] = (uint16_t)kGaveUp;
       *reinterpret_cast<uint32_t *>(my_starts + kHintedBins + 2) = at4[3] + c4[3];
     }
     return;
   }
-  static_assert(kTwoKeys == 1u << 15, "the byte's lowest bit");
-  *reinterpret_cast<u32x2 *>(my_starts + tid * 4) =
-      u32x2{at4[0] | (at4[1] << 16) | ((two4 & 1u) << 15) | ((two4 & 0x100u) << 23),
-            at4[2] | (at4[3] << 16) | ((two4 & 0x10000u) >> 1) | ((two4 & 0x1000000u) << 7)};
+  u32x4 word4;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) word4[e] = at4[e] | (key4[e] == kNoKey ? kTwoKeys : 0u);
+  *reinterpret_cast<u32x2 *>(my_starts + tid * 4) = u32x2{word4[0] | (word4[1] << 16), word4[2] | (word4[3] << 16)};
   if (tid == kThreads - 1) my_starts[kHintedBins] = (uint16_t)(at4[3] + c4[3]);
   *reinterpret_cast<u32x4 *>(&h[tid * 4]) = at4;  // cursors
   __syncthreads();
@@ -1070,8 +1086,8 @@ constexpr uint32_t kFinishCap = 4096;  // entries that a workgroup puts in order
 constexpr uint32_t kMaxCrowds = 64;
 static_assert(kBucketMaxK / (kFinishCap - kFinishCap / 4) + 2 <= kMaxCrowds && kMaxCrowds <= kWave,
               "a lane for every bin that is crowded and selected");
-// Bins with more entries than that, counted from the hint's (by value all that are selected, by index the one of
-// the k-th key), and the entries of the workgroups before this one.
+// Bins with many entries, counted from the hint's (by value all that are selected, by index the one of the k-th
+// key), and the entries of the workgroups before this one.
 struct Crowds {
   uint32_t n, bin[kMaxCrowds];
   uint32_t base[kMaxCrowds];    // by value: entries above the bin
@@ -1080,9 +1096,11 @@ struct Crowds {
   uint32_t above, own_above;    // by index: the same for the bins above
 };
 struct Finish {
-  bool can, gave_up;
+  bool can;
+  uint32_t gave_up;       // as in the state
   uint32_t crowds;        // how many
-  uint32_t limit;         // most entries of a bin
+  uint32_t limit;         // most entries of a bin that is put in order
+  uint32_t many;          // from so many on a bin is looked at for being one key
   const uint16_t *starts;
   const uint64_t *binned;
   int list_cap;
@@ -1115,30 +1133,38 @@ __device__ __forceinline__ bool one_key_each(Crowds &cr, const Finish &fin) {
   const uint16_t *row = fin.starts + (int64_t)(real ? src : 0u) * kStartPitch;
   const uint64_t *list = fin.binned + (int64_t)(real ? src : 0u) * binned_cap(fin.list_cap);
   const Unlisted *unlisted = reinterpret_cast<const Unlisted *>(list);
-  const bool listed = row[kHintedBins] != kGaveUp;
-  uint32_t all = row[kHintedBins];  // candidates
-  if (!listed) all = *reinterpret_cast<const uint32_t *>(row + kHintedBins + 2);
+  struct Piece {
+    uint32_t at, end, all;  // the bin's entries, and all of the workgroup
+    bool listed, two;
+  };
+  const auto piece_of = [&](uint32_t bin) {
+    // (the words of a workgroup with lists are asked for before it is known to have them)
+    const uint32_t word = row[bin], word1 = row[bin + 1u], all = row[kHintedBins];
+    Piece c{word & kStartMask, word1 & kStartMask, all, all != kGaveUp, (word & kTwoKeys) != 0u};
+    if (!c.listed) {
+      c.all = *reinterpret_cast<const uint32_t *>(row + kHintedBins + 2);
+      c.at = unlisted->start[bin] & ~kTwoKeysHere;
+      c.end = bin + 1u < (uint32_t)kHintedBins ? unlisted->start[bin + 1u] & ~kTwoKeysHere : c.all;
+      c.two = (unlisted->start[bin] & kTwoKeysHere) != 0u;
+    }
+    if (!real) c.end = c.at;
+    return c;
+  };
   bool other = false;
   for (uint32_t q = wave / kParts; q < n; q += kWavesPerBlock / kParts) {
-    const uint32_t bin = cr.bin[q];
-    uint32_t at, end, key = 0u;
-    bool two;
-    if (listed) {
-      at = row[bin] & kStartMask;
-      end = bin + 1u < (uint32_t)kHintedBins ? row[bin + 1u] & kStartMask : all;
-      two = (row[bin] & kTwoKeys) != 0u;
-      if (at < end) key = (uint32_t)(list[at] >> 32);
-    } else {
-      at = unlisted->start[bin] & ~kTwoKeysHere;
-      end = bin + 1u < (uint32_t)kHintedBins ? unlisted->start[bin + 1u] & ~kTwoKeysHere : all;
-      two = (unlisted->start[bin] & kTwoKeysHere) != 0u;
-      key = unlisted->key[bin];
-    }
-    const uint32_t cnt = real ? end - at : 0u;
+    const Piece c = piece_of(cr.bin[q]);
+    other = other || (c.two && c.at < c.end);
+  }
+  if (__syncthreads_or(other)) return false;  // (the most frequent end)
+  for (uint32_t q = wave / kParts; q < n; q += kWavesPerBlock / kParts) {
+    const Piece c = piece_of(cr.bin[q]);
+    const uint32_t cnt = c.end - c.at, all = c.all, end = c.end;
+    uint32_t key = 0u;
+    if (cnt != 0u) key = c.listed ? (uint32_t)(list[c.at] >> 32) : unlisted->key[cr.bin[q]];
     const uint64_t has = wave_ballot(cnt != 0u);
     const uint32_t some =
         has != 0ull ? (uint32_t)__builtin_amdgcn_readlane((int)key, __builtin_ctzll(has)) : 0u;
-    other = other || (cnt != 0u && (two || key != some));
+    other = other || (cnt != 0u && (key != some || key == 0u));
     const uint32_t sum = (uint32_t)wave_sum((int)(src < blockIdx.x ? cnt : 0u));
     if (src == blockIdx.x) cr.own[q] = cnt;
     if (lane == 0) {
@@ -1146,7 +1172,7 @@ __device__ __forceinline__ bool one_key_each(Crowds &cr, const Finish &fin) {
       s_sum[q][part] = sum;
     }
     if (FINISH == kFinishByIndex) {
-      const uint32_t over = all - end;
+      const uint32_t over = real ? all - end : 0u;
       const uint32_t above = (uint32_t)wave_sum((int)(src < blockIdx.x ? over : 0u));
       if (src == blockIdx.x) cr.own_above = over;
       if (lane == 0) s_above[part] = above;
@@ -1180,7 +1206,7 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
   __shared__ Pick s_pick;
   __shared__ uint32_t s_bin2;
   __shared__ uint32_t s_base[kHintedBins / kWave];  // entries above every 64th bin from the top
-  __shared__ uint32_t s_big, s_plain, s_at_lo, s_at_hi, s_begin, s_end;
+  __shared__ uint32_t s_big, s_over, s_fix, s_fix_lo, s_fix_end, s_plain, s_at_lo, s_at_hi, s_begin, s_end;
   const Copies cp = copies_of(map);
   const int tid = threadIdx.x, lane = tid & 63;
   // thread t owns the bins 4t .. 4t + 3; of eight copies its words are those of every other one
@@ -1209,7 +1235,7 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
     s_pick.k_rem = k_rem;
     s_pick.found = 0u;
     s_bin2 = 0u;
-    s_big = s_plain = s_at_lo = s_begin = s_end = 0u;
+    s_big = s_over = s_fix = s_plain = s_at_lo = s_begin = s_end = 0u;
     if (FINISH != kNoFinish) cr.n = 0u;
     s_at_hi = cp.used - 1u;
   }
@@ -1227,7 +1253,7 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
         const bool here = !found && r + c[j] >= rank;
         pb = here ? map.nb0 + (uint32_t)(tid * kPer + j) : pb;
         pk = here ? rank - r : pk;
-        if (FINISH == kFinishByIndex && rem_out && here && c[j] > fin->limit) s_big = 1u;
+        if (FINISH == kFinishByIndex && rem_out && here && c[j] > fin->many) s_big = c[j];
         found = found || here;
         r += c[j];
       }
@@ -1256,7 +1282,7 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
           s_at_lo = bin;
           s_end = next;
         }
-        if (r < k_rem && c[j] > fin->limit) s_big = 1u;
+        if (r < k_rem && c[j] > fin->many) s_big = 1u;
       }
       if (boff && bin < cp.used && (cp.used - 1u - bin) % kWave == 0u) s_base[(cp.used - 1u - bin) / kWave] = r;
       r = next;
@@ -1267,14 +1293,19 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
   if (tid == 0) s_pick.total = total;
   __syncthreads();
   if (FINISH != kNoFinish) {
-    fin->can = s_pick.found != 0u;
+    fin->can = s_pick.found != 0u && fin->gave_up < 2u;
     fin->crowds = 0u;
-    if (__builtin_expect(fin->can && (s_big != 0u || fin->gave_up), 0)) {
+    fin->at_lo = s_at_lo;
+    fin->at_hi = s_at_hi;
+    fin->base = s_begin;
+    fin->end = s_end;
+    if (__builtin_expect(fin->can && (s_big != 0u || fin->gave_up != 0u), 0)) {
       if (FINISH == kFinishByIndex) {
         if (tid == 0) {
-          cr.n = s_big;
+          cr.n = s_big != 0u ? 1u : 0u;
           cr.bin[0] = s_pick.bin - map.nb0;
-          s_plain = 1u - s_big;
+          s_plain = s_big != 0u ? 0u : 1u;
+          s_over = s_big > fin->limit ? 1u : 0u;
         }
       } else {
         const uint32_t hi = fin->hi < k_rem ? fin->hi : k_rem;
@@ -1282,15 +1313,18 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
 #pragma unroll
         for (int j = kPer - 1; j >= 0; --j) {
           const uint32_t next = r + c[j], bin = (uint32_t)(tid * kPer + j);
-          if (r < k_rem && c[j] > fin->limit) {
+          if (r < k_rem && c[j] > fin->many) {
             const uint32_t q = atomicAdd(&cr.n, 1u);
             if (q < kMaxCrowds) {
               cr.bin[q] = bin;
               cr.base[q] = r;
             }
-            if (fin->lo < hi && r < hi && next >= hi) {  // (the last bin of the stretch, or one before it)
-              s_at_lo = bin + 1u;
-              s_end = r;
+            if (c[j] > fin->limit) s_over = 1u;
+            // (longer than a stretch: the last bin that starts in it, or one that started before)
+            if (fin->lo < hi && r < hi && next >= hi) {
+              s_fix = 1u;
+              s_fix_lo = bin + 1u;
+              s_fix_end = r;
             }
           } else if (r < k_rem && c[j] != 0u) {
             s_plain = 1u;
@@ -1299,14 +1333,17 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
         }
       }
       __syncthreads();
-      fin->crowds = cr.n;
-      fin->can = cr.n <= kMaxCrowds && !(fin->gave_up && s_plain != 0u);
-      if (fin->can && cr.n != 0u) fin->can = one_key_each<FINISH>(cr, *fin);
+      if (cr.n != 0u && cr.n <= kMaxCrowds && one_key_each<FINISH>(cr, *fin)) {
+        fin->crowds = cr.n;
+        fin->can = fin->gave_up == 0u || s_plain == 0u;
+        if (s_fix != 0u) {
+          fin->at_lo = s_fix_lo;
+          fin->end = s_fix_end;
+        }
+      } else {
+        fin->can = fin->gave_up == 0u && s_over == 0u;
+      }
     }
-    fin->at_lo = s_at_lo;
-    fin->at_hi = s_at_hi;
-    fin->base = s_begin;
-    fin->end = s_end;
     if (fin->can) boff = nullptr;
   }
   // Where the bins at or above the picked one start in value order, and the segment table: as
@@ -1558,11 +1595,16 @@ __device__ __forceinline__ Pick member_hist(
     __shared__ Crowds crowds;
     if (FINISH != kNoFinish) {
       const uint32_t share = ((uint32_t)k + gridDim.x - 1u) / gridDim.x;
-      fin.gave_up = state->gave_up != 0u;
+      fin.gave_up = state->gave_up;
       fin.starts = io.starts;
       fin.binned = io.binned;
       fin.list_cap = list_cap;
       fin.limit = kFinishCap - (FINISH == kFinishByValue ? share : 0u);
+      // (Putting a mass in order takes longer than a look: 2000 equal ones of 20000, us by index and by value,
+      // 28.7 / 29.4 and 18.7 / 21.5.  Bins of lognormal priorities stay well below; a look in vain takes 1.5 us, as in
+      // the last bin of 20000 ascending priorities.)
+      fin.many = FINISH == kFinishByValue ? 512u + share + (uint32_t)k / 64u : 512u + (uint32_t)k / 16u;
+      if (fin.many > fin.limit) fin.many = fin.limit;
       fin.lo = block * share;
       fin.hi = fin.lo + share;
     }
@@ -2832,8 +2874,8 @@ static_assert(kSortThreads >= kSortBins, "a thread per digit in the segment sort
 // A bin that holds more than a workgroup orders is most often a mass of equal priorities -- new entries at the
 // largest one, integers --, which needs no order but the index (store_crowds): as launches / left to the launch
 // behind / finished, by index and by value: all equal 20000 30 / 40 / 29 and 34 / 44 / 32, 1e6 41 / 53 / 33 and
-// 46 / 57 / 37, 1e7 104 / 111 / 72 and 115 / 122 / 82; nine in ten of 1e6 40 / 52 / 33 and 45 / 56 / 36;
-// 65536 of 1e7 integers below 1000 37 / 45 / 31 and 60 / 68 / 44, of 1e7 with 60000 ties by value 53 / 59 / 37.
+// 46 / 57 / 37, 1e7 104 / 111 / 62 and 115 / 122 / 72; nine in ten of 1e6 40 / 52 / 32 and 45 / 56 / 35;
+// 65536 of 1e7 integers below 1000 37 / 45 / 32 and 61 / 68 / 46, of 1e7 with 60000 ties by value 53 / 59 / 37.
 // By value a workgroup takes the bins that start in its stretch of the output; the bin that holds the k-th
 // key is ordered whole and what lies beyond place k is not stored, so no threshold is needed.  By index
 // every workgroup takes the bin of the k-th key, finds the last entry of it that is selected, and from that
