@@ -2899,13 +2899,13 @@ struct FinishOut {
   }
 };
 
-// fin(place, entry) for the m entries, larger ones first, which were counted in cnt (kFinishSlots words) by
+// By value: fin(place, entry) for the m entries, larger ones first, which were counted in cnt (kFinishSlots words) by
 // slot_of(entry): a counting sort by slots, of which most hold an entry or none, and a rank inside the slot.
 // Both buffers hold kFinishCap, cnt two tables of slots.
 // A slot that is crowded -- priorities that are equal: new entries at the largest one -- is cut again, by what its
 // entries differ in (equal priorities: the index), instead of a radix sort of everything, which stays for
 // more than one such slot and for crowds within the crowd: us a call on 300000 priorities with 1808 equal ones
-// above the rest, 1000 by index 40.9 / 27.6 without and with it, 2000 by value 47.6 / 29.2 by segments and here.
+// above the rest, 2000 by value 47.6 / 29.2 by segments and here.
 template <typename Slot, typename Out>
 __device__ __forceinline__ void order_entries(uint64_t *ents, uint64_t *other, uint32_t *cnt, uint32_t m,
                                               int bits, const Slot &slot_of, const Out &fin, SortShared &sh) {
@@ -2991,6 +2991,89 @@ __device__ __forceinline__ void order_entries(uint64_t *ents, uint64_t *other, u
     const uint64_t own = other[i];
     const uint32_t slot = slot_of(own), b = slot > 0u ? cnt[slot - 1u] : 0u;
     fin(b + larger_in(other, b, cnt[slot], own), own);
+  }
+}
+
+// The rank-th largest of the m entries (0 where they are fewer), which were counted in cnt by slot_of(entry): of its
+// slot's entries while these are few, else of their own range cut into slots in turn, so that priorities that
+// lie close together, or are equal, cost a turn or two.  Bound by the latency of barriers and LDS.  us a call by
+// index, all entries of the bin in order as for values (a radix sort for more than one crowded slot) / so:
+// lognormal 65536 of 1e7 33.7 / 32.4, 1024 consecutive ones above the rest of 1e6 33.4 / 26.0, 4000 of 300000 within 1
+// part in 2500 30.9 / 25.1; as launches of their own 33.0, 24.6, 23.7.
+template <typename Slot>
+__device__ __forceinline__ uint64_t ranked_entry(const uint64_t *ents, uint32_t *cnt, uint32_t m, uint32_t rank,
+                                                 const Slot &slot_of) {
+  __shared__ uint32_t s_wsum[kWavesPerBlock], s_slot, s_rank, s_in, s_n;
+  __shared__ uint64_t s_max[kWavesPerBlock], s_min[kWavesPerBlock], s_few[kFinishSlot], s_found;
+  const uint32_t tid = threadIdx.x;
+  const int lane = (int)tid & 63, wave = __builtin_amdgcn_readfirstlane((int)tid >> 6);
+  uint64_t largest = 0ull, smallest = 0ull;  // (of the slot that is cut)
+  int shift = -1;                            // the first turn's slots are slot_of's
+  for (;;) {
+    const u32x2 c2 = reinterpret_cast<const u32x2 *>(cnt)[tid];
+    const uint32_t inc = (uint32_t)wave_inclusive_sum((int)(c2[0] + c2[1]));
+    if (lane == kWave - 1) s_wsum[wave] = inc;
+    if (tid == 0) s_in = s_n = 0u;
+    __syncthreads();
+    const uint32_t start = inc - c2[0] - c2[1] +
+                           (uint32_t)wave_sum((int)(lane < wave ? s_wsum[lane & (kWavesPerBlock - 1)] : 0u));
+    if (start < rank && start + c2[0] + c2[1] >= rank) {  // one thread
+      const bool second = start + c2[0] < rank;
+      s_slot = 2u * tid + (second ? 1u : 0u);
+      s_rank = rank - start - (second ? c2[0] : 0u);
+      s_in = second ? c2[1] : c2[0];
+    }
+    __syncthreads();
+    const uint32_t slot = s_slot, in = s_in;
+    if (in == 0u) return 0ull;
+    rank = s_rank;
+    const auto in_slot = [&](uint64_t own) {
+      if (shift < 0) return slot_of(own) == slot;
+      return own <= largest && own >= smallest && (uint32_t)((largest - own) >> shift) == slot;
+    };
+    if (in <= kFinishSlot) {
+      for (uint32_t i = tid; i < m; i += kThreads)
+        if (in_slot(ents[i])) s_few[atomicAdd(&s_n, 1u)] = ents[i];
+      __syncthreads();
+      if (tid < in && larger_in(s_few, 0u, in, s_few[tid]) + 1u == rank) s_found = s_few[tid];
+      __syncthreads();
+      return s_found;
+    }
+    uint64_t hi = 0ull, lo = ~0ull;
+    for (uint32_t i = tid; i < m; i += kThreads) {
+      const uint64_t own = ents[i];
+      if (in_slot(own)) {
+        hi = own > hi ? own : hi;
+        lo = own < lo ? own : lo;
+      }
+    }
+#pragma unroll
+    for (int step = 1; step < kWave; step *= 2) {
+      const uint64_t a = __shfl_xor((unsigned long long)hi, step), b = __shfl_xor((unsigned long long)lo, step);
+      hi = a > hi ? a : hi;
+      lo = b < lo ? b : lo;
+    }
+    if (lane == 0) {
+      s_max[wave] = hi;
+      s_min[wave] = lo;
+    }
+    reinterpret_cast<u32x2 *>(cnt)[tid] = u32x2{0u, 0u};
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kWavesPerBlock; ++w) {
+      hi = s_max[w] > hi ? s_max[w] : hi;
+      lo = s_min[w] < lo ? s_min[w] : lo;
+    }
+    if (hi == lo) return hi;  // (no two entries are equal: every turn ends with a shorter range)
+    largest = hi;
+    smallest = lo;
+    const int differ = 64 - __builtin_clzll(hi - lo);
+    shift = differ > 11 ? differ - 11 : 0;
+    for (uint32_t i = tid; i < m; i += kThreads) {
+      const uint64_t own = ents[i];
+      if (own <= hi && own >= lo) atomicAdd(&cnt[(uint32_t)((hi - own) >> shift)], 1u);
+    }
+    __syncthreads();
   }
 }
 
@@ -3097,7 +3180,6 @@ __device__ __forceinline__ void finish_selection(
     int64_t *__restrict__ indices_out) {
   __shared__ SortShared sh;
   __shared__ uint32_t s_n, s_red[kWavesPerBlock], s_own[kWavesPerBlock];
-  __shared__ uint64_t s_last;  // by index: the last entry of the picked bin that is selected
   constexpr int kCrowdCounts = 4 * kFinishCap + 2 * kFinishSlots;
   static_assert(kBinsR + kCrowdCounts + kWavesPerBlock * kWave <= kBinsF / 2 && kBinsR % 2 == 0,
                 "the entries fit the LDS that only a failed hint uses");
@@ -3135,10 +3217,7 @@ __device__ __forceinline__ void finish_selection(
   const uint64_t *from = binned + (int64_t)(real ? src : 0u) * binned_cap(list_cap);
   uint32_t c = row[at_lo] & kStartMask, end = row[at_hi + 1u] & kStartMask;
   const uint32_t all = kByValue ? 0u : row[kHintedBins];  // (no wave gave its list up)
-  if (tid == 0) {
-    s_n = 0u;
-    s_last = 0ull;
-  }
+  if (tid == 0) s_n = 0u;
   reinterpret_cast<u32x2 *>(cnt)[tid] = u32x2{0u, 0u};
   if (!real) end = c;
   uint32_t before = 0u;  // by index: this lane's share of the selected entries of earlier lists
@@ -3200,24 +3279,18 @@ __device__ __forceinline__ void finish_selection(
   }
   __syncthreads();
   const uint32_t m = s_n < kFinishCap ? s_n : kFinishCap;
-  const int bits = 32 + key_bits;
   if (kByValue) {
-    order_entries(ents, other, cnt, m, bits, slot_of,
+    order_entries(ents, other, cnt, m, 32 + key_bits, slot_of,
                   FinishOut{p, n, values_out, indices_out, fin.base, lo_key, k}, sh);
     return;
   }
+  // the last entry of the picked bin that is selected, and those of earlier workgroups
+  const uint64_t last = ranked_entry(ents, cnt, m, pick.k_rem, slot_of);
   const int64_t first_index = (int64_t)blockIdx.x * kWavesPerBlock * wave_len;
-  order_entries(
-      ents, other, cnt, m, bits, slot_of,
-      [&](uint32_t i, uint64_t ent) {
-        if (i + 1u == pick.k_rem) s_last = ent;
-        if (i < pick.k_rem && (int64_t)(uint32_t)~(uint32_t)ent < first_index) ++before;
-      },
-      sh);
+  for (uint32_t i = (uint32_t)tid; i < m; i += kThreads)
+    before += ents[i] >= last && (int64_t)(uint32_t)~(uint32_t)ents[i] < first_index ? 1u : 0u;
   const uint32_t wave_before = (uint32_t)wave_sum((int)before);
   if (lane == 0) s_red[wave] = wave_before;
-  __syncthreads();
-  const uint64_t last = s_last;
   auto selected = [&](uint64_t ent, bool valid) {
     const uint32_t key = (uint32_t)(ent >> 32), at = counted_bin(bin_of(map, key), map.nb0);
     const uint64_t own = ((uint64_t)(key - lo_key) << 32) | (uint32_t)~(uint32_t)ent;

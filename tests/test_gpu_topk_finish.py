@@ -218,7 +218,7 @@ def test_neighbours_in_the_input_that_are_neighbours_in_value(oracle, n, k):
     _check(oracle, np.arange(n, dtype=np.float32), k, "0 to n - 1")
 
 
-@pytest.mark.parametrize("crowd", ["stretch", "two values", "neighbours", "two stretches"])
+@pytest.mark.parametrize("crowd", ["stretch", "two values", "neighbours", "two stretches", "close", "two clusters"])
 @pytest.mark.parametrize("ties", [65, 1_025, 3_000])
 def test_a_crowded_slot(oracle, crowd, ties):
     n, k = 300_007, 2_500
@@ -232,6 +232,11 @@ def test_a_crowded_slot(oracle, crowd, ties):
         w[at] = np.where(rng.random(ties) < 0.5, top, np.float32(1.5) * top)
     elif crowd == "neighbours":  # a few ulps apart
         w[at] = (np.full(ties, top).view(np.uint32) + rng.integers(0, 5, ties).astype(np.uint32)).view(np.float32)
+    elif crowd == "close":  # several crowded slots
+        w[at] = top * (1 + rng.random(ties, dtype=np.float32) * np.float32(4e-4))
+    elif crowd == "two clusters":
+        w[at] = (np.full(ties, top).view(np.uint32) + rng.integers(0, 26, ties).astype(np.uint32)).view(np.float32)
+        w[at[:ties // 3]] *= np.float32(1.002)
     else:
         w[5:5 + ties // 2] = top
         w[n - ties // 2:] = top
