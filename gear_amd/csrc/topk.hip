@@ -1082,7 +1082,10 @@ __global__ __launch_bounds__(kThreads) void level0_kernel(const float *__restric
 // and no bin that it has to order holds too many, unless they all have the same key (the crowds), or is missing in
 // the binned lists because a wave gave its list up.
 enum FinishOrder { kNoFinish, kFinishByIndex, kFinishByValue };
-constexpr uint32_t kFinishCap = 4096;  // entries that a workgroup puts in order
+constexpr uint32_t kFinishCap = 4096;  // entries that a workgroup puts in order, by value
+// ... and that it looks through by index, which needs no second buffer: 7000 of 1e7, whose last bin holds some 5000
+// (small samples end below the largest priorities, which share few bins), 34.9 us a call with a limit of 4096, 32.9 so
+constexpr uint32_t kFinishCapByIndex = 2 * kFinishCap;
 constexpr uint32_t kMaxCrowds = 64;
 static_assert(kBucketMaxK / (kFinishCap - kFinishCap / 4) + 2 <= kMaxCrowds && kMaxCrowds <= kWave,
               "a lane for every bin that is crowded and selected");
@@ -1599,7 +1602,7 @@ __device__ __forceinline__ Pick member_hist(
       fin.starts = io.starts;
       fin.binned = io.binned;
       fin.list_cap = list_cap;
-      fin.limit = kFinishCap - (FINISH == kFinishByValue ? share : 0u);
+      fin.limit = FINISH == kFinishByValue ? kFinishCap - share : kFinishCapByIndex;
       // (Putting a mass in order takes longer than a look: 2000 equal ones of 20000, us by index and by value,
       // 28.7 / 29.4 and 18.7 / 21.5.  Bins of lognormal priorities stay well below; a look in vain takes 1.5 us, as in
       // the last bin of 20000 ascending priorities.)
@@ -3183,9 +3186,10 @@ __device__ __forceinline__ void finish_selection(
   constexpr int kCrowdCounts = 4 * kFinishCap + 2 * kFinishSlots;
   static_assert(kBinsR + kCrowdCounts + kWavesPerBlock * kWave <= kBinsF / 2 && kBinsR % 2 == 0,
                 "the entries fit the LDS that only a failed hint uses");
-  uint64_t *ents = reinterpret_cast<uint64_t *>(lds), *other = ents + kFinishCap;
+  uint64_t *ents = reinterpret_cast<uint64_t *>(lds), *other = ents + kFinishCap;  // (one buffer by index)
   uint32_t *cnt = lds + 4 * kFinishCap;  // entries of a slot
   constexpr bool kByValue = FINISH == kFinishByValue;
+  constexpr uint32_t kCap = kByValue ? kFinishCap : kFinishCapByIndex;
   if (__builtin_expect(fin.crowds != 0u, 0)) {
     store_crowds<FINISH>(p, n, k, crowds, pick, map, list, listed, ent_pre, wave_len, lds + kCrowdCounts,
                          values_out, indices_out);
@@ -3244,7 +3248,7 @@ __device__ __forceinline__ void finish_selection(
         uint32_t slot = 0u;
         if (lane == 0) slot = atomicAdd(&s_n, (uint32_t)__popcll(hits));
         slot = (uint32_t)__builtin_amdgcn_readlane((int)slot, 0) + (uint32_t)__popcll(hits & lt_mask);
-        if (hit && slot < kFinishCap) take(slot, e[u]);
+        if (hit && slot < kCap) take(slot, e[u]);
       }
     }
   } else {
@@ -3267,7 +3271,7 @@ __device__ __forceinline__ void finish_selection(
       if (lane == 0) s_n = run;
     }
     __syncthreads();
-    const uint32_t entries = s_n < kFinishCap ? s_n : kFinishCap;
+    const uint32_t entries = s_n < kCap ? s_n : kCap;
     for (uint32_t i = (uint32_t)tid; i < entries; i += kThreads) {
       uint32_t lo = 0u;  // the first piece that ends behind entry i
 #pragma unroll
@@ -3278,7 +3282,7 @@ __device__ __forceinline__ void finish_selection(
     }
   }
   __syncthreads();
-  const uint32_t m = s_n < kFinishCap ? s_n : kFinishCap;
+  const uint32_t m = s_n < kCap ? s_n : kCap;
   if (kByValue) {
     order_entries(ents, other, cnt, m, 32 + key_bits, slot_of,
                   FinishOut{p, n, values_out, indices_out, fin.base, lo_key, k}, sh);

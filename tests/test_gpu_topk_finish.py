@@ -1,6 +1,6 @@
 """Top-k finished by its first level: a workgroup orders the few bins that concern it, fetched from every
 workgroup's binned list.  Edges: bins that hold nearly, exactly and more than a workgroup orders (4096, less its
-share of the output), a slot of equal keys, the zeros, the first and the last place; and what is left to the
+share of the output; by index 8192), a slot of equal keys, the zeros, the first and the last place; and what is left to the
 launch behind it, whose phases hand over inside it, with several of them on the GPU at once."""
 import numpy as np
 import pytest
@@ -241,3 +241,20 @@ def test_a_crowded_slot(oracle, crowd, ties):
         w[5:5 + ties // 2] = top
         w[n - ties // 2:] = top
     _check(oracle, w, k, "%d %s" % (ties, crowd))
+
+
+@pytest.mark.parametrize("together", [4_096, 4_097, 8_192, 8_193])
+def test_the_most_entries_that_level_1_looks_through_by_index(oracle, together):
+    """Of a bin that is not one key."""
+    from gear_amd import ops
+    n, k = 300_007, 2_500
+    w = _values(n, 7)
+    rng = np.random.default_rng(together)
+    top = np.float32(2) * w.max()
+    w[rng.permutation(n)[:together]] = (np.full(together, top).view(np.uint32) +
+                                        rng.integers(0, 5, together).astype(np.uint32)).view(np.float32)
+    _check(oracle, w, k, "%d together" % together)
+    state = ops.TopKState()
+    announce("topk by index, %d together" % together)
+    state.select(torch.from_numpy(w).cuda(), k, sorted_by_value=False)
+    assert _finished(state) == (together <= 8_192)
