@@ -193,7 +193,8 @@ struct State {
   uint32_t low_seg;  // after a failed hint, value order: the segment of the entries below the hint
   uint32_t gave_up;  // level 0: a wave gave its list up, so there are no binned lists (2: for more than one mass)
   uint32_t done;     // level 1 has written the result: nothing is left to do
-  uint32_t pad[37];
+  uint32_t masses;   // level 0: a workgroup with lists met kMass candidates of one key in a bin, and no other
+  uint32_t pad[36];
 };
 static_assert(sizeof(State) == 256, "State is the 256-byte header of the workspace");
 
@@ -264,6 +265,7 @@ struct Unlisted {
   uint32_t key[kHintedBins], start[kHintedBins];  // (kTwoKeysHere in a start)
 };
 constexpr uint32_t kTwoKeysHere = 0x80000000u;
+constexpr uint32_t kMass = 4;  // (of 512 equal ones in all, two a workgroup, some have four)
 static_assert(sizeof(Unlisted) <= 256 * kWavesPerBlock * sizeof(uint64_t), "fits the shortest binned list");
 __host__ __device__ __forceinline__ int binned_cap(int64_t list_cap) {
   return (int)(list_cap < kQueueCap ? list_cap : kQueueCap) * kWavesPerBlock;
@@ -704,6 +706,7 @@ __global__ __launch_bounds__(kThreads) void prep_kernel(const float *__restrict_
   if (tid == 9) state->next_magic = 0ull;  // level 1 of this call leaves the next hint, if any
   if (tid == 10) state->gave_up = 0u;
   if (tid == 11) state->done = 0u;
+  if (tid == 12) state->masses = 0u;
   BinMap map;
   map.uniform = 1u;
   map.a_end = map.b_last = map.nb0 = map.nc0 = map.b_shift = map.c_shift = 0u;
@@ -1022,6 +1025,10 @@ __global__ __launch_bounds__(kThreads) void level0_hinted_kernel(
     }
     return;
   }
+  bool mass_here = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) mass_here = mass_here || (c4[e] >= kMass && key4[e] != kNoKey);
+  if (mass_here) state->masses = 1u;
   u32x4 word4;
 #pragma unroll
   for (int e = 0; e < 4; ++e) word4[e] = at4[e] | (key4[e] == kNoKey ? kTwoKeys : 0u);
@@ -1103,6 +1110,7 @@ struct Finish {
   uint32_t gave_up;       // as in the state
   uint32_t crowds;        // how many
   uint32_t limit;         // most entries of a bin that is put in order
+  uint32_t masses;        // as in the state
   uint32_t many;          // from so many on a bin is looked at for being one key
   const uint16_t *starts;
   const uint64_t *binned;
@@ -1336,9 +1344,11 @@ __device__ __forceinline__ Pick pick_copies(uint32_t k_rem, const CopyWords &wor
         }
       }
       __syncthreads();
-      if (cr.n != 0u && cr.n <= kMaxCrowds && one_key_each<FINISH>(cr, *fin)) {
+      if (fin->gave_up != 0u && s_plain != 0u) {
+        fin->can = false;
+      } else if ((fin->masses | fin->gave_up) != 0u && cr.n != 0u && cr.n <= kMaxCrowds &&
+                 one_key_each<FINISH>(cr, *fin)) {
         fin->crowds = cr.n;
-        fin->can = fin->gave_up == 0u || s_plain == 0u;
         if (s_fix != 0u) {
           fin->at_lo = s_fix_lo;
           fin->end = s_fix_end;
@@ -1599,13 +1609,14 @@ __device__ __forceinline__ Pick member_hist(
     if (FINISH != kNoFinish) {
       const uint32_t share = ((uint32_t)k + gridDim.x - 1u) / gridDim.x;
       fin.gave_up = state->gave_up;
+      fin.masses = state->masses;
       fin.starts = io.starts;
       fin.binned = io.binned;
       fin.list_cap = list_cap;
       fin.limit = FINISH == kFinishByValue ? kFinishCap - share : kFinishCapByIndex;
       // (Putting a mass in order takes longer than a look: 2000 equal ones of 20000, us by index and by value,
-      // 28.7 / 29.4 and 18.7 / 21.5.  Bins of lognormal priorities stay well below; a look in vain takes 1.5 us, as in
-      // the last bin of 20000 ascending priorities.)
+      // 28.7 / 29.4 and 18.7 / 21.5.  A look in vain takes 1 to 2, so there is none unless level 0 met a mass: 7000 and
+      // 16384 of 1e7 lognormal ones by value, whose largest share a bin, 33.9 / 33.5 with it and 31.9 / 32.2 without.)
       fin.many = FINISH == kFinishByValue ? 512u + share + (uint32_t)k / 64u : 512u + (uint32_t)k / 16u;
       if (fin.many > fin.limit) fin.many = fin.limit;
       fin.lo = block * share;

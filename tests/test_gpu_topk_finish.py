@@ -55,7 +55,7 @@ def test_what_level_1_finishes_by_index(oracle, ties, at, finished):
 
 
 @pytest.mark.parametrize("n,k", [(262_144, 1), (262_145, 64), (262_207, 32_768), (1_048_577, 131_072),
-                                 (1_500_001, 255), (1_500_001, 65_537), (5_000_011, 100_000)])
+                                 (1_500_001, 255), (1_500_001, 65_537), (5_000_011, 100_000), (10_000_000, 7_000)])
 def test_sizes(oracle, n, k):
     _check(oracle, _values(n, n + k), k, "lognormal")
 
