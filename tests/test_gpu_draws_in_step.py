@@ -1,6 +1,7 @@
 """A loader's step that draws its batch itself gives what torch's rand or randint of the same generator would have
 given it, and leaves the generator where that call leaves it: at the sizes where the draws move from the
-selection to a launch of their own and from there to torch, for ranges of one entry and beyond 32 bits."""
+selection to a launch of their own and from there to torch, and for ranges of one entry to just beyond 2^28, from
+where torch draws."""
 import os
 
 import pytest
@@ -122,7 +123,35 @@ def test_uniforms_bit_for_bit():
         assert torch.equal(got, torch.searchsorted(prefix, u.double(), right=True).sort().values)
 
 
-def test_a_captured_step_and_a_sampler_of_its_own_draw_with_torch():
+@pytest.mark.parametrize("weighted", [False, True])
+def test_a_captured_step_draws_with_torch(weighted):
+    """The generator's state is not the host's to read then: every replay has the next numbers of it."""
+    ops, num, n = _ops(), 300, 10_000
+    step = _loader(50 + weighted, batch=8)._step
+    table, lengths = _tables(n)
+    prefix = ops.prefix_sum(torch.rand(n, device="cuda") + 0.01) if weighted else None
+    kind = "weighted" if weighted else "uniform"
+    g, twin = torch.Generator("cuda"), torch.Generator("cuda")
+    g.manual_seed(9)
+    twin.manual_seed(9)
+    announce("%s step captured" % kind)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):  # (what is allocated by the first call is allocated)
+        step.run(kind, twin, prefix, table, 5, lengths, False, ops._ws, num)
+    stream.synchronize()
+    twin.manual_seed(9)
+    graph = torch.cuda.CUDAGraph()
+    graph.register_generator_state(g)
+    with torch.cuda.graph(graph, stream=stream):
+        got = step.run(kind, g, prefix, table, 5, lengths, False, ops._ws, num)[0]
+    for _ in range(4):
+        graph.replay()
+        torch.cuda.synchronize()
+        want = step.run(kind, twin, prefix, table, 5, lengths, False, ops._ws, num)[0]
+        assert torch.equal(got, want)
+
+
+def test_a_sampler_with_a_draw_of_its_own():
     loader = _loader(42, batch=16)
     mine = torch.arange(16, device="cuda")
     announce("a sampler whose draw() was replaced")
