@@ -766,8 +766,8 @@ int launch_scan(const In *in, Out *out, int64_t n, void *ws, size_t ws_bytes, hi
   // instead of two, us at 6e7 / 6.8e7 / 1e8 / 1.3e8: 147 / 167 / 240 / 309 against 187 / 213 / 308 /
   // 399; int64 at 4e7 / 6e7: 143 / 210 against 183 / 267).  The chained kernel and the two launches cut
   // the input the same way, so a rescan finds the sums of the last full scan and the bits are the same;
-  // but integers, which have no rescan and the same sums in any order, take 8 granules in two launches
-  // (captured, 4e7 / 6e7: 187 / 276 us, 197 / 281 with 16).
+  // but integers, which have no rescan and the same sums in any order, take 8 granules in several launches
+  // (captured, 4e7 / 6e7: 185 / 271 us, 185 / 274 with 16; beyond 16384 ranges, 1e8: 482 / 438).
   // Beyond 16384 ranges a workgroup has fewer threads than there are groups: three launches of 8 granules.
   // (8-byte elements: ranges of 2 granules would be smaller than the 2048 elements the workspace is laid
   // out for, so they start at 4.)

@@ -178,11 +178,14 @@ int gear_hip_take_i64(const int64_t *table, int64_t n, const int64_t *idx, int64
 
 /* Inclusive prefix sum of fp32 priorities accumulated and written in fp64:
  *     out[i] = sum_{j<=i} (double) in[j]
- * One pass over the input for up to 16384 ranges (n <= 268 M): every workgroup publishes the sum
- * of its range and adds the sums of all earlier ranges, with a bounded wait (a workgroup that
- * waited too long sums the missing range itself and publishes it: same bits, no kernel can
- * hang).  Two launches (range sums, then the scan) for a stream under graph capture and with
- * GEAR_HIP_SCAN_SINGLE_PASS=0; three (a launch in between scans the range sums) beyond that.  The result is bit-identical in all cases and on every run.  Replaces
+ * One pass over the input for up to 16384 ranges (n <= 268 M fp32, 134 M int64): every workgroup publishes
+ * the sum of its range and adds the sums of all earlier ranges -- beyond 6656 ranges those of the earlier ones of its
+ * group of 64 and of all earlier groups --, with a bounded wait (a workgroup that waited too long sums the missing
+ * range itself and publishes it: same bits, no kernel can hang).  For a stream under graph capture and with
+ * GEAR_HIP_SCAN_SINGLE_PASS=0: two launches (range sums, then the scan) up to 6656 ranges, three (the groups' sums
+ * in between) up to 16384.  More ranges: three launches (the ranges' prefix in between).  fp32 beyond 33.5 M is cut
+ * into ranges of 16384 elements, int64 beyond 16.8 M into 8192, or 4096 where it takes several launches.  The result
+ * is bit-identical in all cases and on every run.  Replaces
  * gear::cuda::launch_prefix_sum /
  * one_dimension_prefix_sum (src/cuda/one_dim_prefix_sum.cu:125-273; libgear.core.prefix_sum,
  * :276-278), which is fp32 and only correct for one block.
@@ -345,9 +348,10 @@ int gear_hip_upper_bound_i64(const int64_t *prefix, int64_t n, const void *u, in
  * call draws itself: the numbers that torch's GPU generator of this seed and offset gives to one rand
  * (float32) or randint (int64) call of `num` elements (Philox4x32-10; the caller advances the offset by 4).
  * num <= gear_hip_draw_max() -- as many as the current GPU holds threads at once, gear_hip_draw_max_of(its compute
- * units, threads apiece): torch numbers the elements of larger calls in another way --, bound <= gear_hip_draw_max_bound() (2^28 - 1: from 2^28 on torch's randint takes
- * two words a draw), else GEAR_HIP_ERANGE.  They take the place of the torch.randint
- * and torch.multinomial of gear/sampler/global_sampler.py:121-199. */
+ * units, threads apiece): torch numbers the elements of larger calls in another way --,
+ * bound <= gear_hip_draw_max_bound() (2^28 - 1: from 2^28 on torch's randint takes two words a draw), else
+ * GEAR_HIP_ERANGE.  They take the place of the torch.randint and torch.multinomial of
+ * gear/sampler/global_sampler.py:121-199. */
 int64_t gear_hip_draw_max(void);
 int64_t gear_hip_draw_max_of(int compute_units, int threads_per_unit);
 int64_t gear_hip_draw_max_bound(void);
