@@ -59,6 +59,8 @@ bool one_launch(const int64_t *kin, int64_t *kout, const int64_t *vin, int64_t *
 // of them in every workgroup (20 000 in order: 12.4 us behind 4.7 for the look-up).  The look-up sees a
 // neighbour for the price of another load, so it says so, workgroup by workgroup, and stores its
 // entries where they belong if all of them say so; the sort looks at those words and ends (4.0 + 2.8 us).
+// Entries in no order pay for the look: 4096 / 5000 / 20 000 in 14.1 / 12.7 / 21.6 us by look-up and sort, 15.0 / 13.9 /
+// 22.2 so, where those in order take 14.1 / 12.7 / 14.3 and 10.4 / 9.4 / 9.6.
 // Beyond what one launch sorts nobody looks at such words: an ordinary look-up then, and the sort.
 constexpr int kTakeBlock = 256;
 struct Taken : Src<uint64_t> {
